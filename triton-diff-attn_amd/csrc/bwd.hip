@@ -169,10 +169,10 @@ __global__ __launch_bounds__(256) void bwd_dlambda_kernel(const float* __restric
   }
 
 // ------------------------------------------------------------------------------------------------
-template <int D, int NWAVES = 4>
+template <int D>
 struct DkvCfg {
   static constexpr int DV = 2 * D;
-  static constexpr int NW = NWAVES;            // waves per workgroup, 32 keys each (2: half-size key blocks for small grids)
+  static constexpr int NW = 4;                 // waves per workgroup, 32 keys each
   static constexpr int NT = NW * 64;
   static constexpr int BK = NW * 32;           // keys per workgroup
   static constexpr int BQ = (D <= 64) ? 64 : 32;  // query rows per staged tile
@@ -191,6 +191,7 @@ struct DkvCfg {
   static constexpr int NBUF = 4;
   static constexpr int XBASE = NBUF * QBUF, SBASE = XBASE + NBUF * XBUF;
   static_assert(NBUF * QBUF <= 65536 && NBUF * XBUF <= 65536, "immediate offsets reach every buffer");
+  static constexpr int SMEM = NBUF * STAGE;
 };
 
 // dK_t and dV for one block of keys.  Products are formed as [queries x keys] so that a lane owns
@@ -206,16 +207,13 @@ struct DkvCfg {
 // PADDED: rows n_keys..N-1 are padding.  As queries they read the last real row of Q1 and Q2 (the row the
 // forward used for their logsumexp) and carry dX = 0; as keys they read the last real row of K1, K2, V and
 // their results are not stored.
-template <int D, int MODE, bool CAUSAL, bool DROP, bool PADDED, int NWAVES = 4>
-__global__ __launch_bounds__((DkvCfg<D, NWAVES>::NT)) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dkdv_kernel(BwdParams p) {
-  using C = DkvCfg<D, NWAVES>;
+// The block is number `wg` of `n_wg`; smem: DkvCfg::SMEM halfs of tile memory.
+template <int D, int MODE, bool CAUSAL, bool DROP, bool PADDED>
+__device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg, lds_half* smem) {
+  using C = DkvCfg<D>;
   constexpr int DV = C::DV, NW = C::NW, BK = C::BK, BQ = C::BQ;
   constexpr int NKS = D / 16, NKV = DV / 16, NDT = D / 32, NVT = DV / 32;
   constexpr bool DO_V = (MODE != 2), DO_K = (MODE != 1);
-
-  __shared__ __attribute__((aligned(16))) half_t smem[C::NBUF * C::STAGE];
-  static_assert(sizeof(smem) >= 256 * sizeof(float), "the hosted reduction uses the tile memory");
-  DA_HOST_DLAMBDA(smem)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -224,10 +222,10 @@ __global__ __launch_bounds__((DkvCfg<D, NWAVES>::NT)) __attribute__((amdgpu_wave
   const int n_kt = p.N / BK;
   int bh, kt;
   if constexpr (CAUSAL) {   // the first key block of a unit is seen by the most queries
-    const UnitBlock ub = longest_first(blockIdx.x, p.BH);
+    const UnitBlock ub = longest_first(wg, p.BH);
     bh = ub.unit; kt = ub.rank;
   } else {
-    const int tile = xcd_remap(blockIdx.x, gridDim.x - p.dlam_fold);
+    const int tile = xcd_remap(wg, n_wg);
     bh = tile / n_kt; kt = tile % n_kt;
   }
   const size_t rows = (size_t)p.BH * p.N;
@@ -293,8 +291,8 @@ __global__ __launch_bounds__((DkvCfg<D, NWAVES>::NT)) __attribute__((amdgpu_wave
   constexpr int XH = (XTile::PER + 1) / 2;
 
   auto stage = [&](int qt, int buf, int part) {
-    half_t* bq = smem + buf * (C::QBUF / 2);
-    half_t* bx = smem + (C::XBASE + buf * C::XBUF) / 2;
+    lds_half* bq = smem + buf * (C::QBUF / 2);
+    lds_half* bx = smem + (C::XBASE + buf * C::XBUF) / 2;
     // dX and the statistics come from the workspace, which has all N rows; Q1 and Q2 have n_keys
     const bool past_end = PADDED && (qt + 1) * BQ > p.n_keys;
     if (part == 0) {
@@ -318,7 +316,7 @@ __global__ __launch_bounds__((DkvCfg<D, NWAVES>::NT)) __attribute__((amdgpu_wave
   // different function of the lane for every 16-byte chunk column, so there is one register per chunk
   // column a lane ever reads; everything else (ring buffer, Q1 or Q2, sub-tile, k-step of 16 rows) is a
   // multiple of 16 rows, which the swizzle does not see, and travels in the instruction's immediate offset.
-  const unsigned lds0 = (unsigned)(unsigned long)((DA_LDS char*)smem);
+  const unsigned lds0 = (unsigned)(unsigned long)smem;
   unsigned qb[NKS], xb[NKV], qtr[NDT][2], xtr[NVT][2], stb;
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) qb[ks] = lds0 + 2u * (unsigned)swz_off<D>(j, 16 * ks + 8 * g);
@@ -608,8 +606,8 @@ __global__ __launch_bounds__((DkvCfg<D, NWAVES>::NT)) __attribute__((amdgpu_wave
   const int b0 = head_half ? NBUF / 2 : 0;          // buffer of the first tile
   {
     const int bz = (b0 + NBUF - 1) % NBUF;          // the buffer in front of the first tile's
-    u32x4* zq = reinterpret_cast<u32x4*>(smem + bz * (C::QBUF / 2));
-    u32x4* zx = reinterpret_cast<u32x4*>(smem + (C::XBASE + bz * C::XBUF) / 2);
+    DA_LDS u32x4* zq = (DA_LDS u32x4*)(smem + bz * (C::QBUF / 2));
+    DA_LDS u32x4* zx = (DA_LDS u32x4*)(smem + (C::XBASE + bz * C::XBUF) / 2);
     for (int k = tid; k < C::QBUF / 16; k += C::NT) zq[k] = u32x4{0u, 0u, 0u, 0u};
     for (int k = tid; k < C::XBUF / 16; k += C::NT) zx[k] = u32x4{0u, 0u, 0u, 0u};
   }
@@ -703,14 +701,22 @@ __global__ __launch_bounds__((DkvCfg<D, NWAVES>::NT)) __attribute__((amdgpu_wave
   }
 }
 
+template <int D, int MODE, bool CAUSAL, bool DROP, bool PADDED>
+__global__ __launch_bounds__(DkvCfg<D>::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dkdv_kernel(BwdParams p) {
+  __shared__ __attribute__((aligned(16))) half_t smem[DkvCfg<D>::SMEM];
+  static_assert(sizeof(smem) >= 256 * sizeof(float), "the hosted reduction uses the tile memory");
+  DA_HOST_DLAMBDA(smem)
+  dkdv_block<D, MODE, CAUSAL, DROP, PADDED>(p, blockIdx.x, gridDim.x - p.dlam_fold, (lds_half*)smem);
+}
+
 // ------------------------------------------------------------------------------------------------
-template <int D, int NWAVES>
+template <int D, int NWAVES, bool PIPE>
 struct DqCfg {
   static constexpr int DV = 2 * D;
   static constexpr int NW = NWAVES;            // waves per workgroup, 32 query rows each
   // waves per SIMD the register budget is sized for: the resident Q1, Q2, dX rows and the two dQ
   // accumulators of a D = 128 wave do not fit 256 registers
-  static constexpr int OCC = (D == 128) ? 1 : 2;
+  static constexpr int OCC = (D == 128 || PIPE) ? 1 : 2;
   static constexpr int NT = NW * 64;
   // thread count the register budget is derived from: with fewer than 4 * OCC waves in a workgroup
   // the occupancy attribute alone does not hold the allocator to 512 / OCC registers
@@ -731,6 +737,7 @@ struct DqCfg {
   static constexpr int NBUF = 4;
   static constexpr int KBUF_BYTES = 2 * K_TILE * 2, VBUF_BYTES = V_TILE * 2, VBASE_BYTES = NBUF * KBUF_BYTES;
   static_assert(NBUF * KBUF_BYTES <= 65536 && NBUF * VBUF_BYTES <= 65536, "immediate offsets reach every buffer");
+  static constexpr int SMEM = NBUF * STAGE;
 };
 
 // dQ_t = s * dS_t K_t for one block of query rows.  Every product is formed transposed,
@@ -740,26 +747,17 @@ struct DqCfg {
 // A padded key has a zero K row, but its recomputed "probability" exp(0 - lse) is not small when a
 // row's logsumexp is negative, and its dS can overflow fp16: it must be masked, not multiplied by 0.
 // DROP: dropout on both softmax maps, as in bwd_dkdv_kernel.
-template <int D, int NWAVES, int MASK, bool DROP>
-__global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_waves_per_eu(DqCfg<D, NWAVES>::OCC, DqCfg<D, NWAVES>::OCC))) void bwd_dq_kernel(BwdParams p) {
-  using C = DqCfg<D, NWAVES>;
+// PIPE: one wave per SIMD, pipelined inside the wave.  The block is number `wg` of `n_wg`; smem: DqCfg::SMEM halfs.
+template <int D, int NWAVES, int MASK, bool DROP, bool PIPE>
+__device__ __forceinline__ void dq_block(const BwdParams& p, int wg, int n_wg, lds_half* smem) {
+  using C = DqCfg<D, NWAVES, PIPE>;
   constexpr bool CAUSAL = (MASK == 1), PADDED = (MASK == 2);
   // rows past the real length are neither read from the caller's tensors nor written to the gradients: checked
   // in both masked variants (the causal one serves padded sequences too), compiled out of the plain one
   constexpr bool TAIL = (MASK != 0);
   constexpr int DV = C::DV, NW = C::NW, BM = C::BM, BN = C::BN;
   constexpr int NKS = D / 16, NKV = DV / 16, NDT = D / 32;
-#ifndef DQ_ASM_SCORES
-#define DQ_ASM_SCORES (D == 128 && !DROP)
-#endif
-#ifndef DQ_PIPE
-#define DQ_PIPE (D == 128 && !DROP)
-#endif
-  constexpr bool kPipe = DQ_PIPE;     // the software-pipelined loop of the one-wave-per-SIMD kernel, below
-
-  __shared__ __attribute__((aligned(16))) half_t smem[C::NBUF * C::STAGE];
-  static_assert(sizeof(smem) >= 256 * sizeof(float), "the hosted reduction uses the tile memory");
-  DA_HOST_DLAMBDA(smem)
+  constexpr bool kPipe = PIPE;     // the software-pipelined loop of the one-wave-per-SIMD kernel, below
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -768,10 +766,10 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
   const int n_qt = p.N / BM;
   int bh, qt;
   if constexpr (CAUSAL) {   // the last query block of a unit sees the most keys
-    const UnitBlock ub = longest_first(blockIdx.x, p.BH);
+    const UnitBlock ub = longest_first(wg, p.BH);
     bh = ub.unit; qt = n_qt - 1 - ub.rank;
   } else {
-    const int tile = xcd_remap(blockIdx.x, gridDim.x - p.dlam_fold);
+    const int tile = xcd_remap(wg, n_wg);
     bh = tile / n_qt; qt = tile % n_qt;
   }
   const size_t rows = (size_t)p.BH * p.N;
@@ -832,11 +830,11 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
   // loads a wave issues per iteration (one K1, one K2 and one V tile)
   const int loads_per_iter = 2 * KTile::count(wave) + VTile::count(wave);
   // with padding, the tiles that reach past the last real key are copied with their row index clamped to it
-  auto copy_k = [&](const half_t* gk, int t, half_t* dst) {
+  auto copy_k = [&](const half_t* gk, int t, lds_half* dst) {
     if (TAIL && (t + 1) * BN > p.n_keys) KTile::issue_clamped(gk + (size_t)t * BN * qk_n, dst, wave, lane, k_off, qk_n, p.n_keys - 1 - t * BN);
     else KTile::issue_at(gk + (size_t)t * BN * qk_n, dst, wave, lane, k_off, qk_n);
   };
-  auto copy_v = [&](int t, half_t* dst, auto k0_tag, auto k1_tag) {
+  auto copy_v = [&](int t, lds_half* dst, auto k0_tag, auto k1_tag) {
     constexpr int K0 = decltype(k0_tag)::value, K1 = decltype(k1_tag)::value;
     if (TAIL && (t + 1) * BN > p.n_keys) VTile::template issue_clamped<K0, K1>(gv + (size_t)t * BN * v_n, dst, wave, lane, v_off, v_n, p.n_keys - 1 - t * BN);
     else VTile::template issue_at<K0, K1>(gv + (size_t)t * BN * v_n, dst, wave, lane, v_off, v_n);
@@ -864,14 +862,13 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
   // used.  It does not see the asynchronous tile copies, so its wait for "the newest loads" would in fact be a
   // wait for every tile copy in flight, in every iteration.  Touching the registers here puts that wait in front
   // of the loop, where the first tiles are waited for anyway.
-  // At D = 128 the kernel runs one wave per SIMD, and for a kernel with that register budget the compiler selects
+  // The pipelined form runs one wave per SIMD, and for a kernel with that register budget the compiler selects
   // every MFMA with its C and D operands in AGPRs: right for the dQ accumulators, but each recomputed score
   // and dP value then costs a copy back for the element-wise work (a quarter of the loop's VALU instructions).
   // There the three score products are issued as assembly with their results in VGPRs and the resident
   // Q1, Q2 and dX rows, which are only ever B operands, in AGPRs.  (Not in the dropout instantiations, whose
   // mask arithmetic makes the compiler move operands about: see bwd_dkdv_kernel.)
-  constexpr bool kAsmScores = DQ_ASM_SCORES;
-  if constexpr (kAsmScores) {
+  if constexpr (kPipe) {
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) { keep_in_agpr(qf1[ks]); keep_in_agpr(qf2[ks]); }
 #pragma unroll
@@ -892,7 +889,7 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
   // which the swizzle does not see, and travel in the instructions' immediate offsets.
   const int tr_row = 4 * g + ((lane & 15) >> 2);
   const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  const unsigned lds0 = (unsigned)(unsigned long)((DA_LDS char*)smem);
+  const unsigned lds0 = (unsigned)(unsigned long)smem;
   unsigned kfr[NKS], vfr[NKV], ktr[NDT][2];
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) kfr[ks] = lds0 + 2u * (unsigned)swz_off<D>(j, 16 * ks + 8 * g);
@@ -912,14 +909,8 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
 
   // Where registers allow, a row statistic that is added to every element of a product is the product's
   // initial accumulator value instead: sixteen registers that hold it, for sixteen additions less per sub-tile.
-#ifndef DQ_FOLD_DP
-#define DQ_FOLD_DP (!DROP && (D == 32 || (D == 64 && MASK == 0)))
-#endif
-#ifndef DQ_FOLD_S
-#define DQ_FOLD_S (D == 32)
-#endif
-  constexpr bool kFoldDP = DQ_FOLD_DP;     // dP starts from -delta1 (not with dropout, which masks dP first)
-  constexpr bool kFoldS = DQ_FOLD_S;       // S1, S2 start from the negated logsumexp
+  constexpr bool kFoldDP = !DROP && (D == 32 || (D == 64 && (MASK == 0 || PIPE)));     // dP starts from -delta1 (not with dropout, which masks dP first)
+  constexpr bool kFoldS = (D == 32);       // S1, S2 start from the negated logsumexp
   f16v de1v, nl1v, nl2v;
 #pragma unroll
   for (int r = 0; r < 16; ++r) { de1v[r] = kFoldDP ? de1 : 0.f; nl1v[r] = kFoldS ? nl1 : 0.f; nl2v[r] = kFoldS ? nl2 : 0.f; }
@@ -928,33 +919,37 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
 
   if constexpr (kPipe) {
     // One wave per SIMD has nobody to run its element-wise work under, so the loop is pipelined inside the wave,
-    // as in the dK/dV kernel: while the element-wise work of tile t runs on the VALU, row by row, the score
-    // products of tile t+1 (assembly, results in VGPRs) run on the matrix unit, two per row; the dQ products
-    // of tile t follow.  Tiles are 32 keys (one sub-tile) and are fetched three iterations ahead; the workgroup
-    // meets once per tile.
-    static_assert(kAsmScores && BN == 32 && !kFoldDP && !kFoldS, "the pipelined loop");
+    // as in the dK/dV kernel: while the element-wise work of 32-key sub-tile i runs on the VALU, row by row, the
+    // score products of sub-tile i+1 (assembly, results in VGPRs) run on the matrix unit; the dQ products of
+    // sub-tile i follow.  The workgroup meets once per tile, in the step that scores the tile's first sub-tile; that
+    // step requests the tile after the next.
     struct Scores { f16v s1, s2, dp; };
-    constexpr int NPROD = 2 * NKS + NKV;              // score products per tile: S1 and S2 alternating, then dP
-    // A fragment of product k of the tile in the buffer at byte offsets (KOFF, VOFF)
+    constexpr int SPT = BN / 32, RING = SPT * C::NBUF, HALF = RING / 2;   // sub-tiles per tile, steps per turn of the ring
+    constexpr int NPROD = 2 * NKS + NKV;              // score products per sub-tile: S1 and S2 alternating, then dP
+    // A fragment of product k of the sub-tile at byte offsets (KOFF, VOFF)
     auto prod_frag = [&](auto koff_tag, auto voff_tag, int k) -> h8 {
       constexpr int KOFF = decltype(koff_tag)::value, VOFF = decltype(voff_tag)::value;
       if (k < 2 * NKS) return lds_read_at<h8>(kfr[k / 2], KOFF + (k & 1) * C::K_TILE * 2);
       return lds_read_at<h8>(vfr[k - 2 * NKS], VOFF);
     };
     auto prod_mfma = [&](int k, h8 a, Scores& s) {
-      if (k < 2 * NKS) {
+      if (k < 2) {
+        if (k) s.s2 = kFoldS ? mfma32_bagpr_from(a, qf2[0], nl2v) : mfma32_bagpr_first(a, qf2[0]);
+        else   s.s1 = kFoldS ? mfma32_bagpr_from(a, qf1[0], nl1v) : mfma32_bagpr_first(a, qf1[0]);
+      } else if (k < 2 * NKS) {
         const int ks = k / 2;
-        if (k & 1) s.s2 = ks ? mfma32_bagpr(a, qf2[ks], s.s2) : mfma32_bagpr_first(a, qf2[0]);
-        else       s.s1 = ks ? mfma32_bagpr(a, qf1[ks], s.s1) : mfma32_bagpr_first(a, qf1[0]);
+        if (k & 1) s.s2 = mfma32_bagpr(a, qf2[ks], s.s2);
+        else       s.s1 = mfma32_bagpr(a, qf1[ks], s.s1);
+      } else if (k == 2 * NKS) {
+        s.dp = kFoldDP ? mfma32_bagpr_from(a, xf[0], de1v) : mfma32_bagpr_first(a, xf[0]);
       } else {
-        const int kv = k - 2 * NKS;
-        s.dp = kv ? mfma32_bagpr(a, xf[kv], s.dp) : mfma32_bagpr_first(a, xf[0]);
+        s.dp = mfma32_bagpr(a, xf[k - 2 * NKS], s.dp);
       }
     };
     constexpr int DEPTH = 4;                          // A fragments requested ahead of their product
     Scores sa, sb;
     {
-      // scores of tile 0, nothing to run them under
+      // scores of sub-tile 0, nothing to run them under
       h8 a[NPROD];
       if (head_half) {
 #pragma unroll
@@ -969,18 +964,24 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
       mfma_results_ready(sa.s1, sa.s2, sa.dp);
     }
 
-    auto iteration = [&](int t, auto pos_tag, Scores& cur, Scores& nxt) {
-      constexpr int POS = decltype(pos_tag)::value;
-      constexpr int KCUR = POS * C::KBUF_BYTES;
-      constexpr int PNXT = (POS + 1) % C::NBUF, BFAR = (POS + 3) % C::NBUF;
-      constexpr std::integral_constant<int, PNXT * C::KBUF_BYTES> knext{};
-      constexpr std::integral_constant<int, PNXT * C::VBUF_BYTES> vnext{};
-      const int tf = (t + 3 < n_tiles) ? t + 3 : n_tiles - 1;   // past the end: harmless re-reads
-      copy_k(gk1, tf, k_buf(BFAR));
+    auto step = [&](int i, auto pos_tag, Scores& cur, Scores& nxt) {
+      constexpr int POS = decltype(pos_tag)::value, PNXT = (POS + 1) % RING;
+      constexpr int BNXT = PNXT / SPT, BFAR = (BNXT + 2) % C::NBUF;
+      constexpr bool opens = (PNXT % SPT) == 0;       // this step scores the first sub-tile of a tile
+      constexpr int KCUR = (POS / SPT) * C::KBUF_BYTES + (POS % SPT) * 32 * D * 2;
+      constexpr std::integral_constant<int, BNXT * C::KBUF_BYTES + (PNXT % SPT) * 32 * D * 2> knext{};
+      constexpr std::integral_constant<int, BNXT * C::VBUF_BYTES + (PNXT % SPT) * 32 * DV * 2> vnext{};
+      const int t3 = i / SPT + 3, tf = t3 < n_tiles ? t3 : n_tiles - 1;   // past the end: harmless re-reads
+      if constexpr (opens) {
+        // that tile has landed for everybody, and every wave is done with the tile whose buffer is refilled now
+        wait_async_tiles_except(loads_per_iter);
+        __syncthreads();
+        copy_k(gk1, tf, k_buf(BFAR));
+      }
       if constexpr (CAUSAL) {
-        // only the last tiles of a wave's loop reach past its first row: mask key > query there
+        // only the last sub-tiles of a wave's loop reach past its first row: mask key > query there
         const int wrow0 = qt * BM + wave * 32;
-        const int kbase = t * BN;
+        const int kbase = i * 32;
         if (kbase + 31 > wrow0) {
           const int rel = wrow0 + j - kbase - 4 * g;     // query index minus the key index of register 0
 #pragma unroll
@@ -989,7 +990,7 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
         }
       }
       if constexpr (PADDED) {
-        const int kbase = t * BN;
+        const int kbase = i * 32;
         if (kbase + 32 > p.n_keys) {
           const int rel = p.n_keys - 1 - kbase - 4 * g;   // last real key minus the key index of register 0
 #pragma unroll
@@ -997,7 +998,7 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
             if (8 * (r / 4) + (r % 4) > rel) { cur.s1[r] = -INFINITY; cur.s2[r] = -INFINITY; }
         }
       }
-      // the transposed K fragments of this tile's dQ products are requested here and arrive under the loop below
+      // the transposed K fragments of this sub-tile's dQ products are requested here and arrive under the loop below
       h8 tk1[2][NDT], tk2[2][NDT];
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
@@ -1016,24 +1017,24 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
       for (int k = 0; k < NPROD; ++k) {
         if (k + DEPTH < NPROD) a[k + DEPTH] = prod_frag(knext, vnext, k + DEPTH);
         // the far tile's copies are spread over the products
-        if (k == NPROD / 4) copy_k(gk2, tf, k_buf(BFAR) + C::K_TILE);
-        if (k == NPROD / 2) copy_v(tf, v_buf(BFAR), v_begin, v_mid);
-        if (k == 3 * NPROD / 4) copy_v(tf, v_buf(BFAR), v_mid, v_end);
+        if (opens && k == NPROD / 4) copy_k(gk2, tf, k_buf(BFAR) + C::K_TILE);
+        if (opens && k == NPROD / 2) copy_v(tf, v_buf(BFAR), v_begin, v_mid);
+        if (opens && k == 3 * NPROD / 4) copy_v(tf, v_buf(BFAR), v_mid, v_end);
         prod_mfma(k, a[k], nxt);
-        // element-wise rows of this tile, spread evenly over the products
+        // element-wise rows of this sub-tile, spread evenly over the products
         const int r0 = 16 * k / NPROD, r1 = 16 * (k + 1) / NPROD;
 #pragma unroll
         for (int r = r0; r < r1; ++r) {
-          const float p1 = fast_exp2(cur.s1[r] + nl1);
-          const float p2 = fast_exp2(cur.s2[r] + nl2);
+          const float p1 = fast_exp2(kFoldS ? cur.s1[r] : cur.s1[r] + nl1);
+          const float p2 = fast_exp2(kFoldS ? cur.s2[r] : cur.s2[r] + nl2);
           // in fp32 up to the rounding of dS itself (see the loop of the other head dims)
-          const float dpc = cur.dp[r] + de1;
+          const float dpc = kFoldDP ? cur.dp[r] : cur.dp[r] + de1;
           b1[r / 8][r % 8] = (half_t)(p1 * dpc);
           b2[r / 8][r % 8] = (half_t)(p2 * __builtin_fmaf(-lam, dpc, de2));
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      mfma_results_ready(nxt.s1, nxt.s2, nxt.dp);     // the next iteration's VALU reads them
+      mfma_results_ready(nxt.s1, nxt.s2, nxt.dp);     // the next step's VALU reads them
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -1041,23 +1042,27 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
           dq1[tt] = mfma32(tk1[kk][tt], b1[kk], dq1[tt]);
           dq2[tt] = mfma32(tk2[kk][tt], b2[kk], dq2[tt]);
         }
-      // the next iteration reads tiles t+1 and t+2: only this iteration's loads (tile t+3) may remain in flight
-      wait_async_tiles_except(loads_per_iter);
-      __syncthreads();
     };
 
-    int t = 0;
+    auto half_turn = [&](int i, auto h0_tag) {
+      constexpr int H0 = decltype(h0_tag)::value;
+      step(i, std::integral_constant<int, H0>{}, sa, sb);
+      step(i + 1, std::integral_constant<int, H0 + 1>{}, sb, sa);
+      if constexpr (HALF == 4) {
+        step(i + 2, std::integral_constant<int, H0 + 2>{}, sa, sb);
+        step(i + 3, std::integral_constant<int, H0 + 3>{}, sb, sa);
+      }
+    };
+    const int n_steps = n_tiles * SPT;
+    int i = 0;
     if (head_half) {
-      iteration(0, std::integral_constant<int, 2>{}, sa, sb);
-      iteration(1, std::integral_constant<int, 3>{}, sb, sa);
-      t = 2;
+      half_turn(0, std::integral_constant<int, HALF>{});
+      i = HALF;
     }
 #pragma nounroll
-    for (; t < n_tiles; t += 4) {
-      iteration(t, std::integral_constant<int, 0>{}, sa, sb);
-      iteration(t + 1, std::integral_constant<int, 1>{}, sb, sa);
-      iteration(t + 2, std::integral_constant<int, 2>{}, sa, sb);
-      iteration(t + 3, std::integral_constant<int, 3>{}, sb, sa);
+    for (; i < n_steps; i += RING) {
+      half_turn(i, std::integral_constant<int, 0>{});
+      half_turn(i + HALF, std::integral_constant<int, HALF>{});
     }
   } else {
   // One iteration: tile t, in the buffer at ring position POS; tile t+2 is requested into the buffer two
@@ -1083,32 +1088,13 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
 #pragma unroll
       for (int kv = 0; kv < NKV; ++kv) av[kv] = lds_read_at<h8>(vfr[kv], VCUR + ksub * 32 * DV * 2);
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kAsmScores) {
-        if constexpr (kFoldS) {
-          s1 = mfma32_bagpr_from(ak1[0], qf1[0], nl1v);
-          s2 = mfma32_bagpr_from(ak2[0], qf2[0], nl2v);
-        } else {
-          s1 = mfma32_bagpr_first(ak1[0], qf1[0]);
-          s2 = mfma32_bagpr_first(ak2[0], qf2[0]);
-        }
 #pragma unroll
-        for (int ks = 1; ks < NKS; ++ks) {
-          s1 = mfma32_bagpr(ak1[ks], qf1[ks], s1);
-          s2 = mfma32_bagpr(ak2[ks], qf2[ks], s2);
-        }
-        dp = kFoldDP ? mfma32_bagpr_from(av[0], xf[0], de1v) : mfma32_bagpr_first(av[0], xf[0]);
-#pragma unroll
-        for (int kv = 1; kv < NKV; ++kv) dp = mfma32_bagpr(av[kv], xf[kv], dp);
-        mfma_results_ready(s1, s2, dp);      // the compiler does not know these are matrix instructions
-      } else {
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          s1 = mfma32(ak1[ks], qf1[ks], s1);
-          s2 = mfma32(ak2[ks], qf2[ks], s2);
-        }
-#pragma unroll
-        for (int kv = 0; kv < NKV; ++kv) dp = mfma32(av[kv], xf[kv], dp);
+      for (int ks = 0; ks < NKS; ++ks) {
+        s1 = mfma32(ak1[ks], qf1[ks], s1);
+        s2 = mfma32(ak2[ks], qf2[ks], s2);
       }
+#pragma unroll
+      for (int kv = 0; kv < NKV; ++kv) dp = mfma32(av[kv], xf[kv], dp);
       if (ksub == 0) copy_v(tn, v_buf(BNXT), v_begin, v_mid);
       // with a barrier every second tile all of a tile's copies go out early: they have to land by the next barrier
       if (ksub == (C::PAIR ? 0 : BN / 32 - 1)) copy_v(tn, v_buf(BNXT), v_mid, v_end);
@@ -1144,9 +1130,7 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
         tk1[kk][tt] = join(lds_read_tr_at(ktr[tt][0], off), lds_read_tr_at(ktr[tt][1], off));
         tk2[kk][tt] = join(lds_read_tr_at(ktr[tt][0], off + C::K_TILE * 2), lds_read_tr_at(ktr[tt][1], off + C::K_TILE * 2));
       };
-      // (At D = 128 the masked variants, which also carry the row clamping of padded sequences, are short of
-      // registers in the same way.)
-      constexpr bool kFragmentsAhead = !DROP && !(D == 128 && TAIL);
+      constexpr bool kFragmentsAhead = !DROP;
       if constexpr (kFragmentsAhead) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
@@ -1232,7 +1216,7 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
   // that the global stores are whole 16-byte chunks of consecutive rows.
   constexpr int SROW = D + 8;
   static_assert(NW * 2 * 32 * SROW <= C::NBUF * C::STAGE, "staging blocks fit the tile memory");
-  half_t* const stg = smem + (size_t)wave * 2 * 32 * SROW;
+  lds_half* const stg = smem + (size_t)wave * 2 * 32 * SROW;
 #pragma unroll
   for (int tt = 0; tt < NDT; ++tt)
 #pragma unroll
@@ -1243,8 +1227,8 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
         v1[e] = (half_t)(dq1[tt][4 * r4 + e] * p.sm_scale);
         v2[e] = (half_t)(dq2[tt][4 * r4 + e] * p.sm_scale);
       }
-      *reinterpret_cast<h4*>(stg + j * SROW + 32 * tt + 8 * r4 + 4 * g) = v1;
-      *reinterpret_cast<h4*>(stg + (32 + j) * SROW + 32 * tt + 8 * r4 + 4 * g) = v2;
+      *(DA_LDS h4*)(stg + j * SROW + 32 * tt + 8 * r4 + 4 * g) = v1;
+      *(DA_LDS h4*)(stg + (32 + j) * SROW + 32 * tt + 8 * r4 + 4 * g) = v2;
     }
   __builtin_amdgcn_wave_barrier();   // the rows are read back by other lanes of this wave only
   constexpr int LPR = D / 8;         // lanes per row
@@ -1256,8 +1240,8 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
 #pragma unroll
   for (int k = 0; k < 32 / RPI; ++k) {
     const int row = k * RPI + lane / LPR, ch = lane % LPR;
-    const u32x4 v1 = *reinterpret_cast<const u32x4*>(stg + row * SROW + 8 * ch);
-    const u32x4 v2 = *reinterpret_cast<const u32x4*>(stg + (32 + row) * SROW + 8 * ch);
+    const u32x4 v1 = *(const DA_LDS u32x4*)(stg + row * SROW + 8 * ch);
+    const u32x4 v2 = *(const DA_LDS u32x4*)(stg + (32 + row) * SROW + 8 * ch);
     if (!TAIL || qloc0 + row < p.n_keys) {    // the gradient tensors have no rows past the real length
       *reinterpret_cast<u32x4*>(o1 + (size_t)row * (size_t)p.sdqk.n + 8 * ch) = v1;
       *reinterpret_cast<u32x4*>(o2 + (size_t)row * (size_t)p.sdqk.n + 8 * ch) = v2;
@@ -1265,19 +1249,74 @@ __global__ __launch_bounds__((DqCfg<D, NWAVES>::REG_NT)) __attribute__((amdgpu_w
   }
 }
 
-// ------------------------------------------------------------------------------------------------
+template <int D, int NWAVES, int MASK, bool DROP>
+__global__ __launch_bounds__((DqCfg<D, NWAVES, false>::REG_NT)) __attribute__((amdgpu_waves_per_eu(DqCfg<D, NWAVES, false>::OCC, DqCfg<D, NWAVES, false>::OCC)))
+void bwd_dq_kernel(BwdParams p) {
+  using C = DqCfg<D, NWAVES, false>;
+  __shared__ __attribute__((aligned(16))) half_t smem[C::SMEM];
+  static_assert(sizeof(smem) >= 256 * sizeof(float), "the hosted reduction uses the tile memory");
+  DA_HOST_DLAMBDA(smem)
+  dq_block<D, NWAVES, MASK, DROP, false>(p, blockIdx.x, gridDim.x - p.dlam_fold, (lds_half*)smem);
+}
+
+// dK/dV blocks and dQ blocks in one grid: the two have nothing to wait for in each other, and as launches of their
+// own each leaves the CUs that its last (or only) round of workgroups does not reach idle.  All blocks are four
+// waves at one wave per SIMD, the long ones first: p.n_kv_wg key blocks (at D = 128 twice, for dK and for dV), then
+// p.n_q_wg query blocks.  Measured against separate launches (whole backward, N(0,1) fp16): B1 H16 N128 D128 49 -> 25 us,
+// B2 H16 N512 D64 48 -> 33, B1 H8 N2048 D64 121 -> 80 (causal 134 -> 73), B1 H12 N3584 D128 848 -> 648,
+// B8 H32 N4096 D128 18.5 -> 18.3 ms.
+template <int D, bool CAUSAL, bool PADDED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_pair_kernel(BwdParams p) {
+  constexpr int SK = DkvCfg<D>::SMEM, SQ = DqCfg<D, 4, true>::SMEM;
+  static_assert(DkvCfg<D>::NT == 256, "both kinds of blocks have four waves");
+  __shared__ __attribute__((aligned(16))) half_t smem[SK > SQ ? SK : SQ];
+  DA_HOST_DLAMBDA(smem)
+  int wg = blockIdx.x;
+  const int n_kv = p.n_kv_wg;
+  if (wg < n_kv) {
+    dkdv_block<D, D == 128 ? 2 : 0, CAUSAL, false, PADDED>(p, wg, n_kv, (lds_half*)smem);
+    return;
+  }
+  wg -= n_kv;
+  if constexpr (D == 128) {
+    if (wg < n_kv) {
+      dkdv_block<D, 1, CAUSAL, false, PADDED>(p, wg, n_kv, (lds_half*)smem);
+      return;
+    }
+    wg -= n_kv;
+  }
+  dq_block<D, 4, CAUSAL ? 1 : PADDED ? 2 : 0, false, true>(p, wg, p.n_q_wg, (lds_half*)smem);
+}
+
+// Whether a backward goes into one grid (bwd_pair_kernel) instead of a dK/dV and a dQ launch: a pure function of
+// the sizes and options.  At D = 128 always: its dQ blocks are four waves at one wave per SIMD either way.  At
+// D <= 64 the dQ kernel of its own has eight waves and 256 rows, two waves per SIMD, and is the faster one on a full chip
+// (headline size: 437 us against 510), so it is a matter of rounds.  Microseconds per round of 256 workgroups at
+// N = 2048, D = 64, which scale alike with N and D: 79 for key blocks, 64 for query blocks of this kernel, 109 for
+// 256-row blocks of the dQ kernel; a grid that is dealt from one list ends with a partial round of 25.  The line
+// holds over B*H*N/128 = 192 ... 1280 blocks: measured gains of up to 24 % on its near side, up to 6 % on its far side.
+// Causal blocks differ in length and fill the rounds by themselves: the one grid is faster below 576 blocks
+// (by 5 % at 512, 40 % at 256) and slower above 640 (by 2-5 %).
+template <int D>
+static bool one_grid(const BwdParams& p) {
+  if (p.drop.threshold) return false;      // the dropout instantiations are not pipelined
+  if (D == 128) return true;
+  const bool wide = p.N % 256 == 0;        // the dQ kernel of its own has its 256-row blocks
+  // N an odd multiple of 128: its 128-row variant has one wave per SIMD at D = 64 (LDS), and this one is pipelined
+  if (D == 64 && !wide && (p.stages & 8u)) return true;
+  const long long blocks = (long long)p.BH * (p.N / 128);
+  if ((p.stages & 12u) != 12u) return blocks <= 256;
+  if (p.causal) return blocks <= 576;
+  const long long two = 79 * ((blocks + 255) / 256) + 109 * ((blocks + 511) / 512);
+  const long long one = (D == 32 ? 150 : 143) * blocks / 256 + 25;
+  return one < two;
+}
+
 template <int D>
 static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
   BwdParams p = p_in;
   const int n_prep = bwd_num_partials(p.BH, p.N, D);
   hipError_t e = hipSuccess;
-  // Shape-aware launch geometry (the reference autotunes its tiles per (N, D, Dv), src/kernel.py:12-19): a problem
-  // whose 128-row blocks do not fill the chip once runs in twice as many 64-row workgroups.  A pure function of
-  // (B*H, N, D) and the options: no tuning state.  Only the plain dK/dV instantiation has the small variant
-  // (the dQ kernel was measured with 64-row workgroups too: 15-20 % slower on such grids, so it keeps 128).
-  constexpr int kNumCU = 256;
-  const bool small_grid = D != 128 && !p.causal && !p.drop.threshold && p.n_keys == p.N &&
-                          (long long)p.BH * (p.N / 128) < kNumCU;
   // the d(lambda) reduce rides in the first dK/dV or dQ launch when there is one, else it is a launch of its own
   const int n_lambda = p.lambda_stride ? p.H : 1;
   bool fold = (p.stages & 2u) && (p.stages & 12u);
@@ -1294,15 +1333,24 @@ static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
                        p.dlam_part, n_prep / p.BH, p.BH, p.dlambda, p.lambda_fp32);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  if ((p.stages & 4u) && small_grid) {
-    if constexpr (D != 128) {
-      p.dlam_fold = fold ? n_lambda : 0;
-      fold = false;
-      const dim3 grid(p.BH * (p.N / DkvCfg<D, 2>::BK) + p.dlam_fold), block(DkvCfg<D, 2>::NT);
-      hipLaunchKernelGGL((bwd_dkdv_kernel<D, 0, false, false, false, 2>), grid, block, 0, stream, p);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (!(p.stages & 12u)) return e;
+  const bool padded = p.n_keys < p.N;
+  if (one_grid<D>(p)) {
+    const int blocks = p.BH * (p.N / 128);
+    p.n_kv_wg = (p.stages & 4u) ? blocks : 0;
+    p.n_q_wg = (p.stages & 8u) ? blocks : 0;
+    p.dlam_fold = fold ? n_lambda : 0;
+    const dim3 grid((D == 128 ? 2 : 1) * p.n_kv_wg + p.n_q_wg + p.dlam_fold), block(256);
+    if (p.causal) {
+      if (padded) hipLaunchKernelGGL((bwd_pair_kernel<D, true, true>), grid, block, 0, stream, p);
+      else        hipLaunchKernelGGL((bwd_pair_kernel<D, true, false>), grid, block, 0, stream, p);
+    } else {
+      if (padded) hipLaunchKernelGGL((bwd_pair_kernel<D, false, true>), grid, block, 0, stream, p);
+      else        hipLaunchKernelGGL((bwd_pair_kernel<D, false, false>), grid, block, 0, stream, p);
     }
-  } else if (p.stages & 4u) {
+    return hipGetLastError();
+  }
+  if (p.stages & 4u) {
     const dim3 block(DkvCfg<D>::NT);
     auto launch_mode = [&](auto mode_tag) {
       constexpr int M = decltype(mode_tag)::value;
@@ -1314,13 +1362,13 @@ static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
         if (p.drop.threshold) {
           if (p.causal) hipLaunchKernelGGL((bwd_dkdv_kernel<D, M, true, true, PAD>), grid, block, 0, stream, p);
           else          hipLaunchKernelGGL((bwd_dkdv_kernel<D, M, false, true, PAD>), grid, block, 0, stream, p);
-        } else {
+        } else if constexpr (D != 128) {
           if (p.causal) hipLaunchKernelGGL((bwd_dkdv_kernel<D, M, true, false, PAD>), grid, block, 0, stream, p);
           else          hipLaunchKernelGGL((bwd_dkdv_kernel<D, M, false, false, PAD>), grid, block, 0, stream, p);
         }
       };
-      if (p.n_keys < p.N) launch_padded(std::true_type{});
-      else                launch_padded(std::false_type{});
+      if (padded) launch_padded(std::true_type{});
+      else        launch_padded(std::false_type{});
     };
     if constexpr (D == 128) {
       launch_mode(std::integral_constant<int, 1>{});
@@ -1336,36 +1384,30 @@ static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
     // runs one wave per SIMD and therefore always has four waves).  A grid so small that even its
     // 128-row workgroups all fit on the chip at once is launched that way too: it finishes sooner
     // in twice as many, half as long workgroups.
-    bool wide = false;
-    auto launch_dq = [&](auto nw_tag, dim3 grid, dim3 block) {
+    auto launch_dq = [&](auto nw_tag) {
       constexpr int NWV = decltype(nw_tag)::value;
       p.dlam_fold = fold ? n_lambda : 0;
       fold = false;
-      grid.x += p.dlam_fold;
+      const dim3 grid(p.BH * (p.N / (32 * NWV)) + p.dlam_fold), block(64 * NWV);
       if (p.drop.threshold) {
-        if (p.causal)            hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 1, true>), grid, block, 0, stream, p);
-        else if (p.n_keys < p.N) hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 2, true>), grid, block, 0, stream, p);
-        else                     hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 0, true>), grid, block, 0, stream, p);
-      } else {
-        if (p.causal)            hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 1, false>), grid, block, 0, stream, p);
-        else if (p.n_keys < p.N) hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 2, false>), grid, block, 0, stream, p);
-        else                     hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 0, false>), grid, block, 0, stream, p);
+        if (p.causal)    hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 1, true>), grid, block, 0, stream, p);
+        else if (padded) hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 2, true>), grid, block, 0, stream, p);
+        else             hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 0, true>), grid, block, 0, stream, p);
+      } else if constexpr (D == 32 || (D == 64 && NWV == 8)) {      // the others go into one grid
+        if (p.causal)    hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 1, false>), grid, block, 0, stream, p);
+        else if (padded) hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 2, false>), grid, block, 0, stream, p);
+        else             hipLaunchKernelGGL((bwd_dq_kernel<D, NWV, 0, false>), grid, block, 0, stream, p);
       }
     };
-    if constexpr (D != 128) {
-      if (p.N % 256 == 0 && (long long)p.BH * (p.N / 128) > kNumCU) {
-        wide = true;
-        const dim3 grid(p.BH * (p.N / 256)), block(512);
-        launch_dq(std::integral_constant<int, 8>{}, grid, block);
-      }
+    if constexpr (D == 128) {
+      launch_dq(std::integral_constant<int, 4>{});
+    } else {
+      // without dropout only grids of more than 256 128-row blocks come here
+      if (p.N % 256 == 0 && (!p.drop.threshold || (long long)p.BH * (p.N / 128) > 256)) launch_dq(std::integral_constant<int, 8>{});
+      else launch_dq(std::integral_constant<int, 4>{});
     }
-    if (!wide) {
-      const dim3 grid(p.BH * (p.N / 128)), block(256);
-      launch_dq(std::integral_constant<int, 4>{}, grid, block);
-    }
-    if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  return e;
+  return hipGetLastError();
 }
 
 hipError_t launch_bwd(const BwdParams& p, int D, hipStream_t stream) {

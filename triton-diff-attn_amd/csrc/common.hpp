@@ -55,6 +55,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kEps = 1e-5f;
 
 #define DA_LDS __attribute__((address_space(3)))
+typedef DA_LDS half_t lds_half;      // tile memory: a pointer to it is known to the compiler as an LDS address
 
 __device__ __forceinline__ f16v mfma32(h8 a, h8 b, f16v c) {
 #ifdef DA_BF16
@@ -204,8 +205,8 @@ __device__ __forceinline__ int swz_off(int row, int col) {
 // owns M0: it sets it in front of the statement and knows it is live there.  The s_nop covers the
 // wait state between a write of M0 and a direct-to-LDS load, which the compiler does not insert
 // for an instruction it cannot see.
-__device__ __forceinline__ void async_copy16(const half_t* g_base, unsigned byte_off, half_t* lds_base) {
-  const unsigned lds_addr = (unsigned)(unsigned long)((DA_LDS char*)lds_base);
+__device__ __forceinline__ void async_copy16(const half_t* g_base, unsigned byte_off, lds_half* lds_base) {
+  const unsigned lds_addr = (unsigned)(unsigned long)lds_base;
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :: "v"(byte_off), "s"(g_base), "{m0}"(lds_addr) : "memory");
 }
@@ -243,7 +244,7 @@ struct AsyncTile {
   }
   // issues this wave's instructions k0 .. k1-1 (of PER) for the tile; `off0` = lane_off(wave, lane, stride)
   template <int K0 = 0, int K1 = PER>
-  __device__ static __forceinline__ void issue_at(const half_t* gtile, half_t* lds_tile, int wave, int lane, unsigned off0,
+  __device__ static __forceinline__ void issue_at(const half_t* gtile, lds_half* lds_tile, int wave, int lane, unsigned off0,
                                                   int stride) {
 #pragma unroll
     for (int k = K0; k < K1; ++k) {
@@ -254,7 +255,7 @@ struct AsyncTile {
     }
   }
   template <int K0 = 0, int K1 = PER>
-  __device__ static __forceinline__ void issue(const half_t* gtile, half_t* lds_tile, int wave, int lane, int stride = COLS) {
+  __device__ static __forceinline__ void issue(const half_t* gtile, lds_half* lds_tile, int wave, int lane, int stride = COLS) {
     issue_at<K0, K1>(gtile, lds_tile, wave, lane, lane_off(wave, lane, stride), stride);
   }
   // The same copy for a tile whose global rows end at `last_row` (relative to the tile's first row; it may be
@@ -262,7 +263,7 @@ struct AsyncTile {
   // address past the tensor's last row is formed and the LDS tile holds finite data everywhere.  Used for the
   // last tiles of a sequence whose length is not a multiple of the tile; costs a few VALU instructions per piece.
   template <int K0 = 0, int K1 = PER>
-  __device__ static __forceinline__ void issue_clamped(const half_t* gtile, half_t* lds_tile, int wave, int lane, unsigned off0,
+  __device__ static __forceinline__ void issue_clamped(const half_t* gtile, lds_half* lds_tile, int wave, int lane, unsigned off0,
                                                        int stride, int last_row) {
     const int r_l = lane / CPR;                        // the lane's row inside a piece
 #pragma unroll

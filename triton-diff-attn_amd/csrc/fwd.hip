@@ -76,8 +76,8 @@ void fwd_kernel(FwdParams p) {
   constexpr int NOT = DV / 32;               // 32-row tiles of O^T
 
   __shared__ __attribute__((aligned(16))) half_t smem[C::SMEM];
-  half_t* const sKbuf = smem;                              // [NBUF][K1 tile, K2 tile]
-  half_t* const sVbuf = smem + C::NBUF * C::K_BUF;         // [NBUF][V tile]
+  lds_half* const sKbuf = (lds_half*)smem;                 // [NBUF][K1 tile, K2 tile]
+  lds_half* const sVbuf = sKbuf + C::NBUF * C::K_BUF;      // [NBUF][V tile]
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -50,6 +50,7 @@ struct BwdParamsT {
   int n_keys;                   // rows n_keys..N-1 are padding: ignored as keys, never read from q1..v, y, dy, never written to the gradients
   unsigned stages;              // bit 0 row preprocess, 1 d(lambda) reduce, 2 dK/dV, 3 dQ
   int dlam_fold;                // set by the launcher: extra workgroups at the end of a dK/dV or dQ grid that do the d(lambda) reduce
+  int n_kv_wg, n_q_wg;          // set by the launcher: key blocks and query blocks of a grid that does both dK/dV and dQ
   int H;                        // heads per batch entry: unit bh belongs to head bh % H
   int lambda_stride;            // 0: one lambda; 1: one per head
   int lambda_fp32;              // lambda_scale and dlambda are fp32 instead of the tensors' 16-bit type
