@@ -62,3 +62,29 @@ def asm_mfma_hazards(asm_text, min_wait=3, lookback=8):
                 pending -= written      # a load wrote them last: ordered by s_waitcnt
             wait += 1
     return found
+
+
+def asm_vmem_scalar_hazards(asm_text, min_wait=5, lookback=8):
+    """Inline-assembly memory instructions whose scalar address a vector instruction wrote fewer than `min_wait` wait
+    states before (a v_readlane of a spilled scalar, say): (instruction line, writer line, wait states, writer text).
+    The compiler places these wait states for its own memory instructions only."""
+    scalars = lambda t: {i for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", t) for i in range(int(lo), int(hi) + 1)} | \
+        {int(i) for i in re.findall(r"\bs(\d+)\b", t)}
+    ins = list(instructions(asm_text))
+    found = []
+    for i, (n, s, inside) in enumerate(ins):
+        if not (inside and s.startswith("global_")):
+            continue
+        pending, wait = scalars(s), 0
+        for n2, s2, _ in reversed(ins[max(0, i - lookback):i]):
+            if wait >= min_wait or not pending:
+                break
+            m = re.match(r"s_nop (\d+)", s2)
+            parts = s2.split(None, 1)
+            written = scalars(parts[1].split(",")[0]) & pending if len(parts) > 1 else set()
+            if written and parts[0].startswith("v_"):
+                found.append((n, n2, wait, s2))
+                break
+            pending -= written          # a scalar instruction wrote them last
+            wait += int(m.group(1)) + 1 if m else 1
+    return found

@@ -28,6 +28,21 @@ def test_scanner_flags_a_write_right_before_an_asm_mfma():
     assert isa_scan.registers("v[2:4], a7, s[0:1], v10") == {"v2", "v3", "v4", "a7", "v10"}
 
 
+def test_scanner_flags_a_scalar_address_that_a_vector_instruction_just_wrote():
+    bad = """
+\tv_readlane_b32 s35, v254, 38
+\ts_mov_b32 m0, s7
+\t;;#ASMSTART
+\ts_nop 0
+\tglobal_load_lds_dwordx4 v36, s[34:35]
+\t;;#ASMEND
+"""
+    assert len(isa_scan.asm_vmem_scalar_hazards(bad)) == 1
+    assert isa_scan.asm_vmem_scalar_hazards(bad.replace("s_nop 0", "s_nop 3")) == []
+    moved = bad.replace("s_nop 0", "s_mov_b64 s[2:3], s[34:35]").replace("v36, s[34:35]", "v36, s[2:3]")
+    assert isa_scan.asm_vmem_scalar_hazards(moved) == []
+
+
 def _load_build():
     import importlib.util
     spec = importlib.util.spec_from_file_location("da_build", os.path.join(ROOT, "triton-diff-attn_amd", "build.py"))
@@ -94,6 +109,17 @@ def test_forward_kernels_do_not_spill_in_their_loops(assembly):
             m = re.match(r"\s+s_cbranch_\w+ (\.LBB\w+)", l)
             if m and label_at.get(m.group(1), i) < i:
                 assert not any("scratch_" in x for x in lines[label_at[m.group(1)]:i]), name
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("source", ["bwd_fp16", "bwd_bf16", "fwd_fp16"])
+def test_tile_copies_do_not_read_an_address_too_early(assembly, source):
+    """The base of a direct global->LDS copy, an asm statement, may have been reloaded from a vector register's lanes
+    right in front of it."""
+    text = assembly[source]
+    assert "global_load_lds_dwordx4" in text
+    hazards = isa_scan.asm_vmem_scalar_hazards(text)
+    assert hazards == [], "tile copy right behind the vector write of its base: %s" % hazards[:5]
 
 
 def test_build_rejects_a_spilling_kernel():

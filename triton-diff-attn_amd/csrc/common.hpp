@@ -202,13 +202,17 @@ __device__ __forceinline__ int swz_off(int row, int col) {
 // that the compiler's wait-count insertion does not serialise later, unrelated LDS reads behind
 // it; the caller orders it with wait_async_tiles() and a barrier before the data is read.
 // The LDS base travels in M0, bound as an operand in that physical register, so the compiler
-// owns M0: it sets it in front of the statement and knows it is live there.  The s_nop covers the
-// wait state between a write of M0 and a direct-to-LDS load, which the compiler does not insert
-// for an instruction it cannot see.
+// owns M0: it sets it in front of the statement and knows it is live there.  The global base is first moved to another
+// scalar pair inside the statement.  That fills the wait state between a write of M0 and a direct-to-LDS load, and
+// it stands between the load and a base that a vector instruction has just written: the compiler keeps scalars that
+// do not fit in the lanes of a vector register, and a v_readlane right in front of a memory instruction that reads
+// its result needs five wait states, which the compiler does not insert for an instruction it cannot see.  (A scalar
+// instruction may read that result at once, and a memory instruction a scalar instruction's.)
 __device__ __forceinline__ void async_copy16(const half_t* g_base, unsigned byte_off, lds_half* lds_base) {
   const unsigned lds_addr = (unsigned)(unsigned long)lds_base;
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(byte_off), "s"(g_base), "{m0}"(lds_addr) : "memory");
+  unsigned long base;
+  asm volatile("s_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+               : "=&s"(base) : "v"(byte_off), "s"(g_base), "{m0}"(lds_addr) : "memory");
 }
 
 // Asynchronous copy of a [ROWS x COLS] fp16 tile whose rows are `stride` elements apart in global
