@@ -119,6 +119,14 @@ __device__ __forceinline__ void mfma_results_ready(f16v& x, f16v& y) {
   asm volatile("s_nop 15\n\ts_nop 3" : "+v"(x), "+v"(y));
 }
 
+// The lane number, formed anew where it is asked for: a kernel whose loop has no register to spare neither keeps it
+// nor anything derived from it across the loop.
+__device__ __forceinline__ int lane_again() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // v_permlane32_swap exchanges the upper half of its first register with the lower half of its

@@ -2,7 +2,7 @@
 // lambda-combine and RMSNorm epilogue.  Computes what the reference's forward kernel computes
 // (src/kernel.py:20-207) with a different decomposition:
 //
-//   * a workgroup of 8 waves owns 128 query rows (4 waves and 64 rows for D = 128); waves 0-3 run softmax stream 1 (Q1,K1) and
+//   * a workgroup of 8 waves owns 128 query rows (4 waves and 64 rows for small grids); waves 0-3 run softmax stream 1 (Q1,K1) and
 //     waves 4-7 run stream 2 (Q2,K2) for the same rows, 32 rows per wave.  All 8 waves share
 //     the K1/K2/V tiles, double-buffered in LDS, and the two streams meet only in the epilogue;
 //   * scores are computed transposed, S^T = K * Q^T (K fragments from LDS as the MFMA A operand,
@@ -19,7 +19,7 @@
 namespace DA_NS {
 
 // SMALL: 64 query rows per workgroup (four waves), for problems whose 128-row blocks do not fill the chip and
-// for the D = 128 instantiations that do not fit the register budget of two waves per SIMD.
+// for the D = 128 instantiations with dropout, which do not fit the register budget of two waves per SIMD.
 template <int D, bool SMALL = false>
 struct FwdCfg {
   static constexpr int DV = 2 * D;
@@ -30,7 +30,7 @@ struct FwdCfg {
   static constexpr int NW = 2 * BM / (32 * QS);    // waves per workgroup: half of them per softmax stream
   static constexpr int NT = NW * 64;
   // waves per SIMD the register budget is sized for: two, except in the four-wave D = 128 workgroups, whose
-  // masked and dropout instantiations need more than 256 registers
+  // dropout instantiations need more than 256 registers
   static constexpr int OCC = (D == 128 && SMALL) ? 1 : 2;
   // thread count the register budget is derived from: with fewer than 4 * OCC waves in a workgroup the
   // occupancy attribute alone does not hold the allocator to 512 / OCC registers (the four-wave variant at
@@ -89,6 +89,8 @@ void fwd_kernel(FwdParams p) {
   // rows past the real length are neither read from the caller's tensors nor written to y: checked in both
   // masked variants (the causal one serves padded sequences too), compiled out of the plain one
   constexpr bool TAIL = (MASK != 0);
+  // the masked loop of the 128-row D = 128 workgroup has no register to spare (see the iteration)
+  constexpr bool kLean = TAIL && D == 128 && !SMALL;
   int bh, qt;
   if constexpr (CAUSAL) {   // the last query block of a unit sees the most keys
     const UnitBlock ub = longest_first(blockIdx.x, p.BH);
@@ -156,29 +158,30 @@ void fwd_kernel(FwdParams p) {
   static_assert(!CAUSAL || BM % (2 * BN) == 0, "an even number of key tiles per query block");
   constexpr int VH = (VTile::PER + 1) / 2;   // V instructions are issued in two groups
   const unsigned k_off = KTile::lane_off(wave, lane, qk_n), v_off = VTile::lane_off(wave, lane, v_n);
+  auto tail_lane = [&] { return kLean ? lane_again() : lane; };
   // With padding, the tiles that reach past the last real row are copied with their row index clamped to it.
   // `tail` (a compile-time tag) says whether the call site can meet such a tile at all.
   auto load_k1 = [&](int tk, int buf, auto tail) {
-    if (TAIL && decltype(tail)::value && (tk + 1) * BN > p.n_keys)
-      KTile::issue_clamped(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, lane, k_off, qk_n, p.n_keys - 1 - tk * BN);
+    if (TAIL && decltype(tail)::value && (kLean || (tk + 1) * BN > p.n_keys))
+      KTile::issue_clamped(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, tail_lane(), k_off, qk_n, p.n_keys - 1 - tk * BN);
     else
       KTile::issue_at(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, lane, k_off, qk_n);
   };
   auto load_k2 = [&](int tk, int buf, auto tail) {
-    if (TAIL && decltype(tail)::value && (tk + 1) * BN > p.n_keys)
-      KTile::issue_clamped(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, lane, k_off, qk_n, p.n_keys - 1 - tk * BN);
+    if (TAIL && decltype(tail)::value && (kLean || (tk + 1) * BN > p.n_keys))
+      KTile::issue_clamped(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, tail_lane(), k_off, qk_n, p.n_keys - 1 - tk * BN);
     else
       KTile::issue_at(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, lane, k_off, qk_n);
   };
   auto load_va = [&](int tv, int buf, auto tail) {
-    if (TAIL && decltype(tail)::value && (tv + 1) * BN > p.n_keys)
-      VTile::template issue_clamped<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n, p.n_keys - 1 - tv * BN);
+    if (TAIL && decltype(tail)::value && (kLean || (tv + 1) * BN > p.n_keys))
+      VTile::template issue_clamped<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
     else
       VTile::template issue_at<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n);
   };
   auto load_vb = [&](int tv, int buf, auto tail) {
-    if (TAIL && decltype(tail)::value && (tv + 1) * BN > p.n_keys)
-      VTile::template issue_clamped<VH, VTile::PER>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n, p.n_keys - 1 - tv * BN);
+    if (TAIL && decltype(tail)::value && (kLean || (tv + 1) * BN > p.n_keys))
+      VTile::template issue_clamped<VH, VTile::PER>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
     else
       VTile::template issue_at<VH, VTile::PER>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n);
   };
@@ -282,43 +285,46 @@ void fwd_kernel(FwdParams p) {
     // queue up behind each other at the memory pipeline.
     const int tk = clampt(t + 3);
     const int tv = clampt(t + 2);
+    constexpr bool kTail = TAIL && decltype(tail)::value, kLeanTail = kLean && kTail;
     load_k1(tk, KP, tail);
+
+    // Keys past the diagonal, or past the last real key, are masked: `rel` is the last visible key minus the key
+    // index of register 0, tile 0
+    auto mask_scores = [&](int rel) {
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          s_cur[0][kt][r] = (kt * 32 + 8 * (r / 4) + (r % 4) > rel) ? -INFINITY : s_cur[0][kt][r];
+    };
+    static_assert(!TAIL || QS == 1, "one 32-row block per wave");
+    if constexpr (kLeanTail) {
+      // Before anything else of the iteration is requested, with no branch around it, from a lane number formed
+      // anew, and with all of the iteration's copies, whose clamping takes registers too, in front of it: at D = 128
+      // the loop fills the 256 registers, and kept apart like this the tail fits them as well (with branches, and
+      // the copies spread as below, 260 bytes a lane went to scratch).
+      load_k2(tk, KP, tail); load_va(tv, VP, tail); load_vb(tv, VP, tail);
+      __builtin_amdgcn_sched_barrier(0);
+      const int ln = lane_again();
+      mask_scores((CAUSAL ? qt * BM + qw * 32 + (ln & 31) : p.n_keys - 1) - t * BN - 4 * (ln >> 5));
+      __builtin_amdgcn_sched_barrier(0);
+    }
 
     // K fragments of the next tile are requested first; the row maxima of this tile are reduced
     // while they arrive.
     h8 ka[NKT][NKS];
     read_k(KR * C::KBUF_BYTES, ka);
 
-    if constexpr (CAUSAL) {
-      // only the last tiles of a wave's loop reach past its first row: mask key > query there
-      static_assert(QS == 1, "one 32-row block per wave");
-      const int wrow0 = qt * BM + qw * 32;
-      if ((t + 1) * BN - 1 > wrow0) {
-        const int rel = wrow0 + j - t * BN - 4 * g;      // query index minus the key index of register 0, tile 0
-#pragma unroll
-        for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (kt * 32 + 8 * (r / 4) + (r % 4) > rel) s_cur[0][kt][r] = -INFINITY;
-      }
-    }
-
-    if constexpr (PADDED && decltype(tail)::value) {
-      // only the last tiles hold padding keys
-      if ((t + 1) * BN > p.n_keys) {
-        const int rel = p.n_keys - 1 - t * BN - 4 * g;   // last real key minus the key index of register 0, tile 0
-#pragma unroll
-        for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (kt * 32 + 8 * (r / 4) + (r % 4) > rel) s_cur[0][kt][r] = -INFINITY;
-      }
+    if constexpr (kTail && !kLean) {
+      // only the last tiles of a wave's loop reach past its first row, or hold padding keys
+      if ((t + 1) * BN > (CAUSAL ? qt * BM + qw * 32 + 1 : p.n_keys))
+        mask_scores((CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - t * BN - 4 * g);
     }
 
     // The score product of the next tile goes to the matrix unit first and runs under the row maxima and
     // the exponentials of this tile.  It starts from the running reference as it stands before this
     // tile's update; when the update moves the reference, the few results are corrected with it.
-    load_k2(tk, KP, tail);
+    if constexpr (!kLeanTail) load_k2(tk, KP, tail);
     scores_of(ka, s_nxt, sc_first, sc_split);
 
     float mx[QS];
@@ -430,8 +436,8 @@ void fwd_kernel(FwdParams p) {
 #pragma unroll
     for (int i = 0; i < NPV; ++i) {
       const int kk = i / NOT, tt = i % NOT;
-      if (i == 0) load_va(tv, VP, tail);
-      if (i == NPV / 2) load_vb(tv, VP, tail);
+      if (!kLeanTail && i == 0) load_va(tv, VP, tail);
+      if (!kLeanTail && i == NPV / 2) load_vb(tv, VP, tail);
       if (i + PD < NPV) vfr[i + PD] = vt_frag(i + PD);
 #pragma unroll
       for (int qs = 0; qs < QS; ++qs) o[qs][tt] = mfma32(vfr[i], __builtin_bit_cast(h8, pw[qs][kk]), o[qs][tt]);
@@ -461,10 +467,12 @@ void fwd_kernel(FwdParams p) {
     iteration(t + 2, std::integral_constant<int, 2>{}, tail, s_a, s_b);
     iteration(t + 3, std::integral_constant<int, 3>{}, tail, s_b, s_a);
   };
-  if constexpr (PADDED) {
-    // Padding concerns the last tiles only: an iteration copies K tile t+3, so the first one that can touch a
-    // tile with padding rows is number n_keys / BN - 3.  Whole turns in front of it run without the tests.
-    const int t_tail = p.n_keys / BN - 3;
+  if constexpr (TAIL) {
+    // A mask concerns the last tiles only: with padding, an iteration copies K tile t+3, so the first one that can
+    // touch a tile with padding rows is number n_keys / BN - 3; under the causal mask the workgroup's rows see all
+    // of the tiles in front of its own.  Whole turns in front of both run without the tests.
+    int t_tail = CAUSAL ? qt * (BM / BN) : p.N / BN;
+    if (p.n_keys < p.N) t_tail = min(t_tail, p.n_keys / BN - 3);
 #pragma nounroll
     for (; t + 4 <= t_tail; t += 4) turn(t, no_tail);
   }
@@ -485,6 +493,7 @@ void fwd_kernel(FwdParams p) {
   // hold a row's values in the same lanes and registers, so the exchange is lane to lane.
   // Each pair of waves has one block of tile memory: first it carries the fp32 exchange, then, once the
   // workgroup has met behind the combine, the staged rows of the two waves side by side.
+  const int lane_e = lane_again(), j_e = lane_e & 31, g_e = lane_e >> 5;
   constexpr int SROW = DV + 8;
   float* const xch = reinterpret_cast<float*>(smem + (size_t)qw * C::XCH_BLOCK);
   half_t* const stg_own = smem + (size_t)qw * C::XCH_BLOCK + (st ? 32 * SROW : 0);
@@ -496,7 +505,7 @@ void fwd_kernel(FwdParams p) {
         h4 v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = (half_t)(val[tt][4 * r4 + e] * scale);
-        *reinterpret_cast<h4*>(stg_own + j * SROW + 32 * tt + 8 * r4 + 4 * g) = v;
+        *reinterpret_cast<h4*>(stg_own + j_e * SROW + 32 * tt + 8 * r4 + 4 * g_e) = v;
       }
     (void)qs;
   };
@@ -507,7 +516,7 @@ void fwd_kernel(FwdParams p) {
     constexpr int RPI = 64 / LPR;          // rows per instruction
 #pragma unroll
     for (int k = 0; k < 32 / RPI; ++k) {
-      const int row = k * RPI + lane / LPR, ch = lane % LPR;
+      const int row = k * RPI + lane_e / LPR, ch = lane_e % LPR;
       const u32x4 v = *reinterpret_cast<const u32x4*>(stg_own + row * SROW + 8 * ch);
       if (!TAIL || row < rows) *reinterpret_cast<u32x4*>(gbase + (size_t)row * row_stride + 8 * ch) = v;
     }
@@ -516,11 +525,11 @@ void fwd_kernel(FwdParams p) {
   static_assert(QS == 1, "the epilogue stages one 32-row block per wave");
   const float lsum = pair_sum(l[0]);
   const float inv = (DROP ? p.drop.keep_scale : 1.0f) / lsum;
-  const size_t row = (size_t)bh * p.N + qrow0;
+  const size_t row = (size_t)bh * p.N + qt * BM + qw * 32 + j_e;
   const size_t wave_row0 = (size_t)bh * p.N + qt * BM + qw * 32;
   {
     float* lse = st ? p.lse2 : p.lse1;
-    if (g == 0 && lse) lse[row] = (m[0] + __builtin_log2f(lsum)) * kLn2;
+    if (g_e == 0 && lse) lse[row] = (m[0] + __builtin_log2f(lsum)) * kLn2;
   }
   if (st == 1) {
 #pragma unroll
@@ -530,7 +539,7 @@ void fwd_kernel(FwdParams p) {
         f4v u;
 #pragma unroll
         for (int e = 0; e < 4; ++e) u[e] = o[0][tt][4 * r4 + e] * inv;
-        *reinterpret_cast<f4v*>(xch + ((tt * 4 + r4) * 64 + lane) * 4) = u;
+        *reinterpret_cast<f4v*>(xch + ((tt * 4 + r4) * 64 + lane_e) * 4) = u;
       }
   }
   __syncthreads();
@@ -541,7 +550,7 @@ void fwd_kernel(FwdParams p) {
     for (int tt = 0; tt < NOT; ++tt)
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
-        const f4v u = *reinterpret_cast<const f4v*>(xch + ((tt * 4 + r4) * 64 + lane) * 4);
+        const f4v u = *reinterpret_cast<const f4v*>(xch + ((tt * 4 + r4) * 64 + lane_e) * 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float x = o[0][tt][4 * r4 + e] * inv - lam * u[e];
@@ -561,7 +570,7 @@ void fwd_kernel(FwdParams p) {
       ss = pair_sum(ss);
       const float rr = __builtin_amdgcn_rsqf(ss * (1.0f / DV) + kEps);
       scale = (1.0f - p.lambda_init) * rr;
-      if (g == 0 && p.rinv) p.rinv[row] = rr;
+      if (g_e == 0 && p.rinv) p.rinv[row] = rr;
     }
     stage_rows(0, o[0], scale);
     __builtin_amdgcn_wave_barrier();   // the rows are read back by other lanes of this wave only
@@ -589,19 +598,19 @@ static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   // Shape-aware launch geometry (the reference autotunes its tiles per (N, D, Dv), src/kernel.py:12-19): a problem
   // whose 128-row blocks do not fill the chip once runs in twice as many 64-row, four-wave workgroups.  A pure
   // function of (B*H, N, D) and the options: no tuning state.  At D <= 64 only the plain instantiation has the
-  // small variant.  At D = 128 it is the other way round: only the plain instantiation fits the 256 registers of
-  // the 128-row workgroup (two waves per SIMD); with a mask or dropout the kernel runs in 64-row workgroups at one
-  // wave per SIMD.
+  // small variant.  At D = 128 the masked instantiations gain by the 128-row workgroup from 256 blocks on (us, causal:
+  // B1 H16 N2048 81 -> 75, B1 H32 N2048 159 -> 114, B1 H32 N3001 328 -> 230; N not a multiple of 128: B2 H32 N1000
+  // 142 -> 111), and the dropout instantiations do not fit the 256 registers of the 128-row workgroup
+  // (two waves per SIMD) and always run in 64-row workgroups at one wave per SIMD.
   constexpr int kNumCU = 256;
   const bool small_grid = (long long)p.BH * (p.N / 128) < kNumCU;
   if constexpr (D == 128) {
-    if (!plain || small_grid) {
-      if (p.rms_norm) { if (drop) launch_fwd_c<D, true, true, true>(p, stream); else launch_fwd_c<D, true, false, true>(p, stream); }
-      else            { if (drop) launch_fwd_c<D, false, true, true>(p, stream); else launch_fwd_c<D, false, false, true>(p, stream); }
+    if (drop) {
+      if (p.rms_norm) launch_fwd_c<D, true, true, true>(p, stream); else launch_fwd_c<D, false, true, true>(p, stream);
+    } else if (small_grid) {
+      if (p.rms_norm) launch_fwd_c<D, true, false, true>(p, stream); else launch_fwd_c<D, false, false, true>(p, stream);
     } else {
-      const dim3 grid(p.BH * (p.N / FwdCfg<D>::BM)), block(FwdCfg<D>::NT);
-      if (p.rms_norm) hipLaunchKernelGGL((fwd_kernel<D, true, 0, false, false>), grid, block, 0, stream, p);
-      else            hipLaunchKernelGGL((fwd_kernel<D, false, 0, false, false>), grid, block, 0, stream, p);
+      if (p.rms_norm) launch_fwd_c<D, true, false, false>(p, stream); else launch_fwd_c<D, false, false, false>(p, stream);
     }
     return hipGetLastError();
   } else {
