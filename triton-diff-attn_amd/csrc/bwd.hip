@@ -240,6 +240,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   const float lam = da_abi::lambda_of_unit(p, bh);
   // hash keys of this unit's two softmax streams (used with dropout only)
   const DropoutKey dkey1 = dropout_key(p.drop, 2u * bh), dkey2 = dropout_key(p.drop, 2u * bh + 1);
+  const DropoutSel dsel = dropout_sel_key(key & 1);
 
   // persistent B operands: this lane's key row of K1, K2, V
   h8 kf1[NKS], kf2[NKS], vf[NKV];
@@ -432,11 +433,11 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
       // lane of a key pair
       if ((r & 3) == 0) {
         const unsigned odd = (unsigned)key & 1u;
-        dropout_words_shared(dropout_word(dkey1, (unsigned)p.N / 2, (query >> 1) + odd, (unsigned)key >> 1), odd, t.w1, t.w1b);
-        dropout_words_shared(dropout_word(dkey2, (unsigned)p.N / 2, (query >> 1) + odd, (unsigned)key >> 1), odd, t.w2, t.w2b);
+        dropout_bytes_shared(dropout_word(dkey1, (unsigned)p.N / 2, (query >> 1) + odd, (unsigned)key >> 1), dsel, t.w1, t.w1b);
+        dropout_bytes_shared(dropout_word(dkey2, (unsigned)p.N / 2, (query >> 1) + odd, (unsigned)key >> 1), dsel, t.w2, t.w2b);
       }
-      const bool keep1 = dropout_keep((r & 2) ? t.w1b : t.w1, query, (unsigned)key, p.drop.threshold);
-      const bool keep2 = dropout_keep((r & 2) ? t.w2b : t.w2, query, (unsigned)key, p.drop.threshold);
+      const bool keep1 = dropout_keep_half((r & 2) ? t.w1b : t.w1, r & 1, p.drop.threshold);
+      const bool keep2 = dropout_keep_half((r & 2) ? t.w2b : t.w2, r & 1, p.drop.threshold);
       t.k1[r] = keep1 ? t.p1[r] : 0.f;
       t.k2[r] = keep2 ? t.p2[r] : 0.f;
       if constexpr (DO_K) {
@@ -780,8 +781,15 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int wg, int n_wg, l
   const int qk_n = (int)p.sqk.n, v_n = (int)p.sv.n;
 
   const float lam = da_abi::lambda_of_unit(p, bh);
-  // hash keys of this unit's two softmax streams (used with dropout only)
+  // used with dropout only, as in the forward: hash keys of this unit's two softmax streams, the counter of this
+  // query's first key pair, the counters' lane-dependent low bits, and what a block of eight keys adds
   const DropoutKey dkey1 = dropout_key(p.drop, 2u * bh), dkey2 = dropout_key(p.drop, 2u * bh + 1);
+  const unsigned hquery = (unsigned)(qt * BM + wave * 32 + j);
+  const unsigned hrow = (hquery >> 1) * ((unsigned)p.N / 2), hlow = 2u * (unsigned)g + (hquery & 1u);
+  const DropoutSel dsel = dropout_sel_query(hquery & 1u);
+  unsigned hstep1[4], hstep2[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) { hstep1[v] = dropout_window_step<16>(dkey1, v); hstep2[v] = dropout_window_step<16>(dkey2, v); }
 
   // persistent B operands: this lane's query row of Q1, Q2 (pre-multiplied by sm_scale*log2(e)
   // exactly as in the forward kernel, so the recomputed probabilities match it), dX, and its row
@@ -1140,24 +1148,24 @@ __device__ __forceinline__ void dq_block(const BwdParams& p, int wg, int n_wg, l
       __builtin_amdgcn_sched_barrier(0);
       h8 b1[2], b2[2];
       unsigned w1 = 0, w2 = 0, w1b = 0, w2b = 0;
+      const unsigned hkeys = hrow + (unsigned)(t * (BN / 2) + ksub * 16);
+      const unsigned hwin1 = DROP ? dropout_window<16>(dkey1, hkeys, hlow) : 0u;
+      const unsigned hwin2 = DROP ? dropout_window<16>(dkey2, hkeys, hlow) : 0u;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float p1 = fast_exp2(kFoldS ? s1[r] : s1[r] + nl1);
         const float p2 = fast_exp2(kFoldS ? s2[r] : s2[r] + nl2);
         if constexpr (DROP) {
-          // register r holds key kq + 8*(r/4) + (r%4) of this lane's query; registers r, r+1 (r even)
-          // share the hash words of their 2x2 block
-          const unsigned query = (unsigned)(qt * BM + wave * 32 + j);
-          const unsigned kq = (unsigned)(t * BN + ksub * 32 + 4 * g + 8 * (r / 4) + (r % 4));
-          // the blocks of registers r..r+1 and r+2..r+3 (r a multiple of 4) are neighbours, hashed one by each
-          // lane of a query pair
+          // register r holds key 8*(r/4) + 4g + (r%4) of the sub-tile; registers r, r+1 (r even) share the hash words
+          // of their 2x2 block, and the blocks of registers r..r+1 and r+2..r+3 (r a multiple of 4) are neighbours,
+          // hashed one by each lane of a query pair
           if ((r & 3) == 0) {
-            dropout_words_shared(dropout_word(dkey1, (unsigned)p.N / 2, query >> 1, (kq >> 1) + (query & 1)), query & 1, w1, w1b);
-            dropout_words_shared(dropout_word(dkey2, (unsigned)p.N / 2, query >> 1, (kq >> 1) + (query & 1)), query & 1, w2, w2b);
+            dropout_bytes_shared(dropout_rounds(dkey1, hwin1 + hstep1[r / 4]), dsel, w1, w1b);
+            dropout_bytes_shared(dropout_rounds(dkey2, hwin2 + hstep2[r / 4]), dsel, w2, w2b);
           }
           const float dpk = p.drop.keep_scale * dp[r];
-          const float d1 = dropout_keep((r & 2) ? w1b : w1, query, kq, p.drop.threshold) ? dpk : 0.f;
-          const float d2 = dropout_keep((r & 2) ? w2b : w2, query, kq, p.drop.threshold) ? dpk : 0.f;
+          const float d1 = dropout_keep_half((r & 2) ? w1b : w1, r & 1, p.drop.threshold) ? dpk : 0.f;
+          const float d2 = dropout_keep_half((r & 2) ? w2b : w2, r & 1, p.drop.threshold) ? dpk : 0.f;
           b1[r / 8][r % 8] = (half_t)(p1 * (d1 + de1));                                             // c m1 dP - delta1
           b2[r / 8][r % 8] = (half_t)(p2 * __builtin_fmaf(-lam, d2, __builtin_fmaf(-lam, de1, de2)));   // -lambda c m2 dP - delta2
         } else {

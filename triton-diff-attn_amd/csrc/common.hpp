@@ -339,9 +339,9 @@ __device__ __forceinline__ DropoutKey dropout_key(const DropoutCfg& c, unsigned 
   return {a, b};
 }
 
-__device__ __forceinline__ unsigned dropout_word(const DropoutKey& key, unsigned half_n, unsigned qh, unsigned kh) {
-  unsigned h = (qh * half_n + kh) ^ key.k1;
-  h *= 0x9E3779B1u;
+constexpr unsigned kDropMul = 0x9E3779B1u;
+// the rounds behind the first multiplication
+__device__ __forceinline__ unsigned dropout_rounds(const DropoutKey& key, unsigned h) {
   h ^= h >> 15;
   h += key.k2;
   h *= 0xC2B2AE3Du;
@@ -350,14 +350,54 @@ __device__ __forceinline__ unsigned dropout_word(const DropoutKey& key, unsigned
   h ^= h >> 16;
   return h;
 }
+__device__ __forceinline__ unsigned dropout_word(const DropoutKey& key, unsigned half_n, unsigned qh, unsigned kh) {
+  return dropout_rounds(key, ((qh * half_n + kh) ^ key.k1) * kDropMul);
+}
+// The first multiplication of a run of counters.  Where a kernel's lane walks along the keys, its counters inside a
+// window of W key pairs (W a power of two that divides the counter of the window's start; half_n is a multiple of 64)
+// differ in their low bits only, and (start + i) ^ k1 = (start ^ high bits of k1) + (i ^ low bits of k1), so the product
+// is a sum: one multiplication per window and lane for the start, whose lane-dependent low two bits `low` ride along,
+// and a wave-uniform term per multiple of four key pairs, formed once per kernel.  A 32-bit multiplication takes four
+// times as long as an addition, and a word has three of them.
+template <int W>
+__device__ __forceinline__ unsigned dropout_window(const DropoutKey& key, unsigned start, unsigned low) {
+  return ((start ^ (key.k1 & ~(unsigned)(W - 1))) + (low ^ (key.k1 & 3u))) * kDropMul;
+}
+template <int W>
+__device__ __forceinline__ unsigned dropout_window_step(const DropoutKey& key, int v) {
+  return ((4u * v) ^ (key.k1 & (unsigned)(W - 4))) * kDropMul;
+}
 // The word of a 2x2 block serves two lanes: the kernels hold the block's two queries (or its two keys) in lanes
 // l and l^1.  Of two neighbouring blocks each lane of the pair hashes one -- the even lane the first, the odd
-// lane the second (`mine`) -- and takes the other from its neighbour, which halves the hash work.
+// lane the second (`mine`) -- and takes the other from its neighbour, which halves the hash work.  What a lane needs
+// of each of the two words are two bytes: one v_perm per block picks them from (mine, other), by a selector that
+// depends on the lane's parity, into the low and the high half of a register.
 // Every lane of the wave must be active.
-__device__ __forceinline__ void dropout_words_shared(unsigned mine, bool odd_lane, unsigned& first, unsigned& second) {
+struct DropoutSel { unsigned first, second; };
+// lanes are queries: the bytes of keys k (low half) and k + 1 of the lane's own query
+__device__ __forceinline__ DropoutSel dropout_sel_query(bool odd_lane) {
+  return odd_lane ? DropoutSel{0x0c070c06u, 0x0c030c02u} : DropoutSel{0x0c010c00u, 0x0c050c04u};
+}
+// lanes are keys: the bytes of queries q (low half) and q + 1 of the lane's own key
+__device__ __forceinline__ DropoutSel dropout_sel_key(bool odd_lane) {
+  return odd_lane ? DropoutSel{0x0c070c05u, 0x0c030c01u} : DropoutSel{0x0c020c00u, 0x0c060c04u};
+}
+__device__ __forceinline__ void dropout_bytes_shared(unsigned mine, const DropoutSel& sel, unsigned& first, unsigned& second) {
   const unsigned other = (unsigned)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1 /* quad_perm 1,0,3,2 */, 0xF, 0xF, true);
-  first = odd_lane ? other : mine;
-  second = odd_lane ? mine : other;
+  first = __builtin_amdgcn_perm(other, mine, sel.first);
+  second = __builtin_amdgcn_perm(other, mine, sel.second);
+}
+// keep decisions of the low and the high half of such a register
+__device__ __forceinline__ bool dropout_keep_half(unsigned bytes, int half, unsigned threshold) {
+  return half ? bytes >= (threshold << 16) : (unsigned short)bytes >= (unsigned short)threshold;
+}
+// two packed 16-bit values with the dropped ones cleared: byte - threshold is negative for those, and v_perm spreads
+// the two sign bits over their halves
+__device__ __forceinline__ unsigned dropout_clear_pair(unsigned bytes, unsigned threshold, unsigned values) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  const s2 d = __builtin_bit_cast(s2, bytes) - (s2)(short)threshold;
+  const unsigned w = __builtin_bit_cast(unsigned, d);
+  return values & ~__builtin_amdgcn_perm(w, w, 0x09090808u);
 }
 // keep decision of pair (q, k) from the word of its 2x2 block
 __device__ __forceinline__ bool dropout_keep(unsigned word, unsigned q, unsigned k, unsigned threshold) {

@@ -104,7 +104,14 @@ void fwd_kernel(FwdParams p) {
   const size_t v_base = da_abi::unit_base(p, p.sv, bh);
   const int qk_n = (int)p.sqk.n, v_n = (int)p.sv.n;
   const int qrow0 = qt * BM + qw * 32 * QS + j;   // this lane's query row of block qs is qrow0 + 32*qs
-  const DropoutKey dkey = dropout_key(p.drop, 2u * bh + st);   // hash key of this wave's softmax stream (used with dropout only)
+  // used with dropout only: hash key of this wave's softmax stream, the counter of this query's first key pair, the
+  // counters' lane-dependent low bits, and what a block of eight keys adds inside a tile
+  const DropoutKey dkey = dropout_key(p.drop, 2u * bh + st);
+  const unsigned hrow = (unsigned)(qrow0 >> 1) * ((unsigned)p.N / 2), hlow = (unsigned)(2 * g + (qrow0 & 1));
+  const DropoutSel dsel = dropout_sel_query(qrow0 & 1);
+  unsigned hstep[BN / 8];
+#pragma unroll
+  for (int v = 0; v < BN / 8; ++v) hstep[v] = dropout_window_step<BN / 2>(dkey, v);
 
   // Q fragments (B operand): column j = this lane's query, k = 8g..8g+7 of each 16-wide k-step.
   // They are pre-multiplied by sm_scale*log2(e), so the MFMA result is the score in log2 units.
@@ -297,7 +304,7 @@ void fwd_kernel(FwdParams p) {
         for (int r = 0; r < 16; ++r)
           s_cur[0][kt][r] = (kt * 32 + 8 * (r / 4) + (r % 4) > rel) ? -INFINITY : s_cur[0][kt][r];
     };
-    static_assert(!TAIL || QS == 1, "one 32-row block per wave");
+    static_assert(!(TAIL || DROP) || QS == 1, "one 32-row block per wave");
     if constexpr (kLeanTail) {
       // Before anything else of the iteration is requested, with no branch around it, from a lane number formed
       // anew, and with all of the iteration's copies, whose clamping takes registers too, in front of it: at D = 128
@@ -402,7 +409,8 @@ void fwd_kernel(FwdParams p) {
 #pragma unroll
     for (int qs = 0; qs < QS; ++qs) {
       float rs = 0.f;
-      unsigned word_a = 0, word_b = 0;     // dropout: hash words of two neighbouring 2x2 blocks
+      unsigned word_a = 0, word_b = 0;     // dropout: this query's bytes of the words of two neighbouring 2x2 blocks
+      const unsigned hwin = DROP ? dropout_window<BN / 2>(dkey, hrow + (unsigned)(t * (BN / 2)), hlow) : 0u;
 #pragma unroll
       for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
@@ -415,14 +423,8 @@ void fwd_kernel(FwdParams p) {
           if constexpr (DROP) {
             // registers r, r+1 hold the keys key, key+1 (key even) of this lane's query; the blocks of registers
             // r..r+1 and r+2..r+3 (r a multiple of 4) are neighbours, hashed one by each lane of a query pair
-            const unsigned query = (unsigned)(qrow0 + 32 * qs);
-            const unsigned key = (unsigned)(t * BN + kt * 32 + 8 * (r / 4) + 4 * g + (r % 4));
-            if (r % 4 == 0)
-              dropout_words_shared(dropout_word(dkey, (unsigned)p.N / 2, query >> 1, (key >> 1) + (query & 1)), query & 1,
-                                   word_a, word_b);
-            const unsigned word = (r % 4 == 0) ? word_a : word_b;
-            w2 &= (dropout_keep(word, query, key, p.drop.threshold) ? 0x0000ffffu : 0u) |
-                  (dropout_keep(word, query, key + 1, p.drop.threshold) ? 0xffff0000u : 0u);
+            if (r % 4 == 0) dropout_bytes_shared(dropout_rounds(dkey, hwin + hstep[kt * 4 + r / 4]), dsel, word_a, word_b);
+            w2 = dropout_clear_pair((r % 4 == 0) ? word_a : word_b, p.drop.threshold, w2);
           }
           pw[qs][kt * 2 + r / 8][(r % 8) / 2] = w2;
         }
