@@ -1,0 +1,83 @@
+"""The host side of a call (csrc/host.cpp and kernel.py around it): the call without autograd against the one with it, and
+inputs that cannot go to the kernels as they are against their plain copies, bit for bit."""
+import pytest
+import torch
+
+from util import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _tensors(N=77, dtype=torch.float16):
+    return [t.cuda().to(dtype) for t in make_inputs(2, 3, N, 64, seed=5)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kw", [{}, {"rms_norm": True, "causal": True}, {"dropout_p": 0.25, "dropout_seed": -3},
+                                {"rms_norm": True, "causal": True, "dropout_p": 0.1, "dropout_seed": 2 ** 70 + 1}])
+def test_without_gradients_the_same_bits(kw, dtype):
+    from layers import MultiheadDiffAttnKernel
+    ins = _tensors(dtype=dtype)[:5]
+    lam = torch.tensor([0.5], device="cuda", dtype=dtype)
+    want = MultiheadDiffAttnKernel(*[t.requires_grad_() for t in ins], lam, 0.8, **kw)
+    assert want.requires_grad
+    with torch.no_grad():
+        got = MultiheadDiffAttnKernel(*ins, lam, 0.8, **kw)
+    with torch.inference_mode():
+        inf = MultiheadDiffAttnKernel(*ins, lam, 0.8, **kw)
+    assert not got.requires_grad and torch.equal(got, want) and torch.equal(inf, want)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_inputs_that_need_converting(grad):
+    from layers import MultiheadDiffAttnKernel
+    ins = _tensors()
+    dy = ins.pop()
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+
+    def run(ins, lam):
+        leaves = [t.detach().requires_grad_(grad) for t in ins]
+        y = MultiheadDiffAttnKernel(*leaves, lam, 0.8, True)
+        if not grad:
+            return [y]
+        y.backward(dy)
+        return [y.detach()] + [t.grad for t in leaves]
+
+    want = run(ins, lam)
+    same = lambda got: all(torch.equal(a, b) for a, b in zip(got, want))
+    for l in (0.5, lam.double(), lam.cpu(), lam.reshape(1, 1, 1), torch.full((3,), 0.5, device="cuda", dtype=torch.float16),
+              torch.full((6,), 0.5, device="cuda", dtype=torch.float16)[::2]):
+        assert same(run(ins, l))
+    mixed = list(ins)
+    mixed[1] = ins[1].transpose(1, 2).contiguous().transpose(1, 2)          # not q1's strides
+    assert same(run(mixed, lam))
+    odd = list(ins)
+    odd[4] = torch.nn.functional.pad(ins[4], (0, 4))[..., :128]             # rows not 16-byte aligned
+    odd[0] = ins[0].transpose(2, 3).contiguous().transpose(2, 3)            # columns, not rows, contiguous
+    assert same(run(odd, lam))
+    if grad:                                                                # the upstream gradient likewise
+        dense = dy
+        for dy in (dense.float(), dense.transpose(2, 3).contiguous().transpose(2, 3), dense.transpose(0, 1).contiguous().transpose(0, 1)):
+            leaves = [t.detach().requires_grad_() for t in ins]
+            MultiheadDiffAttnKernel(*leaves, lam, 0.8, True).backward(dy.to(torch.float16) if dy.dtype == torch.float32 else dy)
+            assert same([want[0]] + [t.grad for t in leaves])
+
+
+def test_what_was_refused_stays_refused():
+    from layers import MultiheadDiffAttnKernel
+    q1, q2, k1, k2, v, _ = _tensors()
+    unaligned = torch.empty(v.numel() + 1, device="cuda", dtype=v.dtype)[1:].view_as(v)     # contiguous, not 16-byte aligned
+    with torch.no_grad():
+        for args, error in (((q1, q2, k1, k2, unaligned), RuntimeError), ((q1, q2[:, :2], k1, k2, v), ValueError), ((q1, q2, k1, k2, v[..., :64]), ValueError),
+                            ((q1.float(), q2, k1, k2, v), TypeError), ((q1, q2, k1.bfloat16(), k2, v), TypeError),
+                            ((q1, q2, k1, k2, v.cpu()), ValueError), ((q1[:, :, :0], q2[:, :, :0], k1[:, :, :0], k2[:, :, :0], v[:, :, :0]), ValueError),
+                            ((q1[:0], q2[:0], k1[:0], k2[:0], v[:0]), RuntimeError)):
+            with pytest.raises(error):
+                MultiheadDiffAttnKernel(*args, 0.5)
+        with pytest.raises(ValueError):
+            MultiheadDiffAttnKernel(q1, q2, k1, k2, v, torch.zeros(2, device="cuda"))
+        with pytest.raises(ValueError):
+            MultiheadDiffAttnKernel(q1, q2, k1, k2, v, 0.5, dropout_p=1.0, dropout_seed=1)
+        # a transform goes to the autograd function, which has no rule for it
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(lambda q: MultiheadDiffAttnKernel(q, q2, k1, k2, v, 0.5))(q1[None])

@@ -1,15 +1,17 @@
-"""ctypes binding of libdiffattn.so (C ABI in include/diffattn.h).
+"""ctypes binding of libdiffattn.so (C ABI in include/diffattn.h), and the loader of its extension module.
 
 torch is imported first on purpose: the library resolves the HIP runtime by soname, so it shares
 the runtime (and therefore streams and device pointers) that torch has already loaded.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch  # noqa: F401  (must precede loading the library)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdiffattn.so")
+HOST_PATH = os.path.join(_HERE, "diffattn_host.so")
 
 ABI_VERSION = 7   # the version of include/diffattn.h this binding is written against
 
@@ -77,6 +79,25 @@ def lib():
                 % (handle.diffattn_abi_version(), ABI_VERSION, os.path.join(_HERE, "build.py")))
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """Returns the extension module that runs one operator call on the library (csrc/host.cpp); raises if it has not
+    been built."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise NativeLibraryMissing(
+                "diffattn_host.so is not built: run `python %s`" % os.path.join(_HERE, "build.py"))
+        lib()       # present and of the right version
+        spec = importlib.util.spec_from_file_location("diffattn_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(code):

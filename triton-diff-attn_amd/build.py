@@ -1,4 +1,5 @@
-"""Builds libdiffattn.so (the gfx950 kernels plus their C ABI) in-tree with plain hipcc.
+"""Builds libdiffattn.so (the gfx950 kernels plus their C ABI) and diffattn_host.so (its extension module) in-tree with
+plain hipcc and g++.
 
 Usage: python build.py            (from anywhere; output lands next to this file)
 """
@@ -9,6 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libdiffattn.so")
+HOST = os.path.join(HERE, "diffattn_host.so")
 ABI_EXAMPLE = os.path.join(HERE, "abi_example")
 SOURCES = ["fwd.hip", "bwd.hip", "api.hip"]
 KERNEL_SOURCES = ["fwd.hip", "bwd.hip"]
@@ -77,6 +79,18 @@ def build(verbose=True):
         if verbose and out.strip():
             print(out)
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    # the extension module that runs one operator call: host code only, against the headers of the torch it is loaded into
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
+           *("-I" + d for d in include_paths()), "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + HERE, "-ldiffattn", *("-L" + d for d in library_paths()),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)

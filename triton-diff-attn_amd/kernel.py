@@ -4,22 +4,18 @@ Host-side counterpart of the reference's `_diff_attention` (src/kernel.py:461-57
 name, same `apply` argument order, same 9-slot gradient tuple (the optional arguments `causal`,
 `dropout_p` and `dropout_seed` -- masking and dropout are features the reference lists as missing,
 src/kernel.py:4 -- add a slot each).  The work itself is done by the
-hand-written HIP kernels in libdiffattn.so, reached through its C ABI; if the library is missing
-the call raises -- there is no other path.
+hand-written HIP kernels in libdiffattn.so, called by the extension module diffattn_host (csrc/host.cpp), which
+also allocates the outputs; if either is missing the call raises -- there is no other path.
 """
 import torch
+from torch.autograd import forward_ad
 from torch.autograd.function import once_differentiable
 
 import _native
 
 _SUPPORTED_D = (32, 64, 128)
-_SEQ_MULTIPLE = 128
 _FLAG_RMS_NORM = 1      # DIFFATTN_RMS_NORM
 _FLAG_CAUSAL = 2        # DIFFATTN_CAUSAL
-_FLAG_BF16 = 4          # DIFFATTN_BF16
-_FLAG_LAMBDA_PER_HEAD = 8   # DIFFATTN_LAMBDA_PER_HEAD
-_FLAG_LAMBDA_FP32 = 16      # DIFFATTN_LAMBDA_FP32
-_FLAG_UNPADDED = 32         # DIFFATTN_UNPADDED
 _DTYPES = (torch.float16, torch.bfloat16)
 
 
@@ -97,8 +93,43 @@ def _lambda_tensor(lambda_scale, device, dtype=torch.float16, num_heads=1):
     return torch.tensor([float(lambda_scale)], dtype=dtype, device=device)
 
 
-def _ptr(t):
-    return 0 if t is None else t.data_ptr()
+def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_norm, causal, dropout_p, dropout_seed,
+                 differentiable):
+    """One forward launch on the current stream.  Returns (inputs as the kernels read them: q1, q2, k1, k2, v, lambda),
+    (y, u2, lse1, lse2, rinv, flags, padded length).
+
+    The kernels work on blocks of 128 rows (like the reference's, src/kernel.py:527).  For other lengths they run on
+    the next multiple of 128, redirect reads past the last real row to that row and ignore the padding keys: no tensor
+    is padded or copied here; only what the library keeps for itself (u2, the row statistics, the backward's workspace)
+    is sized for the padded length.  Tensors are read through their strides (the reference passes Q1's and V's to its
+    kernel, src/kernel.py:487-494): a [B,N,H,d] projection output viewed as [B,H,N,d] is not copied.  The four q/k
+    tensors share one set of strides, as in the reference.  What only a backward reads (src/kernel.py:505 saves its
+    counterparts unconditionally) is neither allocated nor written unless `differentiable`."""
+    dropout_p, dropout_seed = float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF
+    flags = (_FLAG_RMS_NORM if rms_norm else 0) | (_FLAG_CAUSAL if causal else 0)
+    forward = _native.host().forward
+    p_ok = 0.0 <= dropout_p <= 255 / 256
+    if p_ok and torch.is_tensor(Q1) and Q1.is_cuda:
+        dev = torch._C._cuda_getDevice()
+        out = forward(Q1, Q2, K1, K2, V, LAMBDA_SCALE, SM_SCALE, LAMBDA_INIT, flags, dropout_p, dropout_seed, differentiable,
+                      dev, torch._C._cuda_getCurrentRawStream(dev))
+        if out is not None:
+            return (Q1, Q2, K1, K2, V, LAMBDA_SCALE), out
+    # something about the inputs stands in the way: an error, a layout, another device, a lambda to be converted
+    B, H, N, D = _check_inputs(Q1, Q2, K1, K2, V)
+    if not p_ok:
+        raise ValueError("dropout_p must lie in [0, 255/256] (got %r)" % dropout_p)
+    q1, q2, k1, k2, v = (_in_place(t) for t in (Q1, Q2, K1, K2, V))
+    if not (q1.stride() == q2.stride() == k1.stride() == k2.stride()):
+        q1, q2, k1, k2 = (t.contiguous() for t in (q1, q2, k1, k2))
+    dev = q1.device
+    lam = _lambda_tensor(LAMBDA_SCALE, dev, Q1.dtype, H)
+    with torch.cuda.device(dev):
+        out = forward(q1, q2, k1, k2, v, lam, SM_SCALE, LAMBDA_INIT, flags, dropout_p, dropout_seed, differentiable,
+                      q1.get_device(), _current_stream(dev))
+    if out is None:
+        raise RuntimeError("the kernels cannot read these tensors: their pointers must be 16-byte aligned")
+    return (q1, q2, k1, k2, v, lam), out
 
 
 class _diff_attention(torch.autograd.Function):
@@ -106,124 +137,55 @@ class _diff_attention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_norm=False, causal=False,
                 dropout_p=0.0, dropout_seed=0):
-        B, H, N, D = _check_inputs(Q1, Q2, K1, K2, V)
-        dropout_p = float(dropout_p)
-        if not 0.0 <= dropout_p <= 255 / 256:
-            raise ValueError("dropout_p must lie in [0, 255/256] (got %r)" % dropout_p)
-        # the same struct goes to the backward: the masks are a function of (seed, position) only
-        dropout = _native.Dropout(dropout_p, int(dropout_seed) & 0xFFFFFFFFFFFFFFFF) if dropout_p > 0 else None
-        lib = _native.lib()
-        dev = Q1.device
-        # The kernels work on blocks of 128 rows (like the reference's, src/kernel.py:527).  For other lengths
-        # they run on the next multiple of 128, redirect reads past the last real row to that row and ignore
-        # the padding keys: no tensor is padded or copied here; only what the library keeps for itself (u2,
-        # the row statistics, the backward's workspace) is sized for the padded length.
-        n_pad = -(-N // _SEQ_MULTIPLE) * _SEQ_MULTIPLE
-        # Tensors are read through their strides (the reference passes Q1's and V's to its kernel,
-        # src/kernel.py:487-494): a [B,N,H,d] projection output viewed as [B,H,N,d] is not copied.
-        # The four q/k tensors share one set of strides, as in the reference.
-        q1, q2, k1, k2, v = (_in_place(t) for t in (Q1, Q2, K1, K2, V))
-        if not (q1.stride() == q2.stride() == k1.stride() == k2.stride()):
-            q1, q2, k1, k2 = (t.contiguous() for t in (q1, q2, k1, k2))
-        lam = _lambda_tensor(LAMBDA_SCALE, dev, Q1.dtype, H)
-        rms_norm = bool(rms_norm)
-        flags = ((_FLAG_RMS_NORM if rms_norm else 0) | (_FLAG_CAUSAL if causal else 0)
-                 | (_FLAG_BF16 if Q1.dtype == torch.bfloat16 else 0)
-                 | (_FLAG_LAMBDA_PER_HEAD if lam.numel() > 1 else 0)
-                 | (_FLAG_LAMBDA_FP32 if lam.dtype == torch.float32 else 0)
-                 | (_FLAG_UNPADDED if n_pad != N else 0))
-
-        y = torch.empty_like(v)         # v's layout when v is a permuted dense buffer, else dense
-        layout = None
-        if not (_is_dense(q1) and _is_dense(v) and _is_dense(y)):
-            layout = _native.Layout(*q1.stride()[:3], *v.stride()[:3], *y.stride()[:3], *y.stride()[:3])
-        # what only a backward reads (src/kernel.py:505 saves its counterparts unconditionally) is neither
-        # allocated nor written when no input asks for a gradient, e.g. under torch.no_grad()
         differentiable = any(ctx.needs_input_grad)
-        u2 = lse1 = lse2 = rinv = None
+        (*qkv, lam), (y, u2, lse1, lse2, rinv, flags, n_pad) = _run_forward(
+            Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_norm, causal, dropout_p, dropout_seed, differentiable)
         if differentiable:
-            u2 = torch.empty((B, H, n_pad, 2 * D), device=dev, dtype=v.dtype)
-            # the two logsumexps and the RMSNorm statistic share one allocation
-            stats = torch.empty((3 if rms_norm else 2, B, H, n_pad), device=dev, dtype=torch.float32)
-            lse1, lse2 = stats[0], stats[1]
-            rinv = stats[2] if rms_norm else None
-
-        if dev.index is not None and dev.index != torch._C._cuda_getDevice():
-            with torch.cuda.device(dev):
-                rc = lib.diffattn_forward_padded(
-                    q1.data_ptr(), q2.data_ptr(), k1.data_ptr(), k2.data_ptr(), v.data_ptr(),
-                    lam.data_ptr(), y.data_ptr(), _ptr(u2), _ptr(lse1), _ptr(lse2), _ptr(rinv),
-                    B, H, n_pad, N, D, float(SM_SCALE), float(LAMBDA_INIT), flags, layout, dropout, _current_stream(dev))
-        else:
-            rc = lib.diffattn_forward_padded(
-                q1.data_ptr(), q2.data_ptr(), k1.data_ptr(), k2.data_ptr(), v.data_ptr(),
-                lam.data_ptr(), y.data_ptr(), _ptr(u2), _ptr(lse1), _ptr(lse2), _ptr(rinv),
-                B, H, n_pad, N, D, float(SM_SCALE), float(LAMBDA_INIT), flags, layout, dropout, _current_stream(dev))
-        _native.check(rc)
-
-        if differentiable:
-            ctx.save_for_backward(q1, q2, k1, k2, v, y, u2, lse1, lse2, rinv, lam)
+            ctx.save_for_backward(*qkv, y, u2, lse1, lse2, rinv, lam)
         ctx.SM_SCALE = float(SM_SCALE)
         ctx.LAMBDA_INIT = float(LAMBDA_INIT)
         ctx.FLAGS = flags
         ctx.N_PAD = n_pad
-        ctx.DROPOUT = dropout
+        # the same dropout goes to the backward: the masks are a function of (seed, position) only
+        ctx.DROPOUT = (float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF)
         ctx.lambda_meta = (LAMBDA_SCALE.dtype, LAMBDA_SCALE.shape) if torch.is_tensor(LAMBDA_SCALE) else None
         return y
 
     @staticmethod
     @once_differentiable        # the gradients are plain kernel outputs: a second derivative raises
     def backward(ctx, dO):
-        q1, q2, k1, k2, v, y, u2, lse1, lse2, rinv, lam = ctx.saved_tensors
-        B, H, N, D = q1.shape
-        n_pad = ctx.N_PAD
-        lib = _native.lib()
-        dev = q1.device
-        if dO.dtype != q1.dtype:
-            dO = dO.to(q1.dtype)
-        dO = _in_place(dO)
-
+        saved = ctx.saved_tensors
+        dev = saved[0].device
         # only the kernels whose outputs some input asked for are launched (stage bits of the C ABI:
         # 1 row preprocess, 2 d(lambda) reduction, 4 dK/dV, 8 dQ)
         need = ctx.needs_input_grad
-        want_q, want_kv = need[0] or need[1], need[2] or need[3] or need[4]
         want_lam = ctx.lambda_meta is not None and need[6]
-        stages = 1 | (2 if want_lam else 0) | (4 if want_kv else 0) | (8 if want_q else 0)
-        # Gradients are written in the memory layout of the tensors they belong to (autograd would otherwise
-        # copy each one into its leaf's layout).  The four q/k gradients share one set of strides, like q1..k2.
-        dq1 = dq2 = dk1 = dk2 = dv = None
-        if want_q:
-            dq1, dq2 = _grad_like(q1), _grad_like(q1)
-        if want_kv:
-            dk1, dk2, dv = _grad_like(q1), _grad_like(q1), _grad_like(v)
-        gqk = dq1 if want_q else dk1        # (a view that is not a permuted dense buffer gets a dense gradient)
-        layout = None
-        if not (_is_dense(q1) and _is_dense(v) and _is_dense(y) and _is_dense(dO)):
-            layout = _native.Layout(*q1.stride()[:3], *v.stride()[:3], *y.stride()[:3], *dO.stride()[:3],
-                                    *(gqk.stride()[:3] if gqk is not None else (0, 0, 0)),
-                                    *(dv.stride()[:3] if dv is not None else (0, 0, 0)))
-        dlam = torch.empty(lam.numel(), device=dev, dtype=lam.dtype) if want_lam else None
-        ws_bytes = lib.diffattn_backward_workspace_bytes(B, H, n_pad, D, ctx.FLAGS)
-        ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+        stages = (1 | (2 if want_lam else 0) | (4 if need[2] or need[3] or need[4] else 0)
+                  | (8 if need[0] or need[1] else 0))
 
         def launch():
-            return lib.diffattn_backward_stages(
-                q1.data_ptr(), q2.data_ptr(), k1.data_ptr(), k2.data_ptr(), v.data_ptr(), lam.data_ptr(),
-                y.data_ptr(), u2.data_ptr(), lse1.data_ptr(), lse2.data_ptr(), _ptr(rinv), dO.data_ptr(),
-                _ptr(dq1), _ptr(dq2), _ptr(dk1), _ptr(dk2), _ptr(dv), _ptr(dlam),
-                ws.data_ptr(), ws_bytes, B, H, n_pad, N, D, ctx.SM_SCALE, ctx.LAMBDA_INIT, ctx.FLAGS, stages,
-                layout, ctx.DROPOUT, _current_stream(dev))
+            return _native.host().backward(*saved, dO, ctx.SM_SCALE, ctx.LAMBDA_INIT, ctx.FLAGS, ctx.N_PAD, *ctx.DROPOUT,
+                                           stages, _current_stream(dev))
 
-        if dev.index is not None and dev.index != torch._C._cuda_getDevice():
+        if dev.index != torch._C._cuda_getDevice():
             with torch.cuda.device(dev):
-                rc = launch()
+                dq1, dq2, dk1, dk2, dv, dlambda = launch()
         else:
-            rc = launch()
-        _native.check(rc)
-
-        dlambda = None
+            dq1, dq2, dk1, dk2, dv, dlambda = launch()
         if want_lam:
             dtype, shape = ctx.lambda_meta
-            dlambda = dlam.to(dtype).reshape(shape)
+            if dlambda.dtype != dtype or dlambda.shape != shape:
+                dlambda = dlambda.to(dtype).reshape(shape)
         # one slot per forward argument: nine, or more when causal / dropout arguments were passed
         return (dq1, dq2, dk1, dk2, dv, None, dlambda) + (None,) * (len(ctx.needs_input_grad) - 7)
+
+
+def diff_attention(*args):
+    """`_diff_attention.apply`, without the autograd machinery where nothing can ask for it: gradients are off, and no
+    transform, tracer, compiler, dispatch mode or forward-mode level is active.  (B1 H16 N77 D64 forward: about a third of
+    the call's host time.)"""
+    if (torch.is_grad_enabled() or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
+        return _diff_attention.apply(*args)
+    args += (False, False, 0.0, 0)[len(args) - 8:]
+    return _run_forward(*args, False)[1][0]

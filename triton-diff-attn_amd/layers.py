@@ -3,7 +3,7 @@ import math
 
 import torch
 
-from kernel import _diff_attention
+from kernel import diff_attention
 # stock-PyTorch comparison lines under the names the reference's benchmark imports from this
 # module (src/benchmark.py:11-17); none of them is used by MultiheadDiffAttnKernel
 from baselines import MultiheadAttn, MultiheadDiffAttn, MultiheadFlashAttn, MultiheadFlashDiffAttn  # noqa: F401
@@ -46,8 +46,8 @@ def MultiheadDiffAttnKernel(
                 raise RuntimeError("dropout under stream capture needs an explicit dropout_seed (the same masks are "
                                    "then applied on every replay of the graph)")
             dropout_seed = int(torch.randint(0, 2 ** 62, (1,)).item())
-        return _diff_attention.apply(q1, q2, k1, k2, v, sm_scale, lambda_scale, lambda_init, rms_norm, bool(causal),
-                                     float(dropout_p), int(dropout_seed))
+        return diff_attention(q1, q2, k1, k2, v, sm_scale, lambda_scale, lambda_init, rms_norm, bool(causal),
+                              float(dropout_p), int(dropout_seed))
     if causal:
-        return _diff_attention.apply(q1, q2, k1, k2, v, sm_scale, lambda_scale, lambda_init, rms_norm, True)
-    return _diff_attention.apply(q1, q2, k1, k2, v, sm_scale, lambda_scale, lambda_init, rms_norm)
+        return diff_attention(q1, q2, k1, k2, v, sm_scale, lambda_scale, lambda_init, rms_norm, True)
+    return diff_attention(q1, q2, k1, k2, v, sm_scale, lambda_scale, lambda_init, rms_norm)
