@@ -50,6 +50,12 @@ PyObject* library_error(int rc) {
   return PyErr_Format(PyExc_RuntimeError, "libdiffattn: %s (code %d)", diffattn_strerror(rc), rc);
 }
 
+// Other threads run while a call allocates and launches: either may wait for the device.
+struct Released {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Released() { PyEval_RestoreThread(state); }
+};
+
 bool numbers_ok() { return !PyErr_Occurred(); }
 
 // forward(q1, q2, k1, k2, v, lambda, sm_scale, lambda_init, flags, dropout_p, dropout_seed, differentiable, device, stream)
@@ -91,22 +97,27 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (lam.numel() > 1) flags |= DIFFATTN_LAMBDA_PER_HEAD;
   if (lam.scalar_type() == at::kFloat) flags |= DIFFATTN_LAMBDA_FP32;
   if (n_pad != N) flags |= DIFFATTN_UNPADDED;
-  at::Tensor y = at::empty_like(v), u2, lse1, lse2, rinv;      // y in v's layout when v is a permuted dense buffer, else dense
-  if (differentiable) {
-    u2 = at::empty({B, H, n_pad, 2 * D}, v.options());
-    // the two logsumexps and the norm statistic share one allocation
-    at::Tensor stats = at::empty({rms ? 3 : 2, B, H, n_pad}, v.options().dtype(at::kFloat));
-    lse1 = stats.select(0, 0); lse2 = stats.select(0, 1);
-    if (rms) rinv = stats.select(0, 2);
+  at::Tensor y, u2, lse1, lse2, rinv;
+  int rc;
+  {
+    const Released released;
+    y = at::empty_like(v);                                     // in v's layout when v is a permuted dense buffer, else dense
+    if (differentiable) {
+      u2 = at::empty({B, H, n_pad, 2 * D}, v.options());
+      // the two logsumexps and the norm statistic share one allocation
+      at::Tensor stats = at::empty({rms ? 3 : 2, B, H, n_pad}, v.options().dtype(at::kFloat));
+      lse1 = stats.select(0, 0); lse2 = stats.select(0, 1);
+      if (rms) rinv = stats.select(0, 2);
+    }
+    diffattn_layout layout = {};
+    const bool dense = is_dense(q[0]) && is_dense(v) && is_dense(y);
+    if (!dense) { put(&layout.qk_b, q[0]); put(&layout.v_b, v); put(&layout.y_b, y); put(&layout.dy_b, y); }
+    const diffattn_dropout drop = {(float)p, seed};
+    rc = diffattn_forward_padded(q[0].data_ptr(), q[1].data_ptr(), q[2].data_ptr(), q[3].data_ptr(), v.data_ptr(),
+                                 lam.data_ptr(), y.data_ptr(), ptr(u2), (float*)ptr(lse1), (float*)ptr(lse2), (float*)ptr(rinv),
+                                 (int)B, (int)H, (int)n_pad, (int)N, (int)D, (float)sm_scale, (float)lambda_init, flags,
+                                 dense ? nullptr : &layout, p > 0 ? &drop : nullptr, stream);
   }
-  diffattn_layout layout = {};
-  const bool dense = is_dense(q[0]) && is_dense(v) && is_dense(y);
-  if (!dense) { put(&layout.qk_b, q[0]); put(&layout.v_b, v); put(&layout.y_b, y); put(&layout.dy_b, y); }
-  const diffattn_dropout drop = {(float)p, seed};
-  const int rc = diffattn_forward_padded(q[0].data_ptr(), q[1].data_ptr(), q[2].data_ptr(), q[3].data_ptr(), v.data_ptr(),
-                                         lam.data_ptr(), y.data_ptr(), ptr(u2), (float*)ptr(lse1), (float*)ptr(lse2), (float*)ptr(rinv),
-                                         (int)B, (int)H, (int)n_pad, (int)N, (int)D, (float)sm_scale, (float)lambda_init, flags,
-                                         dense ? nullptr : &layout, p > 0 ? &drop : nullptr, stream);
   if (rc != DIFFATTN_OK) return library_error(rc);
   return Py_BuildValue("(NNNNNiL)", wrap(y), wrap(u2), wrap(lse1), wrap(lse2), wrap(rinv), flags, (long long)n_pad);
   END_HANDLE_TH_ERRORS
@@ -134,31 +145,35 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* const stream = PyLong_AsVoidPtr(a[19]);
   if (!numbers_ok()) return nullptr;
 
-  at::Tensor dy = t[11];
-  if (dy.scalar_type() != q1.scalar_type()) dy = dy.to(q1.scalar_type());
-  if (!strides_ok(dy)) dy = dy.contiguous();
-  const int64_t B = q1.size(0), H = q1.size(1), N = q1.size(2), D = q1.size(3);
-  const bool want_kv = stages & DIFFATTN_STAGE_DKDV, want_q = stages & DIFFATTN_STAGE_DQ;
   at::Tensor dq1, dq2, dk1, dk2, dv, dlam;
-  if (want_q) { dq1 = at::empty_like(q1); dq2 = at::empty_like(q1); }
-  if (want_kv) { dk1 = at::empty_like(q1); dk2 = at::empty_like(q1); dv = at::empty_like(v); }
-  if (stages & DIFFATTN_STAGE_DLAMBDA) dlam = at::empty({lam.numel()}, lam.options());
-  diffattn_layout layout = {};
-  const bool dense = is_dense(q1) && is_dense(v) && is_dense(y) && is_dense(dy);
-  if (!dense) {
-    put(&layout.qk_b, q1); put(&layout.v_b, v); put(&layout.y_b, y); put(&layout.dy_b, dy);
-    if (want_q || want_kv) put(&layout.dqk_b, want_q ? dq1 : dk1);   // (of a view that is not a permuted dense buffer: dense)
-    if (want_kv) put(&layout.dv_b, dv);
+  int rc;
+  {
+    const Released released;
+    at::Tensor dy = t[11];
+    if (dy.scalar_type() != q1.scalar_type()) dy = dy.to(q1.scalar_type());
+    if (!strides_ok(dy)) dy = dy.contiguous();
+    const int64_t B = q1.size(0), H = q1.size(1), N = q1.size(2), D = q1.size(3);
+    const bool want_kv = stages & DIFFATTN_STAGE_DKDV, want_q = stages & DIFFATTN_STAGE_DQ;
+    if (want_q) { dq1 = at::empty_like(q1); dq2 = at::empty_like(q1); }
+    if (want_kv) { dk1 = at::empty_like(q1); dk2 = at::empty_like(q1); dv = at::empty_like(v); }
+    if (stages & DIFFATTN_STAGE_DLAMBDA) dlam = at::empty({lam.numel()}, lam.options());
+    diffattn_layout layout = {};
+    const bool dense = is_dense(q1) && is_dense(v) && is_dense(y) && is_dense(dy);
+    if (!dense) {
+      put(&layout.qk_b, q1); put(&layout.v_b, v); put(&layout.y_b, y); put(&layout.dy_b, dy);
+      if (want_q || want_kv) put(&layout.dqk_b, want_q ? dq1 : dk1);   // (of a view that is not a permuted dense buffer: dense)
+      if (want_kv) put(&layout.dv_b, dv);
+    }
+    const size_t ws_bytes = diffattn_backward_workspace_bytes((int)B, (int)H, (int)n_pad, (int)D, flags);
+    at::Tensor ws = at::empty({(int64_t)ws_bytes}, q1.options().dtype(at::kByte));
+    const diffattn_dropout drop = {(float)p, seed};
+    rc = diffattn_backward_stages(q1.data_ptr(), t[1].data_ptr(), t[2].data_ptr(), t[3].data_ptr(), v.data_ptr(),
+                                  lam.data_ptr(), y.data_ptr(), u2.data_ptr(), (const float*)lse1.data_ptr(),
+                                  (const float*)lse2.data_ptr(), (const float*)ptr(rinv), dy.data_ptr(),
+                                  ptr(dq1), ptr(dq2), ptr(dk1), ptr(dk2), ptr(dv), ptr(dlam), ws.data_ptr(), ws_bytes,
+                                  (int)B, (int)H, (int)n_pad, (int)N, (int)D, (float)sm_scale, (float)lambda_init, flags,
+                                  stages, dense ? nullptr : &layout, p > 0 ? &drop : nullptr, stream);
   }
-  const size_t ws_bytes = diffattn_backward_workspace_bytes((int)B, (int)H, (int)n_pad, (int)D, flags);
-  at::Tensor ws = at::empty({(int64_t)ws_bytes}, q1.options().dtype(at::kByte));
-  const diffattn_dropout drop = {(float)p, seed};
-  const int rc = diffattn_backward_stages(q1.data_ptr(), t[1].data_ptr(), t[2].data_ptr(), t[3].data_ptr(), v.data_ptr(),
-                                          lam.data_ptr(), y.data_ptr(), u2.data_ptr(), (const float*)lse1.data_ptr(),
-                                          (const float*)lse2.data_ptr(), (const float*)ptr(rinv), dy.data_ptr(),
-                                          ptr(dq1), ptr(dq2), ptr(dk1), ptr(dk2), ptr(dv), ptr(dlam), ws.data_ptr(), ws_bytes,
-                                          (int)B, (int)H, (int)n_pad, (int)N, (int)D, (float)sm_scale, (float)lambda_init, flags,
-                                          stages, dense ? nullptr : &layout, p > 0 ? &drop : nullptr, stream);
   if (rc != DIFFATTN_OK) return library_error(rc);
   return Py_BuildValue("(NNNNNN)", wrap(dq1), wrap(dq2), wrap(dk1), wrap(dk2), wrap(dv), wrap(dlam));
   END_HANDLE_TH_ERRORS
