@@ -18,7 +18,7 @@
 
 namespace DA_NS {
 
-// SMALL: 64 query rows per workgroup (four waves), for problems whose 128-row blocks do not fill the chip and
+// SMALL: 64 query rows per workgroup (four waves), for problems whose 128-row blocks leave much of the chip idle and
 // for the D = 128 instantiations with dropout, which do not fit the register budget of two waves per SIMD.
 template <int D, bool SMALL = false>
 struct FwdCfg {
@@ -159,10 +159,9 @@ void fwd_kernel(FwdParams p) {
   const half_t* gk1 = p.k1 + qk_base;
   const half_t* gk2 = p.k2 + qk_base;
   const half_t* gv = p.v + v_base;
-  // causal: keys beyond the last row of the workgroup are never visited (BM is a multiple of 2*BN,
-  // so the tile count stays even)
-  const int n_tiles = CAUSAL ? (qt + 1) * (BM / BN) : p.N / BN;
-  static_assert(!CAUSAL || BM % (2 * BN) == 0, "an even number of key tiles per query block");
+  // causal: keys beyond the last row of the workgroup are visited only to make the tile count even (64-row
+  // workgroups with 64-key tiles: every other one has a last tile that is masked throughout; N is a multiple of 128)
+  const int n_tiles = CAUSAL ? ((qt + 1) * (BM / BN) + 1) & ~1 : p.N / BN;
   constexpr int VH = (VTile::PER + 1) / 2;   // V instructions are issued in two groups
   const unsigned k_off = KTile::lane_off(wave, lane, qk_n), v_off = VTile::lane_off(wave, lane, v_n);
   auto tail_lane = [&] { return kLean ? lane_again() : lane; };
@@ -596,16 +595,24 @@ static void launch_fwd_c(const FwdParams& p, hipStream_t stream) {
 template <int D>
 static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   const bool drop = p.drop.threshold != 0;
-  const bool plain = !p.causal && !drop && p.n_keys == p.N;
   // Shape-aware launch geometry (the reference autotunes its tiles per (N, D, Dv), src/kernel.py:12-19): a problem
-  // whose 128-row blocks do not fill the chip once runs in twice as many 64-row, four-wave workgroups.  A pure
-  // function of (B*H, N, D) and the options: no tuning state.  At D <= 64 only the plain instantiation has the
-  // small variant.  At D = 128 the masked instantiations gain by the 128-row workgroup from 256 blocks on (us, causal:
-  // B1 H16 N2048 81 -> 75, B1 H32 N2048 159 -> 114, B1 H32 N3001 328 -> 230; N not a multiple of 128: B2 H32 N1000
-  // 142 -> 111), and the dropout instantiations do not fit the 256 registers of the 128-row workgroup
-  // (two waves per SIMD) and always run in 64-row workgroups at one wave per SIMD.
+  // whose 128-row blocks leave half of the chip idle runs in twice as many 64-row, four-wave workgroups.  A pure
+  // function of (B*H, N, D) and the options: no tuning state.  Figures: us of a launch, bf16, 128-row -> 64-row.
+  // Blocks of one length: up to 128 of them (D <= 64, B1 H8 N2000 D64 39.6 -> 33.8, with dropout 57.7 -> 41.1; D32 29.3 ->
+  // 23.3).  The rings of a D >= 64 workgroup fill a CU's LDS whatever its rows, so from 129 on the halves take a second
+  // round (B1 H9 N2048 D64 38.3 -> 56.8, B1 H12 N2048 D64 41.4 -> 56.9, D128 75 -> 105).
+  // Causal blocks differ in length and end with the longest; halves, longest first, are shorter and dealt more
+  // evenly, and the last CUs need not wait for a second round.  D32, two workgroups to a CU: up to 256 (B1 H8 N2048 29.0 ->
+  // 22.4, B1 H16 N2048 29.4 -> 25.3).  D64: up to 256 too (B1 H8 N2048 38.9 -> 30.6, B1 H16 N2048 41.3 -> 39.0, B1 H4
+  // N8192 139 -> 116; 384 blocks 46 -> 61), where a unit is short up to 192 (B1 H18 N1024 23.9 -> 19.7, B1 H24 N1000 24.3
+  // -> 24.1, B1 H31 N1024 27.5 -> 31.2).  D128: below 256 (B1 H16 N2048 75 -> 81, B1 H9 N2048 67 -> 57; B1 H32 N3001
+  // 230 -> 328).
+  // The D = 128 dropout instantiations do not fit the 256 registers of the 128-row workgroup (two waves per SIMD) and
+  // always run in 64-row workgroups at one wave per SIMD.
   constexpr int kNumCU = 256;
-  const bool small_grid = (long long)p.BH * (p.N / 128) < kNumCU;
+  const long long blocks = (long long)p.BH * (p.N / 128);
+  const int causal_limit = D == 128 ? kNumCU - 1 : D == 32 || p.N >= 2048 ? kNumCU : kNumCU * 3 / 4;
+  const bool small_grid = blocks <= (p.causal ? causal_limit : kNumCU / 2);
   if constexpr (D == 128) {
     if (drop) {
       if (p.rms_norm) launch_fwd_c<D, true, true, true>(p, stream); else launch_fwd_c<D, false, true, true>(p, stream);
@@ -616,14 +623,14 @@ static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
     }
     return hipGetLastError();
   } else {
-    if (plain && small_grid) {
-      const dim3 sgrid(p.BH * (p.N / FwdCfg<D, true>::BM)), sblock(FwdCfg<D, true>::NT);
-      if (p.rms_norm) hipLaunchKernelGGL((fwd_kernel<D, true, 0, false, true>), sgrid, sblock, 0, stream, p);
-      else            hipLaunchKernelGGL((fwd_kernel<D, false, 0, false, true>), sgrid, sblock, 0, stream, p);
-      return hipGetLastError();
-    }
-    if (p.rms_norm) { if (drop) launch_fwd_c<D, true, true, false>(p, stream); else launch_fwd_c<D, true, false, false>(p, stream); }
-    else            { if (drop) launch_fwd_c<D, false, true, false>(p, stream); else launch_fwd_c<D, false, false, false>(p, stream); }
+    auto launch = [&](auto drop_tag, auto small_tag) {
+      constexpr bool DR = decltype(drop_tag)::value, SM = decltype(small_tag)::value;
+      if (p.rms_norm) launch_fwd_c<D, true, DR, SM>(p, stream); else launch_fwd_c<D, false, DR, SM>(p, stream);
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if (small_grid) { if (drop) launch(yes, yes); else launch(no, yes); }
+    else            { if (drop) launch(yes, no); else launch(no, no); }
     return hipGetLastError();
   }
 }
