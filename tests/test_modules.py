@@ -146,3 +146,22 @@ def test_attention_dropout_acts_in_training_mode_only():
     assert torch.isfinite(c).all()
     c.float().square().mean().backward()
     assert all(p.grad is not None and torch.isfinite(p.grad).all() for p in layer.parameters())
+
+
+def test_streams_are_the_same_views_either_way():
+    """The fused operator's q and k come from unbind, a custom attention's from select (it may write them in place): the
+    same values, strides and gradients."""
+    torch.manual_seed(2)
+    fused, custom = modules.DiffAttn(64, 2), modules.DiffAttn(64, 2, attention=lambda *a, **k: None)
+    p = torch.randn(2, 24, 2, 2, 16)
+    grads = []
+    for layer in (fused, custom):
+        leaf = p.clone().requires_grad_(True)
+        a, b = layer._streams(leaf * 1)
+        assert a.stride() == b.stride() == p[:, :, :, 0].transpose(1, 2).stride()
+        assert torch.equal(a, p[:, :, :, 0].transpose(1, 2)) and torch.equal(b, p[:, :, :, 1].transpose(1, 2))
+        if layer is custom:
+            a.mul_(1.0)
+        (a.sin().sum() + (b * a).sum()).backward()
+        grads.append(leaf.grad)
+    assert torch.equal(*grads)
