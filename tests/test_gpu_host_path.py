@@ -81,3 +81,36 @@ def test_what_was_refused_stays_refused():
         # a transform goes to the autograd function, which has no rule for it
         with pytest.raises(RuntimeError):
             torch.func.vmap(lambda q: MultiheadDiffAttnKernel(q, q2, k1, k2, v, 0.5))(q1[None])
+
+
+def _odd(t, dim, stride):
+    """t with another stride for its dimension `dim`, of size 1."""
+    s = list(t.stride())
+    s[dim] = stride
+    return torch.empty_strided(t.shape, s, dtype=t.dtype, device=t.device).copy_(t)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("dim,B,H,N", [(0, 1, 3, 77), (1, 2, 1, 77), (2, 2, 3, 1)])
+def test_strides_of_dimensions_of_size_one_do_not_matter(dim, B, H, N, grad):
+    """Slices of a fused projection, or tensors with any other stride that addresses nothing: the bits of plain copies.
+    (A lambda given as a number takes the call the other way into the extension module.)"""
+    from layers import MultiheadDiffAttnKernel
+    ins = [t.cuda() for t in make_inputs(B, H, N, 64, seed=6)]
+    dy = ins.pop()
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+
+    def run(ins, lam):
+        leaves = [t.detach().requires_grad_(grad) for t in ins]
+        y = MultiheadDiffAttnKernel(*leaves, lam, 0.8, True)
+        if grad:
+            y.backward(dy)
+        return [y.detach()] + [t.grad for t in leaves if grad]
+
+    want = run(ins, lam)
+    wide = lambda i: _odd(ins[i], dim, 2 * ins[i].stride(dim))       # as in a fused projection of two
+    for changed in ({0: wide(0)}, {1: _odd(ins[1], dim, 7)}, {2: _odd(ins[2], dim, 8)}, {3: wide(3)},
+                    {0: wide(0), 1: wide(1), 3: _odd(ins[3], dim, 1 << 20)}):
+        mixed = [changed.get(i, t) for i, t in enumerate(ins)]
+        for l in (lam, 0.5):
+            assert all(torch.equal(a, b) for a, b in zip(run(mixed, l), want)), changed.keys()

@@ -14,12 +14,23 @@ namespace {
 
 constexpr int64_t kSeqMultiple = 128;
 
+bool aligned(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
 // Whether the kernels can read t in place: contiguous rows, every other stride a non-negative multiple of 8 elements
 // (16-byte aligned rows), base pointer 16-byte aligned.
 bool strides_ok(const at::Tensor& t) {
   const auto s = t.strides();
   return s[3] == 1 && s[2] >= t.size(3) && s[2] % 8 == 0 && s[0] % 8 == 0 && s[1] % 8 == 0 && s[0] >= 0 && s[1] >= 0 &&
-         s[2] <= (int64_t(1) << 26) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+         s[2] <= (int64_t(1) << 26) && aligned(t);
+}
+
+// Whether b's elements lie where a's do, each from its base pointer: equal sizes and strides, but for the strides of
+// dimensions of size 1, which address nothing (a slice of a fused [1, 2, H, N, d] projection keeps the stride of the whole).
+bool same_layout(const at::Tensor& a, const at::Tensor& b) {
+  if (a.sizes() != b.sizes()) return false;
+  for (int64_t i = 0; i < a.dim(); ++i)
+    if (a.size(i) != 1 && a.stride(i) != b.stride(i)) return false;
+  return true;
 }
 
 bool is_dense(const at::Tensor& t) {
@@ -81,10 +92,11 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const auto type = q[0].scalar_type();
   if (type != at::kHalf && type != at::kBFloat16) Py_RETURN_NONE;
   for (const at::Tensor* t : {&q[0], &q[1], &q[2], &q[3], &v})
-    if (t->scalar_type() != type || t->dim() != 4 || !t->is_cuda() || t->get_device() != device || !strides_ok(*t)) Py_RETURN_NONE;
+    if (t->scalar_type() != type || t->dim() != 4 || !t->is_cuda() || t->get_device() != device) Py_RETURN_NONE;
   const int64_t B = q[0].size(0), H = q[0].size(1), N = q[0].size(2), D = q[0].size(3);
-  for (int i = 1; i < 4; ++i)
-    if (q[i].sizes() != q[0].sizes() || q[i].strides() != q[0].strides()) Py_RETURN_NONE;
+  if (!strides_ok(q[0]) || !strides_ok(v)) Py_RETURN_NONE;
+  for (int i = 1; i < 4; ++i)       // the four q/k tensors are read through the strides of the first
+    if (!same_layout(q[0], q[i]) || !aligned(q[i])) Py_RETURN_NONE;
   if (v.size(0) != B || v.size(1) != H || v.size(2) != N || v.size(3) != 2 * D || (D != 32 && D != 64 && D != 128) || N < 1) Py_RETURN_NONE;
   if (B > INT32_MAX || H > INT32_MAX || N > INT32_MAX - kSeqMultiple) Py_RETURN_NONE;
   if (!lam.is_cuda() || lam.get_device() != device || (lam.scalar_type() != type && lam.scalar_type() != at::kFloat) ||
