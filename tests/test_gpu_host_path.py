@@ -114,3 +114,15 @@ def test_strides_of_dimensions_of_size_one_do_not_matter(dim, B, H, N, grad):
         mixed = [changed.get(i, t) for i, t in enumerate(ins)]
         for l in (lam, 0.5):
             assert all(torch.equal(a, b) for a, b in zip(run(mixed, l), want)), changed.keys()
+
+
+@pytest.mark.parametrize("which", [0, 4])
+def test_a_refusal_says_what_is_wrong(which):
+    """Strides that a copy does not change (torch calls the tensor contiguous as it is) are refused as strides, pointers as
+    pointers."""
+    from layers import MultiheadDiffAttnKernel
+    ins = [t.cuda() for t in make_inputs(2, 3, 1, 64, seed=6)][:5]
+    t = ins[which]
+    for bad, message in ((_odd(t, 2, 8), "strides"), (torch.empty(t.numel() + 1, device="cuda", dtype=t.dtype)[1:].view_as(t), "16-byte aligned")):
+        with pytest.raises(RuntimeError, match=message):
+            MultiheadDiffAttnKernel(*ins[:which], bad, *ins[which + 1:], 0.5)

@@ -69,13 +69,16 @@ struct Released {
 
 bool numbers_ok() { return !PyErr_Occurred(); }
 
-// forward(q1, q2, k1, k2, v, lambda, sm_scale, lambda_init, flags, dropout_p, dropout_seed, differentiable, device, stream)
+// forward(q1, q2, k1, k2, v, lambda, sm_scale, lambda_init, flags, dropout_p, dropout_seed, differentiable, device, stream,
+//         as_is)
 //   -> None when an input is not what the kernels read in place, else (y, u2, lse1, lse2, rinv, flags, n_pad)
+// `as_is`: the caller has copied what copying helps; strides or pointers that the kernels still cannot read go to the library,
+// whose refusal says what is wrong with them.
 // u2, the two logsumexps and, with rms_norm, the norm statistic are what only a backward reads: None unless
 // `differentiable`.  `flags`: DIFFATTN_RMS_NORM and DIFFATTN_CAUSAL from the caller, the others are added here.
 PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 14) return PyErr_Format(PyExc_TypeError, "forward takes 14 arguments");
+  if (n != 15) return PyErr_Format(PyExc_TypeError, "forward takes 15 arguments");
   at::Tensor q[4], v, lam;
   for (int i = 0; i < 4; ++i)
     if (!unpack(a[i], q[i])) Py_RETURN_NONE;
@@ -87,6 +90,7 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const bool differentiable = PyObject_IsTrue(a[11]) == 1;
   const long device = PyLong_AsLong(a[12]);
   void* const stream = PyLong_AsVoidPtr(a[13]);
+  const bool as_is = PyObject_IsTrue(a[14]) == 1;
   if (!numbers_ok()) return nullptr;
 
   const auto type = q[0].scalar_type();
@@ -94,9 +98,9 @@ PyObject* forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (const at::Tensor* t : {&q[0], &q[1], &q[2], &q[3], &v})
     if (t->scalar_type() != type || t->dim() != 4 || !t->is_cuda() || t->get_device() != device) Py_RETURN_NONE;
   const int64_t B = q[0].size(0), H = q[0].size(1), N = q[0].size(2), D = q[0].size(3);
-  if (!strides_ok(q[0]) || !strides_ok(v)) Py_RETURN_NONE;
+  if (!as_is && !(strides_ok(q[0]) && strides_ok(v))) Py_RETURN_NONE;
   for (int i = 1; i < 4; ++i)       // the four q/k tensors are read through the strides of the first
-    if (!same_layout(q[0], q[i]) || !aligned(q[i])) Py_RETURN_NONE;
+    if (!same_layout(q[0], q[i]) || !(as_is || aligned(q[i]))) Py_RETURN_NONE;
   if (v.size(0) != B || v.size(1) != H || v.size(2) != N || v.size(3) != 2 * D || (D != 32 && D != 64 && D != 128) || N < 1) Py_RETURN_NONE;
   if (B > INT32_MAX || H > INT32_MAX || N > INT32_MAX - kSeqMultiple) Py_RETURN_NONE;
   if (!lam.is_cuda() || lam.get_device() != device || (lam.scalar_type() != type && lam.scalar_type() != at::kFloat) ||

@@ -112,7 +112,7 @@ def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_nor
     if p_ok and torch.is_tensor(Q1) and Q1.is_cuda:
         dev = torch._C._cuda_getDevice()
         out = forward(Q1, Q2, K1, K2, V, LAMBDA_SCALE, SM_SCALE, LAMBDA_INIT, flags, dropout_p, dropout_seed, differentiable,
-                      dev, torch._C._cuda_getCurrentRawStream(dev))
+                      dev, torch._C._cuda_getCurrentRawStream(dev), False)
         if out is not None:
             return (Q1, Q2, K1, K2, V, LAMBDA_SCALE), out
     # something about the inputs stands in the way: an error, a layout, another device, a lambda to be converted
@@ -126,9 +126,9 @@ def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_nor
     lam = _lambda_tensor(LAMBDA_SCALE, dev, Q1.dtype, H)
     with torch.cuda.device(dev):
         out = forward(q1, q2, k1, k2, v, lam, SM_SCALE, LAMBDA_INIT, flags, dropout_p, dropout_seed, differentiable,
-                      q1.get_device(), _current_stream(dev))
+                      q1.get_device(), _current_stream(dev), True)
     if out is None:
-        raise RuntimeError("the kernels cannot read these tensors: their pointers must be 16-byte aligned")
+        raise RuntimeError("tensors of this size are out of the kernels' range")
     return (q1, q2, k1, k2, v, lam), out
 
 
