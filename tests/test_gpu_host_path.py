@@ -126,3 +126,16 @@ def test_a_refusal_says_what_is_wrong(which):
     for bad, message in ((_odd(t, 2, 8), "strides"), (torch.empty(t.numel() + 1, device="cuda", dtype=t.dtype)[1:].view_as(t), "16-byte aligned")):
         with pytest.raises(RuntimeError, match=message):
             MultiheadDiffAttnKernel(*ins[:which], bad, *ins[which + 1:], 0.5)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_without_dropout_the_seed_is_not_looked_at(grad):
+    from kernel import _diff_attention
+    ins = [t.requires_grad_(grad) for t in _tensors()[:5]]
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+    want = _diff_attention.apply(*ins, 0.125, lam, 0.8, True)
+    for seed in (None, "unused", float("nan")):
+        y = _diff_attention.apply(*ins, 0.125, lam, 0.8, True, False, 0.0, seed)
+        assert torch.equal(y, want)
+        if grad:
+            y.backward(torch.ones_like(y))

@@ -93,6 +93,12 @@ def _lambda_tensor(lambda_scale, device, dtype=torch.float16, num_heads=1):
     return torch.tensor([float(lambda_scale)], dtype=dtype, device=device)
 
 
+def _dropout(p, seed):
+    """The two dropout arguments as the extension module takes them.  Without dropout there is no seed to look at."""
+    p = float(p)
+    return p, int(seed) & 0xFFFFFFFFFFFFFFFF if p > 0 else 0
+
+
 def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_norm, causal, dropout_p, dropout_seed,
                  differentiable):
     """One forward launch on the current stream.  Returns (inputs as the kernels read them: q1, q2, k1, k2, v, lambda),
@@ -105,7 +111,7 @@ def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_nor
     kernel, src/kernel.py:487-494): a [B,N,H,d] projection output viewed as [B,H,N,d] is not copied.  The four q/k
     tensors share one set of strides, as in the reference.  What only a backward reads (src/kernel.py:505 saves its
     counterparts unconditionally) is neither allocated nor written unless `differentiable`."""
-    dropout_p, dropout_seed = float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF
+    dropout_p, dropout_seed = _dropout(dropout_p, dropout_seed)
     flags = (_FLAG_RMS_NORM if rms_norm else 0) | (_FLAG_CAUSAL if causal else 0)
     forward = _native.host().forward
     p_ok = 0.0 <= dropout_p <= 255 / 256
@@ -147,7 +153,7 @@ class _diff_attention(torch.autograd.Function):
         ctx.FLAGS = flags
         ctx.N_PAD = n_pad
         # the same dropout goes to the backward: the masks are a function of (seed, position) only
-        ctx.DROPOUT = (float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF)
+        ctx.DROPOUT = _dropout(dropout_p, dropout_seed)
         ctx.lambda_meta = (LAMBDA_SCALE.dtype, LAMBDA_SCALE.shape) if torch.is_tensor(LAMBDA_SCALE) else None
         return y
 
