@@ -139,3 +139,13 @@ def test_without_dropout_the_seed_is_not_looked_at(grad):
         assert torch.equal(y, want)
         if grad:
             y.backward(torch.ones_like(y))
+
+
+def test_scales_are_whatever_float_takes():
+    import numpy as np
+    from kernel import _diff_attention
+    ins = _tensors()[:5]
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+    want = _diff_attention.apply(*ins, 0.125, lam, 0.75, True)
+    for sm_scale, lambda_init in (("0.125", "0.75"), (np.float64(0.125), np.float32(0.75)), (torch.tensor(0.125), torch.tensor([0.75], device="cuda"))):
+        assert torch.equal(_diff_attention.apply(*ins, sm_scale, lam, lambda_init, True), want)

@@ -111,6 +111,7 @@ def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_nor
     kernel, src/kernel.py:487-494): a [B,N,H,d] projection output viewed as [B,H,N,d] is not copied.  The four q/k
     tensors share one set of strides, as in the reference.  What only a backward reads (src/kernel.py:505 saves its
     counterparts unconditionally) is neither allocated nor written unless `differentiable`."""
+    SM_SCALE, LAMBDA_INIT = float(SM_SCALE), float(LAMBDA_INIT)
     dropout_p, dropout_seed = _dropout(dropout_p, dropout_seed)
     flags = (_FLAG_RMS_NORM if rms_norm else 0) | (_FLAG_CAUSAL if causal else 0)
     forward = _native.host().forward
