@@ -149,3 +149,39 @@ def test_scales_are_whatever_float_takes():
     want = _diff_attention.apply(*ins, 0.125, lam, 0.75, True)
     for sm_scale, lambda_init in (("0.125", "0.75"), (np.float64(0.125), np.float32(0.75)), (torch.tensor(0.125), torch.tensor([0.75], device="cuda"))):
         assert torch.equal(_diff_attention.apply(*ins, sm_scale, lam, lambda_init, True), want)
+
+
+class _Tagged(torch.Tensor):
+    pass
+
+
+class _Plain(torch.Tensor):
+    """A subclass whose operations return plain tensors."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        with torch._C.DisableTorchFunctionSubclass():
+            return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("lam", [0.5, None])
+def test_a_subclass_of_tensor_is_the_type_of_the_output(lam, grad):
+    from layers import MultiheadDiffAttnKernel
+    ins = _tensors()
+    dy = ins.pop()
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16) if lam is None else lam
+
+    def run(ins):
+        leaves = [t.detach().requires_grad_(grad) for t in ins]
+        with torch.set_grad_enabled(grad):
+            y = MultiheadDiffAttnKernel(*leaves, lam, 0.8, True)
+        if grad:
+            y.backward(dy)
+        return [y] + [t.grad for t in leaves if grad]
+
+    want = run(ins)
+    for given, returned in ((_Tagged, _Tagged), (_Plain, torch.Tensor), (torch.nn.Parameter, torch.Tensor)):
+        got = run(ins[:4] + [ins[4].as_subclass(given) if given is not torch.nn.Parameter else torch.nn.Parameter(ins[4], requires_grad=grad)])
+        assert type(got[0]) is returned and got[0].requires_grad == grad
+        assert all(torch.equal(a.as_subclass(torch.Tensor), b) for a, b in zip(got, want))

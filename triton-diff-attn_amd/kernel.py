@@ -10,6 +10,7 @@ also allocates the outputs; if either is missing the call raises -- there is no 
 import torch
 from torch.autograd import forward_ad
 from torch.autograd.function import once_differentiable
+from torch.overrides import has_torch_function_unary
 
 import _native
 
@@ -99,6 +100,14 @@ def _dropout(p, seed):
     return p, int(seed) & 0xFFFFFFFFFFFFFFFF if p > 0 else 0
 
 
+def _typed_like(V, out):
+    """A forward's outputs with y of the type that torch.empty_like(V) has: for a tensor subclass, what its
+    __torch_function__ makes of it."""
+    if type(V) is not torch.Tensor and has_torch_function_unary(V):
+        return (out[0].as_subclass(type(torch.empty_like(V[:0]))), *out[1:])
+    return out
+
+
 def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_norm, causal, dropout_p, dropout_seed,
                  differentiable):
     """One forward launch on the current stream.  Returns (inputs as the kernels read them: q1, q2, k1, k2, v, lambda),
@@ -121,7 +130,7 @@ def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_nor
         out = forward(Q1, Q2, K1, K2, V, LAMBDA_SCALE, SM_SCALE, LAMBDA_INIT, flags, dropout_p, dropout_seed, differentiable,
                       dev, torch._C._cuda_getCurrentRawStream(dev), False)
         if out is not None:
-            return (Q1, Q2, K1, K2, V, LAMBDA_SCALE), out
+            return (Q1, Q2, K1, K2, V, LAMBDA_SCALE), _typed_like(V, out)
     # something about the inputs stands in the way: an error, a layout, another device, a lambda to be converted
     B, H, N, D = _check_inputs(Q1, Q2, K1, K2, V)
     if not p_ok:
@@ -136,7 +145,7 @@ def _run_forward(Q1, Q2, K1, K2, V, SM_SCALE, LAMBDA_SCALE, LAMBDA_INIT, rms_nor
                       q1.get_device(), _current_stream(dev), True)
     if out is None:
         raise RuntimeError("tensors of this size are out of the kernels' range")
-    return (q1, q2, k1, k2, v, lam), out
+    return (q1, q2, k1, k2, v, lam), _typed_like(V, out)
 
 
 class _diff_attention(torch.autograd.Function):
