@@ -103,7 +103,9 @@ typedef struct diffattn_dropout {
   unsigned long long seed;
 } diffattn_dropout;
 
-/* ABI version of this header; bumped when a signature changes. */
+/* ABI version of this header; bumped when a signature changes.  diffattn_abi_version() is the one the library was built
+ * with: a caller compiled against this header compares the two before its first call. */
+#define DIFFATTN_ABI_VERSION 7
 int diffattn_abi_version(void);
 
 /* Human-readable text for a return code of this library (static storage). */

@@ -3,6 +3,9 @@ argument rejection works without a GPU, and the host wrappers validate their inp
 import ctypes
 import os
 import re
+import shutil
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -31,6 +34,23 @@ def test_library_exports_every_declared_symbol():
         assert hasattr(lib, name), name
         assert name in _native.SYMBOLS, "binding table misses %s" % name
     assert lib.diffattn_abi_version() == 7 == _native.ABI_VERSION
+    assert re.search(r"#define DIFFATTN_ABI_VERSION (\d+)", open(HEADER).read()).group(1) == "7"
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_extension_module_refuses_a_library_of_another_version(tmp_path):
+    """The module finds its library beside itself: here one with the same symbols and a version of its own."""
+    import _native
+    shutil.copy(_native.HOST_PATH, tmp_path / "diffattn_host.so")
+    stub = "int diffattn_abi_version(void) { return VERSION; }\n" + "".join(
+        "int %s(void) { return 0; }\n" % n for n in declared_symbols() if n != "diffattn_abi_version")
+    (tmp_path / "stub.c").write_text(stub)
+    load = "import torch, importlib.util as u; s = u.spec_from_file_location('diffattn_host', %r); u.module_from_spec(s)" % str(tmp_path / "diffattn_host.so")
+    for version, accepted in ((7, True), (6, False), (8, False)):
+        subprocess.run(["g++", "-x", "c", "-shared", "-fPIC", "-DVERSION=%d" % version, str(tmp_path / "stub.c"), "-o", str(tmp_path / "libdiffattn.so")], check=True)
+        run = subprocess.run([sys.executable, "-c", load], capture_output=True, text=True)
+        assert (run.returncode == 0) == accepted, run.stderr
+        assert accepted or "ImportError: libdiffattn has ABI version %d, diffattn_host was built against 7" % version in run.stderr
 
 
 def test_argument_rejection_needs_no_gpu():

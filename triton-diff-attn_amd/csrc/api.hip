@@ -193,7 +193,7 @@ void fill_bwd(da_abi::BwdParamsT<T>& p, const void* q1, const void* q2, const vo
 
 extern "C" {
 
-int diffattn_abi_version(void) { return 7; }
+int diffattn_abi_version(void) { return DIFFATTN_ABI_VERSION; }
 
 const char* diffattn_strerror(int code) {
   switch (code) {

@@ -204,4 +204,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "diffattn_host", nullptr, -1, metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_diffattn_host(void) { return PyModule_Create(&module); }
+// A module that was built against another version of the library would call it with the wrong arguments.
+PyMODINIT_FUNC PyInit_diffattn_host(void) {
+  if (diffattn_abi_version() != DIFFATTN_ABI_VERSION)
+    return PyErr_Format(PyExc_ImportError, "libdiffattn has ABI version %d, diffattn_host was built against %d: rebuild both",
+                        diffattn_abi_version(), DIFFATTN_ABI_VERSION);
+  return PyModule_Create(&module);
+}
