@@ -29,7 +29,7 @@ def kernel_masks(B, H, n_pad, p, seed):
 def run(cpu, lam_value, lambda_init, rms, causal, p, seed):
     from layers import MultiheadDiffAttnKernel
     leaves = [t.cuda().requires_grad_(True) for t in cpu[:5]]
-    lam = torch.tensor([lam_value], dtype=torch.float16, device="cuda", requires_grad=True)
+    lam = torch.tensor([lam_value], dtype=cpu[0].dtype, device="cuda", requires_grad=True)
     y = MultiheadDiffAttnKernel(*leaves, lambda_scale=lam, lambda_init=lambda_init, rms_norm=rms, causal=causal,
                                 dropout_p=p, dropout_seed=seed)
     y.backward(cpu[5].cuda())
