@@ -65,17 +65,18 @@ def asm_mfma_hazards(asm_text, min_wait=3, lookback=8):
 
 
 def asm_vmem_scalar_hazards(asm_text, min_wait=5, lookback=8):
-    """Inline-assembly memory instructions whose scalar address a vector instruction wrote fewer than `min_wait` wait
-    states before (a v_readlane of a spilled scalar, say): (instruction line, writer line, wait states, writer text).
-    The compiler places these wait states for its own memory instructions only."""
+    """Inline-assembly memory instructions with a scalar operand (the address, or for a direct-to-LDS load the LDS base in
+    m0) that a vector instruction wrote fewer than `min_wait` wait states before (a v_readlane of a spilled scalar, say):
+    (instruction line, writer line, wait states, writer text).  The compiler places these wait states for its own memory
+    instructions only."""
     scalars = lambda t: {i for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", t) for i in range(int(lo), int(hi) + 1)} | \
-        {int(i) for i in re.findall(r"\bs(\d+)\b", t)}
+        {int(i) for i in re.findall(r"\bs(\d+)\b", t)} | set(re.findall(r"\bm0\b", t))
     ins = list(instructions(asm_text))
     found = []
     for i, (n, s, inside) in enumerate(ins):
         if not (inside and s.startswith("global_")):
             continue
-        pending, wait = scalars(s), 0
+        pending, wait = scalars(s) | ({"m0"} if s.startswith("global_load_lds_") else set()), 0
         for n2, s2, _ in reversed(ins[max(0, i - lookback):i]):
             if wait >= min_wait or not pending:
                 break

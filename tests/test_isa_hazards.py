@@ -41,6 +41,11 @@ def test_scanner_flags_a_scalar_address_that_a_vector_instruction_just_wrote():
     assert isa_scan.asm_vmem_scalar_hazards(bad.replace("s_nop 0", "s_nop 3")) == []
     moved = bad.replace("s_nop 0", "s_mov_b64 s[2:3], s[34:35]").replace("v36, s[34:35]", "v36, s[2:3]")
     assert isa_scan.asm_vmem_scalar_hazards(moved) == []
+    # the LDS base in m0 is an operand of the copy too
+    m0 = bad.replace("s_mov_b32 m0, s7", "v_readlane_b32 m0, v254, 39").replace("v_readlane_b32 s35", "v_readlane_b32 s9")
+    assert [f[3] for f in isa_scan.asm_vmem_scalar_hazards(m0)] == ["v_readlane_b32 m0, v254, 39"]
+    assert isa_scan.asm_vmem_scalar_hazards(m0.replace("s_nop 0", "s_nop 4")) == []
+    assert isa_scan.asm_vmem_scalar_hazards(m0.replace("\ts_nop 0\n", "\ts_mov_b32 m0, s7\n")) == []
 
 
 def _load_build():
@@ -53,12 +58,12 @@ def _load_build():
 
 @pytest.fixture(scope="module")
 def assembly(tmp_path_factory):
-    """Assembly text of the three compilations the tests below read (backward fp16 and bf16, forward fp16),
-    compiled side by side."""
+    """Assembly text of the four compilations (backward and forward, fp16 and bf16), compiled side by side."""
     build = _load_build()
     tmp = tmp_path_factory.mktemp("isa")
     jobs = {}
-    for key, src, variant in (("bwd_fp16", "bwd.hip", []), ("bwd_bf16", "bwd.hip", ["-DDA_BF16"]), ("fwd_fp16", "fwd.hip", [])):
+    for key, src, variant in (("bwd_fp16", "bwd.hip", []), ("bwd_bf16", "bwd.hip", ["-DDA_BF16"]), ("fwd_fp16", "fwd.hip", []),
+                              ("fwd_bf16", "fwd.hip", ["-DDA_BF16"])):
         out = tmp / (key + ".s")
         cmd = [build.HIPCC] + [f for f in build.FLAGS if f != "-fPIC"] + build.SOURCE_FLAGS.get(src, []) + variant + ["--cuda-device-only", "-S", "-o", str(out),
                                                                               os.path.join(CSRC, src)]
@@ -89,11 +94,12 @@ def test_backward_kernels_have_no_unprotected_asm_mfma(assembly, variant):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-def test_forward_kernels_do_not_spill_in_their_loops(assembly):
+@pytest.mark.parametrize("variant", ["fp16", "bf16"])
+def test_forward_kernels_do_not_spill_in_their_loops(assembly, variant):
     """The forward instantiations without dropout use no scratch memory at all; those with dropout may
     park a value across the main loop, but never inside it."""
     import re
-    kernels = re.findall(r"^(_Z\w*fwd_kernel\w*):[^\n]*\n(.*?)s_endpgm", assembly["fwd_fp16"], re.S | re.M)
+    kernels = re.findall(r"^(_Z\w*fwd_kernel\w*):[^\n]*\n(.*?)s_endpgm", assembly["fwd_" + variant], re.S | re.M)
     # D <= 64: rms_norm x mask x dropout in 128-row and in 64-row workgroups (24 each);
     # D = 128: rms_norm x mask x dropout in 64-row workgroups plus rms_norm x mask in 128-row ones without dropout (18)
     assert len(kernels) == 66
@@ -112,7 +118,7 @@ def test_forward_kernels_do_not_spill_in_their_loops(assembly):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-@pytest.mark.parametrize("source", ["bwd_fp16", "bwd_bf16", "fwd_fp16"])
+@pytest.mark.parametrize("source", ["bwd_fp16", "bwd_bf16", "fwd_fp16", "fwd_bf16"])
 def test_tile_copies_do_not_read_an_address_too_early(assembly, source):
     """The base of a direct global->LDS copy, an asm statement, may have been reloaded from a vector register's lanes
     right in front of it."""
