@@ -147,18 +147,17 @@ def test_host_validation_errors():
     assert _lambda_tensor(torch.tensor([[0.1], [0.2], [0.3]]), torch.device("cpu"), num_heads=3).dtype == torch.float32
     assert _lambda_tensor(torch.tensor([0.5], dtype=torch.float64), torch.device("cpu"), torch.bfloat16).dtype == torch.bfloat16
     assert _lambda_tensor(0.5, torch.device("cpu"), torch.bfloat16).dtype == torch.bfloat16
-    from kernel import _grad_like, _in_place, _is_dense, _strides_ok
-    x = torch.arange(2 * 3 * 5 * 4, dtype=torch.float16).reshape(2, 3, 5, 4)
+    from kernel import _in_place
+    copied = lambda t: _in_place(t) is not t and _in_place(t).is_contiguous()
     wide = torch.zeros(2, 16, 3, 64, dtype=torch.float16)              # a [B,N,H,C] buffer seen as [B,H,N,C]
-    view = wide.transpose(1, 2)
-    assert _strides_ok(view) and _in_place(view) is view and not _is_dense(view) and _is_dense(wide)
-    assert not _strides_ok(x.transpose(2, 3)) and _in_place(x.transpose(2, 3)).is_contiguous()    # last dim strided
-    # a gradient buffer takes the layout of a permuted dense tensor; for a slice of a longer tensor it is a
-    # compact buffer in the same dimension order: either way its own strides go to the kernels
-    assert _grad_like(view).stride() == view.stride()
-    sliced = _grad_like(wide[:, :8].transpose(1, 2)[:, :, :, :32])
-    assert _strides_ok(sliced) and sliced.stride() == (8 * 3 * 32, 32, 3 * 32, 1)
-    assert not _strides_ok(torch.zeros(2, 3, 5, 36, dtype=torch.float16)[..., :32])               # rows not 16-byte aligned
+    for readable in (wide, wide.transpose(1, 2), wide[:, :8].transpose(1, 2)[:, :, :, :32]):
+        assert _in_place(readable) is readable
+    assert copied(wide.transpose(2, 3))                                # last dim strided
+    assert copied(torch.zeros(2, 3, 5, 36, dtype=torch.float16)[..., :32])      # rows not 16-byte aligned
+    assert copied(torch.zeros(2, 3, 5, 40, dtype=torch.float16)[..., 4:36])     # the first row not 16-byte aligned
+    assert copied(wide[:, :, :1].expand(2, 16, 3, 64))                 # rows on top of each other
+    with pytest.raises(TypeError):
+        _in_place(wide[0])
     lam = _lambda_tensor(0.25, torch.device("cpu"))
     assert lam.dtype == torch.float16 and lam.shape == (1,) and lam.item() == 0.25
 

@@ -56,11 +56,120 @@ def test_inputs_that_need_converting(grad):
     odd[0] = ins[0].transpose(2, 3).contiguous().transpose(2, 3)            # columns, not rows, contiguous
     assert same(run(odd, lam))
     if grad:                                                                # the upstream gradient likewise
-        dense = dy
-        for dy in (dense.float(), dense.transpose(2, 3).contiguous().transpose(2, 3), dense.transpose(0, 1).contiguous().transpose(0, 1)):
+        for other in (dy.transpose(2, 3).contiguous().transpose(2, 3), dy.transpose(0, 1).contiguous().transpose(0, 1)):
             leaves = [t.detach().requires_grad_() for t in ins]
-            MultiheadDiffAttnKernel(*leaves, lam, 0.8, True).backward(dy.to(torch.float16) if dy.dtype == torch.float32 else dy)
+            MultiheadDiffAttnKernel(*leaves, lam, 0.8, True).backward(other)
             assert same([want[0]] + [t.grad for t in leaves])
+
+
+@pytest.mark.parametrize("layout", ["dense", "token-major", "sliced", "long"])
+def test_layouts_of_the_results(layout):
+    """y and dv are written in v's layout and the q/k gradients in q1's where those are permuted dense buffers, else
+    compactly in the same order of dimensions; a leaf's gradient then is the buffer the kernel wrote.  The bits are those of
+    dense tensors."""
+    from layers import MultiheadDiffAttnKernel
+    B, H, N, D = 2, 3, 77, 64
+    dense = _tensors(N)
+    dy = dense.pop()
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+
+    def arranged(t):
+        if layout == "dense":
+            return t
+        C = t.shape[-1]
+        rows, width = (N + 3 if layout == "long" else N), (2 * C if layout == "sliced" else C)
+        buf = torch.zeros(B, rows, H, width, device="cuda", dtype=t.dtype)
+        view = buf.transpose(1, 2)[:, :, :N, :C]
+        view.copy_(t)
+        return view
+
+    def run(ins):
+        leaves = [t.detach().requires_grad_() for t in ins]
+        y = MultiheadDiffAttnKernel(*leaves, lam, 0.8, True)
+        return [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+
+    want = run(dense)
+    ins = [arranged(t) for t in dense]
+    got = run(ins)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    strides = lambda C: (H * N * C, N * C, C, 1) if layout == "dense" else (N * H * C, C, H * C, 1)
+    assert [t.stride() for t in got] == [strides(2 * D)] + [strides(D)] * 4 + [strides(2 * D)]
+
+
+def test_an_upstream_gradient_of_another_type():
+    """autograd hands the operator gradients of its output's type; a caller of the extension module may not."""
+    import _native
+    from kernel import _run_forward
+    ins = _tensors()
+    dy = ins.pop()
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+    (*qkv, lam), (y, u2, lse1, lse2, rinv, flags, n_pad) = _run_forward(*ins, 0.125, lam, 0.8, True, False, 0.0, 0, True)
+    stream = torch.cuda.current_stream().cuda_stream
+    back = lambda g: _native.host().backward(*qkv, y, u2, lse1, lse2, rinv, lam, g, 0.125, 0.8, flags, n_pad, 0.0, 0, 15, stream)
+    assert all(torch.equal(a, b) for a, b in zip(back(dy.float()), back(dy)))
+
+
+def test_other_threads_run_during_a_call():
+    """Two threads on streams of their own get the results of one; and a call into the extension module lets go of the
+    interpreter's lock: with a switch interval that never passes, a waiting thread only runs when the calling one does."""
+    import sys
+    import threading
+    import time
+
+    import _native
+    from layers import MultiheadDiffAttnKernel
+    ins = _tensors(640)
+    dy = ins.pop()
+    lam = torch.full((1,), 0.5, device="cuda", dtype=torch.float16)
+
+    def run():
+        leaves = [t.detach().requires_grad_() for t in ins]
+        y = MultiheadDiffAttnKernel(*leaves, lam, 0.8, True)
+        y.backward(dy)
+        return [y.detach()] + [t.grad for t in leaves]
+
+    want = run()
+    torch.cuda.synchronize()
+    wrong = []
+
+    def worker():
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got = run()
+                stream.synchronize()
+                wrong.extend(i for i, (a, b) in enumerate(zip(got, want)) if not torch.equal(a, b))
+
+    threads = [threading.Thread(target=worker) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+    turns, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(0)
+
+    forward = _native.host().forward
+    dev, stream = torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    try:
+        sys.setswitchinterval(1000.0)       # before the thread first waits for the lock
+        thread.start()
+        seen, deadline = turns[0], time.monotonic() + 20
+        while turns[0] == seen and time.monotonic() < deadline:
+            forward(*ins, lam, 0.125, 0.8, 1, 0.0, 0, False, dev, stream, False)
+        ran = turns[0] != seen
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()
+    assert ran
 
 
 def test_what_was_refused_stays_refused():

@@ -69,6 +69,15 @@ struct Released {
 
 bool numbers_ok() { return !PyErr_Occurred(); }
 
+// readable(t) -> whether the kernels can read the 4-dimensional tensor t in place (strides_ok above)
+PyObject* readable(PyObject*, PyObject* o) {
+  HANDLE_TH_ERRORS
+  at::Tensor t;
+  if (!unpack(o, t) || t.dim() != 4) return PyErr_Format(PyExc_TypeError, "readable takes a tensor of four dimensions");
+  return PyBool_FromLong(strides_ok(t));
+  END_HANDLE_TH_ERRORS
+}
+
 // forward(q1, q2, k1, k2, v, lambda, sm_scale, lambda_init, flags, dropout_p, dropout_seed, differentiable, device, stream,
 //         as_is)
 //   -> None when an input is not what the kernels read in place, else (y, u2, lse1, lse2, rinv, flags, n_pad)
@@ -196,6 +205,7 @@ PyObject* backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 PyMethodDef methods[] = {
+    {"readable", (PyCFunction)readable, METH_O, nullptr},
     {"forward", (PyCFunction)(void (*)())forward, METH_FASTCALL, nullptr},
     {"backward", (PyCFunction)(void (*)())backward, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -50,28 +50,9 @@ def _check_inputs(Q1, Q2, K1, K2, V):
     return B, H, N, D
 
 
-def _strides_ok(t):
-    """Whether the kernels can read t in place: contiguous rows, every other stride a non-negative
-    multiple of 8 elements (16-byte aligned rows), base pointer 16-byte aligned."""
-    sb, sh, sn, sc = t.stride()
-    return (sc == 1 and sn >= t.size(3) and sn % 8 == 0 and sb % 8 == 0 and sh % 8 == 0 and sb >= 0 and sh >= 0
-            and sn <= (1 << 26) and t.data_ptr() % 16 == 0)
-
-
 def _in_place(t):
     """t itself when the kernels can read it through its strides, else a dense copy."""
-    return t if _strides_ok(t) else t.contiguous()
-
-
-def _is_dense(t):
-    B, H, N, C = t.shape
-    return t.stride() == (H * N * C, N * C, C, 1)
-
-
-def _grad_like(t):
-    """An uninitialised gradient buffer in t's memory layout when t is a permuted dense buffer (autograd then
-    takes it as it is instead of copying it into the leaf's layout), else dense."""
-    return torch.empty_like(t)
+    return t if _native.host().readable(t) else t.contiguous()
 
 
 def _current_stream(dev):
