@@ -155,15 +155,17 @@ def test_other_threads_run_during_a_call():
             time.sleep(0)
 
     forward = _native.host().forward
+    row = [t[:1, :1, :1].contiguous() for t in ins]
     dev, stream = torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream
     interval = sys.getswitchinterval()
     thread = threading.Thread(target=other)
     try:
         sys.setswitchinterval(1000.0)       # before the thread first waits for the lock
         thread.start()
-        seen, deadline = turns[0], time.monotonic() + 20
-        while turns[0] == seen and time.monotonic() < deadline:
-            forward(*ins, lam, 0.125, 0.8, 1, 0.0, 0, False, dev, stream, False)
+        # the outputs are kept: freeing a tensor lets go of the lock too
+        outputs, seen, deadline = [], turns[0], time.monotonic() + 10
+        while turns[0] == seen and time.monotonic() < deadline and len(outputs) < 20000:
+            outputs.append(forward(*row, lam, 0.125, 0.8, 1, 0.0, 0, False, dev, stream, False))
         ran = turns[0] != seen
     finally:
         sys.setswitchinterval(interval)
