@@ -1,5 +1,5 @@
-"""The forward in 64-row workgroups and on either side of the lines where 128-row ones take over (csrc/fwd.hip,
-launch_fwd_t), against the fp32 oracle: with 64-key tiles, under the causal mask, every other workgroup has an odd number
+"""The forward in 64-row workgroups and on either side of the lines where 128-row ones take over (csrc/dispatch.hpp,
+fwd_64_rows), against the fp32 oracle: with 64-key tiles, under the causal mask, every other workgroup has an odd number
 of key tiles to see and one more that is masked throughout; lengths end in every part of the last two blocks.  The gradients check the saved row statistics."""
 import pytest
 import torch
@@ -24,10 +24,16 @@ pytestmark = pytest.mark.gpu
     (2, 2, 577, False),
     (1, 5, 1000, True),        # several turns without a test
     (1, 5, 1000, False),
-    (1, 192, 128, True),       # either side of the lines between the two
+    (1, 128, 128, True),       # either side of the lines between the two
+    (1, 129, 128, True),
+    (1, 192, 128, True),
     (1, 193, 128, True),
     (1, 256, 128, True),
     (1, 257, 128, True),
+    (1, 21, 1024, True),
+    (1, 22, 1024, True),
+    (1, 28, 1000, True),
+    (1, 29, 1000, True),
     (1, 16, 2048, True),
     (1, 64, 255, False),
     (1, 129, 100, False),

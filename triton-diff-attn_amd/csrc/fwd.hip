@@ -14,6 +14,7 @@
 //     transposing LDS read, using the same key permutation as the accumulator layout.
 #include <type_traits>
 
+#include "dispatch.hpp"
 #include "params.hpp"
 
 namespace DA_NS {
@@ -595,24 +596,9 @@ static void launch_fwd_c(const FwdParams& p, hipStream_t stream) {
 template <int D>
 static hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   const bool drop = p.drop.threshold != 0;
-  // Shape-aware launch geometry (the reference autotunes its tiles per (N, D, Dv), src/kernel.py:12-19): a problem
-  // whose 128-row blocks leave half of the chip idle runs in twice as many 64-row, four-wave workgroups.  A pure
-  // function of (B*H, N, D) and the options: no tuning state.  Figures: us of a launch, bf16, 128-row -> 64-row.
-  // Blocks of one length: up to 128 of them (D <= 64, B1 H8 N2000 D64 39.6 -> 33.8, with dropout 57.7 -> 41.1; D32 29.3 ->
-  // 23.3).  The rings of a D >= 64 workgroup fill a CU's LDS whatever its rows, so from 129 on the halves take a second
-  // round (B1 H9 N2048 D64 38.3 -> 56.8, B1 H12 N2048 D64 41.4 -> 56.9, D128 75 -> 105).
-  // Causal blocks differ in length and end with the longest; halves, longest first, are shorter and dealt more
-  // evenly, and the last CUs need not wait for a second round.  D32, two workgroups to a CU: up to 256 (B1 H8 N2048 29.0 ->
-  // 22.4, B1 H16 N2048 29.4 -> 25.3).  D64: up to 256 too (B1 H8 N2048 38.9 -> 30.6, B1 H16 N2048 41.3 -> 39.0, B1 H4
-  // N8192 139 -> 116; 384 blocks 46 -> 61), where a unit is short up to 192 (B1 H18 N1024 23.9 -> 19.7, B1 H24 N1000 24.3
-  // -> 24.1, B1 H31 N1024 27.5 -> 31.2).  D128: below 256 (B1 H16 N2048 75 -> 81, B1 H9 N2048 67 -> 57; B1 H32 N3001
-  // 230 -> 328).
   // The D = 128 dropout instantiations do not fit the 256 registers of the 128-row workgroup (two waves per SIMD) and
   // always run in 64-row workgroups at one wave per SIMD.
-  constexpr int kNumCU = 256;
-  const long long blocks = (long long)p.BH * (p.N / 128);
-  const int causal_limit = D == 128 ? kNumCU - 1 : D == 32 || p.N >= 2048 ? kNumCU : kNumCU * 3 / 4;
-  const bool small_grid = blocks <= (p.causal ? causal_limit : kNumCU / 2);
+  const bool small_grid = da_abi::fwd_64_rows(D, p.causal, p.N, (long long)p.BH * (p.N / 128));
   if constexpr (D == 128) {
     if (drop) {
       if (p.rms_norm) launch_fwd_c<D, true, true, true>(p, stream); else launch_fwd_c<D, false, true, true>(p, stream);
