@@ -1,10 +1,11 @@
-"""Backwards whose dK/dV and dQ blocks share one grid (csrc/bwd.hip, one_grid), and the ones just past the line where they
+"""Backwards whose dK/dV and dQ blocks share one grid (csrc/dispatch.hpp, bwd_one_grid), and the ones just past the line where they
 become two launches again, against the fp32 oracle: every head dim, masks, ragged lengths, one block to two rounds of
 blocks, and calls that ask for one kind of gradient only."""
 import pytest
 import torch
 
 from oracle import diff_attn_oracle as orc
+from test_gpu_full_grids import check
 from util import GRAD_RTOL, Y_ATOL, make_inputs, max_abs, rel_to_max, run_kernel
 
 pytestmark = pytest.mark.gpu
@@ -21,7 +22,7 @@ NAMES = ("dq1", "dq2", "dk1", "dk2", "dv", "dlambda")
     (1, 2, 1000, True),        # ragged
     (1, 257, 128, False),      # one block more than there are CUs
     (2, 65, 250, False),       # ragged, a second round
-    (4, 72, 256, True),        # 576 and 578 causal blocks: either side of the line at D <= 64
+    (4, 72, 256, True),
     (1, 289, 256, True),
     (2, 128, 256, False),      # 512 and 514 blocks: either side of the line at D <= 64
     (1, 257, 256, False),
@@ -35,6 +36,18 @@ def test_gradients_match_the_oracle(B, H, N, causal, D):
     # 16-bit rounding of the terms they are summed from
     for name, g, r in zip(NAMES, grads, ref[1:]):
         assert rel_to_max(g, r) <= GRAD_RTOL or max_abs(g, r) <= 2e-3, name
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("H,N", [
+    (216, 256), (217, 256),    # 432 and 434 blocks of two to a unit
+    (144, 512), (145, 512),    # 576 and 580 of four
+    (384, 128), (385, 128),    # single ones (at D = 64 always one grid)
+])
+def test_either_side_of_the_causal_lines(H, N, D):
+    ins = make_inputs(1, H, N, D, seed=1500 + N + D)
+    y, grads = run_kernel(*ins[:5], 0.5, 0.8, True, ins[5], causal=True)
+    check(ins, True, y, grads, causal=True)
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])

@@ -1,4 +1,5 @@
-"""The rule that chooses between the 64-row and the 128-row forward (csrc/dispatch.hpp) against measured times, on the CPU."""
+"""The rules that choose between the 64-row and the 128-row forward and between one grid and two launches of a backward
+(csrc/dispatch.hpp) against measured times, on the CPU."""
 import ctypes
 import os
 import shutil
@@ -9,7 +10,7 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "triton-diff-attn_amd", "csrc")
 
 # (D, causal, N, blocks): us of a launch in 64-row and in 128-row workgroups, fp16, MI355X
-MEASURED = {
+FORWARD = {
     (32, True, 128, 256): (7.6, 7.4), (32, True, 256, 192): (8.2, 9.1), (32, True, 512, 256): (10.4, 12.0),
     (32, True, 1024, 240): (15.6, 18.0), (32, True, 2048, 256): (25.3, 29.7),
     (64, True, 128, 128): (8.6, 9.3), (64, True, 128, 136): (15.0, 9.4), (64, True, 128, 192): (15.2, 9.7),
@@ -30,13 +31,40 @@ MEASURED = {
 }
 
 
-@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-def test_the_forward_takes_the_faster_workgroups(tmp_path):
+# (D, causal, N, blocks): time of the whole backward in two launches over that in one grid, fp16, N a multiple of 256 or D = 32
+BACKWARD = {
+    (32, False, 256, 288): 1.17, (32, False, 512, 512): 0.96, (32, False, 1024, 448): 0.93, (32, False, 1024, 576): 1.20,
+    (32, False, 2048, 640): 1.14, (32, False, 2048, 1024): 0.96, (32, False, 4096, 1088): 1.11,
+    (64, False, 256, 192): 1.13, (64, False, 256, 512): 0.94, (64, False, 512, 544): 1.14, (64, False, 1024, 448): 0.94,
+    (64, False, 2048, 256): 1.12, (64, False, 2048, 576): 1.18, (64, False, 2048, 1024): 0.94, (64, False, 4096, 640): 1.11,
+    (32, True, 128, 288): 1.10, (32, True, 128, 448): 0.91, (32, True, 128, 480): 0.94, (32, True, 128, 672): 0.92,
+    (32, True, 256, 288): 1.11, (32, True, 256, 544): 1.16, (32, True, 256, 640): 1.12, (32, True, 256, 704): 1.07,
+    (64, True, 256, 384): 1.13, (64, True, 256, 512): 0.96, (64, True, 256, 576): 1.14, (64, True, 256, 640): 1.11,
+    (64, True, 256, 704): 1.07, (64, True, 256, 1088): 1.10,
+    (64, True, 512, 192): 1.48, (64, True, 512, 528): 1.07, (64, True, 1024, 288): 1.31, (32, True, 1024, 1024): 0.90,
+    (64, True, 2048, 512): 1.10, (64, True, 2048, 576): 1.06, (64, True, 2048, 1280): 0.95, (64, True, 4096, 480): 1.12,
+}
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    tmp = tmp_path_factory.mktemp("rules")
+    (tmp / "rules.cpp").write_text('#include "dispatch.hpp"\nextern "C" {\n'
+                                   "int fwd(int d, int causal, int n, long long blocks) { return da_abi::fwd_64_rows(d, causal, n, blocks); }\n"
+                                   "int bwd(int d, int causal, int n, long long blocks) { return da_abi::bwd_one_grid(d, false, causal, n, blocks, 15u); }\n}\n")
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I" + CSRC, str(tmp / "rules.cpp"), "-o", str(tmp / "rules.so")], check=True)
+    lib = ctypes.CDLL(str(tmp / "rules.so"))
+    for f in (lib.fwd, lib.bwd):
+        f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_longlong]
+    return lib
+
+
+def test_the_forward_takes_the_faster_workgroups(rules):
     """Of every measured pair the rule takes the faster one, or one that is within the 5 % that such a pair moves by."""
-    (tmp_path / "rule.cpp").write_text('#include "dispatch.hpp"\nextern "C" int rule(int d, int causal, int n, long long blocks)'
-                                       " { return da_abi::fwd_64_rows(d, causal, n, blocks); }\n")
-    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I" + CSRC, str(tmp_path / "rule.cpp"), "-o", str(tmp_path / "rule.so")], check=True)
-    rule = ctypes.CDLL(str(tmp_path / "rule.so")).rule
-    rule.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_longlong]
-    slower = {k: (t64, t128) for k, (t64, t128) in MEASURED.items() if (t64 if rule(*k) else t128) > 1.05 * min(t64, t128)}
-    assert not slower
+    assert not {k: (t64, t128) for k, (t64, t128) in FORWARD.items() if (t64 if rules.fwd(*k) else t128) > 1.05 * min(t64, t128)}
+
+
+def test_the_backward_takes_the_faster_grid(rules):
+    assert not {k: gain for k, gain in BACKWARD.items() if (1 / gain if rules.bwd(*k) else gain) > 1.04}

@@ -17,6 +17,7 @@
 // needed besides it, because U1 = X + lambda U2.
 #include <type_traits>
 
+#include "dispatch.hpp"
 #include "params.hpp"
 
 namespace DA_NS {
@@ -1296,30 +1297,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   dq_block<D, 4, CAUSAL ? 1 : PADDED ? 2 : 0, false, true>(p, wg, p.n_q_wg, (lds_half*)smem);
 }
 
-// Whether a backward goes into one grid (bwd_pair_kernel) instead of a dK/dV and a dQ launch: a pure function of
-// the sizes and options.  At D = 128 always: its dQ blocks are four waves at one wave per SIMD either way.  At
-// D <= 64 the dQ kernel of its own has eight waves and 256 rows, two waves per SIMD, and is the faster one on a full chip
-// (headline size: 437 us against 510), so it is a matter of rounds.  Microseconds per round of 256 workgroups at
-// N = 2048, D = 64, which scale alike with N and D: 79 for key blocks, 64 for query blocks of this kernel, 109 for
-// 256-row blocks of the dQ kernel; a grid that is dealt from one list ends with a partial round of 25.  The line
-// holds over B*H*N/128 = 192 ... 1280 blocks: measured gains of up to 24 % on its near side, up to 6 % on its far side.
-// Causal blocks differ in length and fill the rounds by themselves: the one grid is faster below 576 blocks
-// (by 5 % at 512, 40 % at 256) and slower above 640 (by 2-5 %).
-template <int D>
-static bool one_grid(const BwdParams& p) {
-  if (p.drop.threshold) return false;      // the dropout instantiations are not pipelined
-  if (D == 128) return true;
-  const bool wide = p.N % 256 == 0;        // the dQ kernel of its own has its 256-row blocks
-  // N an odd multiple of 128: its 128-row variant has one wave per SIMD at D = 64 (LDS), and this one is pipelined
-  if (D == 64 && !wide && (p.stages & 8u)) return true;
-  const long long blocks = (long long)p.BH * (p.N / 128);
-  if ((p.stages & 12u) != 12u) return blocks <= 256;
-  if (p.causal) return blocks <= 576;
-  const long long two = 79 * ((blocks + 255) / 256) + 109 * ((blocks + 511) / 512);
-  const long long one = (D == 32 ? 150 : 143) * blocks / 256 + 25;
-  return one < two;
-}
-
 template <int D>
 static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
   BwdParams p = p_in;
@@ -1343,7 +1320,7 @@ static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
   }
   if (!(p.stages & 12u)) return e;
   const bool padded = p.n_keys < p.N;
-  if (one_grid<D>(p)) {
+  if (da_abi::bwd_one_grid(D, p.drop.threshold != 0, p.causal, p.N, (long long)p.BH * (p.N / 128), p.stages)) {
     const int blocks = p.BH * (p.N / 128);
     p.n_kv_wg = (p.stages & 4u) ? blocks : 0;
     p.n_q_wg = (p.stages & 8u) ? blocks : 0;

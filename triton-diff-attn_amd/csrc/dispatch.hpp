@@ -1,4 +1,5 @@
-// The launch geometry of a forward as a pure function of its sizes and options.  Plain C++: a test compiles it by itself.
+// The launch geometries of a forward and of a backward as pure functions of the sizes and options.  Plain C++: a test
+// compiles it by itself.
 #pragma once
 
 namespace da_abi {
@@ -29,6 +30,33 @@ constexpr bool fwd_64_rows(int d, bool causal, int n, long long blocks) {
   if (causal && d == 128 && n > 256) limit += (n - 256) / 8;
   const int most = d == 128 ? kNumCU - 1 : kNumCU;
   return blocks <= (limit < most ? limit : most);
+}
+
+// Whether a backward goes into one grid (bwd_pair_kernel) instead of a dK/dV and a dQ launch.  `n`, `blocks`: as above;
+// `stages`: what is asked for (4 dK/dV, 8 dQ).
+// At D = 128 always: its dQ blocks are four waves at one wave per SIMD either way.  At D <= 64 the dQ kernel of its own has
+// eight waves and 256 rows, two waves per SIMD, and is the faster one on a full chip (headline size: 437 us against 510), so
+// it is a matter of rounds.  Microseconds per round of 256 workgroups at N = 2048, D = 64, which scale alike with N and D:
+// 79 for key blocks, 64 for query blocks of the one grid, 109 for 256-row blocks of the dQ kernel; a grid that is dealt from
+// one list ends with a partial round of 25.  Measured over N = 128 ... 4096 and 192 ... 1280 blocks: gains of up to 24 % on
+// the line's near side, up to 6 % on its far side, 7 % in padded sequences.
+// Causal blocks differ in length and fill the rounds by themselves: the one grid is faster below 576 blocks
+// (by 5 % at 512, 40 % at 256) and slower above 640 (by 2-5 %).  Those of a unit of one or two blocks hardly differ: at N = 256
+// the rounds decide as without a mask (us of the whole backward, two launches -> one grid: D64 512 blocks 71 -> 74, 640
+// blocks 95 -> 86, D32 640 blocks 61 -> 55); at N = 128 there is one key block and one query block to a unit, and two launches
+// are ahead from 448 blocks on (D32, 448 blocks 36 -> 39, 512 blocks 40 -> 42; 384 blocks 34 -> 32).
+constexpr bool bwd_one_grid(int d, bool dropout, bool causal, int n, long long blocks, unsigned stages) {
+  if (dropout) return false;          // the dropout instantiations are not pipelined
+  if (d == 128) return true;
+  const bool wide = n % 256 == 0;     // the dQ kernel of its own has its 256-row blocks
+  // n an odd multiple of 128: its 128-row variant has one wave per SIMD at D = 64 (LDS), and this one is pipelined
+  if (d == 64 && !wide && (stages & 8u)) return true;
+  if ((stages & 12u) != 12u) return blocks <= kNumCU;
+  if (causal && n > 256) return blocks <= 576;
+  if (causal && n == 128) return blocks <= 384;
+  const long long two = 79 * ((blocks + 255) / 256) + 109 * ((blocks + 511) / 512);
+  const long long one = (d == 32 ? 150 : 143) * blocks / 256 + 25;
+  return one < two;
 }
 
 }  // namespace da_abi
