@@ -39,7 +39,7 @@ def check(ins, rms_norm, y, grads, **options):
     (2, 40, 961, True),        # one real row in the last tile
 ])
 def test_separate_launches_match_the_oracle(B, H, N, causal, D, dtype):
-    # past the lines of one_grid (576 causal blocks; 512 others are two whole rounds of either launch), on 256-row blocks,
+    # past the lines of bwd_one_grid (576 causal blocks; 512 others are two whole rounds of either launch), on 256-row blocks,
     # and with them past every line of the 64-row forward
     assert (blocks(B, H, N) > 576 if causal else blocks(B, H, N) == 512) and -(-N // 128) % 2 == 0
     ins = [t.to(dtype) for t in make_inputs(B, H, N, D, seed=6000 + N + D)]

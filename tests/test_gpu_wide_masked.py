@@ -1,4 +1,4 @@
-"""The D = 128 forward with a mask in 128-row workgroups (csrc/fwd.hip, launch_fwd_t: from 256 of them on), against the fp32
+"""The D = 128 forward with a mask in 128-row workgroups (csrc/dispatch.hpp, fwd_64_rows: always from 256 of them on), against the fp32
 oracle: one block to several turns of the ring in front of the masked tail, and lengths that end in every part of the
 last block.  The gradients check the saved row statistics."""
 import pytest

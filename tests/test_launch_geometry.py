@@ -25,6 +25,9 @@ FORWARD = {
     (128, True, 512, 192): (28.7, 26.8), (128, True, 640, 160): (25.6, 29.6), (128, True, 640, 205): (35.7, 31.7),
     (128, True, 768, 174): (33.2, 33.9), (128, True, 768, 222): (40.6, 36.2), (128, True, 1024, 192): (37.9, 40.5),
     (128, True, 1536, 192): (46.8, 55.0), (128, True, 2048, 240): (70.8, 74.0),
+    (32, False, 128, 128): (5.2, 6.1), (32, False, 512, 128): (8.7, 10.7), (32, False, 2048, 144): (30.3, 28.4),
+    (32, False, 2048, 192): (31.2, 28.6), (128, False, 128, 128): (11.5, 14.2), (128, False, 512, 144): (37.8, 25.2),
+    (128, False, 2048, 128): (58.5, 67.4), (128, False, 2048, 256): (114.3, 94.2),
     # bf16
     (64, False, 2048, 128): (33.8, 39.6), (64, False, 2048, 144): (56.8, 38.3), (64, False, 2048, 192): (56.9, 41.4),
     (64, True, 8192, 256): (116, 139), (64, True, 2048, 384): (61, 46), (128, True, 3072, 768): (328, 230),

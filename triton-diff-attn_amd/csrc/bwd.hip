@@ -7,11 +7,13 @@
 //                     the four row statistics the main kernels need.
 //   bwd_dkdv_kernel   one workgroup per 128 keys, loops over all query tiles:
 //                     dV += (P1 - lambda P2)^T dX, dK_t += s dS_t^T Q_t      (:410-424)
-//   bwd_dq_kernel     one workgroup per 128 queries, loops over all key tiles:
+//   bwd_dq_kernel     one workgroup per 256 or 128 queries, loops over all key tiles:
 //                     dQ_t += s dS_t K_t                                      (:426-436)
+//   bwd_pair_kernel   blocks of both kinds in one grid: always at D = 128 without dropout, else where
+//                     bwd_one_grid (dispatch.hpp) says so
 //   d(lambda)         fixed-order sum of the partials into one fp16 value (one per head with per-head
-//                     lambda) (:573): one extra workgroup per value at the end of the first dK/dV or dQ
-//                     grid of the call, or bwd_dlambda_kernel when neither of them is launched
+//                     lambda) (:573): one extra workgroup per value at the end of the first grid of dK/dV or dQ
+//                     blocks of the call, or bwd_dlambda_kernel when there is none
 //
 // The pre-norm row X is rebuilt as Y / ((1 - lambda_init) * rinv); only U2 = softmax(S2) V is
 // needed besides it, because U1 = X + lambda U2.
@@ -199,8 +201,9 @@ struct DkvCfg {
 // one key column; P and dS in accumulator layout are then directly the A operands (rows = keys,
 // contraction over queries) of dV = P^T dX and dK_t = dS_t^T Q_t.
 // MODE 0 computes dV, dK1 and dK2 in one pass.  At D = 128 their accumulators plus the resident
-// K1, K2, V rows exceed the 512 registers of a lane, so the work is split in two launches:
-// MODE 1 computes dV only (scores S1, S2; no dP), MODE 2 computes dK1 and dK2 only.
+// K1, K2, V rows exceed the 512 registers of a lane, so there are two kinds of key blocks, side by side in
+// bwd_pair_kernel's grid and with dropout in two launches: MODE 1 computes dV only (scores S1, S2; no dP),
+// MODE 2 computes dK1 and dK2 only.
 // CAUSAL: queries before the key block are skipped and the four sub-tiles on the diagonal are masked.
 // DROP: dropout on both softmax maps, masks regenerated from the hash the forward used.  With the
 // keep mask m_t and c = 1/(1-p):  dS1 = A1 (c m1 dP - delta1),  dS2 = A2 (-lambda c m2 dP - delta2),

@@ -10,9 +10,10 @@ constexpr int kNumCU = 256;
 // (N, D, Dv), src/kernel.py:12-19; there is no tuning state here.)  `n`: the padded sequence length, a multiple of 128;
 // `blocks`: B*H*n/128.  Figures: us of a launch, 128-row -> 64-row.
 // Blocks of one length: up to 128 of them, i.e. where 128-row blocks leave half of the chip idle (bf16, D <= 64, B1 H8
-// N2000 D64 39.6 -> 33.8, with dropout 57.7 -> 41.1; D32 29.3 -> 23.3).  The rings of a D >= 64 workgroup fill a CU's LDS
-// whatever its rows, so from 129 on the halves take a second round (bf16, B1 H9 N2048 D64 38.3 -> 56.8, B1 H12 N2048 D64
-// 41.4 -> 56.9, D128 75 -> 105).
+// N2000 D64 39.6 -> 33.8, with dropout 57.7 -> 41.1; D32 29.3 -> 23.3; fp16, B1 H8 N2048 D128 67.4 -> 58.5).  The rings of a
+// D >= 64 workgroup fill a CU's LDS whatever its rows, so from 129 on the halves take a second round (bf16, B1 H9 N2048 D64
+// 38.3 -> 56.8, B1 H12 N2048 D64 41.4 -> 56.9, D128 75 -> 105); at D32 two share a CU and take turns (fp16, B1 H9 N2048 28.4 ->
+// 30.3, 256 blocks of N = 512 11.1 -> 11.6).
 // Causal blocks differ in length and end with the longest; halves, longest first, are shorter and dealt more evenly.
 //   D32, two workgroups to a CU: up to 256 (bf16, B1 H8 N2048 29.0 -> 22.4, B1 H16 N2048 29.4 -> 25.3; fp16, 256 blocks of
 //   N = 256 9.2 -> 8.0, N = 128 7.4 -> 7.6).
