@@ -1,0 +1,113 @@
+"""The layer as one node (modules._diff_attn_layer, csrc/layer_host.cpp): its kernels and its gradients against the same layer
+taken operation by operation, and which calls it stands for."""
+import copy
+
+import pytest
+import torch
+
+import _native
+import baselines
+import modules
+
+pytestmark = pytest.mark.gpu
+_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,E", [(1, 128), (63, 128), (64, 384), (65, 256), (255, 640), (1000, 384), (4129, 256), (8192, 1024)])
+def test_weight_gradient(T, E, dtype):
+    """Edges of a 64-token slab, one and several splits, an operand with a row stride of its own."""
+    gen = torch.Generator(device="cuda").manual_seed(T + E)
+    a = torch.randn(T, 3 * E, device="cuda", generator=gen).to(dtype)[:, E:2 * E]
+    b = torch.randn(T, E, device="cuda", generator=gen).to(dtype)
+    got = _native.layer().weight_gradient(a, b, torch.cuda.current_stream().cuda_stream)
+    want = a.double().t() @ b.double()
+    # one rounding of the result, and T additions of exact products in fp32
+    bound = _ULP[dtype] * want.abs() + T * 2.0 ** -23 * (a.double().abs().t() @ b.double().abs()) + 2.0 ** -24
+    assert got.dtype == dtype and bool(((got.double() - want).abs() <= bound).all())
+
+
+def _step(layer, x, dy):
+    x = x.clone().requires_grad_(True)
+    layer.zero_grad(set_to_none=True)
+    y = layer(x)
+    y.backward(dy)
+    return dict({n: p.grad for n, p in layer.named_parameters()}, x=x.grad, y=y.detach())
+
+
+def _node(layer, x):
+    return type(layer(x.clone().requires_grad_(True)).grad_fn).__name__
+
+
+@pytest.mark.parametrize("B,N,H,d,causal,per_head,dtype", [
+    (2, 77, 1, 32, False, False, torch.float16),          # E = 64: library weight gradients
+    (1, 1, 2, 32, True, True, torch.bfloat16),
+    (2, 200, 3, 64, True, True, torch.float16),           # E = 384, padded sequence
+    (3, 256, 4, 64, False, True, torch.bfloat16),
+    (2, 130, 2, 128, False, False, torch.float16),
+])
+def test_layer_node_matches_its_operations(B, N, H, d, causal, per_head, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    E = 2 * H * d
+    layer = modules.DiffAttn(E, H, depth=2, causal=causal, per_head_lambda=per_head, device="cuda", dtype=dtype)
+    with torch.no_grad():
+        for name, p in layer.named_parameters():
+            p.normal_(1.0 if name == "head_gain" else 0.0, 0.1 if "lambda" in name or name == "head_gain" else E ** -0.5, generator=gen)
+    single = copy.deepcopy(layer)
+    single.out_proj.register_forward_hook(lambda *a: None)          # a hook: the operations one by one
+    x = torch.randn(B, N, E, device="cuda", generator=gen).to(dtype)
+    dy = torch.randn(B, N, E, device="cuda", generator=gen).add_(0.25).to(dtype)
+    assert _node(layer, x) == "_diff_attn_layerBackward" and _node(single, x) != "_diff_attn_layerBackward"
+    got, want = _step(layer, x, dy), _step(single, x, dy)
+    for name in want:
+        a, b = got[name].double(), want[name].double()
+        assert got[name].dtype == want[name].dtype and got[name].shape == want[name].shape and got[name].stride() == want[name].stride()
+        if N == 1 and name.startswith("lambda"):
+            continue            # zero but for rounding: both softmax maps of a single position are 1, and the norm takes out the factor
+        # either side rounds to 16 bits about four times on the way to any of them.  d(lambda) is a sum of terms of both signs that
+        # leaves a fraction of them: eight times as much (against 64 bits, 24 seeds: the node 4e-3 and 8e-3 off in the two types, the
+        # operations 6e-3 and 1e-2)
+        assert (a - b).norm() <= (64 if name.startswith("lambda") else 8) * _ULP[dtype] * b.norm(), name
+    again = _step(layer, x, dy)
+    assert all(torch.equal(again[n], got[n]) for n in got)
+    with torch.no_grad():
+        assert torch.equal(layer(x), got["y"])
+    # any subset of the gradients is what the whole gives
+    for wanted in (("x",), ("q_proj.weight",), ("k_proj.weight", "head_gain"), ("v_proj.weight", "lambda_k1"), ("out_proj.weight",)):
+        part = copy.deepcopy(layer).requires_grad_(False)
+        for n, p in part.named_parameters():
+            p.requires_grad_(n in wanted)
+        xp = x.clone().requires_grad_("x" in wanted)
+        part(xp).backward(dy)
+        grads = dict({n: p.grad for n, p in part.named_parameters()}, x=xp.grad)
+        assert all(torch.equal(g, got[n]) if n in wanted else g is None for n, g in grads.items()), wanted
+
+
+def test_which_calls_the_node_stands_for():
+    node = "_diff_attn_layerBackward"
+    x = torch.randn(1, 64, 128, device="cuda").half()
+
+    def changed(change, x=x):
+        layer = modules.DiffAttn(128, 1, device="cuda")
+        change(layer)
+        return _node(layer, x)
+
+    assert changed(lambda l: None) == node
+    assert changed(lambda l: None, x.transpose(0, 1)) == node       # any strides of x
+    for change in (lambda l: setattr(l, "q_proj", torch.nn.Sequential(l.q_proj)),
+                   lambda l: setattr(l, "attention", lambda *a, **k: baselines.MultiheadDiffAttn(*a, **k)),
+                   lambda l: l.v_proj.register_full_backward_hook(lambda *a: None),
+                   lambda l: setattr(l, "lambda_scale", lambda: torch.full((1,), 0.5, device="cuda")),
+                   lambda l: torch.nn.utils.parametrizations.weight_norm(l.k_proj),
+                   lambda l: setattr(l, "attention_dropout", 0.5)):
+        assert changed(change) != node
+    layer = modules.DiffAttn(128, 1, device="cuda")
+    y = layer(x.requires_grad_(True))
+    (g,) = torch.autograd.grad(y.float().square().sum(), x, create_graph=True)
+    with pytest.raises(RuntimeError):
+        g.sum().backward()      # as before: no second derivative
+    # saved tensors go through hooks that return other memory
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda()):
+        y2 = layer(x)
+    dy = torch.randn_like(y2)
+    assert torch.equal(torch.autograd.grad(y2, x, dy)[0], torch.autograd.grad(layer(x), x, dy)[0])

@@ -12,6 +12,7 @@ import torch  # noqa: F401  (must precede loading the library)
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdiffattn.so")
 HOST_PATH = os.path.join(_HERE, "diffattn_host.so")
+LAYER_PATH = os.path.join(_HERE, "diffattn_layer.so")
 
 ABI_VERSION = 7   # the version of include/diffattn.h this binding is written against
 
@@ -81,23 +82,32 @@ def lib():
     return _lib
 
 
-_host = None
+_modules = {}
+
+
+def _module(name, path):
+    module = _modules.get(name)
+    if module is None:
+        if not os.path.exists(path):
+            raise NativeLibraryMissing(
+                "%s.so is not built: run `python %s`" % (name, os.path.join(_HERE, "build.py")))
+        lib()       # present and of the right version
+        spec = importlib.util.spec_from_file_location(name, path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _modules[name] = module
+    return module
 
 
 def host():
     """Returns the extension module that runs one operator call on the library (csrc/host.cpp); raises if it has not
     been built."""
-    global _host
-    if _host is None:
-        if not os.path.exists(HOST_PATH):
-            raise NativeLibraryMissing(
-                "diffattn_host.so is not built: run `python %s`" % os.path.join(_HERE, "build.py"))
-        lib()       # present and of the right version
-        spec = importlib.util.spec_from_file_location("diffattn_host", HOST_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        _host = module
-    return _host
+    return _modules.get("diffattn_host") or _module("diffattn_host", HOST_PATH)
+
+
+def layer():
+    """Returns the extension module that runs one step of the layer (csrc/layer_host.cpp); raises if it has not been built."""
+    return _modules.get("diffattn_layer") or _module("diffattn_layer", LAYER_PATH)
 
 
 def check(code):

@@ -1,4 +1,4 @@
-"""Builds libdiffattn.so (the gfx950 kernels plus their C ABI) and diffattn_host.so (its extension module) in-tree with
+"""Builds libdiffattn.so (the gfx950 kernels plus their C ABI), diffattn_host.so and diffattn_layer.so (its extension modules) in-tree with
 plain hipcc and g++.
 
 Usage: python build.py            (from anywhere; output lands next to this file)
@@ -11,9 +11,10 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libdiffattn.so")
 HOST = os.path.join(HERE, "diffattn_host.so")
+LAYER = os.path.join(HERE, "diffattn_layer.so")
 ABI_EXAMPLE = os.path.join(HERE, "abi_example")
-SOURCES = ["fwd.hip", "bwd.hip", "api.hip"]
-KERNEL_SOURCES = ["fwd.hip", "bwd.hip"]
+SOURCES = ["fwd.hip", "bwd.hip", "layer.hip", "api.hip"]
+KERNEL_SOURCES = ["fwd.hip", "bwd.hip", "layer.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -48,7 +49,7 @@ def check_resources(src, remarks):
             continue
         m = re.search(r"fwd_kernelILi\d+ELb\dELi\dELb(\d)", name)       # <D, RMS, MASK, DROP, ...>
         dropout = bool(m) and m.group(1) == "1"
-        if "bwd_" in name or ("fwd_kernel" in name and not dropout):
+        if "bwd_" in name or "wgrad" in name or ("fwd_kernel" in name and not dropout):
             bad.append("%s: %s bytes of scratch per lane" % (name, scratch))
     if bad:
         raise RuntimeError("%s: kernels that must not spill do:\n  %s" % (src, "\n  ".join(bad)))
@@ -82,18 +83,24 @@ def build(verbose=True):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
-    # the extension module that runs one operator call: host code only, against the headers of the torch it is loaded into
+    # the extension modules that run one operator call and one step of the layer: host code only, against the headers of
+    # the torch they are loaded into
     import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
-           *("-I" + d for d in include_paths()), "-I" + sysconfig.get_paths()["include"],
-           os.path.join(CSRC, "host.cpp"), "-o", HOST, "-L" + HERE, "-ldiffattn", *("-L" + d for d in library_paths()),
-           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
+    procs = []
+    for src, out in (("host.cpp", HOST), ("layer_host.cpp", LAYER)):
+        cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+               "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
+               *("-I" + d for d in include_paths()), "-I" + sysconfig.get_paths()["include"],
+               os.path.join(CSRC, src), "-o", out, "-L" + HERE, "-ldiffattn", *("-L" + d for d in library_paths()),
+               "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        procs.append((cmd, subprocess.Popen(cmd)))
+    for cmd, pr in procs:
+        if pr.wait() != 0:
+            raise RuntimeError("%s failed: %s" % (cmd[0], " ".join(cmd)))
     # the C++ example of the C ABI (also driven by a GPU test): links the library, no PyTorch
     cmd = [HIPCC, "--offload-arch=gfx950", "-O2", "-std=c++17", os.path.join(CSRC, "abi_example.cpp"),
            "-L" + HERE, "-ldiffattn", "-Wl,-rpath,$ORIGIN", "-o", ABI_EXAMPLE]

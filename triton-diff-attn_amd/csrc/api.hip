@@ -5,6 +5,7 @@
 #include <cstring>
 
 #include "../../include/diffattn.h"
+#include "layer.hpp"
 #include "params.hpp"
 
 // Scratch of diffattn_backward_static: one copy per GPU, at an address that differs per GPU.  In
@@ -189,6 +190,51 @@ void fill_bwd(da_abi::BwdParamsT<T>& p, const void* q1, const void* q2, const vo
   p.lambda_fp32 = (flags & DIFFATTN_LAMBDA_FP32) ? 1 : 0;
 }
 
+// gain, gain_part: null, or what diffattn_layer_backward takes
+int backward_impl(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
+                             const void* lambda_scale, const void* y, const void* u2,
+                             const float* lse1, const float* lse2, const float* rinv, const void* dy,
+                             void* dq1, void* dq2, void* dk1, void* dk2, void* dv, void* dlambda,
+                             void* workspace, size_t workspace_bytes,
+                             int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
+                             unsigned stage_mask, const diffattn_layout* layout, const diffattn_dropout* dropout,
+                             const void* gain, float* gain_part, void* stream) {
+  if (!q1 || !q2 || !k1 || !k2 || !v || !lambda_scale || !y || !u2 || !lse1 || !lse2 || !dy || !workspace)
+    return DIFFATTN_EINVAL_NULL;
+  if (gain && !gain_part) return DIFFATTN_EINVAL_NULL;
+  // outputs are required by the stages that write them
+  if ((stage_mask & DIFFATTN_STAGE_DLAMBDA) && !dlambda) return DIFFATTN_EINVAL_NULL;
+  if ((stage_mask & DIFFATTN_STAGE_DKDV) && (!dk1 || !dk2 || !dv)) return DIFFATTN_EINVAL_NULL;
+  if ((stage_mask & DIFFATTN_STAGE_DQ) && (!dq1 || !dq2)) return DIFFATTN_EINVAL_NULL;
+  if (flags & ~kKnownFlags) return DIFFATTN_EINVAL_FLAGS;
+  if ((flags & DIFFATTN_RMS_NORM) && !rinv) return DIFFATTN_EINVAL_NULL;
+  if (int e = check_dims(B, H, N, D)) return e;
+  if (n_valid < 1 || n_valid > N) return DIFFATTN_EINVAL_SEQ;
+  const void* ptrs[] = {q1, q2, k1, k2, v, y, u2, dy, dq1, dq2, dk1, dk2, dv, gain};
+  for (const void* q : ptrs)
+    if (!aligned16(q)) return DIFFATTN_EINVAL_ALIGN;
+  Layouts lay;
+  if (int e = resolve_layout(layout, B, H, (flags & DIFFATTN_UNPADDED) ? n_valid : N, D, true, &lay)) return e;
+  da_abi::DropoutCfg drop;
+  if (int e = resolve_dropout(dropout, &drop)) return e;
+  const WsLayout w = ws_layout(B * H, N, D);
+  if (workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return DIFFATTN_EINVAL_WS;
+  char* ws = (char*)workspace;
+  const int n_part = bwd_num_partials(B * H, N, D);
+  if (flags & DIFFATTN_BF16) {
+    da_bf16::BwdParams p;
+    fill_bwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
+             ws + w.dx, ws + w.stat, ws + w.part, n_part, B * H, H, N, n_valid, sm_scale, lambda_init, flags, stage_mask, lay, drop);
+    p.gain = (const __bf16*)gain; p.dgain_part = gain_part;
+    return (int)da_bf16::launch_bwd(p, D, (hipStream_t)stream);
+  }
+  BwdParams p;
+  fill_bwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
+           ws + w.dx, ws + w.stat, ws + w.part, n_part, B * H, H, N, n_valid, sm_scale, lambda_init, flags, stage_mask, lay, drop);
+  p.gain = (const half_t*)gain; p.dgain_part = gain_part;
+  return (int)launch_bwd(p, D, (hipStream_t)stream);
+}
+
 }  // namespace
 
 extern "C" {
@@ -259,37 +305,9 @@ int diffattn_backward_stages(const void* q1, const void* q2, const void* k1, con
                              int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
                              unsigned stage_mask, const diffattn_layout* layout, const diffattn_dropout* dropout,
                              void* stream) {
-  if (!q1 || !q2 || !k1 || !k2 || !v || !lambda_scale || !y || !u2 || !lse1 || !lse2 || !dy || !workspace)
-    return DIFFATTN_EINVAL_NULL;
-  // outputs are required by the stages that write them
-  if ((stage_mask & DIFFATTN_STAGE_DLAMBDA) && !dlambda) return DIFFATTN_EINVAL_NULL;
-  if ((stage_mask & DIFFATTN_STAGE_DKDV) && (!dk1 || !dk2 || !dv)) return DIFFATTN_EINVAL_NULL;
-  if ((stage_mask & DIFFATTN_STAGE_DQ) && (!dq1 || !dq2)) return DIFFATTN_EINVAL_NULL;
-  if (flags & ~kKnownFlags) return DIFFATTN_EINVAL_FLAGS;
-  if ((flags & DIFFATTN_RMS_NORM) && !rinv) return DIFFATTN_EINVAL_NULL;
-  if (int e = check_dims(B, H, N, D)) return e;
-  if (n_valid < 1 || n_valid > N) return DIFFATTN_EINVAL_SEQ;
-  const void* ptrs[] = {q1, q2, k1, k2, v, y, u2, dy, dq1, dq2, dk1, dk2, dv};
-  for (const void* q : ptrs)
-    if (!aligned16(q)) return DIFFATTN_EINVAL_ALIGN;
-  Layouts lay;
-  if (int e = resolve_layout(layout, B, H, (flags & DIFFATTN_UNPADDED) ? n_valid : N, D, true, &lay)) return e;
-  da_abi::DropoutCfg drop;
-  if (int e = resolve_dropout(dropout, &drop)) return e;
-  const WsLayout w = ws_layout(B * H, N, D);
-  if (workspace_bytes < w.total || (reinterpret_cast<uintptr_t>(workspace) & 255u)) return DIFFATTN_EINVAL_WS;
-  char* ws = (char*)workspace;
-  const int n_part = bwd_num_partials(B * H, N, D);
-  if (flags & DIFFATTN_BF16) {
-    da_bf16::BwdParams p;
-    fill_bwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
-             ws + w.dx, ws + w.stat, ws + w.part, n_part, B * H, H, N, n_valid, sm_scale, lambda_init, flags, stage_mask, lay, drop);
-    return (int)da_bf16::launch_bwd(p, D, (hipStream_t)stream);
-  }
-  BwdParams p;
-  fill_bwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
-           ws + w.dx, ws + w.stat, ws + w.part, n_part, B * H, H, N, n_valid, sm_scale, lambda_init, flags, stage_mask, lay, drop);
-  return (int)launch_bwd(p, D, (hipStream_t)stream);
+  return backward_impl(q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
+                       workspace, workspace_bytes, B, H, N, n_valid, D, sm_scale, lambda_init, flags, stage_mask, layout, dropout,
+                       nullptr, nullptr, stream);
 }
 
 int diffattn_backward(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
@@ -333,6 +351,82 @@ int diffattn_dropout_mask(unsigned char* keep, int B, int H, int N, int softmax_
   const dim3 grid((unsigned)(((size_t)N * N + 255) / 256), (unsigned)(B * H));
   hipLaunchKernelGGL(dropout_mask_kernel, grid, dim3(256), 0, (hipStream_t)stream, keep, drop, N, softmax_stream);
   return (int)hipGetLastError();
+}
+
+size_t diffattn_layer_gain_parts(int B, int H, int N, int D) { return check_dims(B, H, N, D) ? 0 : (size_t)bwd_num_partials(B * H, N, D); }
+
+int diffattn_layer_backward(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
+                             const void* lambda_scale, const void* y, const void* u2,
+                             const float* lse1, const float* lse2, const float* rinv, const void* dy,
+                             void* dq1, void* dq2, void* dk1, void* dk2, void* dv, void* dlambda,
+                             void* workspace, size_t workspace_bytes,
+                             int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
+                             unsigned stage_mask, const diffattn_layout* layout, const diffattn_dropout* dropout,
+                             const void* gain, float* gain_part, void* stream) {
+  return backward_impl(q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
+                       workspace, workspace_bytes, B, H, N, n_valid, D, sm_scale, lambda_init, flags, stage_mask, layout, dropout,
+                       gain, gain_part, stream);
+}
+
+int diffattn_layer_pack(const void* w0, const void* w1, const void* w2, void* packed, size_t weight_bytes,
+                        const diffattn_lambda_vectors* vectors, float lambda_init, float* lambda, void* stream) {
+  if (!w0 || !w1 || !w2 || !packed || (lambda && !vectors)) return DIFFATTN_EINVAL_NULL;
+  if (weight_bytes % 16 != 0) return DIFFATTN_EINVAL_DIM;
+  for (const void* q : {w0, w1, w2, (const void*)packed})
+    if (!aligned16(q)) return DIFFATTN_EINVAL_ALIGN;
+  da_abi::LayerPackParams p = {{w0, w1, w2}, packed, weight_bytes, {}, lambda, lambda_init};
+  if (vectors) p.vec = *vectors;
+  return (int)launch_layer_pack(p, (hipStream_t)stream);
+}
+
+static bool wgrad_size_ok(int n_jobs, int T, int E) {
+  return n_jobs >= 1 && n_jobs <= 4 && T >= 1 && E >= da_abi::kWgradTile && E % da_abi::kWgradTile == 0 && E <= (1 << 14);
+}
+
+static da_abi::WgradSplit wgrad_split_of(int n_jobs, int T, int E) {
+  const long long nt = E / da_abi::kWgradTile;
+  return da_abi::wgrad_split(n_jobs * nt * nt, T);
+}
+
+size_t diffattn_layer_wgrad_workspace_bytes(int n_jobs, int T, int E) {
+  if (!wgrad_size_ok(n_jobs, T, E)) return 0;
+  const int splits = wgrad_split_of(n_jobs, T, E).splits;
+  return splits > 1 ? (size_t)splits * n_jobs * E * E * sizeof(float) : 0;
+}
+
+int diffattn_layer_wgrad(const diffattn_wgrad_job* jobs, int n_jobs, int T, int E, void* workspace, size_t workspace_bytes,
+                         int flags, void* stream) {
+  if (!jobs) return DIFFATTN_EINVAL_NULL;
+  if (flags & ~DIFFATTN_BF16) return DIFFATTN_EINVAL_FLAGS;
+  if (!wgrad_size_ok(n_jobs, T, E)) return DIFFATTN_EINVAL_DIM;
+  da_abi::WgradParams p = {};
+  for (int i = 0; i < n_jobs; ++i) {
+    const diffattn_wgrad_job& j = jobs[i];
+    if (!j.a || !j.b || !j.out) return DIFFATTN_EINVAL_NULL;
+    if (!aligned16(j.a) || !aligned16(j.b) || !aligned16(j.out)) return DIFFATTN_EINVAL_ALIGN;
+    for (long long ld : {j.lda, j.ldb})
+      if (ld < E || ld % 8 != 0 || ld > (1LL << 26)) return DIFFATTN_EINVAL_LAYOUT;
+    p.job[i] = {j.a, j.b, j.out, (int)j.lda, (int)j.ldb};
+  }
+  p.n_jobs = n_jobs; p.T = T; p.E = E;
+  p.split = wgrad_split_of(n_jobs, T, E);
+  const size_t need = diffattn_layer_wgrad_workspace_bytes(n_jobs, T, E);
+  if (need && (!workspace || workspace_bytes < need || !aligned16(workspace))) return DIFFATTN_EINVAL_WS;
+  p.part = (float*)workspace;
+  return (int)((flags & DIFFATTN_BF16) ? da_bf16::launch_wgrad(p, (hipStream_t)stream) : launch_wgrad(p, (hipStream_t)stream));
+}
+
+int diffattn_layer_finish(const float* gain_part, int n_part, int width, void* dgain,
+                          const diffattn_lambda_vectors* vectors, const float* dlambda,
+                          float* dq1, float* dk1, float* dq2, float* dk2, int flags, void* stream) {
+  if (dgain && !gain_part) return DIFFATTN_EINVAL_NULL;
+  if (dlambda && (!vectors || !dq1 || !dk1 || !dq2 || !dk2)) return DIFFATTN_EINVAL_NULL;
+  if (flags & ~DIFFATTN_BF16) return DIFFATTN_EINVAL_FLAGS;
+  if (dgain && (n_part < 1 || width < 16 || width % 16 != 0)) return DIFFATTN_EINVAL_DIM;
+  if (!dgain && !dlambda) return DIFFATTN_OK;
+  da_abi::LayerFinishParams p = {gain_part, n_part, width, dgain, {}, dlambda, dq1, dk1, dq2, dk2};
+  if (vectors) p.vec = *vectors;
+  return (int)((flags & DIFFATTN_BF16) ? da_bf16::launch_layer_finish(p, (hipStream_t)stream) : launch_layer_finish(p, (hipStream_t)stream));
 }
 
 }  // extern "C"

@@ -60,4 +60,18 @@ constexpr bool bwd_one_grid(int d, bool dropout, bool causal, int n, long long b
   return one < two;
 }
 
+// A weight gradient of the layer (wgrad_kernel, layer.hip): workgroups per 128 x 128 tile and the 64-token slabs that each
+// of them takes.  `tiles`: of all the weights of the launch.  One workgroup fills a CU's LDS, so tiles are split as far as one
+// round of workgroups goes, but not below four slabs, where starting a workgroup and adding its sums takes longer than they do.
+constexpr int kWgradTile = 128, kWgradSlab = 64;
+struct WgradSplit { int splits, slabs; };
+constexpr WgradSplit wgrad_split(long long tiles, int tokens) {
+  const int all = (tokens + kWgradSlab - 1) / kWgradSlab;
+  long long want = kNumCU / tiles;
+  if (want > all / 4) want = all / 4;
+  if (want < 1) want = 1;
+  const int slabs = (int)((all + want - 1) / want);
+  return {(all + slabs - 1) / slabs, slabs};
+}
+
 }  // namespace da_abi

@@ -36,6 +36,8 @@ struct BwdParamsT {
   const T* y; const T* u2;
   const float* lse1; const float* lse2; const float* rinv;
   const T* dy;
+  const T* gain;                // [2D] the caller's output is y times this, and dy the gradient of that; null: none
+  float* dgain_part;            // [n_part][2D] with gain: per-workgroup partial sums of its gradient
   T* dq1; T* dq2; T* dk1; T* dk2; T* dv;
   T* dlambda;                   // 1 element, or H elements with lambda_stride = 1
   // workspace carve-up

@@ -17,13 +17,60 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
+from torch.autograd.function import once_differentiable
 
+import _native
+from kernel import _DTYPES, _SUPPORTED_D, _current_stream
 from layers import MultiheadDiffAttnKernel
 
 
 def lambda_init_for_depth(depth: int) -> float:
     """The paper's schedule for the initial lambda of layer `depth` (0-based)."""
     return 0.8 - 0.6 * math.exp(-0.3 * depth)
+
+
+class _diff_attn_layer(torch.autograd.Function):
+    """The whole layer as one node: csrc/layer_host.cpp runs it.  (As single operations, B8 H8 N1024 d64 causal fp16: 39
+    launches and 709 us of device time a step, of which the operator and four projections of 90 us in all are forward
+    work.)"""
+
+    @staticmethod
+    def forward(ctx, x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, heads, causal, lambda_init):
+        inputs = (x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2)
+        ctx.options = (heads, causal, lambda_init)
+        differentiable = any(ctx.needs_input_grad)
+        y, *saved = _native.layer().layer_forward(*inputs, *ctx.options, differentiable, _current_stream(x.device))
+        if differentiable:
+            ctx.save_for_backward(*inputs, *saved)
+        return y
+
+    @staticmethod
+    @once_differentiable        # like the operator's: a second derivative raises
+    def backward(ctx, dy):
+        saved = ctx.saved_tensors
+        dev = saved[0].device
+        needed = sum(1 << i for i in range(10) if ctx.needs_input_grad[i])
+
+        def launch():
+            return _native.layer().layer_backward(*saved, dy, *ctx.options, needed, _current_stream(dev))
+
+        if dev.index != torch._C._cuda_getDevice():
+            with torch.cuda.device(dev):
+                grads = launch()
+        else:
+            grads = launch()
+        return (*grads, None, None, None)
+
+
+def _plain(t):
+    return type(t) is torch.Tensor or type(t) is nn.Parameter
+
+
+def _plain_linear(m):
+    """Whether calling m is F.linear with its weight and nothing else: no bias, hooks, wrapper or override."""
+    return (type(m) is nn.Linear and m.bias is None and "forward" not in m.__dict__ and m._compiled_call_impl is None
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
 
 
 class DiffAttn(nn.Module):
@@ -72,7 +119,46 @@ class DiffAttn(nn.Module):
             p1, p2 = p.select(3, 0), p.select(3, 1)
         return p1.transpose(1, 2), p2.transpose(1, 2)
 
+    def _fused_inputs(self, x):
+        """The layer's tensors when one node may stand for all of its operations, else None.  Whatever could see or change a
+        single operation goes through them one by one: a replaced or hooked projection, another `attention`, tensor
+        subclasses, autocast, transforms, tracers, compilers and modes, and what the kernels do not read in place."""
+        if not (_plain(x) and x.is_cuda and x.dtype in _DTYPES and x.dim() == 3 and x.numel() > 0 and self.head_dim in _SUPPORTED_D
+                and self.attention is MultiheadDiffAttnKernel and not (self.training and self.attention_dropout)):
+            return None
+        if (torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or forward_ad._current_level >= 0
+                or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda") or nn.modules.module._has_any_global_hook()):
+            return None
+        cls = type(self)
+        if (cls.lambda_scale is not DiffAttn.lambda_scale or cls._streams is not DiffAttn._streams
+                or "lambda_scale" in self.__dict__ or "_streams" in self.__dict__):
+            return None
+        projections = (self.q_proj, self.k_proj, self.v_proj, self.out_proj)
+        if not all(_plain_linear(m) for m in projections):
+            return None
+        E, H, d, dev = self.embed_dim, self.num_heads, self.head_dim, x.device
+        if x.size(2) != E or dev.index != torch._C._cuda_getDevice() or x.size(0) * H * (x.size(1) + 127) > 1 << 28:
+            return None
+        lambdas = (self.lambda_q1, self.lambda_k1, self.lambda_q2, self.lambda_k2)
+        shape = lambdas[0].shape
+        if shape not in ((d,), (H, d)):
+            return None
+        inputs = (*(m.weight for m in projections), self.head_gain, *lambdas)
+        shapes = ((E, E),) * 4 + ((2 * d,),) + (shape,) * 4
+        dtypes = (x.dtype,) * 5 + (torch.float32,) * 4
+        for t, s, dt in zip(inputs, shapes, dtypes):
+            if not (_plain(t) and t.shape == s and t.dtype == dt and t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0):
+                return None
+        return (x, *inputs)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        fused = self._fused_inputs(x)
+        if fused is not None:
+            options = (self.num_heads, self.causal, self.lambda_init)
+            if torch.is_grad_enabled():
+                return _diff_attn_layer.apply(*fused, *options)
+            return _native.layer().layer_forward(*fused, *options, False, _current_stream(x.device))[0]
         B, N, E = x.shape
         H, d = self.num_heads, self.head_dim
         q1, q2 = self._streams(self.q_proj(x).view(B, N, H, 2, d))
