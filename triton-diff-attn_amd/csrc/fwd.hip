@@ -114,6 +114,9 @@ void fwd_kernel(FwdParams p) {
 #pragma unroll
   for (int v = 0; v < BN / 8; ++v) hstep[v] = dropout_window_step<BN / 2>(dkey, v);
 
+  // Asked for here, with the first tiles: behind the loop its latency would be in nobody's shadow.
+  const float lam_load = da_abi::lambda_of_unit(p, bh);
+
   // Q fragments (B operand): column j = this lane's query, k = 8g..8g+7 of each 16-wide k-step.
   // They are pre-multiplied by sm_scale*log2(e), so the MFMA result is the score in log2 units.
   h8 qf[QS][NKS];
@@ -266,8 +269,9 @@ void fwd_kernel(FwdParams p) {
   load_k1(0, b0, with_tail); load_k2(0, b0, with_tail); load_va(0, b0, with_tail); load_vb(0, b0, with_tail);
   load_k1(clampt(1), b0 + 1, with_tail); load_k2(clampt(1), b0 + 1, with_tail);
   load_va(clampt(1), b0 + 1, with_tail); load_vb(clampt(1), b0 + 1, with_tail);
-  load_k1(clampt(2), (b0 + 2) % 4, with_tail); load_k2(clampt(2), (b0 + 2) % 4, with_tail);
+  if (n_tiles > 2) { load_k1(2, (b0 + 2) % 4, with_tail); load_k2(2, (b0 + 2) % 4, with_tail); }
   wait_async_tiles();
+  const float lam = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, lam_load)));
   __syncthreads();
   f16v s_a[QS][NKT], s_b[QS][NKT];
   {
@@ -545,7 +549,6 @@ void fwd_kernel(FwdParams p) {
       }
   }
   __syncthreads();
-  const float lam = da_abi::lambda_of_unit(p, bh);
   float ss = 0.f;
   if (st == 0) {
 #pragma unroll
