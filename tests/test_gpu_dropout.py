@@ -40,6 +40,7 @@ def run(cpu, lam_value, lambda_init, rms, causal, p, seed):
 @pytest.mark.parametrize("D,N,p,rms,causal", [
     (64, 256, 0.1, True, False),
     (64, 384, 0.5, False, False),
+    (64, 256, 0.9, False, False),       # a keep factor of 10 in the probabilities of the backward
     (32, 256, 0.1, True, True),
     (32, 128, 0.5, True, False),
     (128, 128, 0.1, False, False),

@@ -42,7 +42,7 @@ struct BwdParamsT {
   T* dlambda;                   // 1 element, or H elements with lambda_stride = 1
   // workspace carve-up
   T* dx;                        // [BH,N,2D] gradient w.r.t. the pre-norm rows, 16-bit
-  float* stat;                  // [4][BH*N]: -lse1*log2(e), -lse2*log2(e), -delta1, -(lambda*delta1 + delta2)
+  float* stat;                  // [4][BH*N]: -lse1*log2(e), -lse2*log2(e), -delta1, -(lambda*delta1 + delta2); with dropout otherwise, see dkdv_block
   float* dlam_part;             // [n_part] per-workgroup partial sums of d(lambda)
   int n_part;
   int BH, N;
