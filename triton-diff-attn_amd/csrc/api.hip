@@ -150,8 +150,9 @@ template <class T>
 void fill_fwd(da_abi::FwdParamsT<T>& p, const void* q1, const void* q2, const void* k1, const void* k2,
               const void* v, const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
               int BH, int H, int N, int n_valid, float sm_scale, float lambda_init, int flags, const Layouts& lay,
-              const da_abi::DropoutCfg& drop) {
+              const da_abi::DropoutCfg& drop, const void* gain, void* y_gain) {
   p.drop = drop;
+  p.gain = (const T*)gain; p.y_gain = (T*)y_gain;
   p.sqk = lay.qk; p.sv = lay.v; p.sy = lay.y;
   p.q1 = (const T*)q1; p.q2 = (const T*)q2; p.k1 = (const T*)k1; p.k2 = (const T*)k2;
   p.v = (const T*)v; p.lambda_scale = (const T*)lambda_scale;
@@ -235,6 +236,32 @@ int backward_impl(const void* q1, const void* q2, const void* k1, const void* k2
   return (int)launch_bwd(p, D, (hipStream_t)stream);
 }
 
+// gain, y_gain: null, or what diffattn_layer_forward takes
+int forward_impl(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
+                 const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
+                 int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
+                 const diffattn_layout* layout, const diffattn_dropout* dropout, const void* gain, void* y_gain, void* stream) {
+  if (!q1 || !q2 || !k1 || !k2 || !v || !lambda_scale || !(y || y_gain) || (y_gain && !gain)) return DIFFATTN_EINVAL_NULL;
+  if (flags & ~kKnownFlags) return DIFFATTN_EINVAL_FLAGS;
+  if (int e = check_dims(B, H, N, D)) return e;
+  if (n_valid < 1 || n_valid > N) return DIFFATTN_EINVAL_SEQ;
+  const void* ptrs[] = {q1, q2, k1, k2, v, y, u2, gain, y_gain};
+  for (const void* q : ptrs)
+    if (!aligned16(q)) return DIFFATTN_EINVAL_ALIGN;
+  Layouts lay;
+  if (int e = resolve_layout(layout, B, H, (flags & DIFFATTN_UNPADDED) ? n_valid : N, D, false, &lay)) return e;
+  da_abi::DropoutCfg drop;
+  if (int e = resolve_dropout(dropout, &drop)) return e;
+  if (flags & DIFFATTN_BF16) {
+    da_bf16::FwdParams p;
+    fill_fwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B * H, H, N, n_valid, sm_scale, lambda_init, flags, lay, drop, gain, y_gain);
+    return (int)da_bf16::launch_fwd(p, D, (hipStream_t)stream);
+  }
+  FwdParams p;
+  fill_fwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B * H, H, N, n_valid, sm_scale, lambda_init, flags, lay, drop, gain, y_gain);
+  return (int)launch_fwd(p, D, (hipStream_t)stream);
+}
+
 }  // namespace
 
 extern "C" {
@@ -271,25 +298,8 @@ int diffattn_forward_padded(const void* q1, const void* q2, const void* k1, cons
                             const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
                             int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
                             const diffattn_layout* layout, const diffattn_dropout* dropout, void* stream) {
-  if (!q1 || !q2 || !k1 || !k2 || !v || !lambda_scale || !y) return DIFFATTN_EINVAL_NULL;
-  if (flags & ~kKnownFlags) return DIFFATTN_EINVAL_FLAGS;
-  if (int e = check_dims(B, H, N, D)) return e;
-  if (n_valid < 1 || n_valid > N) return DIFFATTN_EINVAL_SEQ;
-  if (!aligned16(q1) || !aligned16(q2) || !aligned16(k1) || !aligned16(k2) || !aligned16(v) ||
-      !aligned16(y) || !aligned16(u2))
-    return DIFFATTN_EINVAL_ALIGN;
-  Layouts lay;
-  if (int e = resolve_layout(layout, B, H, (flags & DIFFATTN_UNPADDED) ? n_valid : N, D, false, &lay)) return e;
-  da_abi::DropoutCfg drop;
-  if (int e = resolve_dropout(dropout, &drop)) return e;
-  if (flags & DIFFATTN_BF16) {
-    da_bf16::FwdParams p;
-    fill_fwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B * H, H, N, n_valid, sm_scale, lambda_init, flags, lay, drop);
-    return (int)da_bf16::launch_fwd(p, D, (hipStream_t)stream);
-  }
-  FwdParams p;
-  fill_fwd(p, q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B * H, H, N, n_valid, sm_scale, lambda_init, flags, lay, drop);
-  return (int)launch_fwd(p, D, (hipStream_t)stream);
+  return forward_impl(q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B, H, N, n_valid, D, sm_scale, lambda_init, flags,
+                      layout, dropout, nullptr, nullptr, stream);
 }
 
 size_t diffattn_backward_workspace_bytes(int B, int H, int N, int D, int flags) {
@@ -351,6 +361,15 @@ int diffattn_dropout_mask(unsigned char* keep, int B, int H, int N, int softmax_
   const dim3 grid((unsigned)(((size_t)N * N + 255) / 256), (unsigned)(B * H));
   hipLaunchKernelGGL(dropout_mask_kernel, grid, dim3(256), 0, (hipStream_t)stream, keep, drop, N, softmax_stream);
   return (int)hipGetLastError();
+}
+
+int diffattn_layer_forward(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
+                           const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
+                           int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
+                           const diffattn_layout* layout, const diffattn_dropout* dropout,
+                           const void* gain, void* y_gain, void* stream) {
+  return forward_impl(q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B, H, N, n_valid, D, sm_scale, lambda_init, flags,
+                      layout, dropout, gain, y_gain, stream);
 }
 
 size_t diffattn_layer_gain_parts(int B, int H, int N, int D) { return check_dims(B, H, N, D) ? 0 : (size_t)bwd_num_partials(B * H, N, D); }

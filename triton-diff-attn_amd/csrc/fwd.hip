@@ -517,13 +517,25 @@ void fwd_kernel(FwdParams p) {
   };
   // `rows`: how many of the wave's 32 rows exist in the destination (32 unless the sequence is padded and
   // the destination is the caller's tensor, which has no rows past the real length)
-  auto store_rows = [&](half_t* gbase /* first of this wave's 32 rows */, size_t row_stride, int rows) {
+  // `gain`: null, or the factors of the DV features (a lane stores the same eight of every row).  Stored from here the
+  // product costs its bytes once; as a launch of its own it read y back: a layer's step B8 H8 N1024 D64 439 -> 430 us, its
+  // inference 138 -> 134, B2 H8 N512 D32 68 -> 64.
+  auto store_rows = [&](half_t* gbase /* first of this wave's 32 rows */, size_t row_stride, int rows, const half_t* gain) {
     constexpr int LPR = DV / 8;            // lanes per row
     constexpr int RPI = 64 / LPR;          // rows per instruction
+    const int ch = lane_e % LPR;
+    h8 gv = {};
+    if (gain) gv = *reinterpret_cast<const h8*>(gain + 8 * ch);
 #pragma unroll
     for (int k = 0; k < 32 / RPI; ++k) {
-      const int row = k * RPI + lane_e / LPR, ch = lane_e % LPR;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(stg_own + row * SROW + 8 * ch);
+      const int row = k * RPI + lane_e / LPR;
+      u32x4 v = *reinterpret_cast<const u32x4*>(stg_own + row * SROW + 8 * ch);
+      if (gain) {
+        h8 x = __builtin_bit_cast(h8, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = (half_t)((float)x[e] * (float)gv[e]);
+        v = __builtin_bit_cast(u32x4, x);
+      }
       if (!TAIL || row < rows) *reinterpret_cast<u32x4*>(gbase + (size_t)row * row_stride + 8 * ch) = v;
     }
   };
@@ -568,7 +580,7 @@ void fwd_kernel(FwdParams p) {
   if (st == 1) {
     stage_rows(0, o[0], inv);
     __builtin_amdgcn_wave_barrier();   // the rows are read back by other lanes of this wave only
-    if (p.u2) store_rows(p.u2 + wave_row0 * DV, DV, 32);
+    if (p.u2) store_rows(p.u2 + wave_row0 * DV, DV, 32, nullptr);
   } else {
     float scale = 1.0f;
     if (RMS) {
@@ -579,8 +591,10 @@ void fwd_kernel(FwdParams p) {
     }
     stage_rows(0, o[0], scale);
     __builtin_amdgcn_wave_barrier();   // the rows are read back by other lanes of this wave only
-    store_rows(p.y + da_abi::unit_base(p, p.sy, bh) + (size_t)(qt * BM + qw * 32) * (size_t)p.sy.n, (size_t)p.sy.n,
-               p.n_keys - (qt * BM + qw * 32));
+    const size_t out0 = da_abi::unit_base(p, p.sy, bh) + (size_t)(qt * BM + qw * 32) * (size_t)p.sy.n;
+    const int out_rows = p.n_keys - (qt * BM + qw * 32);
+    if (p.y) store_rows(p.y + out0, (size_t)p.sy.n, out_rows, nullptr);
+    if (p.y_gain) store_rows(p.y_gain + out0, (size_t)p.sy.n, out_rows, p.gain);
   }
 }
 

@@ -141,20 +141,21 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     lam = at::empty({t[6].numel() / s.d}, t[6].options());
     const diffattn_lambda_vectors vec = vectors(t + 6, s);
     qkv = at::mm(x2, pack(t + 1, s, &vec, (float)lambda_init, (float*)lam.data_ptr(), stream).t());
-    hd = at::empty({s.T, s.E}, qkv.options());
+    hg = at::empty({s.T, s.E}, qkv.options());
     float* st = nullptr;
     const int64_t rows = s.B * s.H * s.n_pad;
     if (differentiable) {
+      hd = at::empty({s.T, s.E}, qkv.options());
       u2 = at::empty({s.B, s.H, s.n_pad, 2 * s.d}, qkv.options());
       stats = at::empty({3, rows}, qkv.options().dtype(at::kFloat));
       st = (float*)stats.data_ptr();
     }
     const Parts p = parts(qkv, s);
     const diffattn_layout layout = s.layout();
-    check(diffattn_forward_padded(p.q1, p.q2, p.k1, p.k2, p.v, lam.data_ptr(), hd.data_ptr(), differentiable ? u2.data_ptr() : nullptr,
-                                  st, st ? st + rows : nullptr, st ? st + 2 * rows : nullptr, (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d,
-                                  s.sm_scale(), (float)lambda_init, s.flags, &layout, nullptr, stream));
-    hg = at::mul(hd.view({s.T, s.H, 2 * s.d}), gain).view({s.T, s.E});
+    check(diffattn_layer_forward(p.q1, p.q2, p.k1, p.k2, p.v, lam.data_ptr(), differentiable ? hd.data_ptr() : nullptr,
+                                 differentiable ? u2.data_ptr() : nullptr, st, st ? st + rows : nullptr, st ? st + 2 * rows : nullptr,
+                                 (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, &layout,
+                                 nullptr, gain.data_ptr(), hg.data_ptr(), stream));
     y = at::mm(hg, wo.t()).view({s.B, s.N, s.E});
     if (!differentiable) qkv = hd = hg = lam = at::Tensor();
   }

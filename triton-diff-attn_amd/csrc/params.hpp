@@ -13,7 +13,8 @@ template <class T>
 struct FwdParamsT {
   const T* q1; const T* q2; const T* k1; const T* k2; const T* v;
   const T* lambda_scale;        // device memory: one value, or one per head (lambda_stride = 1)
-  T* y;                         // [B,H,N,2D]
+  T* y;                         // [B,H,N,2D] (may be null with y_gain)
+  T* y_gain; const T* gain;     // y, as stored, times one factor per feature, in y's layout, and the [2D] factors; null: not wanted
   T* u2;                        // [B,H,N,2D]  softmax(S2) V, saved for backward (may be null)
   float* lse1; float* lse2;     // [B,H,N] natural-log row logsumexp of the scaled scores (may be null)
   float* rinv;                  // [B,H,N] rsqrt(mean(X^2)+eps), only written when rms_norm (may be null)
