@@ -64,10 +64,9 @@ def test_layer_node_matches_its_operations(B, N, H, d, causal, per_head, dtype):
         assert got[name].dtype == want[name].dtype and got[name].shape == want[name].shape and got[name].stride() == want[name].stride()
         if N == 1 and name.startswith("lambda"):
             continue            # zero but for rounding: both softmax maps of a single position are 1, and the norm takes out the factor
-        # either side rounds to 16 bits about four times on the way to any of them.  d(lambda) is a sum of terms of both signs that
-        # leaves a fraction of them: eight times as much (against 64 bits, 24 seeds: the node 4e-3 and 8e-3 off in the two types, the
-        # operations 6e-3 and 1e-2)
-        assert (a - b).norm() <= (64 if name.startswith("lambda") else 8) * _ULP[dtype] * b.norm(), name
+        # dx and the gain's gradient have up to four roundings on the one side that the other does not have; the rest differ by the
+        # order of fp32 sums, d(lambda), a sum of both signs, included: everything in front of it rounds alike on both sides
+        assert (a - b).norm() <= 8 * _ULP[dtype] * b.norm(), name
     again = _step(layer, x, dy)
     assert all(torch.equal(again[n], got[n]) for n in got)
     with torch.no_grad():

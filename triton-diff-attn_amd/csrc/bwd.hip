@@ -30,7 +30,8 @@ int bwd_num_partials(int BH, int N, int D) { (void)D; return (int)(((long long)B
 
 // ------------------------------------------------------------------------------------------------
 // GAIN: the caller's output was y times a gain per feature, and dy is the gradient of that product: it is multiplied by the
-// gain on the way in (in fp32, not rounded again), and the workgroup leaves the sum of dy * y over its rows, one value per
+// gain on the way in, rounded to 16 bits as the product of two tensors is (d(lambda) is a sum of both signs that leaves little
+// of them, and shows in its third digit whether that rounding was done), and the workgroup leaves the sum of dy * y over its rows, one value per
 // feature, as its partial of the gain's gradient.  (As passes of their own, B8 H8 N1024 D64: 39 us for the two products and
 // the sum, beside 15 us for this kernel.)
 template <int D, bool RMS, bool GAIN = false>
@@ -73,21 +74,16 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdParams p) {
       g8 = *reinterpret_cast<const h8*>(gdy + n * (size_t)p.sdy.n);
     }
     const h8 u8 = *reinterpret_cast<const h8*>(p.u2 + off);
-    float gd[8];         // dy, with the gain in it
+    if constexpr (GAIN) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      gd[e] = (float)g8[e];
-      if constexpr (GAIN) { gpart[e] += gd[e] * (float)y8[e]; gd[e] *= gain[e]; }
+      for (int e = 0; e < 8; ++e) { gpart[e] += (float)g8[e] * (float)y8[e]; g8[e] = (half_t)((float)g8[e] * gain[e]); }
     }
     // dX of the row, and ix with X = ix * Y (the pre-norm row rebuilt from the saved output)
     float dx[8], ix = 1.0f;
     if (RMS) {
       float gy = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        if constexpr (GAIN) gy += gd[e] * (float)y8[e] + gd[e + 1] * (float)y8[e + 1];
-        else gy = dot_pair(h2{g8[e], g8[e + 1]}, h2{y8[e], y8[e + 1]}, gy);
-      }
+      for (int e = 0; e < 8; e += 2) gy = dot_pair(h2{g8[e], g8[e + 1]}, h2{y8[e], y8[e + 1]}, gy);
 #pragma unroll
       for (int msk = LPR / 2; msk >= 1; msk >>= 1) gy += __shfl_xor(gy, msk, 64);
       const float r = p.rinv[row];
@@ -95,7 +91,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdParams p) {
         const float a = c * r, b = r * gy / (c * DV);
         ix = 1.0f / (c * r);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) dx[e] = a * gd[e] - b * (float)y8[e];
+        for (int e = 0; e < 8; ++e) dx[e] = a * (float)g8[e] - b * (float)y8[e];
       } else {
         ix = 0.f;
 #pragma unroll
@@ -103,7 +99,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdParams p) {
       }
     } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dx[e] = gd[e];
+      for (int e = 0; e < 8; ++e) dx[e] = (float)g8[e];
     }
     // The row sums are formed from dX as the other kernels will read it, rounded to 16 bits: dS = A (dP - delta)
     // with dP = dX V^T cancels almost completely where a row attends to a single key, and a delta from the
