@@ -101,6 +101,8 @@ def test_which_calls_the_node_stands_for():
                    lambda l: setattr(l, "attention_dropout", 0.5)):
         assert changed(change) != node
     layer = modules.DiffAttn(128, 1, device="cuda")
+    # under a compiler the choice itself is traced without a break, and the single operations are what it sees
+    assert torch.compile(lambda t: t + (1 if layer._fused_inputs(t) is None else 2), backend="eager", fullgraph=True)(x).equal(x + 1)
     y = layer(x.requires_grad_(True))
     (g,) = torch.autograd.grad(y.float().square().sum(), x, create_graph=True)
     with pytest.raises(RuntimeError):

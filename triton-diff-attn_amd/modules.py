@@ -126,9 +126,9 @@ class DiffAttn(nn.Module):
         if not (_plain(x) and x.is_cuda and x.dtype in _DTYPES and x.dim() == 3 and x.numel() > 0 and self.head_dim in _SUPPORTED_D
                 and self.attention is MultiheadDiffAttnKernel and not (self.training and self.attention_dropout)):
             return None
-        if (torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
+        if (torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or forward_ad._current_level >= 0
-                or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda") or nn.modules.module._has_any_global_hook()):
+                or torch.is_autocast_enabled("cuda") or nn.modules.module._has_any_global_hook()):
             return None
         cls = type(self)
         if (cls.lambda_scale is not DiffAttn.lambda_scale or cls._streams is not DiffAttn._streams
