@@ -112,3 +112,43 @@ def test_which_calls_the_node_stands_for():
         y2 = layer(x)
     dy = torch.randn_like(y2)
     assert torch.equal(torch.autograd.grad(y2, x, dy)[0], torch.autograd.grad(layer(x), x, dy)[0])
+
+
+def _pair(E=256, H=2, seed=0, **options):
+    """A layer that goes as one node, and the same layer operation by operation (a hook sees to that)."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    layer = modules.DiffAttn(E, H, device="cuda", **options)
+    with torch.no_grad():
+        for name, p in layer.named_parameters():
+            p.normal_(1.0 if name == "head_gain" else 0.0, 0.1 if "lambda" in name or name == "head_gain" else E ** -0.5, generator=gen)
+    single = copy.deepcopy(layer)
+    single.out_proj.register_forward_hook(lambda *a: None)
+    x = torch.randn(2, 77, E, device="cuda", generator=gen).to(layer.head_gain.dtype)
+    dy = torch.randn(2, 77, E, device="cuda", generator=gen).add_(0.25).to(x.dtype)
+    return layer, single, x, dy
+
+
+def test_results_may_be_written_in_place():
+    """A residual added to the output, dropout on it and detach_(), an output made without gradients that meets a trainable
+    tensor later, and the gradient of x: none of them is a view of anything."""
+    layer, single, x, dy = _pair()
+    scale = torch.full((1,), 0.5, device="cuda", dtype=x.dtype, requires_grad=True)
+    results = []
+    for l in (layer, single):
+        xg = x.clone().requires_grad_(True)
+        y = l(xg)
+        assert not y._is_view() and y.is_contiguous()
+        y += xg
+        torch.nn.functional.dropout(y, 0.0, True, inplace=True)
+        (g,) = torch.autograd.grad(y, xg, dy)
+        if l is layer:
+            g.mul_(scale)
+        else:
+            g = g * scale
+        with torch.no_grad():
+            n = l(xg)
+        n.mul_(scale)
+        l(xg).detach_().add_(1.0)
+        results.append((y.detach(), g.detach(), n.detach(), torch.autograd.grad(n, scale, dy)[0]))
+    for a, b in zip(*results):
+        assert (a.double() - b.double()).norm() <= 8 * _ULP[x.dtype] * b.double().norm()

@@ -49,6 +49,10 @@ at::Tensor dense(const at::Tensor& t) {
   return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone();
 }
 
+// t in another shape, for a result that nothing else holds.  Autograd would know a view as one made in a custom function, or
+// under no_grad, and refuse to have it written in place, which the output of a layer often is (a residual added to it).
+at::Tensor not_a_view(const at::Tensor& t, at::IntArrayRef sizes) { return at::_unsafe_view(t, sizes); }
+
 // Sizes of a call.  d is the width of a q/k head; a value head is 2d wide and E = 2 H d.
 struct Sizes {
   int64_t B, N, E, H, d, T, n_pad;
@@ -156,7 +160,7 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                  differentiable ? u2.data_ptr() : nullptr, st, st ? st + rows : nullptr, st ? st + 2 * rows : nullptr,
                                  (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, &layout,
                                  nullptr, gain.data_ptr(), hg.data_ptr(), stream));
-    y = at::mm(hg, wo.t()).view({s.B, s.N, s.E});
+    y = not_a_view(at::mm(hg, wo.t()), {s.B, s.N, s.E});
     if (!differentiable) qkv = hd = hg = lam = at::Tensor();
   }
   return Py_BuildValue("(NNNNNNN)", wrap(y), wrap(qkv), wrap(hd), wrap(hg), wrap(u2), wrap(stats), wrap(lam));
@@ -207,7 +211,7 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     dhg.data_ptr(), d.q1, d.q2, d.k1, d.k2, d.v, dlam.data_ptr(), ws.data_ptr(), ws_bytes,
                                     (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, stages,
                                     &layout, nullptr, t[5].data_ptr(), (float*)gpart.data_ptr(), stream));
-      if (want(0)) grad[0] = at::mm(dqkv, pack(t + 1, s, nullptr, 0.f, nullptr, stream)).view(t[0].sizes());
+      if (want(0)) grad[0] = not_a_view(at::mm(dqkv, pack(t + 1, s, nullptr, 0.f, nullptr, stream)), t[0].sizes());
       if (want(5)) grad[5] = at::empty_like(t[5]);
       if (want_lam)
         for (int i = 6; i < 10; ++i) grad[i] = at::empty_like(t[i]);
