@@ -1,6 +1,7 @@
 """The layer as one node (modules._diff_attn_layer, csrc/layer_host.cpp): its kernels and its gradients against the same layer
 taken operation by operation, and which calls it stands for."""
 import copy
+import weakref
 
 import pytest
 import torch
@@ -152,3 +153,37 @@ def test_results_may_be_written_in_place():
         results.append((y.detach(), g.detach(), n.detach(), torch.autograd.grad(n, scale, dy)[0]))
     for a, b in zip(*results):
         assert (a.double() - b.double()).norm() <= 8 * _ULP[x.dtype] * b.double().norm()
+
+
+@pytest.mark.parametrize("wanted", [("x",), ("x", "out_proj.weight"), ("out_proj.weight",), ("head_gain",), ("q_proj.weight",),
+                                    ("lambda_k1",), ("k_proj.weight", "head_gain")])
+def test_only_what_a_gradient_reads_is_saved(wanted):
+    """Inputs that no wanted gradient reads may be written in place before the backward, as with the single operations, and
+    are not held until then."""
+    layer, single, x, dy = _pair()
+    # what each wanted gradient reads of the inputs, by the graph of the single operations
+    reads = {"x": {"q_proj.weight", "k_proj.weight", "v_proj.weight", "out_proj.weight", "head_gain"},
+             "out_proj.weight": set(), "head_gain": {"out_proj.weight"},
+             "q_proj.weight": {"x", "out_proj.weight", "head_gain"}, "k_proj.weight": {"x", "out_proj.weight", "head_gain"},
+             "lambda_k1": {"out_proj.weight", "head_gain", "lambda_q1", "lambda_k1", "lambda_q2", "lambda_k2"}}
+    read = set().union(*(reads[n] for n in wanted))
+    grads = []
+    for l in (layer, single):
+        for n, p in l.named_parameters():
+            p.requires_grad_(n in wanted)
+        xg = x.clone().requires_grad_("x" in wanted) * 1.0
+        y = l(xg)
+        inputs = dict(l.named_parameters(), x=xg)
+        with torch.no_grad():
+            for n, t in inputs.items():
+                if n not in read:
+                    t.add_(1.0)
+        grads.append(torch.autograd.grad(y, [inputs[n] for n in wanted], dy))
+    for a, b in zip(*grads):
+        assert (a.double() - b.double()).norm() <= 8 * _ULP[x.dtype] * b.double().norm()
+    if "x" in wanted:
+        xg = x.clone().requires_grad_(True) * 1.0
+        held = weakref.ref(xg)
+        y = layer(xg)
+        del xg
+        assert held() is None and y.requires_grad

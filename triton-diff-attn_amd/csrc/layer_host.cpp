@@ -28,8 +28,10 @@ PyObject* wrap(const at::Tensor& t) {
   return THPVariable_Wrap(t);
 }
 
-bool tensors(PyObject* const* a, int n, at::Tensor* out) {
+// None is an undefined tensor where `optional` allows it
+bool tensors(PyObject* const* a, int n, at::Tensor* out, bool optional = false) {
   for (int i = 0; i < n; ++i) {
+    if (optional && a[i] == Py_None) continue;
     if (!THPVariable_Check(a[i])) {
       PyErr_Format(PyExc_TypeError, "argument %d must be a tensor", i);
       return false;
@@ -45,6 +47,7 @@ void check(int rc) {
 
 // t as the kernels read it: dense and 16-byte aligned (what autograd's saved-tensor hooks hand back may be neither)
 at::Tensor dense(const at::Tensor& t) {
+  if (!t.defined()) return t;
   at::Tensor c = t.contiguous();
   return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone();
 }
@@ -57,13 +60,13 @@ at::Tensor not_a_view(const at::Tensor& t, at::IntArrayRef sizes) { return at::_
 struct Sizes {
   int64_t B, N, E, H, d, T, n_pad;
   int flags;
-  Sizes(const at::Tensor& x, const at::Tensor& lam, int64_t heads, bool causal)
-      : B(x.size(0)), N(x.size(1)), E(x.size(2)), H(heads), d(E / (2 * heads)), T(B * N),
+  Sizes(at::IntArrayRef x, at::ScalarType type, int64_t n_lambda, int64_t heads, bool causal)
+      : B(x[0]), N(x[1]), E(x[2]), H(heads), d(E / (2 * heads)), T(B * N),
         n_pad((N + kSeqMultiple - 1) / kSeqMultiple * kSeqMultiple) {
     flags = DIFFATTN_RMS_NORM | DIFFATTN_LAMBDA_FP32;
     if (causal) flags |= DIFFATTN_CAUSAL;
-    if (x.scalar_type() == at::kBFloat16) flags |= DIFFATTN_BF16;
-    if (lam.numel() > 1) flags |= DIFFATTN_LAMBDA_PER_HEAD;
+    if (type == at::kBFloat16) flags |= DIFFATTN_BF16;
+    if (n_lambda > 1) flags |= DIFFATTN_LAMBDA_PER_HEAD;
     if (n_pad != N) flags |= DIFFATTN_UNPADDED;
   }
   float sm_scale() const { return (float)(1.0 / std::sqrt((double)d)); }
@@ -122,25 +125,27 @@ std::vector<at::Tensor> weight_gradients(const std::vector<Wgrad>& jobs, int64_t
 // The projections run in the type of the layer, also where a backward is called under autocast.
 const c10::DispatchKeySet kNoAutocast = c10::autocast_dispatch_keyset;
 
-// layer_forward(x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, heads, causal, lambda_init, differentiable, stream)
-//   -> (y, qkv, heads, scaled heads, u2, row statistics, lambda); from qkv on None unless `differentiable`
+// layer_forward(x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, heads, causal, lambda_init, inner, outer, stream)
+//   -> (y, qkv, heads, scaled heads, u2, row statistics, lambda).  `inner`: a backward will go behind the output projection;
+//   without, qkv, heads, u2, the statistics and lambda are None.  `outer`: it will want that projection's weight gradient;
+//   without, the scaled heads are None.
 PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 15) return PyErr_Format(PyExc_TypeError, "layer_forward takes 15 arguments");
+  if (n != 16) return PyErr_Format(PyExc_TypeError, "layer_forward takes 16 arguments");
   at::Tensor t[10];
   if (!tensors(a, 10, t)) return nullptr;
   const int64_t heads = PyLong_AsLongLong(a[10]);
   const bool causal = PyObject_IsTrue(a[11]) == 1;
   const double lambda_init = PyFloat_AsDouble(a[12]);
-  const bool differentiable = PyObject_IsTrue(a[13]) == 1;
-  void* const stream = PyLong_AsVoidPtr(a[14]);
+  const bool inner = PyObject_IsTrue(a[13]) == 1, outer = PyObject_IsTrue(a[14]) == 1;
+  void* const stream = PyLong_AsVoidPtr(a[15]);
   if (PyErr_Occurred()) return nullptr;
   at::Tensor y, qkv, hd, hg, u2, stats, lam;
   {
     const Released released;
     const c10::impl::ExcludeDispatchKeyGuard no_autocast(kNoAutocast);
     const at::Tensor &x = t[0], &wo = t[4], &gain = t[5];
-    const Sizes s(x, t[6].dim() > 1 ? t[6].select(1, 0) : t[6].select(0, 0), heads, causal);
+    const Sizes s(x.sizes(), x.scalar_type(), t[6].dim() > 1 ? t[6].size(0) : 1, heads, causal);
     const at::Tensor x2 = x.reshape({s.T, s.E});
     lam = at::empty({t[6].numel() / s.d}, t[6].options());
     const diffattn_lambda_vectors vec = vectors(t + 6, s);
@@ -148,7 +153,7 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     hg = at::empty({s.T, s.E}, qkv.options());
     float* st = nullptr;
     const int64_t rows = s.B * s.H * s.n_pad;
-    if (differentiable) {
+    if (inner) {
       hd = at::empty({s.T, s.E}, qkv.options());
       u2 = at::empty({s.B, s.H, s.n_pad, 2 * s.d}, qkv.options());
       stats = at::empty({3, rows}, qkv.options().dtype(at::kFloat));
@@ -156,38 +161,42 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     const Parts p = parts(qkv, s);
     const diffattn_layout layout = s.layout();
-    check(diffattn_layer_forward(p.q1, p.q2, p.k1, p.k2, p.v, lam.data_ptr(), differentiable ? hd.data_ptr() : nullptr,
-                                 differentiable ? u2.data_ptr() : nullptr, st, st ? st + rows : nullptr, st ? st + 2 * rows : nullptr,
+    check(diffattn_layer_forward(p.q1, p.q2, p.k1, p.k2, p.v, lam.data_ptr(), inner ? hd.data_ptr() : nullptr,
+                                 inner ? u2.data_ptr() : nullptr, st, st ? st + rows : nullptr, st ? st + 2 * rows : nullptr,
                                  (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, &layout,
                                  nullptr, gain.data_ptr(), hg.data_ptr(), stream));
     y = not_a_view(at::mm(hg, wo.t()), {s.B, s.N, s.E});
-    if (!differentiable) qkv = hd = hg = lam = at::Tensor();
+    if (!inner) qkv = lam = at::Tensor();
+    if (!outer) hg = at::Tensor();
   }
   return Py_BuildValue("(NNNNNNN)", wrap(y), wrap(qkv), wrap(hd), wrap(hg), wrap(u2), wrap(stats), wrap(lam));
   END_HANDLE_TH_ERRORS
 }
 
 // layer_backward(x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, qkv, heads, scaled heads, u2, row statistics, lambda, dy,
-//                heads, causal, lambda_init, needed, stream)
-//   -> the gradients of the first ten arguments; `needed`: bit i says whether argument i's is wanted, None where not
+//                B, N, heads, causal, lambda_init, needed, stream)
+//   -> the gradients of the first ten arguments; `needed`: bit i says whether argument i's is wanted, None where not.
+//   What those do not take may be None: x without one of the q, k and v weights, these without x, and so on.
 PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 22) return PyErr_Format(PyExc_TypeError, "layer_backward takes 22 arguments");
+  if (n != 24) return PyErr_Format(PyExc_TypeError, "layer_backward takes 24 arguments");
   at::Tensor t[17], grad[10];
-  if (!tensors(a, 17, t)) return nullptr;
-  const int64_t heads = PyLong_AsLongLong(a[17]);
-  const bool causal = PyObject_IsTrue(a[18]) == 1;
-  const double lambda_init = PyFloat_AsDouble(a[19]);
-  const unsigned needed = (unsigned)PyLong_AsUnsignedLong(a[20]);
-  void* const stream = PyLong_AsVoidPtr(a[21]);
+  if (!tensors(a, 16, t, true) || !tensors(a + 16, 1, t + 16)) return nullptr;
+  const int64_t B = PyLong_AsLongLong(a[17]), N = PyLong_AsLongLong(a[18]), heads = PyLong_AsLongLong(a[19]);
+  const bool causal = PyObject_IsTrue(a[20]) == 1;
+  const double lambda_init = PyFloat_AsDouble(a[21]);
+  const unsigned needed = (unsigned)PyLong_AsUnsignedLong(a[22]);
+  void* const stream = PyLong_AsVoidPtr(a[23]);
   if (PyErr_Occurred()) return nullptr;
   {
     const Released released;
     const c10::impl::ExcludeDispatchKeyGuard no_autocast(kNoAutocast);
     auto want = [&](int i) { return (needed >> i & 1u) != 0; };
-    const Sizes s(t[0], t[15], heads, causal);
+    // of the tensors that a backward goes through first, one is always there
+    const at::ScalarType type = (t[11].defined() ? t[11] : t[12]).scalar_type();
+    const Sizes s({B, N, t[16].size(2)}, type, t[15].defined() ? t[15].numel() : 1, heads, causal);
     for (int i = 1; i < 16; ++i) t[i] = dense(t[i]);
-    const at::Tensor x2 = dense(t[0].reshape({s.T, s.E})), dy = dense(t[16].to(t[0].scalar_type()).reshape({s.T, s.E}));
+    const at::Tensor x2 = t[0].defined() ? dense(t[0].reshape({s.T, s.E})) : t[0], dy = dense(t[16].to(type).reshape({s.T, s.E}));
     const at::Tensor &qkv = t[10], &hd = t[11], &hg = t[12], &u2 = t[13], &stats = t[14], &lam = t[15];
     const bool want_q = want(0) || want(1), want_kv = want(0) || want(2) || want(3);
     const bool want_lam = want(6) || want(7) || want(8) || want(9);
@@ -211,12 +220,12 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     dhg.data_ptr(), d.q1, d.q2, d.k1, d.k2, d.v, dlam.data_ptr(), ws.data_ptr(), ws_bytes,
                                     (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, stages,
                                     &layout, nullptr, t[5].data_ptr(), (float*)gpart.data_ptr(), stream));
-      if (want(0)) grad[0] = not_a_view(at::mm(dqkv, pack(t + 1, s, nullptr, 0.f, nullptr, stream)), t[0].sizes());
-      if (want(5)) grad[5] = at::empty_like(t[5]);
+      if (want(0)) grad[0] = not_a_view(at::mm(dqkv, pack(t + 1, s, nullptr, 0.f, nullptr, stream)), {s.B, s.N, s.E});
+      if (want(5)) grad[5] = at::empty({2 * s.d}, hd.options());
       if (want_lam)
         for (int i = 6; i < 10; ++i) grad[i] = at::empty_like(t[i]);
       if (want(5) || want_lam) {
-        const diffattn_lambda_vectors vec = vectors(t + 6, s);
+        const diffattn_lambda_vectors vec = want_lam ? vectors(t + 6, s) : diffattn_lambda_vectors{};
         auto f = [&](int i) { return want_lam ? (float*)grad[i].data_ptr() : nullptr; };
         check(diffattn_layer_finish((const float*)gpart.data_ptr(), (int)n_part, (int)(2 * s.d), want(5) ? grad[5].data_ptr() : nullptr, &vec,
                                     want_lam ? (const float*)dlam.data_ptr() : nullptr, f(6), f(7), f(8), f(9), s.flags & DIFFATTN_BF16, stream));

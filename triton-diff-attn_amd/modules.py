@@ -38,18 +38,29 @@ class _diff_attn_layer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, heads, causal, lambda_init):
         inputs = (x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2)
-        ctx.options = (heads, causal, lambda_init)
-        differentiable = any(ctx.needs_input_grad)
-        y, *saved = _native.layer().layer_forward(*inputs, *ctx.options, differentiable, _current_stream(x.device))
-        if differentiable:
-            ctx.save_for_backward(*inputs, *saved)
+        options = (heads, causal, lambda_init)
+        need = ctx.needs_input_grad
+        projections, lambdas = any(need[1:4]), any(need[6:10])
+        operator = need[0] or projections or lambdas        # its gradients are wanted
+        inner = operator or need[5]                         # a gradient behind the output projection is
+        y, *saved = _native.layer().layer_forward(*inputs, *options, inner, need[4], _current_stream(x.device))
+        if inner or need[4]:
+            ctx.options = (*x.shape[:2], *options)
+            # An input is saved where the single operations would save it: what no wanted gradient reads may be written in
+            # place before the backward, and is not held until then.  The gain beside its own gradient alone is such a one,
+            # but the kernel that forms that gradient reads it: its values, without the version that autograd would check.
+            keep = (projections, *(need[0],) * 3, inner, inner, *(lambdas,) * 4)
+            if inner and not operator:
+                gain = gain.data
+            inputs = (x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2)
+            ctx.save_for_backward(*(t if k else None for t, k in zip(inputs, keep)), *saved)
         return y
 
     @staticmethod
     @once_differentiable        # like the operator's: a second derivative raises
     def backward(ctx, dy):
         saved = ctx.saved_tensors
-        dev = saved[0].device
+        dev = dy.device
         needed = sum(1 << i for i in range(10) if ctx.needs_input_grad[i])
 
         def launch():
@@ -158,7 +169,7 @@ class DiffAttn(nn.Module):
             options = (self.num_heads, self.causal, self.lambda_init)
             if torch.is_grad_enabled():
                 return _diff_attn_layer.apply(*fused, *options)
-            return _native.layer().layer_forward(*fused, *options, False, _current_stream(x.device))[0]
+            return _native.layer().layer_forward(*fused, *options, False, False, _current_stream(x.device))[0]
         B, N, E = x.shape
         H, d = self.num_heads, self.head_dim
         q1, q2 = self._streams(self.q_proj(x).view(B, N, H, 2, d))
