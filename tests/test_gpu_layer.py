@@ -187,3 +187,35 @@ def test_only_what_a_gradient_reads_is_saved(wanted):
         y = layer(xg)
         del xg
         assert held() is None and y.requires_grad
+
+
+def test_only_the_gradients_asked_for_are_formed(monkeypatch):
+    """Of a layer that trains as a whole, grad() of some inputs and backward(inputs=...) form what they ask for and nothing
+    else."""
+    layer, _, x, dy = _pair()
+    x.requires_grad_(True)
+    inputs = [x, *(getattr(layer, n).weight for n in ("q_proj", "k_proj", "v_proj", "out_proj")), layer.head_gain,
+              layer.lambda_q1, layer.lambda_k1, layer.lambda_q2, layer.lambda_k2]
+    formed = []
+    native = _native.layer()
+
+    class Recorded:
+        layer_forward, wanted = native.layer_forward, native.wanted
+
+        @staticmethod
+        def layer_backward(*args):
+            formed.append(native.layer_backward(*args))
+            return formed[-1]
+
+    monkeypatch.setattr(_native, "layer", lambda: Recorded)
+    whole = torch.autograd.grad(layer(x), inputs, dy)
+    assert all(g is not None for g in formed.pop())
+    for ids in ((0,), (4,), (1, 2), (5,), (0, 4), (3, 9)):
+        y = layer(x)
+        grads = torch.autograd.grad(y, [inputs[i] for i in ids], dy)
+        for i, g in zip(ids, grads):
+            assert (g.double() - whole[i].double()).norm() <= _ULP[x.dtype] * whole[i].double().norm()
+        assert tuple(i for i, g in enumerate(formed.pop()) if g is not None) == ids
+    layer(x).backward(dy, inputs=[inputs[3]])
+    assert [i for i, g in enumerate(formed.pop()) if g is not None] == [3]
+    assert [i for i, t in enumerate(inputs) if t.grad is not None] == [3]

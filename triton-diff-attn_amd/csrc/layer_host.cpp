@@ -8,6 +8,7 @@
 // Here the operator reads q, k and v where one [tokens, 3E] product left them and writes its gradients into another.
 #include <Python.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -173,9 +174,28 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// wanted(ctx) -> bit i: the backward that is running wants a gradient of the i-th of the first ten tensors of the function
+// that ctx belongs to.  ctx.needs_input_grad is fixed by the forward; grad(loss, x), or a backward with a list of inputs, wants
+// less, and of the single operations the engine would run none behind the rest.
+PyObject* wanted(PyObject*, PyObject* ctx) {
+  HANDLE_TH_ERRORS
+  if (!THPFunction_Check(ctx)) return PyErr_Format(PyExc_TypeError, "wanted takes the context of a function");
+  unsigned bits = 0;
+  THPObjectPtr need(PyObject_GetAttrString(ctx, "needs_input_grad"));
+  if (!need) return nullptr;
+  const std::shared_ptr<torch::autograd::PyNode> node = ((THPFunction*)ctx)->cdata.lock();
+  for (int i = 0; i < 10; ++i) {
+    THPObjectPtr bit(PySequence_GetItem(need.get(), i));
+    if (!bit) return nullptr;
+    if (PyObject_IsTrue(bit.get()) == 1 && (!node || node->task_should_compute_output(i))) bits |= 1u << i;
+  }
+  return PyLong_FromUnsignedLong(bits);
+  END_HANDLE_TH_ERRORS
+}
+
 // layer_backward(x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, qkv, heads, scaled heads, u2, row statistics, lambda, dy,
-//                B, N, heads, causal, lambda_init, needed, stream)
-//   -> the gradients of the first ten arguments; `needed`: bit i says whether argument i's is wanted, None where not.
+//                B, N, heads, causal, lambda_init, wanted, stream)
+//   -> the gradients of the first ten arguments; `wanted`: bit i says whether argument i's is, None where not.
 //   What those do not take may be None: x without one of the q, k and v weights, these without x, and so on.
 PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -185,13 +205,13 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t B = PyLong_AsLongLong(a[17]), N = PyLong_AsLongLong(a[18]), heads = PyLong_AsLongLong(a[19]);
   const bool causal = PyObject_IsTrue(a[20]) == 1;
   const double lambda_init = PyFloat_AsDouble(a[21]);
-  const unsigned needed = (unsigned)PyLong_AsUnsignedLong(a[22]);
+  const unsigned wanted = (unsigned)PyLong_AsUnsignedLong(a[22]);
   void* const stream = PyLong_AsVoidPtr(a[23]);
   if (PyErr_Occurred()) return nullptr;
   {
     const Released released;
     const c10::impl::ExcludeDispatchKeyGuard no_autocast(kNoAutocast);
-    auto want = [&](int i) { return (needed >> i & 1u) != 0; };
+    auto want = [&](int i) { return (wanted >> i & 1u) != 0; };
     // of the tensors that a backward goes through first, one is always there
     const at::ScalarType type = (t[11].defined() ? t[11] : t[12]).scalar_type();
     const Sizes s({B, N, t[16].size(2)}, type, t[15].defined() ? t[15].numel() : 1, heads, causal);
@@ -272,6 +292,7 @@ PyObject* weight_gradient(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"layer_forward", (PyCFunction)(void (*)())layer_forward, METH_FASTCALL, nullptr},
     {"layer_backward", (PyCFunction)(void (*)())layer_backward, METH_FASTCALL, nullptr},
+    {"wanted", (PyCFunction)wanted, METH_O, nullptr},
     {"weight_gradient", (PyCFunction)(void (*)())weight_gradient, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -61,10 +61,10 @@ class _diff_attn_layer(torch.autograd.Function):
     def backward(ctx, dy):
         saved = ctx.saved_tensors
         dev = dy.device
-        needed = sum(1 << i for i in range(10) if ctx.needs_input_grad[i])
+        wanted = _native.layer().wanted(ctx)
 
         def launch():
-            return _native.layer().layer_backward(*saved, dy, *ctx.options, needed, _current_stream(dev))
+            return _native.layer().layer_backward(*saved, dy, *ctx.options, wanted, _current_stream(dev))
 
         if dev.index != torch._C._cuda_getDevice():
             with torch.cuda.device(dev):
