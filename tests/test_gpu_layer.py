@@ -107,7 +107,7 @@ def test_which_calls_the_node_stands_for():
     y = layer(x.requires_grad_(True))
     (g,) = torch.autograd.grad(y.float().square().sum(), x, create_graph=True)
     with pytest.raises(RuntimeError):
-        g.sum().backward()      # as before: no second derivative
+        g.sum().backward()      # the operator's gradients have no derivative
     # saved tensors go through hooks that return other memory
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda()):
         y2 = layer(x)
@@ -219,3 +219,33 @@ def test_only_the_gradients_asked_for_are_formed(monkeypatch):
     layer(x).backward(dy, inputs=[inputs[3]])
     assert [i for i, g in enumerate(formed.pop()) if g is not None] == [3]
     assert [i for i, t in enumerate(inputs) if t.grad is not None] == [3]
+
+
+@pytest.mark.parametrize("frozen", [(), ("q_proj.weight", "k_proj.weight", "v_proj.weight"), ("x",), ("x", "qkv", "lambda")])
+@pytest.mark.parametrize("of", ["out_proj.weight", "head_gain"])
+def test_second_derivatives(of, frozen):
+    """A penalty on the gradient of the output projection or of the gain is differentiable by everything that it depends on,
+    also by an x that nobody holds any more and by tensors of which no values were saved."""
+    layer, single, x, dy = _pair(causal=True)
+    results = []
+    for l in (layer, single):
+        params = dict(l.named_parameters())
+        for n, p in params.items():
+            p.requires_grad_(not any(n.startswith(f) or f == "qkv" and n[:6] in ("q_proj", "k_proj", "v_proj") for f in frozen))
+        leaf = x.clone().requires_grad_("x" not in frozen)
+        factor = torch.ones((), device="cuda", dtype=x.dtype, requires_grad=True)
+        calls = []
+        params[of].register_hook(lambda g: calls.append(1) or 2.0 * g)
+        y = l(leaf * 1.0)
+        (g,) = torch.autograd.grad((y * y * factor).float().sum() / 64, params[of], create_graph=True)
+        assert len(calls) == 1
+        (g.float().square().sum() / 1024).backward()
+        results.append((y, g, factor.grad, leaf.grad, *(p.grad for p in params.values())))
+    tensors = 0
+    for a, b in zip(*results):
+        assert (a is None) == (b is None)
+        if a is not None:
+            tensors += 1
+            # the same operations on values that differ by their last bits
+            assert (a.double() - b.double()).norm() <= 16 * _ULP[x.dtype] * b.double().norm()
+    assert tensors >= 5

@@ -193,6 +193,23 @@ PyObject* wanted(PyObject*, PyObject* ctx) {
   END_HANDLE_TH_ERRORS
 }
 
+// input_edge(ctx, i, like, sizes...) -> a tensor of unset values that stands in autograd's graph where tensor i of the function
+// of ctx does: for a gradient that goes on to an input whose values nobody saved, because no gradient reads them
+PyObject* input_edge(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n < 4 || !THPFunction_Check(a[0]) || !THPVariable_Check(a[2])) return PyErr_Format(PyExc_TypeError, "input_edge takes a context, an index, a tensor and sizes");
+  const long i = PyLong_AsLong(a[1]);
+  std::vector<int64_t> sizes;
+  for (Py_ssize_t k = 3; k < n; ++k) sizes.push_back(PyLong_AsLongLong(a[k]));
+  if (PyErr_Occurred()) return nullptr;
+  const std::shared_ptr<torch::autograd::PyNode> node = ((THPFunction*)a[0])->cdata.lock();
+  TORCH_CHECK(node && i >= 0 && (size_t)i < node->num_outputs(), "no such input");
+  at::Tensor t = at::empty(sizes, THPVariable_Unpack(a[2]).options());
+  if (node->next_edge(i).is_valid()) torch::autograd::impl::set_gradient_edge(t, node->next_edge(i));
+  return wrap(t);
+  END_HANDLE_TH_ERRORS
+}
+
 // layer_backward(x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, qkv, heads, scaled heads, u2, row statistics, lambda, dy,
 //                B, N, heads, causal, lambda_init, wanted, stream)
 //   -> the gradients of the first ten arguments; `wanted`: bit i says whether argument i's is, None where not.
@@ -292,6 +309,7 @@ PyObject* weight_gradient(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"layer_forward", (PyCFunction)(void (*)())layer_forward, METH_FASTCALL, nullptr},
     {"layer_backward", (PyCFunction)(void (*)())layer_backward, METH_FASTCALL, nullptr},
+    {"input_edge", (PyCFunction)(void (*)())input_edge, METH_FASTCALL, nullptr},
     {"wanted", (PyCFunction)wanted, METH_O, nullptr},
     {"weight_gradient", (PyCFunction)(void (*)())weight_gradient, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

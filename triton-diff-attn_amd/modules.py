@@ -18,7 +18,6 @@ import math
 import torch
 from torch import nn
 from torch.autograd import forward_ad
-from torch.autograd.function import once_differentiable
 
 import _native
 from kernel import _DTYPES, _SUPPORTED_D, _current_stream
@@ -30,10 +29,40 @@ def lambda_init_for_depth(depth: int) -> float:
     return 0.8 - 0.6 * math.exp(-0.3 * depth)
 
 
+class _recalled_linear(torch.autograd.Function):
+    """F.linear(x, w) with its value at hand: what autograd needs of it is the graph."""
+
+    @staticmethod
+    def forward(ctx, value, x, w):
+        ctx.save_for_backward(x if ctx.needs_input_grad[2] else None, w if ctx.needs_input_grad[1] else None)
+        return value.view_as(value)
+
+    @staticmethod
+    def backward(ctx, g):
+        x, w = ctx.saved_tensors
+        return None, None if w is None else g @ w, None if x is None else g.flatten(0, 1).t() @ x.flatten(0, 1)
+
+
+class _recalled_gain(torch.autograd.Function):
+    """heads * gain with its value at hand, of heads [tokens, E] that need no gradient"""
+
+    @staticmethod
+    def forward(ctx, value, heads, gain):
+        ctx.save_for_backward(heads)
+        ctx.width = gain.numel()
+        return value.view_as(value)
+
+    @staticmethod
+    def backward(ctx, g):
+        return None, None, (g * ctx.saved_tensors[0]).view(-1, ctx.width).sum(0)
+
+
 class _diff_attn_layer(torch.autograd.Function):
     """The whole layer as one node: csrc/layer_host.cpp runs it.  (As single operations, B8 H8 N1024 d64 causal fp16: 39
     launches and 709 us of device time a step, of which the operator and four projections of 90 us in all are forward
-    work.)"""
+    work.)  A backward that is itself differentiated goes through the single operations, so that what they can differentiate
+    twice still can: the gradients of the output projection and of the gain.  Behind these is the operator, whose gradients
+    are plain kernel outputs; their derivative raises."""
 
     @staticmethod
     def forward(ctx, x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2, heads, causal, lambda_init):
@@ -57,11 +86,12 @@ class _diff_attn_layer(torch.autograd.Function):
         return y
 
     @staticmethod
-    @once_differentiable        # like the operator's: a second derivative raises
     def backward(ctx, dy):
         saved = ctx.saved_tensors
         dev = dy.device
         wanted = _native.layer().wanted(ctx)
+        if torch.is_grad_enabled():         # create_graph
+            return (*_differentiable_gradients(ctx, saved, dy, wanted), None, None, None)
 
         def launch():
             return _native.layer().layer_backward(*saved, dy, *ctx.options, wanted, _current_stream(dev))
@@ -72,6 +102,50 @@ class _diff_attn_layer(torch.autograd.Function):
         else:
             grads = launch()
         return (*grads, None, None, None)
+
+
+def _differentiable_gradients(ctx, saved, dy, wanted):
+    """The gradients of _diff_attn_layer as functions of dy and of its inputs."""
+    B, N, heads, causal, lambda_init = ctx.options
+    E, need = dy.size(-1), ctx.needs_input_grad
+    *inputs, qkv, hd, hg, _, _, lam = saved
+    operator = any(need[:4]) or any(need[6:])           # else the heads are constants
+
+    def at(i, *sizes):
+        """Input i.  What was not saved is not read, and its place in the graph is what counts.  An alias, at which the
+        gradients are taken: hooks on the inputs run where the node's gradients arrive, and not here too."""
+        t = inputs[i]
+        if sizes and (t is None or i == 5 and not operator):
+            t = _native.layer().input_edge(ctx, i, dy, *sizes)
+        inputs[i] = None if t is None else t.view_as(t)
+        return inputs[i]
+
+    with torch.autocast("cuda", enabled=False):
+        wo, gain = at(4, E, E), at(5, E // heads)
+        if operator:
+            x, *weights = at(0, B, N, E), at(1, E, E), at(2, E, E), at(3, E, E)
+            q, k, v = (_recalled_linear.apply(value, x, w) for value, w in zip(qkv.view(B, N, 3, E).unbind(2), weights))
+            q1, q2 = q.view(B, N, heads, 2, -1).transpose(1, 2).unbind(3)
+            k1, k2 = k.view(B, N, heads, 2, -1).transpose(1, 2).unbind(3)
+            vectors = [at(i) for i in range(6, 10)]
+            if vectors[0] is not None:
+                lam = _lambda(*vectors, lambda_init)
+            y = MultiheadDiffAttnKernel(q1, q2, k1, k2, v.view(B, N, heads, -1).transpose(1, 2), lambda_scale=lam,
+                                        lambda_init=lambda_init, rms_norm=True, causal=causal)
+            y = (y * gain).transpose(1, 2)
+        else:
+            y = _recalled_gain.apply(hd if hg is None else hg, hd, gain) if need[5] else hg
+        y = nn.functional.linear(y.reshape(B, N, E), wo)
+        ids = [i for i in range(10) if wanted >> i & 1]
+        grads = [None] * 10
+        for i, g in zip(ids, torch.autograd.grad(y, [inputs[i] for i in ids], dy, create_graph=True)):
+            grads[i] = g
+    return grads
+
+
+def _lambda(q1, k1, q2, k2, lambda_init):
+    """[1], or [num_heads] from vectors per head"""
+    return (torch.exp((q1 * k1).sum(-1)) - torch.exp((q2 * k2).sum(-1)) + lambda_init).reshape(-1)
 
 
 def _plain(t):
@@ -113,9 +187,7 @@ class DiffAttn(nn.Module):
         self.head_gain = nn.Parameter(torch.ones(2 * self.head_dim, **kw))
 
     def lambda_scale(self) -> torch.Tensor:
-        lam = (torch.exp((self.lambda_q1 * self.lambda_k1).sum(-1))
-               - torch.exp((self.lambda_q2 * self.lambda_k2).sum(-1)) + self.lambda_init)
-        return lam.reshape(-1)      # [1], or [num_heads] with per_head_lambda
+        return _lambda(self.lambda_q1, self.lambda_k1, self.lambda_q2, self.lambda_k2, self.lambda_init)
 
     def _streams(self, p: torch.Tensor):
         """[B, N, H, 2, d] -> two [B, H, N, d] views: sub-heads 2h and 2h+1 of the q/k projections are the two softmax
