@@ -46,6 +46,10 @@ def _node(layer, x):
     (2, 200, 3, 64, True, True, torch.float16),           # E = 384, padded sequence
     (3, 256, 4, 64, False, True, torch.bfloat16),
     (2, 130, 2, 128, False, False, torch.float16),
+    (1, 130, 40, 64, True, False, torch.float16),         # E = 5120: the widest layer whose weights are packed
+    (2, 48, 40, 64, True, False, torch.bfloat16),         # ... and where those of few tokens are not, forward
+    (1, 130, 41, 64, False, True, torch.float16),         # E = 5248: a product for each projection
+    (2, 2050, 12, 128, True, False, torch.bfloat16),      # E = 3072 and many tokens: forward only
 ])
 def test_layer_node_matches_its_operations(B, N, H, d, causal, per_head, dtype):
     gen = torch.Generator(device="cuda").manual_seed(N)

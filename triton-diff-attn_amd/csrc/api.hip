@@ -389,7 +389,7 @@ int diffattn_layer_backward(const void* q1, const void* q2, const void* k1, cons
 
 int diffattn_layer_pack(const void* w0, const void* w1, const void* w2, void* packed, size_t weight_bytes,
                         const diffattn_lambda_vectors* vectors, float lambda_init, float* lambda, void* stream) {
-  if (!w0 || !w1 || !w2 || !packed || (lambda && !vectors)) return DIFFATTN_EINVAL_NULL;
+  if ((weight_bytes && (!w0 || !w1 || !w2 || !packed)) || (lambda && !vectors)) return DIFFATTN_EINVAL_NULL;
   if (weight_bytes % 16 != 0) return DIFFATTN_EINVAL_DIM;
   for (const void* q : {w0, w1, w2, (const void*)packed})
     if (!aligned16(q)) return DIFFATTN_EINVAL_ALIGN;

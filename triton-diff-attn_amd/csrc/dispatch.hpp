@@ -60,6 +60,26 @@ constexpr bool bwd_one_grid(int d, bool dropout, bool causal, int n, long long b
   return one < two;
 }
 
+// Whether the layer's three input projections, or their input gradient, are one product with the three weights E x E copied
+// one behind another, instead of a product for each.  One product of 3E fills the chip where one of E does not, and saves two
+// launches; the copy moves 12 E^2 bytes, and a product on few tokens is bound by the 6 E^2 that it reads.  Device time of
+// both, us, fp16 (bf16 the same within 10 %, with the weights of several layers in turn), one product | three:
+//   E 1024, 77 tokens 15 | 19, 1024 22 | 30, 8192 66 | 70;  E 2048: 24 | 29, 40 | 51, 164 | 162;  E 3584: 45 | 58, 94 | 110
+//   E 4096, 32 tokens 50 | 37, 77 54 | 48, 128 56 | 69, 512 83 | 91, 1024 117 | 129, 4096 322 | 299
+//   E 5120, 32 tokens 82 | 57, 77 89 | 65, 128 91 | 100, 512 129 | 147, 1024 189 | 197, 4096 528 | 576
+//   E 5632, 32 tokens 115 | 61, 512 167 | 147, 2048 489 | 338, 4096 712 | 661;  E 8192: 229 | 96, 299 | 249, 697 | 594, 1238 | 1130
+// Up to E 4730 the weights and their copy fit the last-level cache of 256 MB, up to E 5120 most of them do; beyond that both
+// go to memory.  Few tokens at E 4096 to 4608: the three products are the faster ones on the device, but 37 us more of host
+// time, which is what bounds such a call (E 4096, 77 tokens, the layer's forward: 66 us on the device instead of 75, and 102
+// us a call instead of 74; E 5120 77 instead of 123, and 101 instead of 122; E 8192 171 instead of 282 both ways).  At E 3072 to
+// 4096 the single product of many tokens takes a worse library kernel (E 3072, 4096 tokens 216 | 206, 8192 466 | 406; not at E
+// 2560 and from 4608 on).  The input gradient (E 2048, 77 tokens 32 | 34, 4096 110 | 138; E 4096 81 | 68, 353 | 400; E 7168 280 |
+// 162, 1446 | 1111; E 8192 320 | 175, 1382 | 1396) has no such line, and its call with few tokens is bound by host time further up.
+constexpr bool layer_packed(bool backward, long long E, long long tokens) {
+  if (E > 5120) return false;
+  return backward || !((E > 4608 && tokens <= 96) || (E >= 3072 && E <= 4096 && tokens >= 4096));
+}
+
 // A weight gradient of the layer (wgrad_kernel, layer.hip): workgroups per 128 x 128 tile and the 64-token slabs that each
 // of them takes.  `tiles`: of all the weights of the launch.  One workgroup fills a CU's LDS, so tiles are split as far as one
 // round of workgroups goes, but not below four slabs, where starting a workgroup and adding its sums takes longer than they do.

@@ -18,8 +18,9 @@ typedef struct diffattn_lambda_vectors {
   int n, d;
 } diffattn_lambda_vectors;
 
-/* Copies three matrices of weight_bytes (a multiple of 16) each one behind the other to `packed`, and forms lambda
- * (skipped when `lambda` is NULL; then `vectors` may be NULL too). */
+/* Copies three matrices of weight_bytes (a multiple of 16) each one behind the other to `packed` (skipped when weight_bytes
+ * is 0; then the matrices and `packed` may be NULL), and forms lambda (skipped when `lambda` is NULL; then `vectors` may be
+ * NULL too). */
 int diffattn_layer_pack(const void* w0, const void* w1, const void* w2, void* packed, size_t weight_bytes,
                         const diffattn_lambda_vectors* vectors, float lambda_init, float* lambda, void* stream);
 

@@ -13,6 +13,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 
+#include "dispatch.hpp"
 #include "layer_abi.h"
 
 namespace {
@@ -96,6 +97,14 @@ at::Tensor pack(const at::Tensor* w, const Sizes& s, const diffattn_lambda_vecto
   return packed;
 }
 
+// dqkv [T, 3E] times the three weights one below another: a single sum, rounded once, also where it is three products
+at::Tensor input_gradient(const at::Tensor& dqkv, const at::Tensor* w, const Sizes& s, void* stream) {
+  if (da_abi::layer_packed(true, s.E, s.T)) return at::mm(dqkv, pack(w, s, nullptr, 0.f, nullptr, stream));
+  at::Tensor sum = at::mm(dqkv.narrow(1, 0, s.E), w[0], at::kFloat);
+  for (int i = 1; i < 3; ++i) at::addmm_out(sum, sum, dqkv.narrow(1, i * s.E, s.E), w[i], at::kFloat);
+  return sum.to(dqkv.scalar_type());
+}
+
 // out = a^T b for each job, in one launch of the framework's kernel where it is the faster one, else as library products.
 // The library's tiles for few outputs and a long contraction leave most of the chip idle.  One product, fp16, us, library ->
 // kernel: E 256, 8192 tokens 47.5 -> 18.1; E 512, 1000 tokens 18.9 -> 12.1, 16384 99.9 -> 21.4; E 1024, 256 tokens 18.6 -> 8.0, 8192
@@ -150,7 +159,16 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor x2 = x.reshape({s.T, s.E});
     lam = at::empty({t[6].numel() / s.d}, t[6].options());
     const diffattn_lambda_vectors vec = vectors(t + 6, s);
-    qkv = at::mm(x2, pack(t + 1, s, &vec, (float)lambda_init, (float*)lam.data_ptr(), stream).t());
+    if (da_abi::layer_packed(false, s.E, s.T)) {
+      qkv = at::mm(x2, pack(t + 1, s, &vec, (float)lambda_init, (float*)lam.data_ptr(), stream).t());
+    } else {
+      check(diffattn_layer_pack(nullptr, nullptr, nullptr, nullptr, 0, &vec, (float)lambda_init, (float*)lam.data_ptr(), stream));
+      qkv = at::empty({s.T, 3 * s.E}, x.options());
+      for (int i = 0; i < 3; ++i) {
+        at::Tensor out = qkv.narrow(1, i * s.E, s.E);
+        at::mm_out(out, x2, t[1 + i].t());
+      }
+    }
     hg = at::empty({s.T, s.E}, qkv.options());
     float* st = nullptr;
     const int64_t rows = s.B * s.H * s.n_pad;
@@ -257,7 +275,7 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     dhg.data_ptr(), d.q1, d.q2, d.k1, d.k2, d.v, dlam.data_ptr(), ws.data_ptr(), ws_bytes,
                                     (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, stages,
                                     &layout, nullptr, t[5].data_ptr(), (float*)gpart.data_ptr(), stream));
-      if (want(0)) grad[0] = not_a_view(at::mm(dqkv, pack(t + 1, s, nullptr, 0.f, nullptr, stream)), {s.B, s.N, s.E});
+      if (want(0)) grad[0] = not_a_view(input_gradient(dqkv, t + 1, s, stream), {s.B, s.N, s.E});
       if (want(5)) grad[5] = at::empty({2 * s.d}, hd.options());
       if (want_lam)
         for (int i = 6; i < 10; ++i) grad[i] = at::empty_like(t[i]);
