@@ -46,6 +46,7 @@ def _node(layer, x):
     (2, 200, 3, 64, True, True, torch.float16),           # E = 384, padded sequence
     (3, 256, 4, 64, False, True, torch.bfloat16),
     (2, 130, 2, 128, False, False, torch.float16),
+    (2, 2048, 8, 64, True, False, torch.float16),         # E = 1024: one weight in four splits, four in one
     (1, 130, 40, 64, True, False, torch.float16),         # E = 5120: the widest layer whose weights are packed
     (2, 48, 40, 64, True, False, torch.bfloat16),         # ... and where those of few tokens are not, forward
     (1, 130, 41, 64, False, True, torch.float16),         # E = 5248: a product for each projection
@@ -76,7 +77,14 @@ def test_layer_node_matches_its_operations(B, N, H, d, causal, per_head, dtype):
     assert all(torch.equal(again[n], got[n]) for n in got)
     with torch.no_grad():
         assert torch.equal(layer(x), got["y"])
-    # any subset of the gradients is what the whole gives
+    # Any subset of the gradients is what the whole gives, bit for bit but for weights: how the sum over the tokens is split
+    # depends on how many weights want theirs.  Two fp32 sums of the same products that round to different values round to
+    # neighbours, 2 ulp of a half apart at most.
+    def same(n, g):
+        if not n.endswith("weight"):
+            return torch.equal(g, got[n])
+        return (g.double() - got[n].double()).norm() <= 2 * _ULP[dtype] * got[n].double().norm()
+
     for wanted in (("x",), ("q_proj.weight",), ("k_proj.weight", "head_gain"), ("v_proj.weight", "lambda_k1"), ("out_proj.weight",)):
         part = copy.deepcopy(layer).requires_grad_(False)
         for n, p in part.named_parameters():
@@ -84,7 +92,7 @@ def test_layer_node_matches_its_operations(B, N, H, d, causal, per_head, dtype):
         xp = x.clone().requires_grad_("x" in wanted)
         part(xp).backward(dy)
         grads = dict({n: p.grad for n, p in part.named_parameters()}, x=xp.grad)
-        assert all(torch.equal(g, got[n]) if n in wanted else g is None for n, g in grads.items()), wanted
+        assert all(same(n, g) if n in wanted else g is None for n, g in grads.items()), wanted
 
 
 def test_which_calls_the_node_stands_for():

@@ -71,6 +71,24 @@ PACKED = {
     (12288, 200): (563.7, 335.1, 692.0, 543.6), (12288, 2048): (1919.3, 1465.6, 1865.3, 1666.9),
 }
 
+# (weights, E, tokens): us of a layer's weight gradients by wgrad_kernel and as library products, fp16
+WGRAD = {
+    (1, 256, 77): (8.3, 13.9), (1, 256, 16384): (25.5, 91.8), (1, 384, 77): (8.4, 6.6), (1, 384, 1000): (12.3, 14.0),
+    (1, 512, 256): (8.9, 7.1), (1, 512, 1000): (12.7, 14.0), (1, 512, 2048): (15.6, 17.1), (1, 512, 16384): (22.9, 98.5),
+    (1, 640, 256): (8.9, 7.2), (1, 640, 8192): (27.1, 49.7), (1, 768, 1000): (15.4, 14.1), (1, 768, 2048): (18.3, 17.2),
+    (1, 768, 4096): (21.8, 28.5), (1, 1024, 77): (8.6, 6.8), (1, 1024, 1000): (20.6, 14.3), (1, 1024, 2048): (22.2, 18.1),
+    (1, 1024, 4096): (23.7, 30.8), (1, 1152, 1000): (18.7, 17.7), (1, 1152, 2048): (23.5, 21.7), (1, 1152, 4096): (33.0, 34.2),
+    (1, 1280, 1000): (20.3, 17.5), (1, 1280, 8192): (41.4, 65.3), (1, 1536, 77): (9.0, 9.6), (1, 1536, 1000): (15.4, 21.0),
+    (1, 2048, 256): (10.2, 10.7), (1, 2048, 16384): (146.4, 164.3), (1, 2560, 256): (16.5, 14.1),
+    (1, 3072, 8192): (202.7, 158.2), (1, 4096, 1000): (66.9, 43.2), (2, 512, 77): (8.6, 11.9), (2, 1024, 1000): (23.1, 27.2),
+    (2, 1152, 2048): (22.8, 42.0), (2, 2048, 77): (16.7, 18.8), (3, 384, 77): (8.5, 16.9), (3, 1280, 256): (16.8, 22.5),
+    (3, 1792, 8192): (204.8, 235.0), (3, 3072, 2048): (162.0, 143.8), (4, 256, 1000): (12.9, 139.9),
+    (4, 768, 8192): (60.8, 198.2), (4, 1024, 77): (9.7, 23.4), (4, 1024, 8192): (72.6, 211.9), (4, 1152, 77): (15.9, 27.7),
+    (4, 1152, 8192): (147.2, 242.9), (4, 1536, 2048): (64.1, 100.3), (4, 2048, 77): (29.6, 36.0),
+    (4, 2048, 16384): (637.0, 686.0), (4, 2560, 2048): (156.1, 143.4), (4, 2560, 8192): (516.2, 479.6),
+    (4, 3072, 8192): (722.0, 637.6), (4, 4096, 16384): (2576.7, 1875.5),
+}
+
 
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
@@ -80,12 +98,16 @@ def rules(tmp_path_factory):
     (tmp / "rules.cpp").write_text('#include "dispatch.hpp"\nextern "C" {\n'
                                    "int fwd(int d, int causal, int n, long long blocks) { return da_abi::fwd_64_rows(d, causal, n, blocks); }\n"
                                    "int bwd(int d, int causal, int n, long long blocks) { return da_abi::bwd_one_grid(d, false, causal, n, blocks, 15u); }\n"
-                                   "int packed(int backward, long long E, long long tokens) { return da_abi::layer_packed(backward, E, tokens); }\n}\n")
+                                   "int packed(int backward, long long E, long long tokens) { return da_abi::layer_packed(backward, E, tokens); }\n"
+                                   "int wgrad(int weights, long long E, long long tokens) { return da_abi::wgrad_own(weights, E, tokens); }\n"
+                                   "void split(long long tiles, int tokens, int* out) { auto s = da_abi::wgrad_split(tiles, tokens); out[0] = s.splits; out[1] = s.slabs; }\n"
+                                   "}\n")
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I" + CSRC, str(tmp / "rules.cpp"), "-o", str(tmp / "rules.so")], check=True)
     lib = ctypes.CDLL(str(tmp / "rules.so"))
     for f in (lib.fwd, lib.bwd):
         f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_longlong]
-    lib.packed.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
+    lib.packed.argtypes = lib.wgrad.argtypes = [ctypes.c_int, ctypes.c_longlong, ctypes.c_longlong]
+    lib.split.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     return lib
 
 
@@ -95,6 +117,25 @@ def test_the_projections_take_the_faster_products(rules):
         pairs = {k: t[2 * backward:2 * backward + 2] for k, t in PACKED.items()}
         assert not {k: (backward, one, three) for k, (one, three) in pairs.items()
                     if (one if rules.packed(backward, *k) else three) > 1.06 * min(one, three)}
+
+
+def test_the_weight_gradients_take_the_faster_way(rules):
+    """Within 11 %: that of a single weight at 1000 tokens of E 512, on the near side of a line that fits E 1024."""
+    assert not {k: (own, lib) for k, (own, lib) in WGRAD.items() if (own if rules.wgrad(*k) else lib) > 1.11 * min(own, lib)}
+    assert not rules.wgrad(4, 64, 1000) and not rules.wgrad(4, 1088, 1000)      # the kernel's tiles are 128 wide
+
+
+def test_the_split_of_a_weight_gradient(rules):
+    """Every slab of 64 tokens in exactly one split, none without slabs, no split of fewer than four slabs (but for the last,
+    which takes what is left), and no more workgroups than CUs where there is anything to split."""
+    out = (ctypes.c_int * 2)()
+    for tiles in (1, 2, 4, 9, 36, 64, 100, 127, 128, 129, 144, 255, 256, 257, 1024, 4 * 128 * 128):
+        for tokens in (1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 1000, 4095, 4096, 4129, 16384, 100001, 2 ** 31 - 64):
+            rules.split(tiles, tokens, out)
+            splits, slabs = out
+            whole = -(-tokens // 64)
+            assert splits >= 1 and slabs >= 1 and (splits - 1) * slabs < whole <= splits * slabs, (tiles, tokens)
+            assert splits == 1 or (slabs >= 4 and splits * tiles <= 256), (tiles, tokens)
 
 
 def test_the_forward_takes_the_faster_workgroups(rules):

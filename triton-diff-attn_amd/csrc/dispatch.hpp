@@ -94,4 +94,21 @@ constexpr WgradSplit wgrad_split(long long tiles, int tokens) {
   return {(all + slabs - 1) / slabs, slabs};
 }
 
+// Whether a layer's weight gradients go to wgrad_kernel, in one launch, or are a library product each.  The library's tiles
+// for few outputs and a long contraction leave most of the chip idle; from E 2560 on its larger tiles fill the chip and read
+// less.  Device time, us, fp16, library | kernel with the sum of its splits:
+//   four weights: E 256, 77 tokens 52 | 9, 8192 190 | 19;  E 512 23 | 9, 204 | 31;  E 768 23 | 9, 198 | 61;  E 1024 23 | 10, 212 | 73
+//     (946 TFLOP/s), 16384 403 | 141;  E 1152 28 | 16, 243 | 147;  E 1280 28 | 17, 257 | 132;  E 1536 34 | 23, 323 | 202;
+//     E 1792 35 | 29, 311 | 266;  E 2048 36 | 30, 337 | 296, 16384 686 | 637;  E 2560 45 | 47, 2048 143 | 156, 8192 480 | 516 (16384
+//     1494 | 1028);  E 3072 56 | 59, 638 | 722;  E 4096 68 | 102, 961 | 1308
+//   one weight: E 384, 256 tokens 7.0 | 8.7, 1000 14.0 | 12.3;  E 512, 77 tokens 6.7 | 8.6, 2048 17 | 15, 8192 52 | 23, 16384 98 | 23;
+//     E 768, 1000 tokens 14.3 | 15.6, 2048 17.2 | 18.2, 4096 29 | 22;  E 1024, 77 tokens 7.0 | 8.6, 1000 14.5 | 20.8, 2048 17.6 |
+//     22.7, 4096 31 | 24, 8192 56 | 30;  E 1152, 2048 tokens 21.7 | 23.4, 4096 34 | 33;  E 1280, 1000 tokens 17.5 | 20.3, 2048
+//     21.7 | 21.1;  E 1536, 77 tokens 9.6 | 9.0, 1000 21.0 | 15.4;  two weights: the kernel throughout (E 512, 77 tokens 12 | 9)
+// A single short product is a library tile to each CU and no splits to add, while the kernel's are few tiles, split.
+constexpr bool wgrad_own(int weights, long long E, long long tokens) {
+  if (E % kWgradTile != 0 || E > 2048) return false;
+  return weights > 1 || E <= 256 || E >= 1536 || tokens > 2 * E;
+}
+
 }  // namespace da_abi

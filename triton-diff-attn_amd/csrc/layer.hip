@@ -21,8 +21,10 @@ using da_abi::WgradParams;
 // of four LDS buffers, three slabs ahead; waves 0-3 take the first 32 tokens of a slab and waves 4-7 the last 32, each wave
 // a 64 x 64 quarter (four fragments for four products), and the two halves meet in LDS at the end.  Two waves per SIMD
 // hide each other's LDS reads without a second workgroup, whose tile would have to be added through memory.  Bound by the
-// matrix unit where the grid fills the chip (E 2048, 16384 tokens: 148 us, 927 TFLOP/s; a library product of that size 181 us),
-// by the start and end of its workgroups and the sum of the splits where it does not (E 512, 8192 tokens: 23 us, library 53).
+// matrix unit where the grid fills the chip (E 2048, 16384 tokens, one weight: 145 us, 948 TFLOP/s; a library product of that
+// size 165 us), by the start and end of its workgroups and the sum of the splits where it does not (E 512, one weight, with
+// wgrad_reduce_kernel: 23 us at 8192 and at 16384 tokens, library 52 and 98; between E 1024 and 2048 also by a last round that is
+// partly empty: four weights of E 1152, 324 tiles for 256 CUs, 8192 tokens 147 us = 591 TFLOP/s).
 struct WgradCfg {
   static constexpr int TILE = da_abi::kWgradTile, BK = da_abi::kWgradSlab, NW = 8, NT = NW * 64, NBUF = 4;
   static constexpr int BUF = BK * TILE;                              // halfs of one operand's slab

@@ -47,7 +47,8 @@ int diffattn_layer_backward(const void* q1, const void* q2, const void* k1, cons
 
 /* out[E][E] = a^T b over T tokens, a and b [T][E] with row strides lda and ldb (elements, multiples of 8), for up to four
  * jobs of one size; E is a multiple of 128.  The contraction is split between workgroups where the tiles alone do not fill
- * the chip; workspace: diffattn_layer_wgrad_workspace_bytes (0 when nothing is split).  Fixed order: bit-reproducible. */
+ * the chip; workspace: diffattn_layer_wgrad_workspace_bytes (0 when nothing is split).  Bit-reproducible for a
+ * given number of jobs; with more or fewer of them the split, and with it the order of a sum, may be another. */
 typedef struct diffattn_wgrad_job {
   const void *a, *b;
   void* out;

@@ -105,18 +105,14 @@ at::Tensor input_gradient(const at::Tensor& dqkv, const at::Tensor* w, const Siz
   return sum.to(dqkv.scalar_type());
 }
 
-// out = a^T b for each job, in one launch of the framework's kernel where it is the faster one, else as library products.
-// The library's tiles for few outputs and a long contraction leave most of the chip idle.  One product, fp16, us, library ->
-// kernel: E 256, 8192 tokens 47.5 -> 18.1; E 512, 1000 tokens 18.9 -> 12.1, 16384 99.9 -> 21.4; E 1024, 256 tokens 18.6 -> 8.0, 8192
-// 59.1 -> 30.0 (572 TFLOP/s; 291 before), 16384 109.4 -> 46.8; E 2048, 256 tokens 19.5 -> 9.1, 16384 180.6 -> 148.3 (927 TFLOP/s).
-// From E 4096 on the library's larger tiles fill the chip and read less: 256 tokens 19.7 -> 30.3, 8192 256 -> 319, 16384 493 -> 630.
+// out = a^T b for each job: one launch of the framework's kernel, or a library product each
 struct Wgrad { at::Tensor a, b; };
-bool wgrad_own(int64_t E, int64_t T) { return E % 128 == 0 && E <= 2048 && T <= INT32_MAX; }
+bool wgrad_own(const std::vector<Wgrad>& jobs, int64_t E, int64_t T) { return T <= INT32_MAX && da_abi::wgrad_own((int)jobs.size(), E, T); }
 
-std::vector<at::Tensor> weight_gradients(const std::vector<Wgrad>& jobs, int64_t E, int64_t T, int flags, void* stream) {
+std::vector<at::Tensor> weight_gradients(const std::vector<Wgrad>& jobs, int64_t E, int64_t T, int flags, bool own, void* stream) {
   std::vector<at::Tensor> out;
   if (jobs.empty()) return out;
-  if (!wgrad_own(E, T)) {
+  if (!own) {
     for (const Wgrad& j : jobs) out.push_back(at::mm(j.a.t(), j.b));
     return out;
   }
@@ -289,7 +285,7 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (want(i)) { jobs.push_back({dqkv.narrow(1, (i - 1) * s.E, s.E), x2}); which.push_back(i); }
     }
     if (want(4)) { jobs.push_back({dy, hg}); which.push_back(4); }
-    const std::vector<at::Tensor> dw = weight_gradients(jobs, s.E, s.T, s.flags, stream);
+    const std::vector<at::Tensor> dw = weight_gradients(jobs, s.E, s.T, s.flags, wgrad_own(jobs, s.E, s.T), stream);
     for (size_t i = 0; i < dw.size(); ++i) grad[which[i]] = dw[i];
     for (int i = 6; i < 10; ++i)
       if (!want(i)) grad[i] = at::Tensor();
@@ -305,7 +301,7 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// weight_gradient(a, b, stream) -> a^T b for [T, E] tensors, by the kernel that layer_backward uses
+// weight_gradient(a, b, stream) -> a^T b for [T, E] tensors, by the kernel that layer_backward uses for several weights
 PyObject* weight_gradient(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 3) return PyErr_Format(PyExc_TypeError, "weight_gradient takes 3 arguments");
@@ -315,10 +311,12 @@ PyObject* weight_gradient(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (PyErr_Occurred()) return nullptr;
   TORCH_CHECK(t[0].dim() == 2 && t[0].sizes() == t[1].sizes() && t[0].is_cuda() && t[1].device() == t[0].device() &&
               t[0].scalar_type() == t[1].scalar_type() && (t[0].scalar_type() == at::kHalf || t[0].scalar_type() == at::kBFloat16) &&
-              t[0].stride(1) == 1 && t[1].stride(1) == 1 && t[0].size(0) > 0, "two 16-bit [T, E] tensors with contiguous rows");
+              t[0].stride(1) == 1 && t[1].stride(1) == 1 && t[0].size(0) > 0 && t[0].size(0) <= INT32_MAX,
+              "two 16-bit [T, E] tensors with contiguous rows");
   {
     const Released released;
-    out = weight_gradients({{t[0], t[1]}}, t[0].size(1), t[0].size(0), t[0].scalar_type() == at::kBFloat16 ? DIFFATTN_BF16 : 0, stream)[0];
+    out = weight_gradients({{t[0], t[1]}}, t[0].size(1), t[0].size(0), t[0].scalar_type() == at::kBFloat16 ? DIFFATTN_BF16 : 0,
+                           da_abi::wgrad_own(4, t[0].size(1), t[0].size(0)), stream)[0];
   }
   return wrap(out);
   END_HANDLE_TH_ERRORS
