@@ -58,12 +58,12 @@ def _load_build():
 
 @pytest.fixture(scope="module")
 def assembly(tmp_path_factory):
-    """Assembly text of the four compilations (backward and forward, fp16 and bf16), compiled side by side."""
+    """Assembly text of the six compilations (backward, forward and layer, fp16 and bf16), compiled side by side."""
     build = _load_build()
     tmp = tmp_path_factory.mktemp("isa")
     jobs = {}
     for key, src, variant in (("bwd_fp16", "bwd.hip", []), ("bwd_bf16", "bwd.hip", ["-DDA_BF16"]), ("fwd_fp16", "fwd.hip", []),
-                              ("fwd_bf16", "fwd.hip", ["-DDA_BF16"])):
+                              ("fwd_bf16", "fwd.hip", ["-DDA_BF16"]), ("layer_fp16", "layer.hip", []), ("layer_bf16", "layer.hip", ["-DDA_BF16"])):
         out = tmp / (key + ".s")
         cmd = [build.HIPCC] + [f for f in build.FLAGS if f != "-fPIC"] + build.SOURCE_FLAGS.get(src, []) + variant + ["--cuda-device-only", "-S", "-o", str(out),
                                                                               os.path.join(CSRC, src)]
@@ -118,7 +118,7 @@ def test_forward_kernels_do_not_spill_in_their_loops(assembly, variant):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-@pytest.mark.parametrize("source", ["bwd_fp16", "bwd_bf16", "fwd_fp16", "fwd_bf16"])
+@pytest.mark.parametrize("source", ["bwd_fp16", "bwd_bf16", "fwd_fp16", "fwd_bf16", "layer_fp16", "layer_bf16"])
 def test_tile_copies_do_not_read_an_address_too_early(assembly, source):
     """The base of a direct global->LDS copy, an asm statement, may have been reloaded from a vector register's lanes
     right in front of it."""
@@ -126,6 +126,14 @@ def test_tile_copies_do_not_read_an_address_too_early(assembly, source):
     assert "global_load_lds_dwordx4" in text
     hazards = isa_scan.asm_vmem_scalar_hazards(text)
     assert hazards == [], "tile copy right behind the vector write of its base: %s" % hazards[:5]
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("variant", ["fp16", "bf16"])
+def test_the_weight_gradient_does_not_spill(assembly, variant):
+    """A spilled base of its tile copies would be reloaded lane by lane right in front of them."""
+    text = assembly["layer_" + variant]
+    assert "wgrad_kernel" in text and "scratch_" not in text and "v_pk_fma_f32" not in text
 
 
 def test_build_rejects_a_spilling_kernel():
