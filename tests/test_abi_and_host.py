@@ -179,3 +179,21 @@ def test_drop_in_signature_matches_reference():
                                      "causal", "dropout_p", "dropout_seed"]
     assert fsig.parameters["causal"].default is False
     assert issubclass(_diff_attention, torch.autograd.Function)
+
+
+def test_layer_functions_reject_what_has_no_kernel():
+    import _native
+    lib = _native.lib()
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) & ~255) + 256
+    f, vp = ctypes.c_float, ctypes.c_void_p
+    rms, gain = 1, vp(p)
+
+    def backward(flags, gain):
+        return lib.diffattn_layer_backward(*[vp(p)] * 19, ctypes.c_size_t(1 << 30), 1, 1, 128, 128, 64, f(0.125), f(0.8), flags, 15,
+                                           None, gain, vp(p), None)
+
+    assert backward(0, gain) == -6                # the gain multiplies normalised heads
+    assert backward(rms, None) == -1
+    assert lib.diffattn_layer_pack(None, None, None, None, ctypes.c_size_t(256), None, f(0.8), None, None) == -1
+    assert lib.diffattn_layer_pack(vp(p), vp(p), vp(p), vp(p), ctypes.c_size_t(24), None, f(0.8), None, None) == -2

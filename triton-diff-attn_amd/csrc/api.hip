@@ -366,10 +366,9 @@ int diffattn_dropout_mask(unsigned char* keep, int B, int H, int N, int softmax_
 int diffattn_layer_forward(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
                            const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
                            int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
-                           const diffattn_layout* layout, const diffattn_dropout* dropout,
-                           const void* gain, void* y_gain, void* stream) {
+                           const diffattn_layout* layout, const void* gain, void* y_gain, void* stream) {
   return forward_impl(q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, B, H, N, n_valid, D, sm_scale, lambda_init, flags,
-                      layout, dropout, gain, y_gain, stream);
+                      layout, nullptr, gain, y_gain, stream);
 }
 
 size_t diffattn_layer_gain_parts(int B, int H, int N, int D) { return check_dims(B, H, N, D) ? 0 : (size_t)bwd_num_partials(B * H, N, D); }
@@ -380,10 +379,12 @@ int diffattn_layer_backward(const void* q1, const void* q2, const void* k1, cons
                              void* dq1, void* dq2, void* dk1, void* dk2, void* dv, void* dlambda,
                              void* workspace, size_t workspace_bytes,
                              int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
-                             unsigned stage_mask, const diffattn_layout* layout, const diffattn_dropout* dropout,
+                             unsigned stage_mask, const diffattn_layout* layout,
                              const void* gain, float* gain_part, void* stream) {
+  if (!gain) return DIFFATTN_EINVAL_NULL;
+  if (!(flags & DIFFATTN_RMS_NORM)) return DIFFATTN_EINVAL_FLAGS;      // the gain is that of the normalised heads
   return backward_impl(q1, q2, k1, k2, v, lambda_scale, y, u2, lse1, lse2, rinv, dy, dq1, dq2, dk1, dk2, dv, dlambda,
-                       workspace, workspace_bytes, B, H, N, n_valid, D, sm_scale, lambda_init, flags, stage_mask, layout, dropout,
+                       workspace, workspace_bytes, B, H, N, n_valid, D, sm_scale, lambda_init, flags, stage_mask, layout, nullptr,
                        gain, gain_part, stream);
 }
 

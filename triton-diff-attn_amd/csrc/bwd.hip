@@ -37,6 +37,7 @@ int bwd_num_partials(int BH, int N, int D) { (void)D; return (int)(((long long)B
 template <int D, bool RMS, bool GAIN = false>
 __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdParams p) {
   constexpr int DV = 2 * D, LPR = DV / 8, RPP = 256 / LPR;
+  static_assert(RMS || !GAIN, "a gain multiplies normalised heads");
   __shared__ float red[GAIN ? RPP * DV : 256];
   const int tid = threadIdx.x, sub = tid % LPR, rloc = tid / LPR;
   // the 64 rows of a workgroup belong to one (batch, head) unit: N is a multiple of 128
@@ -1348,10 +1349,8 @@ static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
   bool fold = (p.stages & 2u) && (p.stages & 12u);
   p.dlam_fold = 0;
   if (p.stages & 1u) {
-    if (p.gain && p.rms_norm)
+    if (p.gain)         // of normalised heads
       hipLaunchKernelGGL((bwd_prep_kernel<D, true, true>), dim3(n_prep), dim3(256), 0, stream, p);
-    else if (p.gain)
-      hipLaunchKernelGGL((bwd_prep_kernel<D, false, true>), dim3(n_prep), dim3(256), 0, stream, p);
     else if (p.rms_norm)
       hipLaunchKernelGGL((bwd_prep_kernel<D, true>), dim3(n_prep), dim3(256), 0, stream, p);
     else

@@ -225,6 +225,7 @@ __device__ __forceinline__ LambdaTerms lambda_terms(const diffattn_lambda_vector
   return {expf(s1), expf(s2)};
 }
 
+#ifndef DA_BF16       // it copies bytes: one build serves both types
 // the last workgroup forms lambda, the others copy the three weights one after another (16 bytes a thread and turn)
 __global__ __launch_bounds__(256) void layer_pack_kernel(LayerPackParams p) {
   if (blockIdx.x == gridDim.x - 1) {
@@ -248,6 +249,7 @@ hipError_t launch_layer_pack(const LayerPackParams& p, hipStream_t stream) {
   hipLaunchKernelGGL(layer_pack_kernel, dim3((unsigned)(want < 2048 ? want : 2048) + 1), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
+#endif
 
 // ---- the last sums of a backward -----------------------------------------------------------------
 // d(gain): workgroup b sums columns 16b .. 16b+15 of the partials, 64 rows of them at a time, then a tree in a fixed order.

@@ -48,6 +48,5 @@ hipError_t launch_layer_finish(const da_abi::LayerFinishParams& p, hipStream_t s
 }  // namespace da
 namespace da_bf16 {
 hipError_t launch_wgrad(const da_abi::WgradParams& p, hipStream_t stream);
-hipError_t launch_layer_pack(const da_abi::LayerPackParams& p, hipStream_t stream);
 hipError_t launch_layer_finish(const da_abi::LayerFinishParams& p, hipStream_t stream);
 }  // namespace da_bf16

@@ -24,15 +24,14 @@ typedef struct diffattn_lambda_vectors {
 int diffattn_layer_pack(const void* w0, const void* w1, const void* w2, void* packed, size_t weight_bytes,
                         const diffattn_lambda_vectors* vectors, float lambda_init, float* lambda, void* stream);
 
-/* diffattn_forward_padded that also, or with y NULL only, writes y * gain (2D values of the tensors' type, one per feature),
+/* diffattn_forward_padded without dropout that also, or with y NULL only, writes y * gain (2D values of the tensors' type, one per feature),
  * formed from y as it is stored and rounded once more, to y_gain, in the layout of y. */
 int diffattn_layer_forward(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
                            const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
                            int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
-                           const diffattn_layout* layout, const diffattn_dropout* dropout,
-                           const void* gain, void* y_gain, void* stream);
+                           const diffattn_layout* layout, const void* gain, void* y_gain, void* stream);
 
-/* diffattn_backward_stages for an output that the caller has multiplied by `gain` (2D values of the tensors' type, one per
+/* diffattn_backward_stages without dropout, with DIFFATTN_RMS_NORM in `flags`, for an output that the caller has multiplied by `gain` (2D values of the tensors' type, one per
  * feature): dy is the gradient of y * gain.  gain_part: diffattn_layer_gain_parts(B, H, N, D) rows of 2D fp32 values, the
  * partial sums of the gain's gradient, written by DIFFATTN_STAGE_PREP. */
 size_t diffattn_layer_gain_parts(int B, int H, int N, int D);
@@ -42,7 +41,7 @@ int diffattn_layer_backward(const void* q1, const void* q2, const void* k1, cons
                             void* dq1, void* dq2, void* dk1, void* dk2, void* dv, void* dlambda,
                             void* workspace, size_t workspace_bytes,
                             int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,
-                            unsigned stage_mask, const diffattn_layout* layout, const diffattn_dropout* dropout,
+                            unsigned stage_mask, const diffattn_layout* layout,
                             const void* gain, float* gain_part, void* stream);
 
 /* out[E][E] = a^T b over T tokens, a and b [T][E] with row strides lda and ldb (elements, multiples of 8), for up to four

@@ -179,7 +179,7 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     check(diffattn_layer_forward(p.q1, p.q2, p.k1, p.k2, p.v, lam.data_ptr(), inner ? hd.data_ptr() : nullptr,
                                  inner ? u2.data_ptr() : nullptr, st, st ? st + rows : nullptr, st ? st + 2 * rows : nullptr,
                                  (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, &layout,
-                                 nullptr, gain.data_ptr(), hg.data_ptr(), stream));
+                                 gain.data_ptr(), hg.data_ptr(), stream));
     y = not_a_view(at::mm(hg, wo.t()), {s.B, s.N, s.E});
     if (!inner) qkv = lam = at::Tensor();
     if (!outer) hg = at::Tensor();
@@ -270,7 +270,7 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
       check(diffattn_layer_backward(p.q1, p.q2, p.k1, p.k2, p.v, lam.data_ptr(), hd.data_ptr(), u2.data_ptr(), st, st + rows, st + 2 * rows,
                                     dhg.data_ptr(), d.q1, d.q2, d.k1, d.k2, d.v, dlam.data_ptr(), ws.data_ptr(), ws_bytes,
                                     (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, stages,
-                                    &layout, nullptr, t[5].data_ptr(), (float*)gpart.data_ptr(), stream));
+                                    &layout, t[5].data_ptr(), (float*)gpart.data_ptr(), stream));
       if (want(0)) grad[0] = not_a_view(input_gradient(dqkv, t + 1, s, stream), {s.B, s.N, s.E});
       if (want(5)) grad[5] = at::empty({2 * s.d}, hd.options());
       if (want_lam)
