@@ -53,6 +53,26 @@ def test_extension_module_refuses_a_library_of_another_version(tmp_path):
         assert accepted or "ImportError: libdiffattn has ABI version %d, diffattn_host was built against 7" % version in run.stderr
 
 
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_layer_module_refuses_a_library_of_another_version(tmp_path):
+    """Its functions have a version beside that of the operator's."""
+    import _native
+    shutil.copy(_native.LAYER_PATH, tmp_path / "diffattn_layer.so")
+    header = os.path.join(ROOT, "triton-diff-attn_amd", "csrc", "layer_abi.h")
+    current = int(re.search(r"#define DIFFATTN_LAYER_VERSION (\d+)", open(header).read()).group(1))
+    text = re.sub(r"/\*.*?\*/", "", open(header).read(), flags=re.S)
+    names = (set(re.findall(r"\b(diffattn_[a-z_]+)\s*\(", text)) | set(declared_symbols())) - {"diffattn_abi_version", "diffattn_layer_version"}
+    (tmp_path / "stub.c").write_text("int diffattn_abi_version(void) { return ABI; }\nint diffattn_layer_version(void) { return LAYER; }\n"
+                                     + "".join("int %s(void) { return 0; }\n" % n for n in sorted(names)))
+    load = "import torch, importlib.util as u; s = u.spec_from_file_location('diffattn_layer', %r); u.module_from_spec(s)" % str(tmp_path / "diffattn_layer.so")
+    for abi, layer, accepted in ((7, current, True), (7, current - 1, False), (7, current + 1, False), (8, current, False)):
+        subprocess.run(["g++", "-x", "c", "-shared", "-fPIC", "-DABI=%d" % abi, "-DLAYER=%d" % layer, str(tmp_path / "stub.c"),
+                        "-o", str(tmp_path / "libdiffattn.so")], check=True)
+        run = subprocess.run([sys.executable, "-c", load], capture_output=True, text=True)
+        assert (run.returncode == 0) == accepted, run.stderr
+        assert accepted or "ImportError: libdiffattn has" in run.stderr and "rebuild both" in run.stderr
+
+
 def test_argument_rejection_needs_no_gpu():
     import _native
     lib = _native.lib()

@@ -363,6 +363,8 @@ int diffattn_dropout_mask(unsigned char* keep, int B, int H, int N, int softmax_
   return (int)hipGetLastError();
 }
 
+int diffattn_layer_version(void) { return DIFFATTN_LAYER_VERSION; }
+
 int diffattn_layer_forward(const void* q1, const void* q2, const void* k1, const void* k2, const void* v,
                            const void* lambda_scale, void* y, void* u2, float* lse1, float* lse2, float* rinv,
                            int B, int H, int N, int n_valid, int D, float sm_scale, float lambda_init, int flags,

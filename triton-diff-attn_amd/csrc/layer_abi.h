@@ -8,9 +8,14 @@
 
 #include "../../include/diffattn.h"
 
+/* The version of the functions below, raised with every change to their arguments; those of diffattn.h have their own. */
+#define DIFFATTN_LAYER_VERSION 2
+
 #ifdef __cplusplus
 extern "C" {
 #endif
+
+int diffattn_layer_version(void);
 
 /* lambda[o] = exp(q1[o] . k1[o]) - exp(q2[o] . k2[o]) + lambda_init, o < n, vectors of d fp32 values */
 typedef struct diffattn_lambda_vectors {

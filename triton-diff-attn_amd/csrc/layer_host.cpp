@@ -334,8 +334,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "diffattn_layer", nullptr, -1, meth
 
 }  // namespace
 
-// A module that was built against another version of the library would call it with the wrong arguments.
+// A module that was built against another version of the library would call it with the wrong arguments.  The layer's
+// functions change without those of diffattn.h, so both versions are asked for.
 PyMODINIT_FUNC PyInit_diffattn_layer(void) {
+  if (diffattn_layer_version() != DIFFATTN_LAYER_VERSION)
+    return PyErr_Format(PyExc_ImportError, "libdiffattn has version %d of the layer's functions, diffattn_layer was built against %d: rebuild both",
+                        diffattn_layer_version(), DIFFATTN_LAYER_VERSION);
   if (diffattn_abi_version() != DIFFATTN_ABI_VERSION)
     return PyErr_Format(PyExc_ImportError, "libdiffattn has ABI version %d, diffattn_layer was built against %d: rebuild both",
                         diffattn_abi_version(), DIFFATTN_ABI_VERSION);
