@@ -261,3 +261,26 @@ def test_second_derivatives(of, frozen):
             # the same operations on values that differ by their last bits
             assert (a.double() - b.double()).norm() <= 16 * _ULP[x.dtype] * b.double().norm()
     assert tensors >= 5
+
+
+def test_replacements_of_the_linear_class_are_seen(monkeypatch):
+    """What replaces nn.Linear.forward, nn.Linear.__call__ or F.linear for all modules at once is called for the four
+    projections, as without the node."""
+    layer, _, x, _ = _pair()
+    calls = []
+
+    def recorded(f):
+        def call(*args):
+            calls.append(1)
+            return f(*args)
+        return call
+
+    with torch.no_grad():
+        want = layer(x)
+        for owner, name in ((torch.nn.Linear, "forward"), (torch.nn.Linear, "__call__"), (torch.nn.functional, "linear")):
+            with monkeypatch.context() as m:
+                m.setattr(owner, name, recorded(getattr(owner, name)), raising=True)
+                got = layer(x)
+            assert len(calls) == 4, name
+            calls.clear()
+            assert (got.double() - want.double()).norm() <= 8 * _ULP[x.dtype] * want.double().norm()

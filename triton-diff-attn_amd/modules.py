@@ -152,6 +152,15 @@ def _plain(t):
     return type(t) is torch.Tensor or type(t) is nn.Parameter
 
 
+_LINEAR_SOURCE = nn.modules.linear.__file__
+
+
+def _linear_is_its_own():
+    """Whether nn.Linear and F.linear are torch's: profilers and quantizers replace them for every module at once."""
+    return (getattr(getattr(nn.Linear.forward, "__code__", None), "co_filename", None) == _LINEAR_SOURCE
+            and nn.Linear.__call__ is nn.Module._wrapped_call_impl and nn.functional.linear is torch._C._nn.linear)
+
+
 def _plain_linear(m):
     """Whether calling m is F.linear with its weight and nothing else: no bias, hooks, wrapper or override."""
     return (type(m) is nn.Linear and m.bias is None and "forward" not in m.__dict__ and m._compiled_call_impl is None
@@ -218,7 +227,7 @@ class DiffAttn(nn.Module):
                 or "lambda_scale" in self.__dict__ or "_streams" in self.__dict__):
             return None
         projections = (self.q_proj, self.k_proj, self.v_proj, self.out_proj)
-        if not all(_plain_linear(m) for m in projections):
+        if not (_linear_is_its_own() and all(_plain_linear(m) for m in projections)):
             return None
         E, H, d, dev = self.embed_dim, self.num_heads, self.head_dim, x.device
         if x.size(2) != E or dev.index != torch._C._cuda_getDevice() or x.size(0) * H * (x.size(1) + 127) > 1 << 28:
