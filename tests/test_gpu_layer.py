@@ -284,3 +284,22 @@ def test_replacements_of_the_linear_class_are_seen(monkeypatch):
             assert len(calls) == 4, name
             calls.clear()
             assert (got.double() - want.double()).norm() <= 8 * _ULP[x.dtype] * want.double().norm()
+
+
+@pytest.mark.parametrize("which", ["x", "dy", "weight"])
+def test_pending_negations(which):
+    """A tensor with the negative bit set is stored with the other sign, which a kernel cannot see."""
+    layer, single, x, dy = _pair()
+    if which == "x":
+        x = torch._neg_view(-x)
+    elif which == "dy":
+        dy = torch._neg_view(-dy)
+    else:
+        for l in (layer, single):
+            l.k_proj.weight = torch.nn.Parameter(torch._neg_view(-l.k_proj.weight.detach()))
+    grads = []
+    for l in (layer, single):
+        y = l(x)
+        grads.append((y, *torch.autograd.grad(y, [p for p in l.parameters() if p.dtype == x.dtype], dy)))
+    for a, b in zip(*grads):
+        assert (a.double() - b.double()).norm() <= 8 * _ULP[x.dtype] * b.double().norm()

@@ -47,10 +47,11 @@ void check(int rc) {
   TORCH_CHECK(rc == DIFFATTN_OK, "libdiffattn: ", diffattn_strerror(rc), " (code ", rc, ")");
 }
 
-// t as the kernels read it: dense and 16-byte aligned (what autograd's saved-tensor hooks hand back may be neither)
+// t as the kernels read it: dense, 16-byte aligned (what autograd's saved-tensor hooks hand back may be neither) and without
+// a pending negation, which only torch's own operations know of
 at::Tensor dense(const at::Tensor& t) {
   if (!t.defined()) return t;
-  at::Tensor c = t.contiguous();
+  at::Tensor c = t.resolve_neg().contiguous();
   return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone();
 }
 

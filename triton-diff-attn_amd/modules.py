@@ -240,7 +240,8 @@ class DiffAttn(nn.Module):
         shapes = ((E, E),) * 4 + ((2 * d,),) + (shape,) * 4
         dtypes = (x.dtype,) * 5 + (torch.float32,) * 4
         for t, s, dt in zip(inputs, shapes, dtypes):
-            if not (_plain(t) and t.shape == s and t.dtype == dt and t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            if not (_plain(t) and t.shape == s and t.dtype == dt and t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    and not t.is_neg()):
                 return None
         return (x, *inputs)
 
