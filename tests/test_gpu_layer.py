@@ -303,3 +303,95 @@ def test_pending_negations(which):
         grads.append((y, *torch.autograd.grad(y, [p for p in l.parameters() if p.dtype == x.dtype], dy)))
     for a, b in zip(*grads):
         assert (a.double() - b.double()).norm() <= 8 * _ULP[x.dtype] * b.double().norm()
+
+
+def _exact(layer, x, dy):
+    """The layer's step in 64 bits, from its formula."""
+    p = {n: t.detach().double().requires_grad_(True) for n, t in layer.named_parameters()}
+    x = x.double().requires_grad_(True)
+    B, N, E = x.shape
+    H, d = layer.num_heads, layer.head_dim
+    q, k = ((x @ p[n + "_proj.weight"].t()).view(B, N, H, 2, d).permute(3, 0, 2, 1, 4) for n in "qk")
+    v = (x @ p["v_proj.weight"].t()).view(B, N, H, 2 * d).transpose(1, 2)
+    mask = torch.ones(N, N, device=x.device, dtype=torch.bool).tril() if layer.causal else torch.ones(N, N, device=x.device, dtype=torch.bool)
+    a = torch.softmax((q @ k.transpose(-1, -2) / d ** 0.5).masked_fill(~mask, float("-inf")), -1)
+    lam = (torch.exp((p["lambda_q1"] * p["lambda_k1"]).sum(-1)) - torch.exp((p["lambda_q2"] * p["lambda_k2"]).sum(-1)) + layer.lambda_init)
+    heads = a[0] @ v - lam.reshape(-1, 1, 1) * (a[1] @ v)
+    heads = heads * torch.rsqrt(heads.square().mean(-1, keepdim=True) + 1e-5) * (1 - layer.lambda_init) * p["head_gain"]
+    y = heads.transpose(1, 2).reshape(B, N, E) @ p["out_proj.weight"].t()
+    y.backward(dy.double())
+    return dict({n: t.grad for n, t in p.items()}, x=x.grad, y=y.detach())
+
+
+@pytest.mark.parametrize("E,H,N,options", [
+    (384, 3, 200, dict(causal=True, per_head_lambda=True)), (512, 2, 256, dict(dtype=torch.bfloat16)), (64, 1, 77, dict(causal=True)),
+    (5248, 41, 130, dict(per_head_lambda=True)), (5632, 44, 32, dict(causal=True, dtype=torch.bfloat16)),
+])
+def test_layer_node_is_as_exact_as_its_operations(E, H, N, options):
+    """Against 64 bits: no output or gradient is further off than that of the single operations, but for the chance of the
+    roundings (a tenth) and what is less than a quarter of a rounding of the result."""
+    layer, single, _, _ = _pair(E, H, depth=2, **options)
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x, dy = (torch.randn(2, N, E, device="cuda", generator=gen).add_(m).to(layer.head_gain.dtype) for m in (0.0, 0.25))
+    want, got, ref = _exact(layer, x, dy), _step(layer, x, dy), _step(single, x, dy)
+    off = {n: [((g[n].double() - w).norm() / w.norm()).item() for g in (got, ref)] for n, w in want.items()}
+    assert not {n: o for n, o in off.items() if o[0] > 1.1 * o[1] + _ULP[x.dtype] / 4}
+
+
+def test_layer_graph_replays_match_eager():
+    """A training step of the layer captured: no call of it allocates outside torch's allocator, synchronises or clears
+    memory with a memset, so every replay gives the eager result, with eager work and a synchronisation in between."""
+    for E, H, N in ((384, 3, 200), (5632, 44, 32)):          # with packed projections and with three products
+        layer, _, _, _ = _pair(E, H, causal=True)
+        gen = torch.Generator(device="cuda").manual_seed(1)
+        x, dy, x2 = (torch.randn(2, N, E, device="cuda", generator=gen).half() for _ in range(3))
+        want = [_step(layer, t, dy) for t in (x, x2)]
+        params = dict(layer.named_parameters())
+        leaf = x.clone().requires_grad_(True)
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            for _ in range(2):
+                torch.autograd.grad(layer(leaf), [*params.values(), leaf], dy)
+            torch.cuda.synchronize()
+            with torch.cuda.graph(graph, stream=stream):
+                y = layer(leaf)
+                grads = torch.autograd.grad(y, [*params.values(), leaf], dy)
+        for i in (0, 1, 0, 1):
+            with torch.no_grad():
+                leaf.copy_((x, x2)[i])
+            graph.replay()
+            torch.cuda.synchronize()
+            for n, g in zip((*params, "x"), grads):
+                assert torch.equal(g, want[i][n]), n
+            assert torch.equal(y, want[i]["y"])
+            _ = (x[0] @ x[0].t()).float().sum().item()
+
+
+def test_layer_on_streams_of_several_threads():
+    """Two threads that train the same layer's values on streams of their own get what one gets on the default stream."""
+    import threading
+    layer, _, x, dy = _pair(512, 4, causal=True)
+    want = _step(layer, x, dy)
+    torch.cuda.synchronize()
+    wrong = []
+
+    def worker():
+        own, stream = copy.deepcopy(layer), torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got = _step(own, x, dy)
+                with torch.no_grad():
+                    got["again"] = own(x)
+                stream.synchronize()
+                wrong.extend(n for n in want if not torch.equal(got[n], want[n]))
+                if not torch.equal(got["again"], want["y"]):
+                    wrong.append("without gradients")
+
+    threads = [threading.Thread(target=worker) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
