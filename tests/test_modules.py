@@ -165,3 +165,11 @@ def test_streams_are_the_same_views_either_way():
         (a.sin().sum() + (b * a).sum()).backward()
         grads.append(leaf.grad)
     assert torch.equal(*grads)
+
+
+def test_the_node_asks_a_stand_in_for_its_context_only_what_needs_a_gradient():
+    """Compiled autograd calls a function's backward with a stand-in for its context, which is no node of the engine's."""
+    import types
+    import _native
+    need = (True, False, True, True, True, False, False, False, False, True, False, False, False)
+    assert _native.layer().wanted(types.SimpleNamespace(needs_input_grad=need)) == sum(1 << i for i in range(10) if need[i])

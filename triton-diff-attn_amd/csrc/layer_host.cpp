@@ -191,14 +191,15 @@ PyObject* layer_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // wanted(ctx) -> bit i: the backward that is running wants a gradient of the i-th of the first ten tensors of the function
 // that ctx belongs to.  ctx.needs_input_grad is fixed by the forward; grad(loss, x), or a backward with a list of inputs, wants
-// less, and of the single operations the engine would run none behind the rest.
+// less, and of the single operations the engine would run none behind the rest.  (A stand-in for the context, as compiled
+// autograd has one, is no node that the engine could be asked about: all that needs a gradient is wanted.)
 PyObject* wanted(PyObject*, PyObject* ctx) {
   HANDLE_TH_ERRORS
-  if (!THPFunction_Check(ctx)) return PyErr_Format(PyExc_TypeError, "wanted takes the context of a function");
   unsigned bits = 0;
   THPObjectPtr need(PyObject_GetAttrString(ctx, "needs_input_grad"));
   if (!need) return nullptr;
-  const std::shared_ptr<torch::autograd::PyNode> node = ((THPFunction*)ctx)->cdata.lock();
+  std::shared_ptr<torch::autograd::PyNode> node;
+  if (THPFunction_Check(ctx)) node = ((THPFunction*)ctx)->cdata.lock();
   for (int i = 0; i < 10; ++i) {
     THPObjectPtr bit(PySequence_GetItem(need.get(), i));
     if (!bit) return nullptr;
