@@ -257,13 +257,13 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     std::vector<int> which;
     at::Tensor dqkv, dlam, gpart;
     if (want_q || want_kv || want_lam || want(5)) {
-      const at::Tensor dhg = at::mm(dy, t[4]);
+      at::Tensor dhg = at::mm(dy, t[4]);
       dqkv = at::empty({s.T, 3 * s.E}, qkv.options());
       dlam = at::empty_like(lam);
       const int64_t n_part = (int64_t)diffattn_layer_gain_parts((int)s.B, (int)s.H, (int)s.n_pad, (int)s.d), rows = s.B * s.H * s.n_pad;
       gpart = at::empty({n_part, 2 * s.d}, lam.options());
       const size_t ws_bytes = diffattn_backward_workspace_bytes((int)s.B, (int)s.H, (int)s.n_pad, (int)s.d, s.flags);
-      const at::Tensor ws = at::empty({(int64_t)ws_bytes}, qkv.options().dtype(at::kByte));
+      at::Tensor ws = at::empty({(int64_t)ws_bytes}, qkv.options().dtype(at::kByte));
       const unsigned stages = DIFFATTN_STAGE_PREP | (want_lam ? DIFFATTN_STAGE_DLAMBDA : 0u) | (want_kv ? DIFFATTN_STAGE_DKDV : 0u) |
                               (want_q ? DIFFATTN_STAGE_DQ : 0u);
       const Parts p = parts(qkv, s), d = parts(dqkv, s);
@@ -273,6 +273,8 @@ PyObject* layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     dhg.data_ptr(), d.q1, d.q2, d.k1, d.k2, d.v, dlam.data_ptr(), ws.data_ptr(), ws_bytes,
                                     (int)s.B, (int)s.H, (int)s.n_pad, (int)s.N, (int)s.d, s.sm_scale(), (float)lambda_init, s.flags, stages,
                                     &layout, t[5].data_ptr(), (float*)gpart.data_ptr(), stream));
+      dhg.reset();        // what follows on this stream may have their memory
+      ws.reset();
       if (want(0)) grad[0] = not_a_view(input_gradient(dqkv, t + 1, s, stream), {s.B, s.N, s.E});
       if (want(5)) grad[5] = at::empty({2 * s.d}, hd.options());
       if (want_lam)
