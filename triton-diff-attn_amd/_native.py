@@ -1,4 +1,4 @@
-"""ctypes binding of libdiffattn.so (C ABI in include/diffattn.h), and the loader of its extension module.
+"""ctypes binding of libdiffattn.so (C ABI in include/diffattn.h), and the loader of its extension modules.
 
 torch is imported first on purpose: the library resolves the HIP runtime by soname, so it shares
 the runtime (and therefore streams and device pointers) that torch has already loaded.

@@ -243,7 +243,8 @@ struct DkvCfg {
 // c into the statistics, so that P_t = c A_t comes out of the exponential and, with K_t = m_t P_t,
 // dS1 = K1 dP - P1 delta1/c,  dS2 = -lambda K2 dP - P2 delta2/c,  dV = (K1 - lambda K2)^T dX.  398 vector instructions
 // a 32-query step instead of 476 with c, two masks of dP and statistic 3 formed in the loop; B4 H32 N2048 D64 fp16 878 -> 869 us
-// and dQ 567 -> 555: most of what was saved the one wave of a SIMD spends on other waits.  (Masks by sign bits instead of
+// and dQ 567 -> 555: the wave issued 5 % shorter, and 3 of that came back as waits.  It issues for 67 % of its time, for 17 % a
+// unit does not take its next instruction and for 16 % it waits for LDS data or a barrier.  (Masks by sign bits instead of
 // compare and select, and the two streams' hashes in step, change nothing on top of it.)
 // PADDED: rows n_keys..N-1 are padding.  As queries they read the last real row of Q1 and Q2 (the row the
 // forward used for their logsumexp) and carry dX = 0; as keys they read the last real row of K1, K2, V and

@@ -5,7 +5,7 @@
 // What the module's own graph of single operations spent beside the operator and its eight large products, B8 H8 N1024 d64
 // causal fp16, in us of 709: four weight gradients 221 (library tiles of 64 x 64), the two q/k gradients put side by side 30,
 // the three input gradients added up 17, the gain and its gradient 47, lambda and its gradients some 45 in 18 launches.
-// Here the operator reads q, k and v where one [tokens, 3E] product left them and writes its gradients into another.
+// Here the operator reads q, k and v from one [tokens, 3E] buffer that the projections fill and writes its gradients into another.
 #include <Python.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_function.h>
