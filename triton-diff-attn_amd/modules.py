@@ -69,7 +69,7 @@ class _diff_attn_layer(torch.autograd.Function):
         inputs = (x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2)
         options = (heads, causal, lambda_init)
         need = ctx.needs_input_grad
-        projections, lambdas = any(need[1:4]), any(need[6:10])
+        projections, lambdas = need[1] or need[2] or need[3], need[6] or need[7] or need[8] or need[9]
         operator = need[0] or projections or lambdas        # its gradients are wanted
         inner = operator or need[5]                         # a gradient behind the output projection is
         y, *saved = _native.layer().layer_forward(*inputs, *options, inner, need[4], _current_stream(x.device))
@@ -78,11 +78,10 @@ class _diff_attn_layer(torch.autograd.Function):
             # An input is saved where the single operations would save it: what no wanted gradient reads may be written in
             # place before the backward, and is not held until then.  The gain beside its own gradient alone is such a one,
             # but the kernel that forms that gradient reads it: its values, without the version that autograd would check.
-            keep = (projections, *(need[0],) * 3, inner, inner, *(lambdas,) * 4)
-            if inner and not operator:
-                gain = gain.data
-            inputs = (x, wq, wk, wv, wo, gain, lq1, lk1, lq2, lk2)
-            ctx.save_for_backward(*(t if k else None for t, k in zip(inputs, keep)), *saved)
+            none = (None,) * 4
+            ctx.save_for_backward(x if projections else None, *((wq, wk, wv) if need[0] else none[:3]),
+                                  *((wo, gain if operator else gain.data) if inner else none[:2]),
+                                  *((lq1, lk1, lq2, lk2) if lambdas else none), *saved)
         return y
 
     @staticmethod
