@@ -24,6 +24,18 @@
 
 namespace DA_NS {
 
+#define DA_INLINE __attribute__((always_inline))
+
+// f(0), f(1), ... f(N-1), each with its number as a compile-time constant.  (A loop with an unroll pragma stays a loop beyond some
+// 16 000 instructions, and the arrays that its number indexes then lie in scratch memory.)
+template <int N, class F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (N > 0) {
+    each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
 constexpr int kPrepRows = 64;   // rows per workgroup of the preprocess kernel = one d(lambda) partial
 
 int bwd_num_partials(int BH, int N, int D) { (void)D; return (int)(((long long)BH * N) / kPrepRows); }
@@ -204,13 +216,17 @@ __global__ __launch_bounds__(256) void bwd_dlambda_kernel(const float* __restric
   }
 
 // ------------------------------------------------------------------------------------------------
-template <int D>
+template <int D, bool CAUSAL>
 struct DkvCfg {
   static constexpr int DV = 2 * D;
   static constexpr int NW = 4;                 // waves per workgroup, 32 keys each
   static constexpr int NT = NW * 64;
   static constexpr int BK = NW * 32;           // keys per workgroup
-  static constexpr int BQ = (D <= 64) ? 64 : 32;  // query rows per staged tile
+  // Query rows per staged tile.  The workgroup meets once per tile: with 32 rows at D = 64 twice as often, which costs 1.6 % (671 ->
+  // 682 us at B4 H32 N2048).  Causal blocks take it all the same: with 64 rows a loop may begin in three ways (an odd half turn of
+  // the ring, masked or not), and at the place where they join 110 to 300 bytes a lane went to scratch; with 32 a turn of the ring is
+  // four sub-tiles, as is the diagonal block.
+  static constexpr int BQ = (D <= 64 && !CAUSAL) ? 64 : 32;
   static constexpr int Q_TILE = BQ * D;        // halfs (swizzled, unpadded)
   static constexpr int X_TILE = BQ * DV;
   static constexpr int STAT = 4 * BQ * 2;      // 4 float arrays, counted in halfs
@@ -218,11 +234,10 @@ struct DkvCfg {
   // LDS map in bytes: the ring buffers of each kind of tile are contiguous, so that any buffer of a kind
   // is within the 64 KiB reach of an LDS instruction's immediate offset from one per-lane address
   static constexpr int QBUF = 2 * Q_TILE * 2, XBUF = X_TILE * 2, SBUF = STAT * 2;   // one ring buffer of Q1|Q2, dX, statistics
-  // A staged tile is read until half a step after its last sub-tile was scored while the tile after
-  // the next is already being fetched, which takes three buffers; there are four so that the ring
-  // position of every step is known at compile time (the loop is unrolled over one turn of the ring,
-  // and the number of steps is a multiple of four): every LDS address is then a per-lane register
-  // plus an immediate offset, with no address arithmetic inside the loop.
+  // A staged tile is read from half a step before its first sub-tile is scored until half a step after its last one was,
+  // while another is being fetched.  The ring has four so that the position of every step is known at compile time (the loop is
+  // unrolled over one turn of the ring, and the number of steps is a multiple of four): every LDS address is then a per-lane
+  // register plus an immediate offset, with no address arithmetic inside the loop.
   static constexpr int NBUF = 4;
   static constexpr int XBASE = NBUF * QBUF, SBASE = XBASE + NBUF * XBUF;
   static_assert(NBUF * QBUF <= 65536 && NBUF * XBUF <= 65536, "immediate offsets reach every buffer");
@@ -252,7 +267,7 @@ struct DkvCfg {
 // The block is number `wg` of `n_wg`; smem: DkvCfg::SMEM halfs of tile memory.
 template <int D, int MODE, bool CAUSAL, bool DROP, bool PADDED>
 __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg, lds_half* smem) {
-  using C = DkvCfg<D>;
+  using C = DkvCfg<D, CAUSAL>;
   constexpr int DV = C::DV, NW = C::NW, BK = C::BK, BQ = C::BQ;
   constexpr int NKS = D / 16, NKV = DV / 16, NDT = D / 32, NVT = DV / 32;
   constexpr bool DO_V = (MODE != 2), DO_K = (MODE != 1);
@@ -333,7 +348,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   const unsigned stat_off = (unsigned)(((size_t)(lane / (BQ / 4)) * rows + 4 * (lane % (BQ / 4))) * sizeof(float));
   constexpr int XH = (XTile::PER + 1) / 2;
 
-  auto stage = [&](int qt, int buf, int part) {
+  auto stage = [&](int qt, int buf, int part) DA_INLINE {
     lds_half* bq = smem + buf * (C::QBUF / 2);
     lds_half* bx = smem + (C::XBASE + buf * C::XBUF) / 2;
     // dX and the statistics come from the workspace, which has all N rows; Q1 and Q2 have n_keys
@@ -422,7 +437,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   // VALU instruction may write an operand right in front of one (an assembly scan in the tests checks that).
   // The dropout instantiations, whose mask arithmetic makes the compiler shuffle operands, issue ordinary
   // (compiler-visible) matrix instructions instead: the compiler then places every wait state itself.
-  auto prod_mfma = [&](int k, h8 a, Scores& out) {
+  auto prod_mfma = [&](int k, h8 a, Scores& out) DA_INLINE {
     if (!DO_K || (k & 1)) {
       const int t = DO_K ? (k >> 1) : k, ks = t >> 1;
       if (t & 1) out.s2 = DROP ? mfma32(a, kf2[ks], out.s2) : mfma32_bagpr(a, kf2[ks], out.s2);
@@ -442,19 +457,21 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
     if constexpr (DO_K) mfma_results_ready(s.s1, s.s2, s.dp);
     else mfma_results_ready(s.s1, s.s2);
   };
-  auto init_scores = [&](int buf, int qs, Scores& out) {
+  // initial accumulator values of the rows 4*r4 .. 4*r4+3
+  auto init_rows = [&](int buf, int qs, Scores& out, int r4) DA_INLINE {
+    const f4v a = stat4(buf, qs, 0, r4), bq = stat4(buf, qs, 1, r4);
 #pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const f4v a = stat4(buf, qs, 0, r4), bq = stat4(buf, qs, 1, r4);
+    for (int e = 0; e < 4; ++e) { out.s1[4 * r4 + e] = a[e]; out.s2[4 * r4 + e] = bq[e]; }
+    if constexpr (DO_K) {
+      // with dropout the mask applies to dP alone, so -delta1 cannot ride in the accumulator
+      const f4v cq = DROP ? f4v{0.f, 0.f, 0.f, 0.f} : stat4(buf, qs, 2, r4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { out.s1[4 * r4 + e] = a[e]; out.s2[4 * r4 + e] = bq[e]; }
-      if constexpr (DO_K) {
-        // with dropout the mask applies to dP alone, so -delta1 cannot ride in the accumulator
-        const f4v cq = DROP ? f4v{0.f, 0.f, 0.f, 0.f} : stat4(buf, qs, 2, r4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) out.dp[4 * r4 + e] = cq[e];
-      }
+      for (int e = 0; e < 4; ++e) out.dp[4 * r4 + e] = cq[e];
     }
+  };
+  auto init_scores = [&](int buf, int qs, Scores& out) DA_INLINE {
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) init_rows(buf, qs, out, r4);
   };
   // Element-wise work of accumulator register r (query row 8*(r/4) + 4g + (r%4)), split in three
   // stages that are issued one product apart, so that no VALU instruction waits on the one
@@ -462,7 +479,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   struct RowTmp { float p1[16], p2[16], u[16], ds1[16], ds2[16], pc[16], k1[16], k2[16]; unsigned w1, w2, w1b, w2b; };
   // `rel` (masked steps only) = key index minus the query index of register 0 of the sub-tile:
   // register r holds query 8*(r/4) + (r%4) relative to that, and a query before its key sees nothing
-  auto ew1 = [&](int r, const f4v& st3, const f4v& st2, const Scores& in, RowTmp& t, auto masked_tag, int rel, int qbase) {
+  auto ew1 = [&](int r, const f4v& st3, const f4v& st2, const Scores& in, RowTmp& t, auto masked_tag, int rel, int qbase) DA_INLINE {
     t.p1[r] = fast_exp2(in.s1[r]);
     t.p2[r] = fast_exp2(in.s2[r]);
     if constexpr (decltype(masked_tag)::value) {
@@ -497,7 +514,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
       asm volatile("" : "+v"(t.p1[r]), "+v"(t.p2[r]));
     }
   };
-  auto ew2 = [&](int r, const Scores& in, RowTmp& t) {
+  auto ew2 = [&](int r, const Scores& in, RowTmp& t) DA_INLINE {
     if constexpr (DROP) {
       if constexpr (DO_K) {
         t.ds1[r] = __builtin_fmaf(t.k1[r], in.dp[r], t.p1[r]);
@@ -517,7 +534,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
     else if constexpr (DO_K) asm volatile("" : "+v"(t.ds1[r]), "+v"(t.ds2[r]));
     else asm volatile("" : "+v"(t.pc[r]));
   };
-  auto ew3 = [&](int r, const RowTmp& t, Packed& out) {   // r odd: packs rows r-1 and r
+  auto ew3 = [&](int r, const RowTmp& t, Packed& out) DA_INLINE {   // r odd: packs rows r-1 and r
     if constexpr (DO_V) { out.pc[r / 8][r % 8 - 1] = (half_t)t.pc[r - 1]; out.pc[r / 8][r % 8] = (half_t)t.pc[r]; }
     if constexpr (DO_K) {
       out.d1[r / 8][r % 8 - 1] = (half_t)t.ds1[r - 1]; out.d1[r / 8][r % 8] = (half_t)t.ds1[r];
@@ -526,7 +543,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   };
   // slot s of the skewed schedule: stage 1 of row s, stage 2 of row s-1, stage 3 of the pair ending at row s-2
   auto ew_slot = [&](int s, const f4v (&st)[4], const f4v (&st2)[4], const Scores& in, RowTmp& t, Packed& out, auto masked_tag,
-                     int rel, int qbase) {
+                     int rel, int qbase) DA_INLINE {
     if (s < 16) ew1(s, st[s / 4], st2[s / 4], in, t, masked_tag, rel, qbase);
     if (s >= 1 && s - 1 < 16) ew2(s - 1, in, t);
     if (s >= 2 && s - 2 < 16 && ((s - 2) & 1)) ew3(s - 2, t, out);
@@ -549,7 +566,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
     const int off = buf * C::QBUF + (t2 & 1) * C::Q_TILE * 2 + row0 * D * 2;
     return join(lds_tr(qtr[t2 >> 1][0], off), lds_tr(qtr[t2 >> 1][1], off));
   };
-  auto acc_mfma = [&](int m, h8 bfrag, const Packed& in) {
+  auto acc_mfma = [&](int m, h8 bfrag, const Packed& in) DA_INLINE {
     const int kk = m / NACC1, slot = m % NACC1;
     if (slot < NSV) { dv[slot] = mfma32(in.pc[kk], bfrag, dv[slot]); return; }
     const int t2 = slot - NSV;
@@ -567,87 +584,125 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   constexpr int NBUF = C::NBUF, RING = SPT * NBUF, HALF = RING / 2;
   static_assert(HALF % 2 == 0 && 4 % HALF == 0, "half a turn is an even number of steps and divides the step count");
 
-  // One step.  Chunk k holds score product k of sub-tile (bufn, qsn), every RATIO-th chunk also
-  // accumulate product (k/RATIO + NACC/2) % NACC -- the upper query half of sub-tile (bufp, qsp)
-  // during the first half of the step, then the lower query half of sub-tile (bufc, qsc) -- and
-  // every chunk its share of the element-wise rows of sub-tile (bufc, qsc).  `pk` holds the packed operands: its lower half is written during the first half
-  // of the step and read during the second, its upper half is written during the second half and
+  // One step.  Chunk k holds score product k of sub-tile i+1, every RATIO-th chunk also
+  // accumulate product (k/RATIO + NACC/2) % NACC -- the upper query half of sub-tile i-1
+  // during the first half of the step, then the lower query half of sub-tile i -- and
+  // every chunk its share of the element-wise rows of sub-tile i.  `pk` holds the packed operands: its lower half is written
+  // during the first half of the step and read during the second, its upper half is written during the second half and
   // read during the first half of the next step.
+  // One wave per SIMD has nobody to hide the start of a step behind, so a step finds the first fragments of its products and
+  // the initial values of its accumulators in registers: the step in front of it requested them, the initial values in the rows of
+  // scores that it was done with.  For that the tile of sub-tile i+2 has to be there from the middle of step i on, where the workgroup
+  // meets; it is requested behind the meeting of the step before (a tile of two sub-tiles: of two steps before).  When a step
+  // requested all that at its own start, and the workgroup met there, behind copies requested as late as a quarter of a step before,
+  // its products began 300 cycles late and a wave of the D = 128 kernel waited for 31 % of its time: us, key blocks alone, before ->
+  // now, fp16: B2 H32 N4096 D128 3000 -> 2610, B4 H32 N2048 D64 687 -> 671, B2 H16 N8192 D32 1439 -> 1423; with the query blocks
+  // in one grid B8 H32 N4096 D128 18.2 -> 16.1 ms, B1 H8 N2048 D64 79 -> 75 us, B2 H16 N512 D32 causal 18.1 -> 17.2.
   static_assert(NPROD % 16 == 0 || 16 % NPROD == 0, "rows are spread evenly over the products");
   constexpr int AHEAD = kShort ? 1 : 3;        // B fragments requested ahead of their product (4: no faster)
-  auto fused = [&](int bufn, int qsn, Scores& s_nxt, int bufc, int qsc, const Scores& s_cur, Packed& pk,
-                   int bufp, int qsp, int tile_next, auto buf_next_tag, auto fetch_tag, auto masked_tag, int rel, int qbase) {
-    constexpr int buf_next = decltype(buf_next_tag)::value;
-    constexpr bool fetch = decltype(fetch_tag)::value;
+  // What a step finds requested by the step in front of it: the first fragments of its products and the statistics of its
+  // first rows; its score accumulators hold their initial values.
+  struct First { h8 a[DEPTH], b[AHEAD]; f4v st; };
+  constexpr bool kCarry = !kShort;             // where registers are short a step requests its own
+  First first;
+  // the accumulate products of a step in their order: the upper query half of sub-tile (bufp, qsp), then the lower one of (bufc, qsc)
+  auto step_bfrag = [&](int bufp, int qsp, int bufc, int qsc, int ja) -> h8 {
+    const int m = (ja + NACC / 2) % NACC;
+    return (ja < NACC / 2) ? acc_frag(bufp, qsp, m) : acc_frag(bufc, qsc, m);
+  };
+  auto request_first = [&](auto pos_tag) DA_INLINE {     // for the step at ring position POS
+    constexpr int POS = decltype(pos_tag)::value;
+    constexpr int SUBN = (POS + 1) % SPT, SUBC = POS % SPT, SUBP = (POS + RING - 1) % SPT;
+    constexpr int BUFN = ((POS + 1) / SPT) % NBUF, BUFC = POS / SPT, BUFP = ((POS + RING - 1) / SPT) % NBUF;
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k) first.a[k] = prod_frag(BUFN, SUBN, k);
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) first.b[k] = step_bfrag(BUFP, SUBP, BUFC, SUBC, k);
+    if constexpr (DO_K) first.st = stat4(BUFC, SUBC, 3, 0);
+  };
+  auto step = [&](int i, auto pos_tag, Scores& s_cur, Scores& s_nxt, Packed& pk, auto masked_tag) DA_INLINE {
+    constexpr int POS = decltype(pos_tag)::value;
+    // sub-tiles i-1 (p), i (c), i+1 (n) and i+2 (f)
+    constexpr int SUBF = (POS + 2) % SPT, SUBN = (POS + 1) % SPT, SUBC = POS % SPT, SUBP = (POS + RING - 1) % SPT;
+    constexpr int BUFF = ((POS + 2) / SPT) % NBUF, BUFN = ((POS + 1) / SPT) % NBUF, BUFC = POS / SPT, BUFP = ((POS + RING - 1) / SPT) % NBUF;
+    constexpr bool meets = (SUBF == 0);
+    const int rel = key - 32 * i - 4 * g, qbase = 32 * i + 4 * g;
+    // Past the end the last tile is fetched and scored again and the result is never used.
+    const int far = i / SPT + (SPT == 1 ? 3 : 2);
+    const int tile_far = far < n_qt ? far : n_qt - 1;
+    constexpr int BUF_FAR = (POS / SPT + (SPT == 1 ? 3 : 2)) % NBUF;
     constexpr int NSLOT = 18;                  // 16 rows + 2 slots of pipeline drain
     constexpr int LEAD = 2;                    // slots run before the first product
     // rows 0..7 are packed by slot 9, which must precede the first product that reads them
     static_assert(LEAD + (NSLOT - LEAD) * (NPROD / 2) / NPROD > 9, "lower half packed before it is read");
-    auto bfrag = [&](int ja) -> h8 {
-      const int m = (ja + NACC / 2) % NACC;
-      return (ja < NACC / 2) ? acc_frag(bufp, qsp, m) : acc_frag(bufc, qsc, m);
-    };
     h8 a[NPROD], bf[NACC];
     f4v st[4], st2[4];
     RowTmp tmp;
-    init_scores(bufn, qsn, s_nxt);
-#pragma unroll
-    for (int k = 0; k < DEPTH; ++k) a[k] = prod_frag(bufn, qsn, k);
-    if constexpr (DO_K) st[0] = stat4(bufc, qsc, 3, 0);
-    if constexpr (DO_K && DROP) {
-#pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) st2[r4] = stat4(bufc, qsc, 2, r4);
+    if constexpr (!kCarry) {
+      init_scores(BUFN, SUBN, s_nxt);
+      request_first(pos_tag);
     }
 #pragma unroll
-    for (int k = 0; k < AHEAD; ++k) bf[k] = bfrag(k);
-    // the first slots run while the initial accumulator values and the first fragments arrive
+    for (int k = 0; k < DEPTH; ++k) a[k] = first.a[k];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) bf[k] = first.b[k];
+    st[0] = first.st;
+    if constexpr (DO_K && DROP) {
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) st2[r4] = stat4(BUFC, SUBC, 2, r4);
+    }
 #pragma unroll
     for (int s = 0; s < LEAD; ++s) ew_slot(s, st, st2, s_cur, tmp, pk, masked_tag, rel, qbase);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 0; k < NPROD; ++k) {
-      if (k + DEPTH < NPROD) a[k + DEPTH] = prod_frag(bufn, qsn, k + DEPTH);
-      if (k % RATIO == 0 && k / RATIO + AHEAD < NACC) bf[k / RATIO + AHEAD] = bfrag(k / RATIO + AHEAD);
+    each<NPROD>([&](auto k_tag) DA_INLINE {
+      constexpr int k = decltype(k_tag)::value;
+      if constexpr (k == NPROD / 2 && meets) {
+        // The tile of sub-tile i+2 has landed for everybody, and everybody is done with sub-tile i-1.
+        wait_async_tiles();
+        __syncthreads();
+      }
+      if constexpr (k + DEPTH < NPROD) a[k + DEPTH] = prod_frag(BUFN, SUBN, k + DEPTH);
+      else if constexpr (kCarry) first.a[k + DEPTH - NPROD] = prod_frag(BUFF, SUBF, k + DEPTH - NPROD);
+      if constexpr (k % RATIO == 0) {
+        constexpr int ja = k / RATIO + AHEAD;
+        if constexpr (ja < NACC) bf[ja] = step_bfrag(BUFP, SUBP, BUFC, SUBC, ja);
+        else if constexpr (kCarry) first.b[ja - NACC] = step_bfrag(BUFC, SUBC, BUFN, SUBN, ja - NACC);
+      }
       // statistics of the next row group, requested a quarter of a step ahead of their use
-      if (DO_K && k % (NPROD / 4) == 0 && k / (NPROD / 4) < 3) st[k / (NPROD / 4) + 1] = stat4(bufc, qsc, 3, k / (NPROD / 4) + 1);
-      // the next tile's fetch is spread over the products so that the waves do not queue up at the memory pipeline
-      if (fetch && k % (NPROD / 4) == 1) stage(tile_next, buf_next, k / (NPROD / 4));
+      if constexpr (DO_K && k % (NPROD / 4) == 0) {
+        constexpr int r4 = k / (NPROD / 4) + 1;
+        if constexpr (r4 < 4) st[r4] = stat4(BUFC, SUBC, 3, r4);
+        else if constexpr (kCarry) first.st = stat4(BUFN, SUBN, 3, 0);
+      }
+      // the fetch of a tile is spread over the products so that the waves do not queue up at the memory pipeline
+      if constexpr (SPT == 1) {
+        if constexpr (k >= NPROD / 2 && (k - NPROD / 2) % (NPROD / 8) == 0) stage(tile_far, BUF_FAR, (k - NPROD / 2) / (NPROD / 8));
+      } else {
+        if constexpr (SUBC == 0 && k >= NPROD / 2 && k % (NPROD / 4) == 1) stage(tile_far, BUF_FAR, k / (NPROD / 4) - 2);
+        if constexpr (SUBC == 1 && k < NPROD / 2 && k % (NPROD / 4) == 1) stage(tile_far, BUF_FAR, k / (NPROD / 4) + 2);
+      }
+      if constexpr (k % RATIO == 0) acc_mfma((k / RATIO + NACC / 2) % NACC, bf[k / RATIO], pk);
       prod_mfma(k, a[k], s_nxt);
-      if (k % RATIO == 0) acc_mfma((k / RATIO + NACC / 2) % NACC, bf[k / RATIO], pk);
       // slots LEAD .. NSLOT-1 spread over the products
-      const int s0 = LEAD + (NSLOT - LEAD) * k / NPROD, s1 = LEAD + (NSLOT - LEAD) * (k + 1) / NPROD;
+      constexpr int s0 = LEAD + (NSLOT - LEAD) * k / NPROD, s1 = LEAD + (NSLOT - LEAD) * (k + 1) / NPROD;
 #pragma unroll
       for (int s = s0; s < s1; ++s) ew_slot(s, st, st2, s_cur, tmp, pk, masked_tag, rel, qbase);
+      // rows that are done with take the initial values of sub-tile i+2 (a row's last use is in the slot behind its own)
+      if constexpr (kCarry && k >= NPROD / 2) {
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          if (s1 > 4 * r4 + 4 && !(s0 > 4 * r4 + 4 && k > NPROD / 2)) init_rows(BUFF, SUBF, s_cur, r4);
+      }
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
     // the next step's VALU reads these results right away
     results_ready(s_nxt);
-  };
-
-  // step i at ring position POS: sub-tile i+1 is scored, sub-tile i gets its element-wise work, and the
-  // accumulate products run over the upper half of sub-tile i-1 and the lower half of sub-tile i
-  auto step = [&](int i, auto pos_tag, const Scores& s_cur, Scores& s_nxt, Packed& pk, auto masked_tag) {
-    constexpr int POS = decltype(pos_tag)::value;
-    constexpr int SUBN = (POS + 1) % SPT, SUBC = POS % SPT, SUBP = (POS + RING - 1) % SPT;
-    constexpr int BUFN = ((POS + 1) / SPT) % NBUF, BUFC = POS / SPT, BUFP = ((POS + RING - 1) / SPT) % NBUF;
-    constexpr bool opens = (SUBN == 0);
-    const int tn = (i + 1) / SPT;
-    if constexpr (opens) {
-      // sub-tile i+1 opens tile tn: its data must have landed; tile tn+1 is fetched during this step
-      wait_async_tiles();
-      __syncthreads();
-    }
-    // Past the end the last tile is fetched and scored again and the result is never used.  In front of
-    // the first sub-tile the all-zero upper operand half is accumulated against the zero-filled last buffer.
-    const int tl = (tn + 1 < n_qt) ? tn + 1 : n_qt - 1;
-    fused(BUFN, SUBN, s_nxt, BUFC, SUBC, s_cur, pk, BUFP, SUBP, tl, std::integral_constant<int, (BUFN + 1) % NBUF>{},
-          std::integral_constant<bool, opens>{}, masked_tag, key - 32 * i - 4 * g, 32 * i + 4 * g);
   };
 
   // prologue: the last buffer, which the first step reads as "the sub-tile before the first", is cleared
   // (uninitialised LDS could hold NaN patterns, and 0 * NaN would poison the sums); the first tile is
   // fetched, then the second starts; scores of the first sub-tile
-  const bool head_half = (HALF == 4) && (((n_sub - i0) / HALF) & 1);   // with HALF == 2 the steps are whole turns
+  const bool head_half = HALF == 4 && ((n_sub / HALF) & 1);
   const int b0 = head_half ? NBUF / 2 : 0;          // buffer of the first tile
   {
     const int bz = (b0 + NBUF - 1) % NBUF;          // the buffer in front of the first tile's
@@ -656,12 +711,16 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
     for (int k = tid; k < C::QBUF / 16; k += C::NT) zq[k] = u32x4{0u, 0u, 0u, 0u};
     for (int k = tid; k < C::XBUF / 16; k += C::NT) zx[k] = u32x4{0u, 0u, 0u, 0u};
   }
+  const int t1 = min(t0 + 1, n_qt - 1), t2 = min(t0 + 2, n_qt - 1);
   stage(t0, b0, 0); stage(t0, b0, 1); stage(t0, b0, 2); stage(t0, b0, 3);
+  // the first step's second product reads the second tile where a tile is one sub-tile, else the tile in front of it
+  if constexpr (SPT == 1) { stage(t1, b0 + 1, 0); stage(t1, b0 + 1, 1); stage(t1, b0 + 1, 2); stage(t1, b0 + 1, 3); }
   wait_async_tiles();
   __syncthreads();
   {
-    const int t1 = (t0 + 1 < n_qt) ? t0 + 1 : t0;
-    stage(t1, b0 + 1, 0); stage(t1, b0 + 1, 1); stage(t1, b0 + 1, 2); stage(t1, b0 + 1, 3);
+    constexpr int NEXT = SPT == 1 ? 2 : 1;
+    const int tn = SPT == 1 ? t2 : t1, bn = (b0 + NEXT) % NBUF;
+    stage(tn, bn, 0); stage(tn, bn, 1); stage(tn, bn, 2); stage(tn, bn, 3);
   }
   Scores sa, sb;
   Packed pk;
@@ -669,54 +728,56 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
     for (int e = 0; e < 8; ++e) { pk.pc[kk][e] = (half_t)0.f; pk.d1[kk][e] = (half_t)0.f; pk.d2[kk][e] = (half_t)0.f; }
-  if (head_half) {
-    init_scores(NBUF / 2, 0, sa);
+  auto begin = [&](auto pos_tag) DA_INLINE {
+    constexpr int POS = decltype(pos_tag)::value;
+    init_scores(POS / SPT, 0, sa);
 #pragma unroll
-    for (int k = 0; k < NPROD; ++k) prod_mfma(k, prod_frag(NBUF / 2, 0, k), sa);
-  } else {
-    init_scores(0, 0, sa);
-#pragma unroll
-    for (int k = 0; k < NPROD; ++k) prod_mfma(k, prod_frag(0, 0, k), sa);
-  }
+    for (int k = 0; k < NPROD; ++k) prod_mfma(k, prod_frag(POS / SPT, 0, k), sa);
+    if constexpr (kCarry) {
+      init_scores((POS + 1) / SPT, (POS + 1) % SPT, sb);
+      request_first(pos_tag);
+    }
+  };
+  if (head_half) begin(std::integral_constant<int, HALF>{});
+  else begin(std::integral_constant<int, 0>{});
   results_ready(sa);
 
   // two steps, starting at the even ring position P0 with the scores of sub-tile i in sa
-  auto two_steps = [&](int i, auto p0_tag, auto masked_tag) {
+  auto two_steps = [&](int i, auto p0_tag, auto masked_tag) DA_INLINE {
     constexpr int P0 = decltype(p0_tag)::value;
     step(i, std::integral_constant<int, P0>{}, sa, sb, pk, masked_tag);
     step(i + 1, std::integral_constant<int, P0 + 1>{}, sb, sa, pk, masked_tag);
   };
-  auto half_turn = [&](int i, auto h0_tag, auto masked_tag) {
+  auto half_turn = [&](int i, auto h0_tag, auto masked_tag) DA_INLINE {
     constexpr int H0 = decltype(h0_tag)::value;
     two_steps(i, std::integral_constant<int, H0>{}, masked_tag);
     if constexpr (HALF == 4) two_steps(i + 2, std::integral_constant<int, H0 + 2>{}, masked_tag);
   };
-  // The steps, a multiple of four, are an odd or even number of half turns; the loop below runs whole
-  // turns, so an odd half turn comes first, at the ring's second half (the prologue has put the first
-  // tile into the buffer that goes with it).  With the causal mask the key block's own four sub-tiles
-  // come first and straddle the diagonal: wave w masks sub-tiles i0 .. i0+w.
-  static_assert(!CAUSAL || BK == 128, "four diagonal sub-tiles per key block");
+  // The steps are a multiple of four.  Where a turn has eight the loop runs whole turns, and an odd half turn comes first,
+  // at the ring's second half (the prologue has put the first tile into the buffer that goes with it).  With the causal mask
+  // a turn has four: the key block's own four sub-tiles come first and straddle the diagonal, wave w masks sub-tiles i0 .. i0+w.
+  static_assert(!CAUSAL || (BK == 128 && RING == 4), "four diagonal sub-tiles per key block, one turn of the ring");
   constexpr std::integral_constant<int, 0> first_half{};
   constexpr std::integral_constant<int, HALF> second_half{};
-  constexpr std::integral_constant<bool, CAUSAL> head_masked{};
   int i = i0;
   if (head_half) {
-    half_turn(i, second_half, head_masked);
+    half_turn(i, second_half, std::false_type{});
     i += HALF;
-  } else if constexpr (CAUSAL) {
+  }
+  if constexpr (CAUSAL) {
     half_turn(i, first_half, std::true_type{});
-    half_turn(i + HALF, second_half, std::integral_constant<bool, HALF == 2>{});
+    half_turn(i + HALF, second_half, std::true_type{});
     i += RING;
   }
 #pragma nounroll
-  while (i < n_sub) {
+  for (; i < n_sub; i += RING) {
     half_turn(i, first_half, std::false_type{});
     half_turn(i + HALF, second_half, std::false_type{});
-    i += RING;
   }
   // upper query half of the last sub-tile, at the last ring position
 #pragma unroll
-  for (int m = NACC / 2; m < NACC; ++m) acc_mfma(m, acc_frag((RING - 1) / SPT, (RING - 1) % SPT, m), pk);
+  for (int m = NACC / 2; m < NACC; ++m)
+    acc_mfma(m, kCarry && m - NACC / 2 < AHEAD ? first.b[m - NACC / 2] : acc_frag((RING - 1) / SPT, (RING - 1) % SPT, m), pk);
 
   wait_async_tiles();   // the re-fetch issued by the last step has nothing left to land in after the kernel
   // accumulator tile tt: column = 32*tt + j (feature), register r = key row 8*(r/4) + 4g + (r%4)
@@ -747,8 +808,8 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
 }
 
 template <int D, int MODE, bool CAUSAL, bool DROP, bool PADDED>
-__global__ __launch_bounds__(DkvCfg<D>::NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dkdv_kernel(BwdParams p) {
-  __shared__ __attribute__((aligned(16))) half_t smem[DkvCfg<D>::SMEM];
+__global__ __launch_bounds__((DkvCfg<D, CAUSAL>::NT)) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dkdv_kernel(BwdParams p) {
+  __shared__ __attribute__((aligned(16))) half_t smem[DkvCfg<D, CAUSAL>::SMEM];
   static_assert(sizeof(smem) >= 256 * sizeof(float), "the hosted reduction uses the tile memory");
   DA_HOST_DLAMBDA(smem)
   dkdv_block<D, MODE, CAUSAL, DROP, PADDED>(p, blockIdx.x, gridDim.x - p.dlam_fold, (lds_half*)smem);
@@ -1319,8 +1380,8 @@ void bwd_dq_kernel(BwdParams p) {
 // B8 H32 N4096 D128 18.5 -> 18.3 ms.
 template <int D, bool CAUSAL, bool PADDED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_pair_kernel(BwdParams p) {
-  constexpr int SK = DkvCfg<D>::SMEM, SQ = DqCfg<D, 4, true>::SMEM;
-  static_assert(DkvCfg<D>::NT == 256, "both kinds of blocks have four waves");
+  constexpr int SK = DkvCfg<D, CAUSAL>::SMEM, SQ = DqCfg<D, 4, true>::SMEM;
+  static_assert(DkvCfg<D, false>::NT == 256, "both kinds of blocks have four waves");
   __shared__ __attribute__((aligned(16))) half_t smem[SK > SQ ? SK : SQ];
   DA_HOST_DLAMBDA(smem)
   int wg = blockIdx.x;
@@ -1381,12 +1442,12 @@ static hipError_t launch_bwd_t(const BwdParams& p_in, hipStream_t stream) {
     return hipGetLastError();
   }
   if (p.stages & 4u) {
-    const dim3 block(DkvCfg<D>::NT);
+    const dim3 block(DkvCfg<D, false>::NT);
     auto launch_mode = [&](auto mode_tag) {
       constexpr int M = decltype(mode_tag)::value;
       p.dlam_fold = fold ? n_lambda : 0;
       fold = false;
-      const dim3 grid(p.BH * (p.N / DkvCfg<D>::BK) + p.dlam_fold);
+      const dim3 grid(p.BH * (p.N / DkvCfg<D, false>::BK) + p.dlam_fold);
       auto launch_padded = [&](auto padded_tag) {
         constexpr bool PAD = decltype(padded_tag)::value;
         if (p.drop.threshold) {
