@@ -597,7 +597,7 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   // requested all that at its own start, and the workgroup met there, behind copies requested as late as a quarter of a step before,
   // its products began 300 cycles late and a wave of the D = 128 kernel waited for 31 % of its time: us, key blocks alone, before ->
   // now, fp16: B2 H32 N4096 D128 3000 -> 2610, B4 H32 N2048 D64 687 -> 671, B2 H16 N8192 D32 1439 -> 1423; with the query blocks
-  // in one grid B8 H32 N4096 D128 18.2 -> 16.1 ms, B1 H8 N2048 D64 79 -> 75 us, B2 H16 N512 D32 causal 18.1 -> 17.2.
+  // in one grid B8 H32 N4096 D128 18.1 -> 16.7 ms, B1 H8 N2048 D64 79 -> 75 us, B2 H16 N512 D32 causal 18.1 -> 17.2.
   static_assert(NPROD % 16 == 0 || 16 % NPROD == 0, "rows are spread evenly over the products");
   constexpr int AHEAD = kShort ? 1 : 3;        // B fragments requested ahead of their product (4: no faster)
   // What a step finds requested by the step in front of it: the first fragments of its products and the statistics of its

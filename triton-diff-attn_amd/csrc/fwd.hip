@@ -60,6 +60,7 @@ struct FwdCfg {
 };
 
 constexpr float kRescaleThreshold = 8.0f;   // log2 units: probabilities stay below 2^8 between updates of the row max
+constexpr float kRescaleSum = 16384.0f;     // D = 32: a lane's share of a tile's row sum, which no probability of it exceeds, between those updates
 
 // MASK: 0 none; 1 causal (key <= query); 2 the last keys of the sequence are padding (key < n_keys).
 // With the causal mask the padding needs no extra test: a padded key lies after every real query.
@@ -92,6 +93,8 @@ void fwd_kernel(FwdParams p) {
   constexpr bool TAIL = (MASK != 0);
   // the masked loop of the 128-row D = 128 workgroup has no register to spare (see the iteration)
   constexpr bool kLean = TAIL && D == 128 && !SMALL;
+  // P*V runs one tile behind the exponentials (late_iteration)
+  constexpr bool kLate = D == 32;
   int bh, qt;
   if constexpr (CAUSAL) {   // the last query block of a unit sees the most keys
     const UnitBlock ub = longest_first(blockIdx.x, p.BH);
@@ -268,11 +271,40 @@ void fwd_kernel(FwdParams p) {
   // prologue: K tiles 0..2 and V tiles 0..1; scores of tile 0
   load_k1(0, b0, with_tail); load_k2(0, b0, with_tail); load_va(0, b0, with_tail); load_vb(0, b0, with_tail);
   load_k1(clampt(1), b0 + 1, with_tail); load_k2(clampt(1), b0 + 1, with_tail);
-  load_va(clampt(1), b0 + 1, with_tail); load_vb(clampt(1), b0 + 1, with_tail);
+  if constexpr (!kLate) { load_va(clampt(1), b0 + 1, with_tail); load_vb(clampt(1), b0 + 1, with_tail); }
   if (n_tiles > 2) { load_k1(2, (b0 + 2) % 4, with_tail); load_k2(2, (b0 + 2) % 4, with_tail); }
+  if constexpr (kLate) {
+    // the V tile in front of the first one, which the first iteration multiplies with zero probabilities
+    DA_LDS u32x4* z = (DA_LDS u32x4*)(sVbuf + ((b0 + 3) % 4) * C::V_TILE);
+    for (int k = tid; k < C::V_TILE / 8; k += C::NT) z[k] = u32x4{0u, 0u, 0u, 0u};
+  }
   wait_async_tiles();
   const float lam = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, lam_load)));
   __syncthreads();
+  // Keys past the diagonal, or past the last real key, are masked: `rel` is the last visible key minus the key
+  // index of register 0, tile 0
+  auto mask_scores = [&](f16v (&s)[QS][NKT], int rel) {
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        s[0][kt][r] = (kt * 32 + 8 * (r / 4) + (r % 4) > rel) ? -INFINITY : s[0][kt][r];
+  };
+  // the largest score of this lane
+  auto lane_max = [&](const f16v (&s)[NKT]) {
+    float mx0 = fmaxf(s[0][0], s[0][1]), mx1 = fmaxf(s[0][2], s[0][3]);
+    float mx2 = fmaxf(s[0][4], s[0][5]), mx3 = fmaxf(s[0][6], s[0][7]);
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+      for (int r = (kt == 0 ? 8 : 0); r < 16; r += 8) {
+        mx0 = fmaxf(mx0, fmaxf(s[kt][r + 0], s[kt][r + 1]));
+        mx1 = fmaxf(mx1, fmaxf(s[kt][r + 2], s[kt][r + 3]));
+        mx2 = fmaxf(mx2, fmaxf(s[kt][r + 4], s[kt][r + 5]));
+        mx3 = fmaxf(mx3, fmaxf(s[kt][r + 6], s[kt][r + 7]));
+      }
+    return fmaxf(fmaxf(mx0, mx1), fmaxf(mx2, mx3));
+  };
   f16v s_a[QS][NKT], s_b[QS][NKT];
   {
     h8 ka[NKT][NKS];
@@ -280,6 +312,136 @@ void fwd_kernel(FwdParams p) {
     else read_k(0, ka);
     scores(ka, s_a);
   }
+  // P of the tile in front of the current one
+  u32x4 pw[NKK];
+  if constexpr (kLate) {
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) pw[kk] = u32x4{0u, 0u, 0u, 0u};
+    // the first tile's row maxima are the reference to begin with
+    if constexpr (TAIL) {
+      if (BN > (CAUSAL ? qt * BM + qw * 32 + 1 : p.n_keys)) mask_scores(s_a, (CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - 4 * g);
+    }
+    m[0] = pair_max(lane_max(s_a[0]));
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_a[0][kt][r] -= m[0];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) negm[0][r] = -m[0];
+    asm volatile("" : "+v"(negm[0]));
+  }
+  constexpr int NPV = NKK * NOT;
+  auto vt_frag_at = [&](int i, int voff) {
+    const int kk = i / NOT, tt = i % NOT;
+    return join(lds_read_tr_at(vtr[tt][0], voff + 16 * kk * DV * 2), lds_read_tr_at(vtr[tt][1], voff + 16 * kk * DV * 2));
+  };
+  constexpr int KA = 4, VA = 3;              // K and V^T fragments requested ahead of their products
+  h8 kfirst[KA], vfirst[VA];                 // the first ones of the next iteration
+  auto k_frag_at = [&](int i, int koff) { return lds_read_at<h8>(kb[i % NKS], koff + (i / NKS) * 32 * D * 2); };
+  auto request_first = [&](int koff, int voff) {
+#pragma unroll
+    for (int i = 0; i < KA && i < NSC; ++i) kfirst[i] = k_frag_at(i, koff);
+#pragma unroll
+    for (int i = 0; i < VA; ++i) vfirst[i] = vt_frag_at(i, voff);
+  };
+  // One iteration at D = 32, where the vector instructions of a tile take longer than its matrix instructions and the two waves of
+  // a SIMD leave each barrier in step: the exponentials of tile t, the score product of tile t+1 and the P*V product of tile t-1,
+  // none of which depends on another, interleaved in one basic block.  Row maxima are formed for the first tile only: the
+  // row sum of the rounded probabilities, which is formed anyway, says afterwards whether they left the range of the 16-bit type with
+  // room to spare, and then this tile's are formed again.  The first fragments of an iteration are requested in the one before it, or where
+  // the workgroup meets between them right behind the meeting.  K tile t+3 goes to the buffer of tile t-1, whose scores were formed two
+  // iterations ago, V tile t+1 to that of tile t-3, multiplied two iterations ago; one meeting in two iterations lies in between.
+  // fp16, us, before -> now: B4 H32 N2048 277 -> 259, B1 H16 N16384 1903 -> 1786, B2 H16 N8192 922 -> 870.  Not at D = 64, which is
+  // bound by power (1.7 GHz of 2.4: 425 us both ways at B4 H32 N2048), nor at D = 128, where it spills.
+  auto late_iteration = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
+    constexpr int POS = decltype(pos_tag)::value;
+    constexpr int KR = (POS + 1) % 4, KP = (POS + 3) % 4, VR = (POS + 3) % 4, VP = (POS + 1) % 4;
+    constexpr int VOFF = VR * C::VBUF_BYTES, KOFF = KR * C::KBUF_BYTES;
+    const int tk = clampt(t + 3), tv = clampt(t + 1);
+    constexpr bool kTail = TAIL && decltype(tail)::value;
+    load_k1(tk, KP, tail);
+    h8 ka[NSC], vfr[NPV];
+#pragma unroll
+    for (int i = 0; i < VA; ++i) vfr[i] = vfirst[i];
+#pragma unroll
+    for (int i = 0; i < KA && i < NSC; ++i) ka[i] = kfirst[i];
+    if constexpr (kTail) {
+      if ((t + 1) * BN > (CAUSAL ? qt * BM + qw * 32 + 1 : p.n_keys))
+        mask_scores(s_cur, (CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - t * BN - 4 * g);
+    }
+    u32x4 pn[NKK];
+    float rs = 0.f;
+    const unsigned hwin = DROP ? dropout_window<BN / 2>(dkey, hrow + (unsigned)(t * (BN / 2)), hlow) : 0u;
+    unsigned word_a = 0, word_b = 0;
+    auto pair_of = [&](int e) {      // registers 2 (e % 8) and the next of 32-key block e / 8
+      const int kt = e / 8, r = 2 * (e % 8);
+      h2 e2;
+      e2[0] = (half_t)fast_exp2(s_cur[0][kt][r]);
+      e2[1] = (half_t)fast_exp2(s_cur[0][kt][r + 1]);
+      rs = add_pair(e2, rs);
+      unsigned w2 = __builtin_bit_cast(unsigned, e2);
+      if constexpr (DROP) {
+        if (r % 4 == 0) dropout_bytes_shared(dropout_rounds(dkey, hwin + hstep[kt * 4 + r / 4]), dsel, word_a, word_b);
+        w2 = dropout_clear_pair((r % 4 == 0) ? word_a : word_b, p.drop.threshold, w2);
+      }
+      pn[kt * 2 + r / 8][(r % 8) / 2] = w2;
+    };
+    constexpr int NM = NPV + NSC;     // matrix products of an iteration
+    int npv = 0, nsc = 0, ne = 0;
+#pragma unroll
+    for (int c = 0; c < NM; ++c) {
+      // products alternate NPV : NSC
+      const int pv_due = (c + 1) * NPV / NM;
+      if (npv < pv_due) {
+        const int i = npv++;
+        if (i + VA < NPV) vfr[i + VA] = vt_frag_at(i + VA, VOFF);
+        o[0][i % NOT] = mfma32(vfr[i], __builtin_bit_cast(h8, pw[i / NOT]), o[0][i % NOT]);
+      } else {
+        const int i = nsc++;
+        if (i + KA < NSC) ka[i + KA] = k_frag_at(i + KA, KOFF);
+        const int kt = i / NKS, ks = i % NKS;
+        if (ks == 0) s_nxt[0][kt] = negm[0];
+        s_nxt[0][kt] = mfma32(ka[i], qf[0][ks], s_nxt[0][kt]);
+      }
+      if (c == NM / 4) load_k2(tk, KP, tail);
+      if (c == NM / 2) load_va(tv, VP, tail);
+      if (c == 3 * NM / 4) load_vb(tv, VP, tail);
+      const int e1 = (c + 1) * (8 * NKT) / NM;
+      while (ne < e1) pair_of(ne++);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!(POS & 1)) request_first(((POS + 2) % 4) * C::KBUF_BYTES, POS * C::VBUF_BYTES);
+    __builtin_amdgcn_sched_barrier(0);
+    if (__any(rs > kRescaleSum)) {
+      const float d = fmaxf(pair_max(lane_max(s_cur[0])), 0.f);
+      const float alpha = fast_exp2(-d);
+      m[0] += d;
+      l[0] *= alpha;
+#pragma unroll
+      for (int tt = 0; tt < NOT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[0][tt][r] *= alpha;
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { s_cur[0][kt][r] -= d; s_nxt[0][kt][r] -= d; }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) negm[0][r] = -m[0];
+      asm volatile("" : "+v"(negm[0]));
+      rs = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8 * NKT; ++e) pair_of(e);
+    }
+    l[0] += rs;
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) pw[kk] = pn[kk];
+    if constexpr (POS & 1) {
+      wait_async_tiles();
+      __syncthreads();
+      request_first(((POS + 2) % 4) * C::KBUF_BYTES, POS * C::VBUF_BYTES);
+    }
+  };
+  static_assert(!kLate || (C::PAIR && QS == 1), "a meeting every second tile");
 
   // One iteration: softmax of tile t (scores in s_cur) and its P*V product, overlapped with the score
   // product of tile t+1 (into s_nxt).
@@ -299,15 +461,6 @@ void fwd_kernel(FwdParams p) {
     constexpr bool kTail = TAIL && decltype(tail)::value, kLeanTail = kLean && kTail;
     load_k1(tk, KP, tail);
 
-    // Keys past the diagonal, or past the last real key, are masked: `rel` is the last visible key minus the key
-    // index of register 0, tile 0
-    auto mask_scores = [&](int rel) {
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s_cur[0][kt][r] = (kt * 32 + 8 * (r / 4) + (r % 4) > rel) ? -INFINITY : s_cur[0][kt][r];
-    };
     static_assert(!(TAIL || DROP) || QS == 1, "one 32-row block per wave");
     if constexpr (kLeanTail) {
       // Before anything else of the iteration is requested, with no branch around it, from a lane number formed
@@ -317,7 +470,7 @@ void fwd_kernel(FwdParams p) {
       load_k2(tk, KP, tail); load_va(tv, VP, tail); load_vb(tv, VP, tail);
       __builtin_amdgcn_sched_barrier(0);
       const int ln = lane_again();
-      mask_scores((CAUSAL ? qt * BM + qw * 32 + (ln & 31) : p.n_keys - 1) - t * BN - 4 * (ln >> 5));
+      mask_scores(s_cur, (CAUSAL ? qt * BM + qw * 32 + (ln & 31) : p.n_keys - 1) - t * BN - 4 * (ln >> 5));
       __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -329,7 +482,7 @@ void fwd_kernel(FwdParams p) {
     if constexpr (kTail && !kLean) {
       // only the last tiles of a wave's loop reach past its first row, or hold padding keys
       if ((t + 1) * BN > (CAUSAL ? qt * BM + qw * 32 + 1 : p.n_keys))
-        mask_scores((CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - t * BN - 4 * g);
+        mask_scores(s_cur, (CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - t * BN - 4 * g);
     }
 
     // The score product of the next tile goes to the matrix unit first and runs under the row maxima and
@@ -340,20 +493,7 @@ void fwd_kernel(FwdParams p) {
 
     float mx[QS];
 #pragma unroll
-    for (int qs = 0; qs < QS; ++qs) {
-      float mx0 = fmaxf(s_cur[qs][0][0], s_cur[qs][0][1]), mx1 = fmaxf(s_cur[qs][0][2], s_cur[qs][0][3]);
-      float mx2 = fmaxf(s_cur[qs][0][4], s_cur[qs][0][5]), mx3 = fmaxf(s_cur[qs][0][6], s_cur[qs][0][7]);
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int r = (kt == 0 ? 8 : 0); r < 16; r += 8) {
-          mx0 = fmaxf(mx0, fmaxf(s_cur[qs][kt][r + 0], s_cur[qs][kt][r + 1]));
-          mx1 = fmaxf(mx1, fmaxf(s_cur[qs][kt][r + 2], s_cur[qs][kt][r + 3]));
-          mx2 = fmaxf(mx2, fmaxf(s_cur[qs][kt][r + 4], s_cur[qs][kt][r + 5]));
-          mx3 = fmaxf(mx3, fmaxf(s_cur[qs][kt][r + 6], s_cur[qs][kt][r + 7]));
-        }
-      mx[qs] = fmaxf(fmaxf(mx0, mx1), fmaxf(mx2, mx3));
-    }
+    for (int qs = 0; qs < QS; ++qs) mx[qs] = lane_max(s_cur[qs]);
     float mxall = mx[0];
 #pragma unroll
     for (int qs = 1; qs < QS; ++qs) mxall = fmaxf(mxall, mx[qs]);
@@ -393,7 +533,6 @@ void fwd_kernel(FwdParams p) {
     // V^T fragments are requested PD products ahead of the product that uses them (measured: 2 and
     // 3 are 1.3 % faster than the single product the compiler picks by itself, 5 and 7 are not); the
     // first ones here, so that they arrive under the exponentials
-    constexpr int NPV = NKK * NOT;
     constexpr int PD = DROP ? 1 : 3;           // dropout: registers are short
     auto vt_frag = [&](int i) {
       const int kk = i / NOT, tt = i % NOT;
@@ -460,18 +599,26 @@ void fwd_kernel(FwdParams p) {
     }
   };
 
+  if constexpr (kLate) {
+    if (head_half) request_first(3 * C::KBUF_BYTES, 1 * C::VBUF_BYTES);
+    else request_first(1 * C::KBUF_BYTES, 3 * C::VBUF_BYTES);
+  }
+  auto one = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
+    if constexpr (kLate) late_iteration(t, pos_tag, tail, s_cur, s_nxt);
+    else iteration(t, pos_tag, tail, s_cur, s_nxt);
+  };
   // the tile count is even (N is a multiple of 128, tiles are at most 64 keys)
   int t = 0;
   if (head_half) {
-    iteration(0, std::integral_constant<int, 2>{}, with_tail, s_a, s_b);
-    iteration(1, std::integral_constant<int, 3>{}, with_tail, s_b, s_a);
+    one(0, std::integral_constant<int, 2>{}, with_tail, s_a, s_b);
+    one(1, std::integral_constant<int, 3>{}, with_tail, s_b, s_a);
     t = 2;
   }
   auto turn = [&](int t, auto tail) {
-    iteration(t, std::integral_constant<int, 0>{}, tail, s_a, s_b);
-    iteration(t + 1, std::integral_constant<int, 1>{}, tail, s_b, s_a);
-    iteration(t + 2, std::integral_constant<int, 2>{}, tail, s_a, s_b);
-    iteration(t + 3, std::integral_constant<int, 3>{}, tail, s_b, s_a);
+    one(t, std::integral_constant<int, 0>{}, tail, s_a, s_b);
+    one(t + 1, std::integral_constant<int, 1>{}, tail, s_b, s_a);
+    one(t + 2, std::integral_constant<int, 2>{}, tail, s_a, s_b);
+    one(t + 3, std::integral_constant<int, 3>{}, tail, s_b, s_a);
   };
   if constexpr (TAIL) {
     // A mask concerns the last tiles only: with padding, an iteration copies K tile t+3, so the first one that can
@@ -485,6 +632,13 @@ void fwd_kernel(FwdParams p) {
 #pragma nounroll
   for (; t < n_tiles; t += 4) turn(t, with_tail);
 
+  if constexpr (kLate) {
+    // the last tile's product
+    constexpr int VOFF = 3 * C::VBUF_BYTES;
+#pragma unroll
+    for (int i = 0; i < NPV; ++i)
+      o[0][i % NOT] = mfma32(i < VA ? vfirst[i] : vt_frag_at(i, VOFF), __builtin_bit_cast(h8, pw[i / NOT]), o[0][i % NOT]);
+  }
   wait_async_tiles();   // the staging blocks below reuse the tile memory the last prefetches write to
   __syncthreads();
   // ---- epilogue ----------------------------------------------------------------------------
