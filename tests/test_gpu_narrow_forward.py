@@ -1,4 +1,5 @@
-"""The forward at D = 32 (P*V one tile behind the exponentials, row sums watched instead of row maxima) at its edges: one to ten
+"""The forward with P*V one tile behind the exponentials and row sums watched instead of row maxima (D = 32, and D = 64 in small
+grids without the causal mask) at its edges: one to ten
 tiles of 64 keys with an even and an odd number of turns of its ring, sequences that end inside a tile, and scores that grow along
 the keys by 0, 3 and 20 powers of two a tile, so that the reference moves never, now and then, and at every tile, in the last case
 past the range of fp16.  The growth is the product of one feature of the queries (4) and of the keys (a whole number per tile), both
@@ -16,9 +17,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("growth", [0, 3, 20])
+@pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("H,N", [(2, 1), (2, 64), (2, 77), (3, 128), (2, 200), (2, 384), (1, 640), (160, 256), (300, 77)])
-def test_forward_of_narrow_heads(H, N, growth, causal, dtype):
-    q1, q2, k1, k2, v, dy = (t.to(dtype) for t in make_inputs(1, H, N, 32, seed=N + growth))
+def test_forward_of_narrow_heads(H, N, D, growth, causal, dtype):
+    q1, q2, k1, k2, v, dy = (t.to(dtype) for t in make_inputs(1, H, N, D, seed=N + growth))
     if growth:
         tile = (torch.arange(N) // 64).to(dtype) * growth
         for q, k in ((q1, k1), (q2, k2)):
@@ -33,7 +35,7 @@ def test_forward_of_narrow_heads(H, N, growth, causal, dtype):
     # scales and rounds the queries: a logit of L powers of two differs by up to 2 L u between the two, a probability by as much
     # times ln 2.  Where that stays below a fifth of the tolerance, dv tells whether the statistics are right.
     unit = 2.0 ** -12 if dtype == torch.float16 else 2.0 ** -9
-    logit = growth * ((N - 1) // 64) * 4 * 32 ** -0.5 * 1.4427
+    logit = growth * ((N - 1) // 64) * 4 * D ** -0.5 * 1.4427
     if 2 * logit * unit * 0.6931 > 1e-2:
         return
     assert rel_to_max(grads[4], ref[5]) <= (GRAD_RTOL if dtype == torch.float16 else 8e-2), "dv"

@@ -45,8 +45,9 @@ struct FwdCfg {
   // address is then a per-lane register plus an immediate offset, with no arithmetic inside the loop.
   static constexpr int NBUF = 4;
   // A barrier every second tile instead of every tile (the ring allows it): measured in one GPU call,
-  // 3.3 % faster at D = 32, 3 % slower at D = 64 and 5 % slower at D = 128.
-  static constexpr bool PAIR = (D == 32);
+  // 3.3 % faster at D = 32, 3 % slower at D = 64 and 5 % slower at D = 128.  In the 64-row workgroups at D = 64, whose waves have a
+  // SIMD each, it is the faster one, too (causal, B1 H4 N8192 124.4 -> 122.2 us, B1 H8 N2048 32.8 -> 31.6).
+  static constexpr bool PAIR = (D == 32 || (D == 64 && SMALL));
   static constexpr int KBUF_BYTES = K_BUF * 2, VBUF_BYTES = V_TILE * 2, VBASE_BYTES = NBUF * KBUF_BYTES;
   static_assert(NBUF * KBUF_BYTES <= 65536 && NBUF * VBUF_BYTES <= 65536, "immediate offsets reach every buffer");
   static constexpr int TILES = NBUF * (K_BUF + V_TILE);
@@ -60,7 +61,7 @@ struct FwdCfg {
 };
 
 constexpr float kRescaleThreshold = 8.0f;   // log2 units: probabilities stay below 2^8 between updates of the row max
-constexpr float kRescaleSum = 16384.0f;     // D = 32: a lane's share of a tile's row sum, which no probability of it exceeds, between those updates
+constexpr float kRescaleSum = 16384.0f;     // of late_iteration: a lane's share of a tile's row sum, which no probability of it exceeds, between those updates
 
 // MASK: 0 none; 1 causal (key <= query); 2 the last keys of the sequence are padding (key < n_keys).
 // With the causal mask the padding needs no extra test: a padded key lies after every real query.
@@ -93,8 +94,8 @@ void fwd_kernel(FwdParams p) {
   constexpr bool TAIL = (MASK != 0);
   // the masked loop of the 128-row D = 128 workgroup has no register to spare (see the iteration)
   constexpr bool kLean = TAIL && D == 128 && !SMALL;
-  // P*V runs one tile behind the exponentials (late_iteration)
-  constexpr bool kLate = D == 32;
+  // P*V runs one tile behind the exponentials (late_iteration).  (The causal 64-row workgroup at D = 64 went to scratch that way.)
+  constexpr bool kLate = D == 32 || (D == 64 && SMALL && MASK != 1);
   int bh, qt;
   if constexpr (CAUSAL) {   // the last query block of a unit sees the most keys
     const UnitBlock ub = longest_first(blockIdx.x, p.BH);
@@ -305,12 +306,30 @@ void fwd_kernel(FwdParams p) {
       }
     return fmaxf(fmaxf(mx0, mx1), fmaxf(mx2, mx3));
   };
+  constexpr int NPV = NKK * NOT;
+  auto vt_frag_at = [&](int i, int voff) {
+    const int kk = i / NOT, tt = i % NOT;
+    return join(lds_read_tr_at(vtr[tt][0], voff + 16 * kk * DV * 2), lds_read_tr_at(vtr[tt][1], voff + 16 * kk * DV * 2));
+  };
+  constexpr int KA = 4, VA = 3;              // K and V^T fragments requested ahead of their products
+  h8 kfirst[KA], vfirst[VA];                 // the first ones of the next iteration
+  auto k_frag_at = [&](int i, int koff) { return lds_read_at<h8>(kb[i % NKS], koff + (i / NKS) * 32 * D * 2); };
+  auto request_first = [&](int koff, int voff) {
+#pragma unroll
+    for (int i = 0; i < KA && i < NSC; ++i) kfirst[i] = k_frag_at(i, koff);
+#pragma unroll
+    for (int i = 0; i < VA; ++i) vfirst[i] = vt_frag_at(i, voff);
+  };
   f16v s_a[QS][NKT], s_b[QS][NKT];
   {
     h8 ka[NKT][NKS];
     if (head_half) read_k(2 * C::KBUF_BYTES, ka);
     else read_k(0, ka);
     scores(ka, s_a);
+  }
+  if constexpr (kLate) {
+    if (head_half) request_first(3 * C::KBUF_BYTES, 1 * C::VBUF_BYTES);
+    else request_first(1 * C::KBUF_BYTES, 3 * C::VBUF_BYTES);
   }
   // P of the tile in front of the current one
   u32x4 pw[NKK];
@@ -330,29 +349,18 @@ void fwd_kernel(FwdParams p) {
     for (int r = 0; r < 16; ++r) negm[0][r] = -m[0];
     asm volatile("" : "+v"(negm[0]));
   }
-  constexpr int NPV = NKK * NOT;
-  auto vt_frag_at = [&](int i, int voff) {
-    const int kk = i / NOT, tt = i % NOT;
-    return join(lds_read_tr_at(vtr[tt][0], voff + 16 * kk * DV * 2), lds_read_tr_at(vtr[tt][1], voff + 16 * kk * DV * 2));
-  };
-  constexpr int KA = 4, VA = 3;              // K and V^T fragments requested ahead of their products
-  h8 kfirst[KA], vfirst[VA];                 // the first ones of the next iteration
-  auto k_frag_at = [&](int i, int koff) { return lds_read_at<h8>(kb[i % NKS], koff + (i / NKS) * 32 * D * 2); };
-  auto request_first = [&](int koff, int voff) {
-#pragma unroll
-    for (int i = 0; i < KA && i < NSC; ++i) kfirst[i] = k_frag_at(i, koff);
-#pragma unroll
-    for (int i = 0; i < VA; ++i) vfirst[i] = vt_frag_at(i, voff);
-  };
   // One iteration at D = 32, where the vector instructions of a tile take longer than its matrix instructions and the two waves of
-  // a SIMD leave each barrier in step: the exponentials of tile t, the score product of tile t+1 and the P*V product of tile t-1,
-  // none of which depends on another, interleaved in one basic block.  Row maxima are formed for the first tile only: the
-  // row sum of the rounded probabilities, which is formed anyway, says afterwards whether they left the range of the 16-bit type with
-  // room to spare, and then this tile's are formed again.  The first fragments of an iteration are requested in the one before it, or where
-  // the workgroup meets between them right behind the meeting.  K tile t+3 goes to the buffer of tile t-1, whose scores were formed two
-  // iterations ago, V tile t+1 to that of tile t-3, multiplied two iterations ago; one meeting in two iterations lies in between.
-  // fp16, us, before -> now: B4 H32 N2048 277 -> 259, B1 H16 N16384 1903 -> 1786, B2 H16 N8192 922 -> 870.  Not at D = 64, which is
-  // bound by power (1.7 GHz of 2.4: 425 us both ways at B4 H32 N2048), nor at D = 128, where it spills.
+  // a SIMD leave each barrier in step, and of the 64-row workgroups at D = 64, which have one wave to a SIMD: the exponentials of tile t,
+  // the score product of tile t+1 and the P*V product of tile t-1, none of which depends on another, interleaved in one basic block.
+  // Row maxima are formed for the first tile only: the row sum of the rounded probabilities, which is formed anyway, says afterwards
+  // whether they left the range of the 16-bit type with room to spare, and then this tile's are formed again.  The first fragments of an
+  // iteration are requested in the one before it, or where the workgroup meets between them right behind the meeting.  K tile t+3 goes
+  // to the buffer of tile t-1, whose scores were formed two iterations ago, V tile t+1 to that of tile t-3, multiplied two
+  // iterations ago; the one meeting in two iterations lies in between.
+  // fp16, us, before -> now: D32 B4 H32 N2048 277 -> 259, B1 H16 N16384 1903 -> 1786, B1 H2 N4096 37.0 -> 31.5, B1 H8 N2048 22.5 -> 20.2;
+  // D64 in 64-row workgroups B1 H8 N2048 37.3 -> 35.3, N2000 38.8 -> 36.3, B1 H4 N1000 19.3 -> 18.0, B1 H16 N512 11.9 -> 11.4.  Not for
+  // the 128-row workgroups at D = 64, which are bound by power (1.7 GHz of 2.4: 425 us both ways at B4 H32 N2048), nor at D = 128,
+  // where it spills.
   auto late_iteration = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
     constexpr int POS = decltype(pos_tag)::value;
     constexpr int KR = (POS + 1) % 4, KP = (POS + 3) % 4, VR = (POS + 3) % 4, VP = (POS + 1) % 4;
@@ -599,10 +607,6 @@ void fwd_kernel(FwdParams p) {
     }
   };
 
-  if constexpr (kLate) {
-    if (head_half) request_first(3 * C::KBUF_BYTES, 1 * C::VBUF_BYTES);
-    else request_first(1 * C::KBUF_BYTES, 3 * C::VBUF_BYTES);
-  }
   auto one = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
     if constexpr (kLate) late_iteration(t, pos_tag, tail, s_cur, s_nxt);
     else iteration(t, pos_tag, tail, s_cur, s_nxt);
