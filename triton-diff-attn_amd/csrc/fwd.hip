@@ -272,12 +272,14 @@ void fwd_kernel(FwdParams p) {
   // prologue: K tiles 0..2 and V tiles 0..1; scores of tile 0
   load_k1(0, b0, with_tail); load_k2(0, b0, with_tail); load_va(0, b0, with_tail); load_vb(0, b0, with_tail);
   load_k1(clampt(1), b0 + 1, with_tail); load_k2(clampt(1), b0 + 1, with_tail);
-  if constexpr (!kLate) { load_va(clampt(1), b0 + 1, with_tail); load_vb(clampt(1), b0 + 1, with_tail); }
+  if (!kLate || head_half) { load_va(clampt(1), b0 + 1, with_tail); load_vb(clampt(1), b0 + 1, with_tail); }
   if (n_tiles > 2) { load_k1(2, (b0 + 2) % 4, with_tail); load_k2(2, (b0 + 2) % 4, with_tail); }
   if constexpr (kLate) {
-    // the V tile in front of the first one, which the first iteration multiplies with zero probabilities
-    DA_LDS u32x4* z = (DA_LDS u32x4*)(sVbuf + ((b0 + 3) % 4) * C::V_TILE);
-    for (int k = tid; k < C::V_TILE / 8; k += C::NT) z[k] = u32x4{0u, 0u, 0u, 0u};
+    // the V tile in front of the first one, which the loop's first iteration multiplies with zero probabilities
+    if (!head_half) {
+      DA_LDS u32x4* z = (DA_LDS u32x4*)(sVbuf + 3 * C::V_TILE);
+      for (int k = tid; k < C::V_TILE / 8; k += C::NT) z[k] = u32x4{0u, 0u, 0u, 0u};
+    }
   }
   wait_async_tiles();
   const float lam = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, lam_load)));
@@ -314,9 +316,12 @@ void fwd_kernel(FwdParams p) {
   constexpr int KA = 4, VA = 3;              // K and V^T fragments requested ahead of their products
   h8 kfirst[KA], vfirst[VA];                 // the first ones of the next iteration
   auto k_frag_at = [&](int i, int koff) { return lds_read_at<h8>(kb[i % NKS], koff + (i / NKS) * 32 * D * 2); };
-  auto request_first = [&](int koff, int voff) {
+  auto request_first_k = [&](int koff) {
 #pragma unroll
     for (int i = 0; i < KA && i < NSC; ++i) kfirst[i] = k_frag_at(i, koff);
+  };
+  auto request_first = [&](int koff, int voff) {
+    request_first_k(koff);
 #pragma unroll
     for (int i = 0; i < VA; ++i) vfirst[i] = vt_frag_at(i, voff);
   };
@@ -328,7 +333,7 @@ void fwd_kernel(FwdParams p) {
     scores(ka, s_a);
   }
   if constexpr (kLate) {
-    if (head_half) request_first(3 * C::KBUF_BYTES, 1 * C::VBUF_BYTES);
+    if (head_half) request_first_k(3 * C::KBUF_BYTES);
     else request_first(1 * C::KBUF_BYTES, 3 * C::VBUF_BYTES);
   }
   // P of the tile in front of the current one
@@ -361,19 +366,27 @@ void fwd_kernel(FwdParams p) {
   // D64 in 64-row workgroups B1 H8 N2048 37.3 -> 35.3, N2000 38.8 -> 36.3, B1 H4 N1000 19.3 -> 18.0, B1 H16 N512 11.9 -> 11.4.  Not for
   // the 128-row workgroups at D = 64, which are bound by power (1.7 GHz of 2.4: 425 us both ways at B4 H32 N2048), nor at D = 128,
   // where it spills.
-  auto late_iteration = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
+  // `opening`: the first iteration where half a turn comes first, which is compiled by itself: there is no product to make up for, V
+  // tile 1 was requested with the first tiles, and the scores are masked.  With them it cost sequences of up to 128 keys, which
+  // have no other iterations to win it back in, 2 to 7 % against
+  // the loop this one replaced (`iteration`); us, fp16, that loop -> with them -> now: D32 H16 N77 causal 6.25 -> 6.67 -> 6.07, N128 causal
+  // 5.87 -> 6.22 -> 5.77, D64 H16 N77 8.07 -> 8.27 -> 7.77, N128 6.51 -> 6.60 -> 6.39 (with dropout 7.10 -> 7.29 -> 7.20).
+  auto late_iteration = [&](int t, auto pos_tag, auto tail, auto opening, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
     constexpr int POS = decltype(pos_tag)::value;
+    constexpr bool kOpening = decltype(opening)::value;
     constexpr int KR = (POS + 1) % 4, KP = (POS + 3) % 4, VR = (POS + 3) % 4, VP = (POS + 1) % 4;
     constexpr int VOFF = VR * C::VBUF_BYTES, KOFF = KR * C::KBUF_BYTES;
     const int tk = clampt(t + 3), tv = clampt(t + 1);
     constexpr bool kTail = TAIL && decltype(tail)::value;
     load_k1(tk, KP, tail);
     h8 ka[NSC], vfr[NPV];
+    if constexpr (!kOpening) {
 #pragma unroll
-    for (int i = 0; i < VA; ++i) vfr[i] = vfirst[i];
+      for (int i = 0; i < VA; ++i) vfr[i] = vfirst[i];
+    }
 #pragma unroll
     for (int i = 0; i < KA && i < NSC; ++i) ka[i] = kfirst[i];
-    if constexpr (kTail) {
+    if constexpr (kTail && !kOpening) {
       if ((t + 1) * BN > (CAUSAL ? qt * BM + qw * 32 + 1 : p.n_keys))
         mask_scores(s_cur, (CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - t * BN - 4 * g);
     }
@@ -394,12 +407,12 @@ void fwd_kernel(FwdParams p) {
       }
       pn[kt * 2 + r / 8][(r % 8) / 2] = w2;
     };
-    constexpr int NM = NPV + NSC;     // matrix products of an iteration
+    constexpr int NV = kOpening ? 0 : NPV, NM = NV + NSC;     // matrix products of an iteration
     int npv = 0, nsc = 0, ne = 0;
 #pragma unroll
     for (int c = 0; c < NM; ++c) {
-      // products alternate NPV : NSC
-      const int pv_due = (c + 1) * NPV / NM;
+      // products alternate NV : NSC
+      const int pv_due = (c + 1) * NV / NM;
       if (npv < pv_due) {
         const int i = npv++;
         if (i + VA < NPV) vfr[i + VA] = vt_frag_at(i + VA, VOFF);
@@ -412,8 +425,8 @@ void fwd_kernel(FwdParams p) {
         s_nxt[0][kt] = mfma32(ka[i], qf[0][ks], s_nxt[0][kt]);
       }
       if (c == NM / 4) load_k2(tk, KP, tail);
-      if (c == NM / 2) load_va(tv, VP, tail);
-      if (c == 3 * NM / 4) load_vb(tv, VP, tail);
+      if (!kOpening && c == NM / 2) load_va(tv, VP, tail);
+      if (!kOpening && c == 3 * NM / 4) load_vb(tv, VP, tail);
       const int e1 = (c + 1) * (8 * NKT) / NM;
       while (ne < e1) pair_of(ne++);
       __builtin_amdgcn_sched_barrier(0);
@@ -607,22 +620,24 @@ void fwd_kernel(FwdParams p) {
     }
   };
 
-  auto one = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
-    if constexpr (kLate) late_iteration(t, pos_tag, tail, s_cur, s_nxt);
+  auto one = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT], auto opening) {
+    if constexpr (kLate) late_iteration(t, pos_tag, tail, opening, s_cur, s_nxt);
     else iteration(t, pos_tag, tail, s_cur, s_nxt);
   };
+  constexpr std::true_type opens{};
+  constexpr std::false_type follows{};
   // the tile count is even (N is a multiple of 128, tiles are at most 64 keys)
   int t = 0;
   if (head_half) {
-    one(0, std::integral_constant<int, 2>{}, with_tail, s_a, s_b);
-    one(1, std::integral_constant<int, 3>{}, with_tail, s_b, s_a);
+    one(0, std::integral_constant<int, 2>{}, with_tail, s_a, s_b, opens);
+    one(1, std::integral_constant<int, 3>{}, with_tail, s_b, s_a, follows);
     t = 2;
   }
   auto turn = [&](int t, auto tail) {
-    one(t, std::integral_constant<int, 0>{}, tail, s_a, s_b);
-    one(t + 1, std::integral_constant<int, 1>{}, tail, s_b, s_a);
-    one(t + 2, std::integral_constant<int, 2>{}, tail, s_a, s_b);
-    one(t + 3, std::integral_constant<int, 3>{}, tail, s_b, s_a);
+    one(t, std::integral_constant<int, 0>{}, tail, s_a, s_b, follows);
+    one(t + 1, std::integral_constant<int, 1>{}, tail, s_b, s_a, follows);
+    one(t + 2, std::integral_constant<int, 2>{}, tail, s_a, s_b, follows);
+    one(t + 3, std::integral_constant<int, 3>{}, tail, s_b, s_a, follows);
   };
   if constexpr (TAIL) {
     // A mask concerns the last tiles only: with padding, an iteration copies K tile t+3, so the first one that can
