@@ -351,14 +351,17 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   auto stage = [&](int qt, int buf, int part) DA_INLINE {
     lds_half* bq = smem + buf * (C::QBUF / 2);
     lds_half* bx = smem + (C::XBASE + buf * C::XBUF) / 2;
-    // dX and the statistics come from the workspace, which has all N rows; Q1 and Q2 have n_keys
-    const bool past_end = PADDED && (qt + 1) * BQ > p.n_keys;
+    // dX and the statistics come from the workspace, which has all N rows; Q1 and Q2 have n_keys.  With padding every copy of
+    // theirs is clamped: a branch per copy cut the products of a step apart, and with the twice as many copies of 32-row tiles
+    // causal blocks had become slower by it than they were with 64-row ones.  us of a whole backward, fp16, with 64-row tiles and
+    // branches -> 32-row tiles and branches -> now: D32 H8 N130 causal 15.9 -> 16.7 -> 15.6, H4 N3000 76.5 -> 75.7 -> 72.7; D64 H4 N3000
+    // causal 107.8 -> 111.0 -> 105.3; 64-row tiles as before: D32 H4 N3000 75.9 -> 72.2 -> 70.1, D64 107.8 -> 104.2 -> 101.0, H16 N77 18.7 -> 19.1 -> 18.1.
     if (part == 0) {
-      if (past_end) QTile::issue_clamped(gq1 + (size_t)qt * BQ * qk_n, bq, wave, lane, q_off, qk_n, p.n_keys - 1 - qt * BQ);
+      if constexpr (PADDED) QTile::issue_clamped(gq1 + (size_t)qt * BQ * qk_n, bq, wave, lane, q_off, qk_n, p.n_keys - 1 - qt * BQ);
       else QTile::issue_at(gq1 + (size_t)qt * BQ * qk_n, bq, wave, lane, q_off, qk_n);
       if (wave == 0 && lane < BQ) async_copy16(reinterpret_cast<const half_t*>(gstat + (size_t)qt * BQ), stat_off, smem + (C::SBASE + buf * C::SBUF) / 2);
     } else if (part == 1) {
-      if (past_end) QTile::issue_clamped(gq2 + (size_t)qt * BQ * qk_n, bq + C::Q_TILE, wave, lane, q_off, qk_n, p.n_keys - 1 - qt * BQ);
+      if constexpr (PADDED) QTile::issue_clamped(gq2 + (size_t)qt * BQ * qk_n, bq + C::Q_TILE, wave, lane, q_off, qk_n, p.n_keys - 1 - qt * BQ);
       else QTile::issue_at(gq2 + (size_t)qt * BQ * qk_n, bq + C::Q_TILE, wave, lane, q_off, qk_n);
     } else if (part == 2) {
       XTile::template issue<0, XH>(gx + (size_t)qt * BQ * DV, bx, wave, lane);

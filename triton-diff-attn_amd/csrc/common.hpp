@@ -11,6 +11,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "tile_rows.hpp"
 
 // The sources are compiled twice into one library: as they stand for fp16 tensors (namespace da),
 // and with -DDA_BF16 for bf16 tensors (namespace da_bf16).  "half" in comments means the 16-bit
@@ -272,22 +273,21 @@ struct AsyncTile {
   }
   // The same copy for a tile whose global rows end at `last_row` (relative to the tile's first row; it may be
   // negative when the whole tile lies past the end): a row beyond it reads row `last_row` instead, so no
-  // address past the tensor's last row is formed and the LDS tile holds finite data everywhere.  Used for the
-  // last tiles of a sequence whose length is not a multiple of the tile; costs a few VALU instructions per piece.
+  // address past the tensor's last row is formed and the LDS tile holds finite data everywhere.  For the last tiles of a sequence
+  // whose length is not a multiple of the tile; a tile in front of them is copied as it is.  Costs a minimum and an addition per piece.
   template <int K0 = 0, int K1 = PER>
   __device__ static __forceinline__ void issue_clamped(const half_t* gtile, lds_half* lds_tile, int wave, int lane, unsigned off0,
                                                        int stride, int last_row) {
-    const int r_l = lane / CPR;                        // the lane's row inside a piece
+    const int row_bytes = stride * 2;
+    const unsigned down = (unsigned)((lane / CPR) * row_bytes);        // the lane's row inside a piece, in bytes
 #pragma unroll
     for (int k = K0; k < K1; ++k) {
       const int inst = wave + NW * k;
       if (NINST % NW == 0 || inst < NINST) {
-        const int first = inst * RPP;                                  // first row of the piece
-        const int base_row = first < last_row ? first : last_row;     // wave-uniform
-        const int room = last_row - base_row;                          // rows the piece may advance: >= 0
-        const int back = r_l > room ? r_l - room : 0;                  // rows this lane steps back
-        const unsigned off = (kOneOffset ? off0 : lane_off(inst, lane, stride)) - (unsigned)(back * stride * 2);
-        async_copy16(gtile + (long long)base_row * stride, off, lds_tile + inst * 512);
+        const da_abi::PieceRows at = da_abi::clamp_piece(inst * RPP, last_row, RPP);
+        const unsigned most = (unsigned)(at.most * row_bytes);
+        const unsigned off = ((kOneOffset ? off0 : lane_off(inst, lane, stride)) - down) + (down < most ? down : most);
+        async_copy16(gtile + (long long)at.base * stride, off, lds_tile + inst * 512);
       }
     }
   }
