@@ -24,18 +24,6 @@
 
 namespace DA_NS {
 
-#define DA_INLINE __attribute__((always_inline))
-
-// f(0), f(1), ... f(N-1), each with its number as a compile-time constant.  (A loop with an unroll pragma stays a loop beyond some
-// 16 000 instructions, and the arrays that its number indexes then lie in scratch memory.)
-template <int N, class F>
-__device__ __forceinline__ void each(F&& f) {
-  if constexpr (N > 0) {
-    each<N - 1>(f);
-    f(std::integral_constant<int, N - 1>{});
-  }
-}
-
 constexpr int kPrepRows = 64;   // rows per workgroup of the preprocess kernel = one d(lambda) partial
 
 int bwd_num_partials(int BH, int N, int D) { (void)D; return (int)(((long long)BH * N) / kPrepRows); }

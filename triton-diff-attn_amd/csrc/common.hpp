@@ -11,6 +11,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include "tile_rows.hpp"
 
 // The sources are compiled twice into one library: as they stand for fp16 tensors (namespace da),
@@ -34,6 +35,18 @@ struct DropoutCfg {
 }  // namespace da_abi
 
 namespace DA_NS {
+
+#define DA_INLINE __attribute__((always_inline))
+
+// f(0), f(1), ... f(N-1), each with its number as a compile-time constant.  (A loop with an unroll pragma stays a loop beyond some
+// 16 000 instructions, and the arrays that its number indexes then lie in scratch memory.)
+template <int N, class F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (N > 0) {
+    each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
 
 #ifdef DA_BF16
 typedef __bf16 half_t;

@@ -19,6 +19,7 @@
 
 namespace DA_NS {
 
+
 // SMALL: 64 query rows per workgroup (four waves), for problems whose 128-row blocks leave much of the chip idle and
 // for the D = 128 instantiations with dropout, which do not fit the register budget of two waves per SIMD.
 template <int D, bool SMALL = false>
@@ -62,6 +63,8 @@ struct FwdCfg {
 
 constexpr float kRescaleThreshold = 8.0f;   // log2 units: probabilities stay below 2^8 between updates of the row max
 constexpr float kRescaleSum = 16384.0f;     // of late_iteration: a lane's share of a tile's row sum, which no probability of it exceeds, between those updates
+constexpr float kRescaleWatch = 14.0f;      // log2 units, of a watching late_iteration: no probability there exceeds 2^14
+constexpr int kWatchMoves = 3;              // moves in a turn of four tiles that make a wave watch
 
 // MASK: 0 none; 1 causal (key <= query); 2 the last keys of the sequence are padding (key < n_keys).
 // With the causal mask the padding needs no extra test: a padded key lies after every real query.
@@ -96,6 +99,7 @@ void fwd_kernel(FwdParams p) {
   constexpr bool kLean = TAIL && D == 128 && !SMALL;
   // P*V runs one tile behind the exponentials (late_iteration).  (The causal 64-row workgroup at D = 64 went to scratch that way.)
   constexpr bool kLate = D == 32 || (D == 64 && SMALL && MASK != 1);
+  constexpr bool kWatch = D == 32;      // with watching iterations
   int bh, qt;
   if constexpr (CAUSAL) {   // the last query block of a unit sees the most keys
     const UnitBlock ub = longest_first(blockIdx.x, p.BH);
@@ -178,25 +182,25 @@ void fwd_kernel(FwdParams p) {
   // clamped: the four branches of an iteration cut its interleaved products apart and cost more than the eight instructions.  us,
   // fp16, with them -> without: D32 H8 N1000 12.6 -> 12.1, causal 13.0 -> 12.4, H16 N77 5.45 -> 5.11, causal N512 9.4 -> 9.0; D64 H16 N77 7.6 ->
   // 7.1, H8 N1000 18.4 -> 17.9; with dropout 8.6 -> 8.1.
-  auto load_k1 = [&](int tk, int buf, auto tail) {
+  auto load_k1 = [&](int tk, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tk + 1) * BN > p.n_keys))
       KTile::issue_clamped(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, tail_lane(), k_off, qk_n, p.n_keys - 1 - tk * BN);
     else
       KTile::issue_at(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, lane, k_off, qk_n);
   };
-  auto load_k2 = [&](int tk, int buf, auto tail) {
+  auto load_k2 = [&](int tk, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tk + 1) * BN > p.n_keys))
       KTile::issue_clamped(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, tail_lane(), k_off, qk_n, p.n_keys - 1 - tk * BN);
     else
       KTile::issue_at(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, lane, k_off, qk_n);
   };
-  auto load_va = [&](int tv, int buf, auto tail) {
+  auto load_va = [&](int tv, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tv + 1) * BN > p.n_keys))
       VTile::template issue_clamped<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
     else
       VTile::template issue_at<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n);
   };
-  auto load_vb = [&](int tv, int buf, auto tail) {
+  auto load_vb = [&](int tv, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tv + 1) * BN > p.n_keys))
       VTile::template issue_clamped<VH, VTile::PER>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
     else
@@ -235,7 +239,7 @@ void fwd_kernel(FwdParams p) {
   };
   // Score products number I0 .. I1-1 of a tile, counted in issue order: 32-key tile kt, k-step ks is number
   // kt * NKS + ks.  The first product of a 32-key tile starts from the running reference.
-  auto scores_of = [&](const h8 (&ka)[NKT][NKS], f16v (&s)[QS][NKT], auto i0, auto i1) {
+  auto scores_of = [&](const h8 (&ka)[NKT][NKS], f16v (&s)[QS][NKT], auto i0, auto i1) DA_INLINE {
 #pragma unroll
     for (int i = decltype(i0)::value; i < decltype(i1)::value; ++i) {
       const int kt = i / NKS, ks = i % NKS;
@@ -289,7 +293,7 @@ void fwd_kernel(FwdParams p) {
   __syncthreads();
   // Keys past the diagonal, or past the last real key, are masked: `rel` is the last visible key minus the key
   // index of register 0, tile 0
-  auto mask_scores = [&](f16v (&s)[QS][NKT], int rel) {
+  auto mask_scores = [&](f16v (&s)[QS][NKT], int rel) DA_INLINE {
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
@@ -297,7 +301,7 @@ void fwd_kernel(FwdParams p) {
         s[0][kt][r] = (kt * 32 + 8 * (r / 4) + (r % 4) > rel) ? -INFINITY : s[0][kt][r];
   };
   // the largest score of this lane
-  auto lane_max = [&](const f16v (&s)[NKT]) {
+  auto lane_max = [&](const f16v (&s)[NKT]) DA_INLINE {
     float mx0 = fmaxf(s[0][0], s[0][1]), mx1 = fmaxf(s[0][2], s[0][3]);
     float mx2 = fmaxf(s[0][4], s[0][5]), mx3 = fmaxf(s[0][6], s[0][7]);
 #pragma unroll
@@ -312,22 +316,23 @@ void fwd_kernel(FwdParams p) {
     return fmaxf(fmaxf(mx0, mx1), fmaxf(mx2, mx3));
   };
   constexpr int NPV = NKK * NOT;
-  auto vt_frag_at = [&](int i, int voff) {
+  auto vt_frag_at = [&](int i, int voff) DA_INLINE {
     const int kk = i / NOT, tt = i % NOT;
     return join(lds_read_tr_at(vtr[tt][0], voff + 16 * kk * DV * 2), lds_read_tr_at(vtr[tt][1], voff + 16 * kk * DV * 2));
   };
   constexpr int KA = 4, VA = 3;              // K and V^T fragments requested ahead of their products
   h8 kfirst[KA], vfirst[VA];                 // the first ones of the next iteration
-  auto k_frag_at = [&](int i, int koff) { return lds_read_at<h8>(kb[i % NKS], koff + (i / NKS) * 32 * D * 2); };
-  auto request_first_k = [&](int koff) {
+  auto k_frag_at = [&](int i, int koff) DA_INLINE { return lds_read_at<h8>(kb[i % NKS], koff + (i / NKS) * 32 * D * 2); };
+  auto request_first_k = [&](int koff) DA_INLINE {
 #pragma unroll
     for (int i = 0; i < KA && i < NSC; ++i) kfirst[i] = k_frag_at(i, koff);
   };
-  auto request_first = [&](int koff, int voff) {
+  auto request_first = [&](int koff, int voff) DA_INLINE {
     request_first_k(koff);
 #pragma unroll
     for (int i = 0; i < VA; ++i) vfirst[i] = vt_frag_at(i, voff);
   };
+  int moves = 0;           // kWatch: how often the reference moved in this turn of the ring
   f16v s_a[QS][NKT], s_b[QS][NKT];
   {
     h8 ka[NKT][NKS];
@@ -357,6 +362,7 @@ void fwd_kernel(FwdParams p) {
     for (int r = 0; r < 16; ++r) negm[0][r] = -m[0];
     asm volatile("" : "+v"(negm[0]));
   }
+  enum Kind { kFollows, kOpens, kWatches };
   // One iteration at D = 32, where the vector instructions of a tile take longer than its matrix instructions and the two waves of
   // a SIMD leave each barrier in step, and of the 64-row workgroups at D = 64, which have one wave to a SIMD: the exponentials of tile t,
   // the score product of tile t+1 and the P*V product of tile t-1, none of which depends on another, interleaved in one basic block.
@@ -369,14 +375,27 @@ void fwd_kernel(FwdParams p) {
   // D64 in 64-row workgroups B1 H8 N2048 37.3 -> 35.3, N2000 38.8 -> 36.3, B1 H4 N1000 19.3 -> 18.0, B1 H16 N512 11.9 -> 11.4.  Not for
   // the 128-row workgroups at D = 64, which are bound by power (1.7 GHz of 2.4: 425 us both ways at B4 H32 N2048), nor at D = 128,
   // where it spills.
-  // `opening`: the first iteration where half a turn comes first, which is compiled by itself: there is no product to make up for, V
+  // `kind`: what the iteration leaves out or looks for.
+  // kWatches (D = 32): scores that move the reference at one tile may do so at most of them, and to form a tile's probabilities a second
+  // time takes half as long as a tile.  Behind a turn of the ring with three such moves a wave goes on with iterations that look at
+  // the row maxima ahead of the exponentials, where a move costs no second ones.  (A look in every iteration, behind a branch, cost
+  // small grids whose reference never moves 1 to 4 %; a way back to the first kind of iteration went to scratch; at two moves a turn
+  // scores with a deviation of 4 to 6 lose 5 %, at four the gain is half.)  us, fp16, scores of a standard deviation of 1, 6, 9, 16 and
+  // 36, row maxima at every tile (`iteration`) | never, probabilities a second time | now:
+  //   B4 H16 N2048  126 133 136 142 147 | 122 130 143 165 186 | 120 131 146 153 151;  causal 78 82 86 89 91 | 76 82 90 103 112 | 75 83 91 96 95
+  //   B1 H8 N2048  23.4 24.4 25.2 26.1 26.5 | 20.3 23.0 25.4 28.5 30.2 | 20.2 23.4 25.8 27.0 26.7;  N8192 230 228 226 235 245 | 216 221 227 249 279 |
+  //   216 223 241 255 251;  scores that grow by 14 powers of two a tile, B4 H16 N2048 157 | 203 | 164
+  // Not at D = 64, where the second loop costs launches whose reference never moves more (H16 N256 8.25 -> 8.42, N512 11.05 -> 11.23) than
+  // such scores are worth: B1 H8 N2048, deviation of 9 and 16, 35.1 35.9 | 35.4 39.5, with it 35.2 36.5; sequences of up to four tiles
+  // have no second turn (N256, deviation of 16, 9.1 | 9.7).
+  // kOpens: the first iteration where half a turn comes first, which is compiled by itself: there is no product to make up for, V
   // tile 1 was requested with the first tiles, and the scores are masked.  With them it cost sequences of up to 128 keys, which
   // have no other iterations to win it back in, 2 to 7 % against
   // the loop this one replaced (`iteration`); us, fp16, that loop -> with them -> now: D32 H16 N77 causal 6.25 -> 6.67 -> 6.07, N128 causal
   // 5.87 -> 6.22 -> 5.77, D64 H16 N77 8.07 -> 8.27 -> 7.77, N128 6.51 -> 6.60 -> 6.39 (with dropout 7.10 -> 7.29 -> 7.20).
-  auto late_iteration = [&](int t, auto pos_tag, auto tail, auto opening, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
+  auto late_iteration = [&](int t, auto pos_tag, auto tail, auto kind, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) DA_INLINE {
     constexpr int POS = decltype(pos_tag)::value;
-    constexpr bool kOpening = decltype(opening)::value;
+    constexpr bool kOpening = decltype(kind)::value == kOpens, kWatching = decltype(kind)::value == kWatches;
     constexpr int KR = (POS + 1) % 4, KP = (POS + 3) % 4, VR = (POS + 3) % 4, VP = (POS + 1) % 4;
     constexpr int VOFF = VR * C::VBUF_BYTES, KOFF = KR * C::KBUF_BYTES;
     const int tk = clampt(t + 3), tv = clampt(t + 1);
@@ -393,11 +412,39 @@ void fwd_kernel(FwdParams p) {
       if ((t + 1) * BN > (CAUSAL ? qt * BM + qw * 32 + 1 : p.n_keys))
         mask_scores(s_cur, (CAUSAL ? qt * BM + qw * 32 + j : p.n_keys - 1) - t * BN - 4 * g);
     }
+    // The reference moves up by d.  P*V of the tiles in front of this one is complete at the end of the iteration only, where
+    // `lower` brings it and the row sum to the new reference.
+    float d = 0.f;
+    auto raise = [&](float largest) DA_INLINE {
+      d = fmaxf(pair_max(largest), 0.f);
+      m[0] += d;
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s_cur[0][kt][r] -= d;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) negm[0][r] = -m[0];
+      asm volatile("" : "+v"(negm[0]));
+    };
+    auto lower = [&]() DA_INLINE {
+      const float alpha = fast_exp2(-d);
+      l[0] *= alpha;
+#pragma unroll
+      for (int tt = 0; tt < NOT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[0][tt][r] *= alpha;
+    };
+    bool moved = false;
+    if constexpr (kWatching) {
+      const float largest = lane_max(s_cur[0]);
+      moved = __any(largest > kRescaleWatch);
+      if (moved) raise(largest);
+    }
     u32x4 pn[NKK];
     float rs = 0.f;
     const unsigned hwin = DROP ? dropout_window<BN / 2>(dkey, hrow + (unsigned)(t * (BN / 2)), hlow) : 0u;
     unsigned word_a = 0, word_b = 0;
-    auto pair_of = [&](int e) {      // registers 2 (e % 8) and the next of 32-key block e / 8
+    auto pair_of = [&](int e) DA_INLINE {      // registers 2 (e % 8) and the next of 32-key block e / 8
       const int kt = e / 8, r = 2 * (e % 8);
       h2 e2;
       e2[0] = (half_t)fast_exp2(s_cur[0][kt][r]);
@@ -411,47 +458,37 @@ void fwd_kernel(FwdParams p) {
       pn[kt * 2 + r / 8][(r % 8) / 2] = w2;
     };
     constexpr int NV = kOpening ? 0 : NPV, NM = NV + NSC;     // matrix products of an iteration
-    int npv = 0, nsc = 0, ne = 0;
-#pragma unroll
-    for (int c = 0; c < NM; ++c) {
+    each<NM>([&](auto c_tag) DA_INLINE {
       // products alternate NV : NSC
-      const int pv_due = (c + 1) * NV / NM;
-      if (npv < pv_due) {
-        const int i = npv++;
-        if (i + VA < NPV) vfr[i + VA] = vt_frag_at(i + VA, VOFF);
-        o[0][i % NOT] = mfma32(vfr[i], __builtin_bit_cast(h8, pw[i / NOT]), o[0][i % NOT]);
+      constexpr int c = decltype(c_tag)::value, npv = c * NV / NM, nsc = c - npv;
+      if constexpr ((c + 1) * NV / NM > npv) {
+        if constexpr (npv + VA < NPV) vfr[npv + VA] = vt_frag_at(npv + VA, VOFF);
+        o[0][npv % NOT] = mfma32(vfr[npv], __builtin_bit_cast(h8, pw[npv / NOT]), o[0][npv % NOT]);
       } else {
-        const int i = nsc++;
-        if (i + KA < NSC) ka[i + KA] = k_frag_at(i + KA, KOFF);
-        const int kt = i / NKS, ks = i % NKS;
-        if (ks == 0) s_nxt[0][kt] = negm[0];
-        s_nxt[0][kt] = mfma32(ka[i], qf[0][ks], s_nxt[0][kt]);
+        if constexpr (nsc + KA < NSC) ka[nsc + KA] = k_frag_at(nsc + KA, KOFF);
+        constexpr int kt = nsc / NKS, ks = nsc % NKS;
+        if constexpr (ks == 0) s_nxt[0][kt] = negm[0];
+        s_nxt[0][kt] = mfma32(ka[nsc], qf[0][ks], s_nxt[0][kt]);
       }
-      if (c == NM / 4) load_k2(tk, KP, tail);
-      if (!kOpening && c == NM / 2) load_va(tv, VP, tail);
-      if (!kOpening && c == 3 * NM / 4) load_vb(tv, VP, tail);
-      const int e1 = (c + 1) * (8 * NKT) / NM;
-      while (ne < e1) pair_of(ne++);
+      if constexpr (c == NM / 4) load_k2(tk, KP, tail);
+      if constexpr (!kOpening && c == NM / 2) load_va(tv, VP, tail);
+      if constexpr (!kOpening && c == 3 * NM / 4) load_vb(tv, VP, tail);
+#pragma unroll
+      for (int e = c * (8 * NKT) / NM; e < (c + 1) * (8 * NKT) / NM; ++e) pair_of(e);
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
     if constexpr (!(POS & 1)) request_first(((POS + 2) % 4) * C::KBUF_BYTES, POS * C::VBUF_BYTES);
     __builtin_amdgcn_sched_barrier(0);
-    if (__any(rs > kRescaleSum)) {
-      const float d = fmaxf(pair_max(lane_max(s_cur[0])), 0.f);
-      const float alpha = fast_exp2(-d);
-      m[0] += d;
-      l[0] *= alpha;
-#pragma unroll
-      for (int tt = 0; tt < NOT; ++tt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[0][tt][r] *= alpha;
+    if constexpr (kWatching) {
+      if (moved) lower();
+    } else if (__builtin_expect(__any(rs > kRescaleSum), 0)) {
+      ++moves;
+      raise(lane_max(s_cur[0]));
 #pragma unroll
       for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) { s_cur[0][kt][r] -= d; s_nxt[0][kt][r] -= d; }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) negm[0][r] = -m[0];
-      asm volatile("" : "+v"(negm[0]));
+        for (int r = 0; r < 16; ++r) s_nxt[0][kt][r] -= d;
+      lower();
       rs = 0.f;
 #pragma unroll
       for (int e = 0; e < 8 * NKT; ++e) pair_of(e);
@@ -474,7 +511,7 @@ void fwd_kernel(FwdParams p) {
   // buffer POS+2 (tile t-2, likewise), all modulo NBUF.
   // `tail`: the iteration can meet tiles that reach past the last real key (their copies are clamped and, in
   // the padded variant, their keys masked); iterations that cannot are compiled without those tests.
-  auto iteration = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) {
+  auto iteration = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) DA_INLINE {
     constexpr int POS = decltype(pos_tag)::value;
     constexpr int KR = (POS + 1) % 4, KP = (POS + 3) % 4, VR = POS, VP = (POS + 2) % 4;
     // Asynchronous prefetch straight into LDS, two iterations ahead: K tile t+3 and V tile t+2.
@@ -623,24 +660,25 @@ void fwd_kernel(FwdParams p) {
     }
   };
 
-  auto one = [&](int t, auto pos_tag, auto tail, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT], auto opening) {
-    if constexpr (kLate) late_iteration(t, pos_tag, tail, opening, s_cur, s_nxt);
+  auto one = [&](int t, auto pos_tag, auto tail, auto kind, f16v (&s_cur)[QS][NKT], f16v (&s_nxt)[QS][NKT]) DA_INLINE {
+    if constexpr (kLate) late_iteration(t, pos_tag, tail, kind, s_cur, s_nxt);
     else iteration(t, pos_tag, tail, s_cur, s_nxt);
   };
-  constexpr std::true_type opens{};
-  constexpr std::false_type follows{};
+  constexpr std::integral_constant<int, kOpens> opens{};
+  constexpr std::integral_constant<int, kFollows> follows{};
+  constexpr std::integral_constant<int, kWatches> watches{};
   // the tile count is even (N is a multiple of 128, tiles are at most 64 keys)
   int t = 0;
   if (head_half) {
-    one(0, std::integral_constant<int, 2>{}, with_tail, s_a, s_b, opens);
-    one(1, std::integral_constant<int, 3>{}, with_tail, s_b, s_a, follows);
+    one(0, std::integral_constant<int, 2>{}, with_tail, opens, s_a, s_b);
+    one(1, std::integral_constant<int, 3>{}, with_tail, follows, s_b, s_a);
     t = 2;
   }
-  auto turn = [&](int t, auto tail) {
-    one(t, std::integral_constant<int, 0>{}, tail, s_a, s_b, follows);
-    one(t + 1, std::integral_constant<int, 1>{}, tail, s_b, s_a, follows);
-    one(t + 2, std::integral_constant<int, 2>{}, tail, s_a, s_b, follows);
-    one(t + 3, std::integral_constant<int, 3>{}, tail, s_b, s_a, follows);
+  auto turn = [&](int t, auto tail, auto kind) DA_INLINE {
+    one(t, std::integral_constant<int, 0>{}, tail, kind, s_a, s_b);
+    one(t + 1, std::integral_constant<int, 1>{}, tail, kind, s_b, s_a);
+    one(t + 2, std::integral_constant<int, 2>{}, tail, kind, s_a, s_b);
+    one(t + 3, std::integral_constant<int, 3>{}, tail, kind, s_b, s_a);
   };
   if constexpr (TAIL) {
     // A mask concerns the last tiles only: with padding, an iteration copies K tile t+3, so the first one that can
@@ -649,10 +687,16 @@ void fwd_kernel(FwdParams p) {
     int t_tail = CAUSAL ? qt * (BM / BN) : p.N / BN;
     if (p.n_keys < p.N) t_tail = min(t_tail, p.n_keys / BN - 3);
 #pragma nounroll
-    for (; t + 4 <= t_tail; t += 4) turn(t, no_tail);
+    for (; t + 4 <= t_tail && !(kWatch && moves >= kWatchMoves); t += 4) { moves = 0; turn(t, no_tail, follows); }
   }
 #pragma nounroll
-  for (; t < n_tiles; t += 4) turn(t, with_tail);
+  for (; t < n_tiles && !(kWatch && moves >= kWatchMoves); t += 4) { moves = 0; turn(t, with_tail, follows); }
+  if constexpr (kWatch) {
+    if (__builtin_expect(moves >= kWatchMoves, 0)) {
+#pragma nounroll
+      for (; t < n_tiles; t += 4) turn(t, with_tail, watches);
+    }
+  }
 
   if constexpr (kLate) {
     // the last tile's product
