@@ -31,7 +31,8 @@ def test_large_logits(scale, D):
 
 
 def test_growing_row_maximum():
-    # keys sorted so that every later tile raises the row maximum: the rescale path runs on every tile
+    # keys sorted so that every later tile raises the row maximum.  The reference moves at some of the eight tiles, by either of the
+    # forward's criteria (at every tile it does in test_gpu_moving_reference.py).
     q1, q2, k1, k2, v, dy = make_inputs(1, 1, 512, 64, seed=42)
     ramp = torch.linspace(0.2, 3.0, 512).reshape(1, 1, 512, 1)
     k1 = (k1.abs() * ramp).half(); q1 = q1.abs().half()

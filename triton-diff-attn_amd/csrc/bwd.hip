@@ -223,9 +223,11 @@ struct DkvCfg {
   // is within the 64 KiB reach of an LDS instruction's immediate offset from one per-lane address
   static constexpr int QBUF = 2 * Q_TILE * 2, XBUF = X_TILE * 2, SBUF = STAT * 2;   // one ring buffer of Q1|Q2, dX, statistics
   // A staged tile is read from half a step before its first sub-tile is scored until half a step after its last one was,
-  // while another is being fetched.  The ring has four so that the position of every step is known at compile time (the loop is
-  // unrolled over one turn of the ring, and the number of steps is a multiple of four): every LDS address is then a per-lane
-  // register plus an immediate offset, with no address arithmetic inside the loop.
+  // while another is being fetched.  With one sub-tile per tile that takes the ring's four buffers: behind its meeting, step i reads tiles i
+  // and i+1 and the first fragments of i+2, and tile i+3 is on its way into the buffer of i-1.  With two sub-tiles per tile three would
+  // do.  The position of every step is known at compile time (the loop is unrolled over one turn of the ring, and the number
+  // of steps is a multiple of four): every LDS address is then a per-lane register plus an immediate offset, with no address
+  // arithmetic inside the loop.
   static constexpr int NBUF = 4;
   static constexpr int XBASE = NBUF * QBUF, SBASE = XBASE + NBUF * XBUF;
   static_assert(NBUF * QBUF <= 65536 && NBUF * XBUF <= 65536, "immediate offsets reach every buffer");
@@ -587,8 +589,9 @@ __device__ __forceinline__ void dkdv_block(const BwdParams& p, int wg, int n_wg,
   // meets; it is requested behind the meeting of the step before (a tile of two sub-tiles: of two steps before).  When a step
   // requested all that at its own start, and the workgroup met there, behind copies requested as late as a quarter of a step before,
   // its products began 300 cycles late and a wave of the D = 128 kernel waited for 31 % of its time: us, key blocks alone, before ->
-  // now, fp16: B2 H32 N4096 D128 3000 -> 2610, B4 H32 N2048 D64 687 -> 671, B2 H16 N8192 D32 1439 -> 1423; with the query blocks
-  // in one grid B8 H32 N4096 D128 18.1 -> 16.7 ms, B1 H8 N2048 D64 79 -> 75 us, B2 H16 N512 D32 causal 18.1 -> 17.2.
+  // now, fp16: B2 H32 N4096 D128 3000 -> 2610, B4 H32 N2048 D64 687 -> 671, B2 H16 N8192 D32 1439 -> 1423 and, on another card,
+  // 1365 -> 1388, which is even; with the query blocks in one grid B8 H32 N4096 D128 18.1 -> 16.7 ms, B1 H8 N2048 D64 79 -> 75 us, B2 H16
+  // N512 D32 causal 18.1 -> 17.2.
   static_assert(NPROD % 16 == 0 || 16 % NPROD == 0, "rows are spread evenly over the products");
   constexpr int AHEAD = kShort ? 1 : 3;        // B fragments requested ahead of their product (4: no faster)
   // What a step finds requested by the step in front of it: the first fragments of its products and the statistics of its
@@ -825,10 +828,10 @@ struct DqCfg {
   static constexpr int STAGE = 2 * K_TILE + V_TILE;
   // A ring of four buffers whose position is a compile-time constant in every iteration (the loop body is one
   // turn of the ring), laid out by tile kind so that an instruction's immediate offset reaches every buffer.
-  // Tiles are fetched two iterations ahead.  With a barrier per tile three buffers would do; four let the
-  // workgroup meet every second tile only (a tile's buffer is refilled two tiles after it was read, which is
-  // always past one barrier), so the two waves of a SIMD, which leave a barrier in step, have twice as long to
-  // drift apart and overlap one's matrix products with the other's element-wise work.  Measured in one GPU call
+  // Tiles are fetched two iterations ahead, in the pipelined form three, which takes the four buffers.  In the other form with a
+  // barrier per tile three would do; four let the workgroup meet every second tile only (a tile's buffer is refilled two tiles
+  // after it was read, which is always past one barrier), so the two waves of a SIMD, which leave a barrier in step, have twice
+  // as long to drift apart and overlap one's matrix products with the other's element-wise work.  Measured in one GPU call
   // against a barrier per tile: 3.6 % faster at D = 128, 0.8 % at D = 32, 2 % slower at D = 64.
   static constexpr bool PAIR = (D != 64);      // a barrier every second tile
   static constexpr int NBUF = 4;

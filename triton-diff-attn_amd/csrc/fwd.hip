@@ -19,7 +19,6 @@
 
 namespace DA_NS {
 
-
 // SMALL: 64 query rows per workgroup (four waves), for problems whose 128-row blocks leave much of the chip idle and
 // for the D = 128 instantiations with dropout, which do not fit the register budget of two waves per SIMD.
 template <int D, bool SMALL = false>
@@ -41,9 +40,10 @@ struct FwdCfg {
   static constexpr int K_TILE = BN * D;            // halfs, one stream (swizzled, unpadded)
   static constexpr int V_TILE = BN * DV;
   static constexpr int K_BUF = 2 * K_TILE;         // K1 and K2 of one tile
-  // Ring depth.  Tiles are fetched two iterations ahead, which takes three buffers; there are four so that
-  // the loop can be unrolled over one turn of the ring with every buffer known at compile time: an LDS
-  // address is then a per-lane register plus an immediate offset, with no arithmetic inside the loop.
+  // Ring depth.  The loop is unrolled over one turn of the ring with every buffer known at compile time: an LDS address is then a
+  // per-lane register plus an immediate offset, with no arithmetic inside the loop.  Where the workgroup meets every second tile all
+  // four buffers are in use (in one iteration and the next, K tiles t+1 and t+2 are read while t+3 and t+4 arrive, V tiles t-1 and t, or t and
+  // t+1, while the next two do); where it meets every tile three would do.
   static constexpr int NBUF = 4;
   // A barrier every second tile instead of every tile (the ring allows it): measured in one GPU call,
   // 3.3 % faster at D = 32, 3 % slower at D = 64 and 5 % slower at D = 128.  In the 64-row workgroups at D = 64, whose waves have a
@@ -256,8 +256,8 @@ void fwd_kernel(FwdParams p) {
   };
   // How many of the next tile's score products are issued ahead of the row maxima of this one; the rest follow
   // the reference update and run under the first exponentials, which have no other matrix work beside them.
-  // The split is between 32-key tiles.  Measured against all of them ahead, inside one GPU call each: the
-  // first of two tiles ahead -2.5 % at D = 64 (0.442 -> 0.432 ms) and -1 % at D = 32; none ahead the same at
+  // The split is between 32-key tiles (D = 32 has late_iteration and no split).  Measured against all of them ahead, inside one GPU
+  // call each: the first of two tiles ahead -2.5 % at D = 64 (0.442 -> 0.432 ms); none ahead the same at
   // D = 64 and +0.7 % at D = 128; a D = 128 tile is a single 32-key tile, and splitting it in the middle
   // of its k-steps cost 1.5 %, so it stays whole and ahead.
   constexpr int SC_EARLY = DROP ? NSC : ((NKT + 1) / 2) * NKS;
