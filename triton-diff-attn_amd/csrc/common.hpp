@@ -287,19 +287,28 @@ struct AsyncTile {
   // The same copy for a tile whose global rows end at `last_row` (relative to the tile's first row; it may be
   // negative when the whole tile lies past the end): a row beyond it reads row `last_row` instead, so no
   // address past the tensor's last row is formed and the LDS tile holds finite data everywhere.  For the last tiles of a sequence
-  // whose length is not a multiple of the tile; a tile in front of them is copied as it is.  Costs a minimum and an addition per piece.
-  template <int K0 = 0, int K1 = PER>
+  // whose length is not a multiple of the tile; a tile in front of them is copied as it is.  Costs a minimum and an addition per piece
+  // beside the lane's way down, which is formed once.  LEAN: where no register holds that between the copies, the way back up is formed
+  // instead (the masked 128-row forward at D = 128, bf16, us, that way -> with the way down: H32 N3072 causal 216.1 -> 217.2, N3001 372.9 ->
+  // 374.2; its 64-row one, which has the registers, H16 N500 22.8 -> 22.4, H4 N3001 causal 79.9 -> 79.4).
+  template <int K0 = 0, int K1 = PER, bool LEAN = false>
   __device__ static __forceinline__ void issue_clamped(const half_t* gtile, lds_half* lds_tile, int wave, int lane, unsigned off0,
                                                        int stride, int last_row) {
-    const int row_bytes = stride * 2;
-    const unsigned down = (unsigned)((lane / CPR) * row_bytes);        // the lane's row inside a piece, in bytes
+    const int row = lane / CPR, row_bytes = stride * 2;                // the lane's row inside a piece
+    const unsigned down = (unsigned)(row * row_bytes);
 #pragma unroll
     for (int k = K0; k < K1; ++k) {
       const int inst = wave + NW * k;
       if (NINST % NW == 0 || inst < NINST) {
         const da_abi::PieceRows at = da_abi::clamp_piece(inst * RPP, last_row, RPP);
-        const unsigned most = (unsigned)(at.most * row_bytes);
-        const unsigned off = ((kOneOffset ? off0 : lane_off(inst, lane, stride)) - down) + (down < most ? down : most);
+        unsigned off = kOneOffset ? off0 : lane_off(inst, lane, stride);
+        if constexpr (LEAN) {
+          const int room = last_row - at.base, back = row > room ? row - room : 0;      // as with at.most: a lane's row is in the piece
+          off -= (unsigned)(back * stride * 2);
+        } else {
+          const unsigned most = (unsigned)(at.most * row_bytes);
+          off = (off - down) + (down < most ? down : most);
+        }
         async_copy16(gtile + (long long)at.base * stride, off, lds_tile + inst * 512);
       }
     }

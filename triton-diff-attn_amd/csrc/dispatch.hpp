@@ -8,7 +8,9 @@ constexpr int kNumCU = 256;
 
 // Whether a forward runs in 64-row, four-wave workgroups instead of 128-row ones.  (The reference autotunes its tiles per
 // (N, D, Dv), src/kernel.py:12-19; there is no tuning state here.)  `n`: the padded sequence length, a multiple of 128;
-// `blocks`: B*H*n/128.  Figures: us of a launch, 128-row -> 64-row.
+// `blocks`: B*H*n/128.  Figures: us of a launch, 128-row -> 64-row.  (The lines were taken before P*V ran one tile behind in D = 32 and in
+// 64-row blocks at D = 64.  Measured again since, at 52 pairs about them, each takes the side that is ahead: D32 B1 H9 N2048 26.4 -> 27.3,
+// 256 causal blocks of N = 128 8.0 -> 7.8; D64 B1 H8 N2048 39.2 -> 30.1, B1 H9 39.9 -> 53.1.)
 // Blocks of one length: up to 128 of them, i.e. where 128-row blocks leave half of the chip idle (bf16, D <= 64, B1 H8
 // N2000 D64 39.6 -> 33.8, with dropout 57.7 -> 41.1; D32 29.3 -> 23.3; fp16, B1 H8 N2048 D128 67.4 -> 58.5).  The rings of a
 // D >= 64 workgroup fill a CU's LDS whatever its rows, so from 129 on the halves take a second round (bf16, B1 H9 N2048 D64
@@ -40,7 +42,8 @@ constexpr bool fwd_64_rows(int d, bool causal, int n, long long blocks) {
 // it is a matter of rounds.  Microseconds per round of 256 workgroups at N = 2048, D = 64, which scale alike with N and D:
 // 79 for key blocks, 64 for query blocks of the one grid, 109 for 256-row blocks of the dQ kernel; a grid that is dealt from
 // one list ends with a partial round of 25.  Measured over N = 128 ... 4096 and 192 ... 1280 blocks: gains of up to 24 % on
-// the line's near side, up to 6 % on its far side, 7 % in padded sequences.
+// the line's near side, up to 6 % on its far side, 7 % in padded sequences; again with the key blocks' requests across steps, at 37 pairs
+// about the lines: two launches over one grid within 0.04 of what it was.
 // Causal blocks differ in length and fill the rounds by themselves: the one grid is faster below 576 blocks
 // (by 5 % at 512, 40 % at 256) and slower above 640 (by 2-5 %).  Those of a unit of one or two blocks hardly differ: at N = 256
 // the rounds decide as without a mask (us of the whole backward, two launches -> one grid: D64 512 blocks 71 -> 74, 640

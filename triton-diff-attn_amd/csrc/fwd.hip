@@ -184,25 +184,27 @@ void fwd_kernel(FwdParams p) {
   // 7.1, H8 N1000 18.4 -> 17.9; with dropout 8.6 -> 8.1.
   auto load_k1 = [&](int tk, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tk + 1) * BN > p.n_keys))
-      KTile::issue_clamped(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, tail_lane(), k_off, qk_n, p.n_keys - 1 - tk * BN);
+      KTile::template issue_clamped<0, KTile::PER, kLean>(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, tail_lane(), k_off, qk_n,
+                                                          p.n_keys - 1 - tk * BN);
     else
       KTile::issue_at(gk1 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF, wave, lane, k_off, qk_n);
   };
   auto load_k2 = [&](int tk, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tk + 1) * BN > p.n_keys))
-      KTile::issue_clamped(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, tail_lane(), k_off, qk_n, p.n_keys - 1 - tk * BN);
+      KTile::template issue_clamped<0, KTile::PER, kLean>(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, tail_lane(), k_off,
+                                                          qk_n, p.n_keys - 1 - tk * BN);
     else
       KTile::issue_at(gk2 + (size_t)tk * BN * qk_n, sKbuf + buf * C::K_BUF + C::K_TILE, wave, lane, k_off, qk_n);
   };
   auto load_va = [&](int tv, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tv + 1) * BN > p.n_keys))
-      VTile::template issue_clamped<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
+      VTile::template issue_clamped<0, VH, kLean>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
     else
       VTile::template issue_at<0, VH>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n);
   };
   auto load_vb = [&](int tv, int buf, auto tail) DA_INLINE {
     if (TAIL && decltype(tail)::value && (kLean || kLate || (tv + 1) * BN > p.n_keys))
-      VTile::template issue_clamped<VH, VTile::PER>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
+      VTile::template issue_clamped<VH, VTile::PER, kLean>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, tail_lane(), v_off, v_n, p.n_keys - 1 - tv * BN);
     else
       VTile::template issue_at<VH, VTile::PER>(gv + (size_t)tv * BN * v_n, sVbuf + buf * C::V_TILE, wave, lane, v_off, v_n);
   };
